@@ -716,45 +716,42 @@ int launch_decode(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t*
 }
 
 // ---- projection launcher -----------------------------------------------------------
-template <int D, int DH, int NKS>
-int launch_project_rows(const rfa::half_t* x, const rfa::ProjectArgs& pa, const rfa::half_t* wf, int R, int H, int np,
-                        float scale, hipStream_t st) {
-    // rows of x in registers; split the H * np pairs of a row tile over enough groups to fill the CUs
-    using Cfg = rfa::ProjectRowCfg<D, DH, NKS>;
-    auto kern = rfa::k_project_phi_rows<D, DH, NKS>;
+template <int D, int DH, int BM>
+int launch_project_tiles(const rfa::half_t* x, const rfa::ProjectArgs& pa, const rfa::half_t* wf, int R, int E, int H,
+                         int np, float scale, hipStream_t st) {
+    using Cfg = rfa::ProjectCfg<D, DH, BM>;
+    auto kern = rfa::k_project_phi<D, DH, BM>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
-    const int nrt = (R + Cfg::BM - 1) / Cfg::BM;
-    const int pairs = H * np;
-    int ngroups = (device_cus() + nrt - 1) / nrt;
-    if (ngroups > pairs) ngroups = pairs;
-    const int ppg = (pairs + ngroups - 1) / ngroups;
-    ngroups = (pairs + ppg - 1) / ppg;
-    const int64_t grid = (int64_t)8 * ((nrt + 7) / 8) * ngroups;
-    RFA_LAUNCH(PROJECT_PHI, kern, dim3((unsigned)grid), dim3(rfa::kThreads), Cfg::kLds, st, x, pa, wf, R, H, np, ngroups,
-               ppg, scale);
+    const int tiles_c = (H * np + Cfg::PPT - 1) / Cfg::PPT;
+    const int64_t tiles = (int64_t)((R + BM - 1) / BM) * tiles_c;
+    const int64_t grid = rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds);
+    RFA_LAUNCH(PROJECT_PHI, kern, dim3((unsigned)grid), dim3(rfa::kThreads), Cfg::kLds, st, x, pa, wf, R, E, H, np, tiles_c,
+               (int)tiles, scale);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
 
+// Rows per tile.  256 rows read the fewest operand bytes per product; a lower tile has more workgroups
+// and a shorter epilogue, but stages w' for fewer rows: 64 until 128 gives every CU a tile, then 128
+// until the busiest CU would have 5/3 as many tiles of 128 as of 256 (5/4 where w' is the larger
+// operand, D > d).  Measured, us for 256 / 128 / 64 rows (tiles of 256 in brackets):
+// 8192 x 512 -> 3 x 512 (384) 30.1 / 28.2 / 35; 16384 x 512 -> 2 x 512 (512) 33.3 / 36.7 / 43;
+// 8192 x 1024 -> 3 x 1024 (768) 82.6 / 88 / 121; 4096 x 768 -> 3 x 768, D 128 (288) 35.2 / 39.7 / 49;
+// 8192 x 512 -> 512 (128) 19.9 / 14.3 / 14.4; 1024 x 1024 -> 3 x 1024 (96) 28.2 / 20.4 / 19.6;
+// 512 x 512 -> 3 x 512 (24) 18.0 / 12.1 / 9.6; 160 x 512 -> 512 (4) 17.0 / 11.3 / 8.5.
 template <int D, int DH>
 int launch_project_phi(const rfa::half_t* x, const rfa::ProjectArgs& pa, const rfa::half_t* wf, int R, int E, int H,
                        int np, float scale, hipStream_t st) {
-    if constexpr (DH == 64 && D <= 64) {
-        if (tune::get(tune::PROJECT_STREAMING) <= 0) {
-            if (E == 128) return launch_project_rows<D, DH, 4>(x, pa, wf, R, H, np, scale, st);
-            if (E == 256) return launch_project_rows<D, DH, 8>(x, pa, wf, R, H, np, scale, st);
-            if (E == 384) return launch_project_rows<D, DH, 12>(x, pa, wf, R, H, np, scale, st);
-            if (E == 512) return launch_project_rows<D, DH, 16>(x, pa, wf, R, H, np, scale, st);
-        }
-    }
-    using Cfg = rfa::ProjectCfg<D, DH>;
-    auto kern = rfa::k_project_phi<D, DH>;
-    if (int rc = set_lds(kern, Cfg::kLds)) return rc;
-    const int nrt = (R + Cfg::BM - 1) / Cfg::BM;
-    const int64_t grid = (int64_t)8 * ((nrt + 7) / 8) * H * np;
-    RFA_LAUNCH(PROJECT_PHI, kern, dim3((unsigned)grid), dim3(rfa::kThreads), Cfg::kLds, st, x, pa, wf, R, E, H, np, scale);
-    RFA_HIP_TRY(hipGetLastError());
-    return RFA_OK;
+    const int knob = tune::get(tune::PROJECT_STREAMING);
+    const int64_t tiles_c = ((int64_t)H * np * DH + 127) / 128;
+    const int64_t cus = device_cus(), t128 = (int64_t)((R + 127) / 128) * tiles_c, t256 = (int64_t)((R + 255) / 256) * tiles_c;
+    int rows = t128 < cus ? 64 : 128;
+    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= (D > DH ? 4 : 3) * ((t128 + cus - 1) / cus)) rows = 256;
+    if (knob >= 0) rows = knob == 0 ? 64 : (knob == 1 ? 256 : 128);
+    if (E > (1 << 23)) rows = 64;      // the rows of a tile are addressed with 32-bit byte offsets
+    if (rows == 256) return launch_project_tiles<D, DH, 256>(x, pa, wf, R, E, H, np, scale, st);
+    if (rows == 128) return launch_project_tiles<D, DH, 128>(x, pa, wf, R, E, H, np, scale, st);
+    return launch_project_tiles<D, DH, 64>(x, pa, wf, R, E, H, np, scale, st);
 }
 
 // ---- weight-gradient plan -------------------------------------------------------------
@@ -1777,7 +1774,7 @@ int rfa_project_feature_map(const void* x, const void* const* weights, const voi
     if (R == 0) return RFA_OK;
     if (!x || !weights || !y) return fail(RFA_ERR_NULL_POINTER, "rfa_project_feature_map: NULL tensor pointer");
     if (!aligned16(x)) return fail(RFA_ERR_ALIGNMENT, "rfa_project_feature_map: tensors must be 16-byte aligned");
-    if ((int64_t)8 * ((R + 127) / 128 + 7) / 8 * H * np > (int64_t(1) << 31) - 1)
+    if ((int64_t)((R + 63) / 64) * H * np > (int64_t(1) << 31) - 9 || E > (1 << 25))
         return fail(RFA_ERR_BAD_SHAPE, "rfa_project_feature_map: sizes exceed the supported range");
     rfa::ProjectArgs pa{};
     bool any_phi = false;

@@ -42,24 +42,9 @@ __device__ __forceinline__ void wave_lds_order() {
     asm volatile("" ::: "memory");
 }
 
-// Copy this wave's 16 staged rows (F halves each, row stride ld in LDS) to global rows
-// r0 .. r0+15 of a [R, H, F] tensor at head h: every store instruction writes whole rows,
-// 16 bytes per lane.
-template <int F>
-__device__ __forceinline__ void wave_rows_s2g(const half_t* Ss, int ld, half_t* __restrict__ dst, int r0, int R,
-                                              int H, int h, int lane) {
-    constexpr int PPR = F / 8;        // 16-byte pieces per row
-    constexpr int RPI = 64 / PPR;     // rows per instruction
-    static_assert(PPR <= 64 && 64 % PPR == 0, "row too long for one wave");
-#pragma unroll
-    for (int k = 0; k < 16 / RPI; ++k) {
-        const int lr = k * RPI + lane / PPR, pc = lane % PPR;
-        const uint4 val = *reinterpret_cast<const uint4*>(Ss + lr * ld + pc * 8);
-        if (r0 + lr < R) *reinterpret_cast<uint4*>(dst + ((int64_t)(r0 + lr) * H + h) * F + pc * 8) = val;
-    }
-}
-
-// Same, for a destination whose rows lie `rs` halves apart: dst points at this head's first column.
+// Copy this wave's 16 staged rows (F halves each, row stride ld in LDS) to global rows r0 .. r0+15 that
+// lie `rs` halves apart (dst points at this head's first column): every store instruction writes
+// whole rows, 16 bytes per lane.
 template <int F>
 __device__ __forceinline__ void wave_rows_s2g_strided(const half_t* Ss, int ld, half_t* __restrict__ dst, int64_t rs,
                                                       int r0, int R, int lane) {

@@ -35,67 +35,68 @@ __device__ __forceinline__ T pick3(T const (&a)[kMaxProjections], int p) {
     return p == 0 ? a[0] : (p == 1 ? a[1] : a[2]);
 }
 
-template <int D, int DH>
+template <int D, int DH, int BM_>
 struct ProjectCfg {
-    static_assert(D % 32 == 0 && DH % 64 == 0, "D multiple of 32, DH multiple of 64");
-    static constexpr int BM = 128;                 // rows of x per workgroup
-    static constexpr int BK = 64;                  // contraction step
-    static constexpr int LDX = BK + lds_pad(BK);
+    static_assert(D % 32 == 0 && (DH == 64 || DH == 128), "D multiple of 32, DH 64 or 128");
+    static constexpr int BM = BM_;                 // rows of x per workgroup
+    static constexpr int BN = 128;                 // output columns: one head of 128 or two of 64
+    static constexpr int BK = 32;                  // contraction step: one MFMA deep
+    static constexpr int kStages = 3;              // 4 to 6 measured no faster at any size
+    static constexpr int PPT = BN / DH;            // heads per tile
+    static constexpr int WR = 4 / PPT;             // waves along the rows; a wave owns whole heads
+    static constexpr int RW = BM / WR;             // rows of a wave
+    static constexpr int NR = RW / 16, NC = DH / 16;
+    static constexpr int XI = BM / 64, WI = BN / 64;    // 1 KiB pieces of a stage per wave: x, W
+    static constexpr int kStageHalves = (BM + BN) * BK;
     static constexpr int LDW = DH + lds_pad(DH);   // rows of w'
-    static constexpr int LDP = (2 * D > DH ? 2 * D : DH) + 16;   // staging rows of y / phi
-    static constexpr int kStageHalves = (BM + DH) * LDX;         // x tile, then W tile
-    static constexpr size_t kLoopLds = (size_t)2 * kStageHalves * 2;
-    static constexpr size_t kEpiLds = (size_t)(D * LDW + 4 * 16 * LDP) * 2;
+    static constexpr size_t kLoopLds = (size_t)kStages * kStageHalves * 2;
+    static constexpr size_t kEpiLds = (size_t)PPT * D * LDW * 2;
     static constexpr size_t kLds = kLoopLds > kEpiLds ? kLoopLds : kEpiLds;
+    static_assert(kLds <= 80 * 1024, "two workgroups per CU");
 };
 
-// One contraction step of the operands: [rows][BK] sub-tiles of x (clamped to the last row) and
-// of W, 16-byte pieces, piece -> (row, 16-byte column); global -> registers -> LDS.
-template <int XP, int WP, int BK>
-__device__ __forceinline__ void project_load_stage(uint4 (&xr)[XP], uint4 (&wr)[WP], const half_t* __restrict__ x,
-                                                   const half_t* __restrict__ wp, int row0, int R, int E, int k0,
-                                                   int tid) {
-#pragma unroll
-    for (int it = 0; it < XP; ++it) {
-        const int pc = tid + kThreads * it;
-        const int r = min(row0 + pc / (BK / 8), R - 1);
-        xr[it] = *reinterpret_cast<const uint4*>(x + (int64_t)r * E + k0 + (pc % (BK / 8)) * 8);
-    }
-#pragma unroll
-    for (int it = 0; it < WP; ++it) {
-        const int pc = tid + kThreads * it;
-        wr[it] = *reinterpret_cast<const uint4*>(wp + (int64_t)(pc / (BK / 8)) * E + k0 + (pc % (BK / 8)) * 8);
-    }
+// 64 lanes x 16 bytes, global -> LDS without registers: lane l's bytes land at lds + 16 l
+__device__ __forceinline__ void dma16(const char* g, half_t* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
-template <int XP, int WP, int BK, int BM, int LDX>
-__device__ __forceinline__ void project_store_stage(const uint4 (&xr)[XP], const uint4 (&wr)[WP], half_t* Xs, int tid) {
-    half_t* Wsm = Xs + BM * LDX;
-#pragma unroll
-    for (int it = 0; it < XP; ++it) {
-        const int pc = tid + kThreads * it;
-        *reinterpret_cast<uint4*>(Xs + (pc / (BK / 8)) * LDX + (pc % (BK / 8)) * 8) = xr[it];
-    }
-#pragma unroll
-    for (int it = 0; it < WP; ++it) {
-        const int pc = tid + kThreads * it;
-        *reinterpret_cast<uint4*>(Wsm + (pc / (BK / 8)) * LDX + (pc % (BK / 8)) * 8) = wr[it];
-    }
+// All but the last N direct loads of this wave have landed and its LDS reads are done; then the
+// workgroup barrier: everyone's share of the stage is in place, the stage before it is free.
+template <int N>
+__device__ __forceinline__ void stage_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// Workgroup -> (row tile, head, projection).  Workgroups are dealt to the 8 XCDs round-robin
-// by their index; the mapping gives each XCD its own row tiles, so that the H * np workgroups
-// that share a tile of x find it in that XCD's L2, while the (small) weights are read by all.
-// grid = 8 * ceil(nrt / 8) * H * np.
-template <int D, int DH>
-__global__ __launch_bounds__(kThreads) void k_project_phi(
+// One 128-column tile (one head of 128 or two of 64) of BM rows per workgroup of four waves.
+//
+// What bounds it: at large sizes the matrix pipes and the operand path L2 -> LDS behind them; where
+// a tile has few contraction steps (E = 512: 16), its start and the stores of y and phi.  So:
+// operands go to LDS directly (no registers, no store instructions), three stages of 32 deep in a
+// ring, one barrier per step; two (256 rows) or three (128) workgroups share a CU, so that one's
+// epilogue runs under another's products.  A wave owns BM / 2 rows x 64 columns (or BM / 4 x 128):
+// with 256 rows 12 operand reads for 32 MFMAs, 48 KB of LDS traffic per 512 clocks of the matrix pipes.
+//
+// Measured (us; q, k, v projections with phi(q), phi(k); before: rows of x in registers for E <= 512,
+// a register-staged two-buffer loop otherwise):
+//   8192 rows, E 512, 8 heads of 64, D 64       42.1 -> 28.2      8192, 1024, 8 of 128, D 128   112 -> 83
+//   32768, 1024, 16 of 64, D 64                  964 -> 304 (678 TFLOP/s)      512, 512   12.4 -> 9.6
+//
+// LDS stage: x tile [BM][32], then W tile [128][32] halves, no padding (a direct load writes 1 KiB
+// in lane order); the four 16-byte pieces of row r are stored rotated, piece c at c ^ ((r >> 2) & 3),
+// which spreads a wave's operand read (16 rows x 16 bytes per 16 lanes) over all banks.  The rows of
+// W sit in pair order (pair_pos), so that accumulator tiles 2p, 2p + 1 give lane (i, G) the 8
+// consecutive columns 32 p + 8 G of row i: y goes out in 16-byte pieces, is the operand of the
+// feature product as it stands, and phi goes out the same way; nothing passes through LDS again.
+//
+// Tiles are numbered row tile by row tile; each XCD gets a contiguous range of numbers, so that
+// the tiles that share rows of x meet in its L2.   grid = 8 * ceil(tiles / 8).
+template <int D, int DH, int BM_>
+__global__ __launch_bounds__(kThreads, 2) void k_project_phi(
     const half_t* __restrict__ x, ProjectArgs pa, const half_t* __restrict__ wf, int R, int E, int H, int np,
-    float scale) {
-    using Cfg = ProjectCfg<D, DH>;
-    constexpr int BM = Cfg::BM, BK = Cfg::BK, LDX = Cfg::LDX, LDW = Cfg::LDW, LDP = Cfg::LDP;
-    constexpr int NCT = DH / 16;                       // column tiles of the output
-    constexpr int XP = BM * BK / 8 / kThreads;         // 16-byte pieces per thread and stage: x
-    constexpr int WP = DH * BK / 8 / kThreads;         //                                      W
+    int tiles_c, int tiles, float scale) {
+    using Cfg = ProjectCfg<D, DH, BM_>;
+    constexpr int BM = Cfg::BM, BK = Cfg::BK, STAGES = Cfg::kStages, NR = Cfg::NR, NC = Cfg::NC, LDW = Cfg::LDW;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
@@ -103,311 +104,152 @@ __global__ __launch_bounds__(kThreads) void k_project_phi(
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, G = lane >> 4;
 
-    const int per_tile = H * np;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int rt_idx = xcd + 8 * (slot / per_tile);
-    const int hp = slot % per_tile;
-    const int h = hp % H, p = hp / H;
-    const int row0 = rt_idx * BM;
-    if (row0 >= R) return;                             // whole workgroup: padding of the grid
+    const int per_xcd = (tiles + kXcds - 1) / kXcds;
+    const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (tile >= tiles) return;                         // whole workgroup: padding of the grid
+    const int row0 = (tile / tiles_c) * BM;
+    const int hp0 = (tile % tiles_c) * Cfg::PPT;       // (projection, head) pairs: hp -> hp / H, hp % H
+    const int pairs = H * np;
 
-    const half_t* __restrict__ wp = pick3(pa.w, p) + (int64_t)h * DH * E;
+    // ---- direct-load addresses: wave-uniform base + 32-bit lane offset, set up once
+    const char* xbase = reinterpret_cast<const char*>(x + (int64_t)row0 * E);
+    unsigned xoff[Cfg::XI], woff[Cfg::WI];
+#pragma unroll
+    for (int it = 0; it < Cfg::XI; ++it) {
+        const int r = (wv * Cfg::XI + it) * 16 + (lane >> 2);
+        xoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(E * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+    }
+    // W rows 32 wv .. of the tile: 32-row groups never straddle a head
+    const int hp_ld = min(hp0 + 32 * wv / DH, pairs - 1);
+    const char* wbase = reinterpret_cast<const char*>(
+        pick3(pa.w, hp_ld / H) + ((int64_t)(hp_ld % H) * DH + (32 * wv) % DH) * E);
+#pragma unroll
+    for (int it = 0; it < Cfg::WI; ++it) {
+        const int r = it * 16 + (lane >> 2);           // LDS row within the group; it holds column pair_inv
+        const int c = (r & 3) | ((r & 16) >> 2) | ((r & 12) << 1);
+        woff[it] = (unsigned)c * (unsigned)(E * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+    }
+    half_t* const xdst = smem + wv * Cfg::XI * 512;
+    half_t* const wdst = smem + BM * BK + wv * Cfg::WI * 512;
+    auto load_stage = [&](int kk, int buf) {
+        const char* xb = xbase + (int64_t)kk * (BK * 2);
+        const char* wb = wbase + (int64_t)kk * (BK * 2);
+#pragma unroll
+        for (int it = 0; it < Cfg::XI; ++it) dma16(xb + xoff[it], xdst + buf * Cfg::kStageHalves + it * 512);
+#pragma unroll
+        for (int it = 0; it < Cfg::WI; ++it) dma16(wb + woff[it], wdst + buf * Cfg::kStageHalves + it * 512);
+    };
+    constexpr int kPerStage = Cfg::XI + Cfg::WI;
 
-    uint4 xr[XP], wr[WP];
-    // y^T tiles (m = output column, n = row): wave wv owns rows [32 wv, +32) of the tile
-    f4 acc[2][NCT];
+    // y^T tiles (m = output column in pair order, n = row) of this wave's rows and head
+    const int wr = wv / Cfg::PPT, wc = wv % Cfg::PPT;
+    f4 acc[NR][NC];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < NR; ++a)
 #pragma unroll
-        for (int c = 0; c < NCT; ++c) acc[a][c] = f4_zero();
+        for (int c = 0; c < NC; ++c) acc[a][c] = f4_zero();
+
+    // operand rows of this lane inside a stage: row (16 t + i), piece G
+    const int piece = (G ^ ((i >> 2) & 3)) * 8;
+    const half_t* const xop = smem + (wr * Cfg::RW + i) * BK + piece;
+    const half_t* const wop = smem + BM * BK + (wc * DH + i) * BK + piece;
 
     const int nk = E / BK;
-    project_load_stage<XP, WP, BK>(xr, wr, x, wp, row0, R, E, 0, tid);
-    project_store_stage<XP, WP, BK, BM, LDX>(xr, wr, smem, tid);
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
+    int buf = 0;
     for (int kk = 0; kk < nk; ++kk) {
-        // branch-free prefetch: the last step re-reads its own operands and stores them to the idle buffer
-        project_load_stage<XP, WP, BK>(xr, wr, x, wp, row0, R, E, min((kk + 1) * BK, E - BK), tid);
-        const half_t* Xs = smem + (kk & 1) * Cfg::kStageHalves;
-        const half_t* Wsm = Xs + BM * LDX;
+        // stage kk has landed (the STAGES - 2 after it may still be on their way), stage kk - 1 is free
+        stage_barrier<(STAGES - 2) * kPerStage>();
+        // the last steps re-request the last stage's columns into buffers nobody reads again
+        load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
+        const half_t* xs = xop + buf * Cfg::kStageHalves;
+        const half_t* wsm = wop + buf * Cfg::kStageHalves;
+        h8 wa[NC], xb[NR];
 #pragma unroll
-        for (int ks = 0; ks < BK / 32; ++ks) {
-            const h8 xb0 = row8(Xs, LDX, 32 * wv + i, 32 * ks, G);
-            const h8 xb1 = row8(Xs, LDX, 32 * wv + 16 + i, 32 * ks, G);
+        for (int c = 0; c < NC; ++c) wa[c] = *reinterpret_cast<const h8*>(wsm + c * 16 * BK);
 #pragma unroll
-            for (int ct = 0; ct < NCT; ++ct) {
-                const h8 wa = row8(Wsm, LDX, 16 * ct + i, 32 * ks, G);
-                acc[0][ct] = mfma32(wa, xb0, acc[0][ct]);
-                acc[1][ct] = mfma32(wa, xb1, acc[1][ct]);
-            }
-        }
-        project_store_stage<XP, WP, BK, BM, LDX>(xr, wr, smem + ((kk + 1) & 1) * Cfg::kStageHalves, tid);
-        __syncthreads();
+        for (int a = 0; a < NR; ++a) xb[a] = *reinterpret_cast<const h8*>(xs + a * 16 * BK);
+        __builtin_amdgcn_s_setprio(1);      // the other workgroup's loads and epilogue give way: 2 % at full size
+#pragma unroll
+        for (int a = 0; a < NR; ++a)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[a][c] = mfma32(wa[c], xb[a], acc[a][c]);
+        __builtin_amdgcn_s_setprio(0);
+        buf = buf == STAGES - 1 ? 0 : buf + 1;
     }
 
-    // ---- epilogue: the stage buffers are free now
-    half_t* Wfs = smem;                                   // w' of this head
-    half_t* Ps = smem + D * LDW + wv * 16 * LDP;          // this wave's 16 staging rows
-    half_t* phi = pick3(pa.phi, p);
-    if (phi) {
-        load_w_to_lds<D, DH>(Wfs, wf + (int64_t)h * D * DH, tid);
-        __syncthreads();
-    }
-    const half_t* bias = pick3(pa.b, p);
-    half_t* y = pick3(pa.y, p);
+    // ---- epilogue: the ring becomes the place of w' (rows in pair order)
+    stage_barrier<0>();
+    const int hp = hp0 + wc;
+    const bool live = hp < pairs;                      // an odd number of 64-wide heads leaves half a tile
+    const int hpc = live ? hp : pairs - 1;
+    const int p = hpc / H, h = hpc % H;
+    half_t* const y = pick3(pa.y, p);
+    half_t* const phi = pick3(pa.phi, p);
+    const half_t* const bias = pick3(pa.b, p);
+    if (wf) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const int r0 = row0 + 32 * wv + 16 * a;
-        h8 op[DH / 32];      // the rounded tile as the B operand of the feature projection, split slot order
+        for (int u = 0; u < Cfg::PPT; ++u) {
+            const int hu = min(hp0 + u, pairs - 1);
+            if (pick3(pa.phi, hu / H))
+                load_w_pair_order<D, DH, kThreads>(smem + u * D * LDW, wf + (int64_t)(hu % H) * D * DH, tid);
+        }
+    }
+    h8 bv[NC / 2];
+#pragma unroll
+    for (int c = 0; c < NC / 2; ++c) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bv[c][e] = (half_t)0.f;
+        if (bias) {
+            const h4* b4 = reinterpret_cast<const h4*>(bias + h * DH + 32 * c + 8 * G);    // 8-byte aligned
+            bv[c] = __builtin_shufflevector(b4[0], b4[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+    __syncthreads();
+    if (!live) return;
+    const half_t* const Wfs = smem + wc * D * LDW;
+#pragma unroll
+    for (int a = 0; a < NR; ++a) {
+        const int r = row0 + wr * Cfg::RW + 16 * a + i;
+        const int64_t at = (int64_t)r * H + h;
+        h8 op[NC / 2];       // the rounded row pieces: y as stored, and the operand of the feature product
         float ss = 0.f;
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-            f4 t = acc[a][ct];
-            if (bias) {
-                const h4 bv = *reinterpret_cast<const h4*>(bias + h * DH + 16 * ct + 4 * G);
+        for (int c = 0; c < NC / 2; ++c) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) t[e] += (float)bv[e];
-            }
-            const h4 yh = to_h4(t);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                ss += (float)yh[e] * (float)yh[e];
-                op[ct / 2][4 * (ct % 2) + e] = yh[e];
-            }
-            if (y) *reinterpret_cast<h4*>(Ps + i * LDP + 16 * ct + 4 * G) = yh;
+            for (int e = 0; e < 8; ++e) op[c][e] = (half_t)(acc[a][2 * c + e / 4][e % 4] + (float)bv[c][e]);
+            ss += dot_h8(__builtin_bit_cast(uint4, op[c]), __builtin_bit_cast(uint4, op[c]));
         }
-        if (y) {        // NULL: the caller keeps only phi(y) (no backward pass will ask for y)
-            wave_lds_order();
-            wave_rows_s2g<DH>(Ps, LDP, y, r0, R, H, h, lane);
-            wave_lds_order();
+        if (y && r < R) {    // NULL: the caller keeps only phi(y) (no backward pass will ask for y)
+#pragma unroll
+            for (int c = 0; c < NC / 2; ++c) *reinterpret_cast<h8*>(y + at * DH + 32 * c + 8 * G) = op[c];
         }
         if (phi) {
             ss = sum_over_groups(ss);
-            const float inv = 1.0f / (sqrtf(ss) + 1e-3f);
+            const float inv_turns = rcp_nr(__builtin_amdgcn_sqrtf(ss) + 1e-3f) * 0.15915494309189535f;
 #pragma unroll
-            for (int jt = 0; jt < D / 16; ++jt) {
-                f4 u = f4_zero();     // u^T tile (m = feature j, n = row); contraction in split slot order
+            for (int t = 0; t < D / 32; ++t) {
+                f4 u[2] = {f4_zero(), f4_zero()};      // u^T tiles 2t, 2t + 1 (m = feature, n = row)
 #pragma unroll
-                for (int pr = 0; pr < DH / 32; ++pr) {
-                    u = mfma32(row_split8(Wfs, LDW, 16 * jt + i, 32 * pr, G), op[pr], u);
-                }
-                h4 sv, cv;
+                for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                    for (int c = 0; c < NC / 2; ++c)
+                        u[q] = mfma32(row8(Wfs, LDW, 32 * t + 16 * q + i, 32 * c, G), op[c], u[q]);
+                h8 sv, cv;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
                     float s_, c_;
-                    fast_sincos(u[e] * inv, s_, c_);
+                    sincos_turns(u[e / 4][e % 4] * inv_turns, s_, c_);
                     sv[e] = (half_t)(scale * s_);
                     cv[e] = (half_t)(scale * c_);
                 }
-                *reinterpret_cast<h4*>(Ps + i * LDP + 16 * jt + 4 * G) = sv;
-                *reinterpret_cast<h4*>(Ps + i * LDP + D + 16 * jt + 4 * G) = cv;
-            }
-            wave_lds_order();
-            wave_rows_s2g<2 * D>(Ps, LDP, phi, r0, R, H, h, lane);
-            wave_lds_order();
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Same computation for narrow inputs (E = 32 * NKS <= 512, DH = 64): a workgroup keeps its 128
-// rows of x in registers for its whole life -- wave w holds rows [32w, 32w + 32) as MFMA B
-// operands, 2 * NKS registers of 8 halves -- and walks a list of (head, projection) pairs whose
-// weight rows ([DH][E] each) arrive whole in a two-buffer LDS ring, one pair ahead.  No barrier
-// inside a pair's contraction or its epilogue.
-//   grid = 8 * ceil(nrt / 8) * ngroups; group g of a row tile takes pairs [g * ppg, (g + 1) * ppg)
-//   of the H * np pairs, pair index hp -> head hp / np, projection hp % np.
-// LDS: [ring: 2 x DH x (E + 8); first used to stage the x tile][staging rows of the waves][w' of the head]
-// ---------------------------------------------------------------------------
-// 16 bytes as a native vector: assignments are plain vector loads and stores (the uint4 class
-// is copied with memcpy, which keeps registers that stay in flight across loop iterations in
-// private memory)
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-template <int D, int DH, int NKS>
-struct ProjectRowCfg {
-    static_assert(DH == 64, "one 64-wide head per pair");
-    static constexpr int BM = 128, E = 32 * NKS;
-    static constexpr int LDE = E + 8;
-    static constexpr int LDW = DH + lds_pad(DH);
-    static constexpr int LDP = (2 * D > DH ? 2 * D : DH) + 16;
-    static constexpr int kSliceHalves = DH * LDE;
-    static constexpr int SP = DH * E / 8 / kThreads;        // 16-byte pieces per thread and slice
-    static constexpr size_t kLds = (size_t)(2 * kSliceHalves + 4 * 16 * LDP + D * LDW) * 2;
-    static_assert(2 * kSliceHalves >= BM * LDE, "the x tile is staged in the ring");
-    static_assert(kLds <= 160 * 1024, "LDS budget");
-};
-
-template <int D, int DH, int NKS>
-__global__ __launch_bounds__(kThreads) void k_project_phi_rows(
-    const half_t* __restrict__ x, ProjectArgs pa, const half_t* __restrict__ wf, int R, int H, int np,
-    int ngroups, int ppg, float scale) {
-    using Cfg = ProjectRowCfg<D, DH, NKS>;
-    constexpr int BM = Cfg::BM, E = Cfg::E, LDE = Cfg::LDE, LDW = Cfg::LDW, LDP = Cfg::LDP, SP = Cfg::SP;
-    constexpr int NCT = DH / 16, PPR = E / 8;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    half_t* ring = reinterpret_cast<half_t*>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = lane & 15, G = lane >> 4;
-    half_t* Ps = ring + 2 * Cfg::kSliceHalves + wv * 16 * LDP;
-    half_t* Wfs = ring + 2 * Cfg::kSliceHalves + 4 * 16 * LDP;
-
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int row0 = (xcd + 8 * (slot / ngroups)) * BM;
-    const int grp = slot % ngroups;
-    const int pairs = H * np;
-    const int hp_begin = grp * ppg, hp_end = min(hp_begin + ppg, pairs);
-    if (row0 >= R || hp_begin >= hp_end) return;
-    RFA_TICK_INIT();
-
-    // weight rows of pair hp: piece -> (row, 16-byte column)
-    u32x4 wr[SP];
-    auto slice_g2r = [&](int hp) {
-        const half_t* __restrict__ src = pick3(pa.w, hp % np) + (int64_t)(hp / np) * DH * E;
-#pragma unroll
-        for (int it = 0; it < SP; ++it) wr[it] = *reinterpret_cast<const u32x4*>(src + (int64_t)(tid + kThreads * it) * 8);
-    };
-    auto slice_r2s = [&](half_t* buf) {
-#pragma unroll
-        for (int it = 0; it < SP; ++it) {
-            const int pc = tid + kThreads * it;
-            *reinterpret_cast<u32x4*>(buf + (pc / PPR) * LDE + (pc % PPR) * 8) = wr[it];
-        }
-    };
-    // Workgroups of different row tiles walk their pairs in rotated order, so that the CUs of an
-    // XCD do not all ask the L2 for the same weight rows at the same time.
-    const int cnt = hp_end - hp_begin;
-    const int rot = (row0 / BM) % cnt;
-    auto pair_at = [&](int j) { return hp_begin + (j + rot) % cnt; };
-    slice_g2r(pair_at(0));
-
-    // x tile -> ring (coalesced rows) -> this wave's rows as B operands
-    {
-        constexpr int XP = BM * PPR / kThreads, BATCH = XP % 16 == 0 ? 16 : 8;
-        static_assert(XP % BATCH == 0, "x tile pieces");
-#pragma unroll
-        for (int base = 0; base < XP; base += BATCH) {
-            u32x4 v[BATCH];
-#pragma unroll
-            for (int b = 0; b < BATCH; ++b) {
-                const int pc = tid + kThreads * (base + b);
-                const int r = min(row0 + pc / PPR, R - 1);
-                v[b] = *reinterpret_cast<const u32x4*>(x + (int64_t)r * E + (pc % PPR) * 8);
-            }
-#pragma unroll
-            for (int b = 0; b < BATCH; ++b) {
-                const int pc = tid + kThreads * (base + b);
-                *reinterpret_cast<u32x4*>(ring + (pc / PPR) * LDE + (pc % PPR) * 8) = v[b];
-            }
-        }
-    }
-    __syncthreads();
-    h8 xb[2][NKS];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) xb[a][ks] = row8(ring, LDE, 32 * wv + 16 * a + i, 32 * ks, G);
-    __syncthreads();
-    slice_r2s(ring);
-    // wf is NULL when no projection asks for phi
-    int h_loaded = pair_at(0) / np;
-    if (wf) load_w_to_lds<D, DH>(Wfs, wf + (int64_t)h_loaded * D * DH, tid);
-    __syncthreads();
-    RFA_TICK(0);
-
-    for (int j = 0; j < cnt; ++j) {
-        const int hp = pair_at(j);
-        const int h = hp / np, p = hp % np;
-        const half_t* Ws = ring + (j & 1) * Cfg::kSliceHalves;
-        // the bias before the weight prefetch: loads return in order, and the epilogue must not
-        // have to wait for the next pair's weights to see its bias
-        const half_t* bias = pick3(pa.b, p);
-        h4 bv[NCT];
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bv[ct][e] = (half_t)0.f;
-            if (bias) bv[ct] = *reinterpret_cast<const h4*>(bias + h * DH + 16 * ct + 4 * G);
-        }
-        const int hp_next = pair_at(min(j + 1, cnt - 1));     // the last pair re-reads its own rows
-        slice_g2r(hp_next);
-
-        f4 acc[2][NCT];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int c = 0; c < NCT; ++c) acc[a][c] = f4_zero();
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-            for (int ct = 0; ct < NCT; ++ct) {
-                const h8 wa = row8(Ws, LDE, 16 * ct + i, 32 * ks, G);
-                acc[0][ct] = mfma32(wa, xb[0][ks], acc[0][ct]);
-                acc[1][ct] = mfma32(wa, xb[1][ks], acc[1][ct]);
-            }
-        RFA_TICK(1);
-
-        half_t* phi = pick3(pa.phi, p);
-        half_t* y = pick3(pa.y, p);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int r0 = row0 + 32 * wv + 16 * a;
-            h8 op[DH / 32];
-            float ss = 0.f;
-#pragma unroll
-            for (int ct = 0; ct < NCT; ++ct) {
-                f4 t = acc[a][ct];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t[e] += (float)bv[ct][e];
-                const h4 yh = to_h4(t);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    ss += (float)yh[e] * (float)yh[e];
-                    op[ct / 2][4 * (ct % 2) + e] = yh[e];
+                if (r < R) {
+                    *reinterpret_cast<h8*>(phi + at * (2 * D) + 32 * t + 8 * G) = sv;
+                    *reinterpret_cast<h8*>(phi + at * (2 * D) + D + 32 * t + 8 * G) = cv;
                 }
-                if (y) *reinterpret_cast<h4*>(Ps + i * LDP + 16 * ct + 4 * G) = yh;
-            }
-            if (y) {
-                wave_lds_order();
-                wave_rows_s2g<DH>(Ps, LDP, y, r0, R, H, h, lane);
-                wave_lds_order();
-            }
-            if (phi) {
-                ss = sum_over_groups(ss);
-                const float inv = 1.0f / (sqrtf(ss) + 1e-3f);
-#pragma unroll
-                for (int jt = 0; jt < D / 16; ++jt) {
-                    f4 u = f4_zero();
-#pragma unroll
-                    for (int pr = 0; pr < DH / 32; ++pr)
-                        u = mfma32(row_split8(Wfs, LDW, 16 * jt + i, 32 * pr, G), op[pr], u);
-                    h4 sv, cv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float s_, c_;
-                        fast_sincos(u[e] * inv, s_, c_);
-                        sv[e] = (half_t)(scale * s_);
-                        cv[e] = (half_t)(scale * c_);
-                    }
-                    *reinterpret_cast<h4*>(Ps + i * LDP + 16 * jt + 4 * G) = sv;
-                    *reinterpret_cast<h4*>(Ps + i * LDP + D + 16 * jt + 4 * G) = cv;
-                }
-                wave_lds_order();
-                wave_rows_s2g<2 * D>(Ps, LDP, phi, r0, R, H, h, lane);
-                wave_lds_order();
             }
         }
-        RFA_TICK(2);
-        __syncthreads();                              // everyone is done with this pair's buffer and w'
-        const int h_next = hp_next / np;
-        if (h_next != h_loaded) {
-            h_loaded = h_next;
-            if (wf) load_w_to_lds<D, DH>(Wfs, wf + (int64_t)h_next * D * DH, tid);
-        }
-        slice_r2s(ring + ((j + 1) & 1) * Cfg::kSliceHalves);
-        __syncthreads();
-        RFA_TICK(3);
     }
 }
 

@@ -41,8 +41,7 @@ def _linear64(x, w, b, H, d):
 @pytest.mark.parametrize("streaming", [False, True])
 @pytest.mark.parametrize("L,B,E,H,d,D", SHAPES)
 def test_qkv_projection_with_feature_map(L, B, E, H, d, D, streaming, knobs):
-    """Both kernels: the one that keeps its rows of x in LDS (picked when they fit) and the one
-    that streams x and the weights together (forced by the "project_streaming" knob)."""
+    """The tile height picked by itself and the tallest one (the "project_streaming" knob)."""
     from rfa_amd import rfa_hip
     knobs(project_streaming=1 if streaming else -1)
     x, ws, bs = _inputs(L, B, E, H, d, 900 + L, 3)
@@ -64,6 +63,27 @@ def test_qkv_projection_with_feature_map(L, B, E, H, d, D, streaming, knobs):
             assert (phi - own).abs().max().item() <= 2e-3
             ref = O.random_project(want.half().float(), wf.float())
             assert (phi - ref).abs().max().item() <= 4e-3
+
+
+# rows around the three tile heights, one and several contraction rounds of the three-stage ring, odd
+# numbers of 64-wide heads (half a column tile), every (d, D)
+@pytest.mark.parametrize("rows_knob", [0, 1, 2])
+@pytest.mark.parametrize("R,E,H,d,D,n", [(1, 64, 1, 64, 32, 1), (63, 128, 3, 64, 64, 1), (65, 64, 3, 64, 128, 3), (127, 192, 1, 128, 32, 2),
+                                         (129, 64, 2, 128, 64, 1), (255, 128, 1, 128, 128, 3), (257, 320, 5, 64, 64, 2), (513, 64, 2, 64, 32, 3)])
+def test_projection_tile_edges(R, E, H, d, D, n, rows_knob, knobs):
+    from rfa_amd import rfa_hip
+    knobs(project_streaming=rows_knob)
+    x, ws, bs = _inputs(R, 1, E, H, d, 970 + R, n)
+    wf = (_randn(H, D, d, seed=79) * 0.9).half()
+    want_phi = [p != n - 1 or n == 1 for p in range(n)]
+    print(f"project tile edges R={R} E={E} H={H} d={d} D={D} n={n} knob={rows_knob}", flush=True)
+    ys, phis = rfa_hip.project_feature_map(x.cuda(), [w.cuda() for w in ws], [b.cuda() for b in bs], want_phi, wf.cuda(), H, O.SCALE)
+    for p in range(n):
+        want = _linear64(x, ws[p], bs[p], H, d)
+        assert ((ys[p].double().cpu() - want).abs() <= 1.5e-3 * want.abs().clamp_min(1.0)).all(), p
+        if want_phi[p]:
+            own = O.random_project(ys[p].float().cpu(), wf.float())
+            assert (phis[p].float().cpu() - own).abs().max().item() <= 2e-3
 
 
 @pytest.mark.parametrize("streaming", [False, True])
