@@ -757,21 +757,23 @@ int launch_project_phi(const rfa::half_t* x, const rfa::ProjectArgs& pa, const r
 // ---- weight-gradient plan -------------------------------------------------------------
 struct WGradPlan {
     int nsplit;            // row splits (partials to add)
-    int rows_per_split;    // multiple of 64
+    int rows_per_split;    // multiple of 32
 };
 
-// About 256-512 workgroups: 8 splits (one per XCD) times as many as the tile count leaves room for.
+// Two workgroups per CU, but at least 16 steps of 32 rows each: every split writes and re-reads an fp32
+// copy of dW, and its ring has to fill first.  Measured (us, 8192 rows) for 4 / 8 / 10 / 16 / 32 splits:
+// 512 -> 3 x 512 (48 tiles) 34.8 / 27.0 / 25.8 / 29.5 / 40.8; 1024 -> 1024 (64) 36.3 / 29.9 / 34.1 / 37.0 /
+// 50.1; 512 -> 512 (16) 32.4 / 23.9 / 22.7 / 23.2 / 24.9; 1000 rows, 384 -> 3 x 384 (27): 4 -> 14.0, 16 -> 22.6.
 WGradPlan make_wgrad_plan(int64_t R, int Eo, int Ei, int np) {
     const int64_t tiles = (int64_t)np * (Eo / 128) * (Ei / 128);
-    const int64_t nchunks = (R + 63) / 64;
-    int64_t want = 8 * ((32 + tiles - 1) / tiles);
+    const int64_t nsteps = (R + 31) / 32;
+    int64_t want = std::min<int64_t>(2 * (int64_t)device_cus() / tiles, nsteps / 16);
     if (want > 64) want = 64;
-    if (want > nchunks) want = nchunks;
     if (want < 1) want = 1;
-    const int64_t cps = (nchunks + want - 1) / want;
+    const int64_t sps = (nsteps + want - 1) / want;
     WGradPlan p;
-    p.rows_per_split = (int)(cps * 64);
-    p.nsplit = (int)((nchunks + cps - 1) / cps);
+    p.rows_per_split = (int)(sps * 32);
+    p.nsplit = (int)((nsteps + sps - 1) / sps);
     if (p.nsplit < 1) p.nsplit = 1;
     return p;
 }
@@ -1835,13 +1837,13 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
                     workspace ? workspace_bytes : (size_t)0);
     float* part = static_cast<float*>(workspace);
     float* bpart = part + (size_t)pl.nsplit * np * E_out * E_in;
-    const int per_split = np * (E_out / 128) * (E_in / 128);
-    const int64_t grid = (int64_t)8 * ((pl.nsplit + 7) / 8) * per_split;
-    if (grid > (int64_t(1) << 30)) return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_weight_grad: sizes exceed the supported range");
+    const int64_t work = (int64_t)pl.nsplit * np * (E_out / 128) * (E_in / 128);
+    if (work > (int64_t(1) << 30)) return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_weight_grad: sizes exceed the supported range");
+    const unsigned grid = (unsigned)(rfa::kXcds * ((work + rfa::kXcds - 1) / rfa::kXcds));
     auto kern = rfa::k_weight_grad_partial;
     if (int rc = set_lds(kern, rfa::WeightGradCfg::kLds)) return rc;
     // R = 0: every split is empty and the partials come out as zeros
-    RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3((unsigned)grid), dim3(rfa::kThreads), rfa::WeightGradCfg::kLds, st,
+    RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3(grid), dim3(rfa::kThreads), rfa::WeightGradCfg::kLds, st,
                static_cast<const rfa::half_t*>(x), wa, part, bpart, (int)R, E_out, E_in, np, pl.nsplit, pl.rows_per_split);
     const int64_t threads = (int64_t)np * ((int64_t)E_out * E_in + E_out) / 4;
     RFA_LAUNCH(WGRAD_REDUCE, rfa::k_weight_grad_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(rfa::kThreads), 0, st,

@@ -61,6 +61,14 @@ __device__ __forceinline__ void dma16(const char* g, half_t* lds) {
                                      (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
+// The same through a wave-uniform base and a 32-bit lane offset, hidden from the compiler: it makes every
+// transposing LDS read wait for all direct loads it knows of (which a ring of stages must not)
+__device__ __forceinline__ void dma16_opaque(const half_t* base, unsigned off_bytes, const half_t* lds) {
+    const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) half_t*)lds;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(off_bytes), "s"(base) : "memory", "m0");
+}
+
 // All but the last N direct loads of this wave have landed and its LDS reads are done; then the
 // workgroup barrier: everyone's share of the stage is in place, the stage before it is free.
 template <int N>
@@ -271,122 +279,152 @@ struct WeightGradArgs {
 };
 
 struct WeightGradCfg {
-    static constexpr int TO = 128, TI = 128, C = 64;       // tile of dW, rows per step
-    static constexpr int LD = 128 + lds_pad(128);
-    static constexpr int kTile = C * LD;                   // halves
-    static constexpr size_t kLds = (size_t)2 * 2 * kTile * 2;
-    static constexpr int kPieces = C * 128 / 8 / kThreads; // 16-byte pieces per thread and tile
+    static constexpr int TO = 128, TI = 128, C = 32;       // tile of dW, rows per step: one MFMA deep
+    static constexpr int kStages = 3;                      // 4 and 5 measured the same
+    static constexpr int NO = TO / 32, NI = TI / 32;       // 16-wide tiles of a wave: 64 x 64
+    static constexpr int kStageHalves = C * (TO + TI);
+    static constexpr size_t kLds = (size_t)kStages * kStageHalves * 2;
+    static constexpr int YI = C * TO / 2048, XI = C * TI / 2048;   // 1 KiB pieces of a stage per wave
 };
 
-// rows [r0, r0 + 64) x columns [c0, c0 + 128) of a [R, E] matrix -> registers; rows at or past
-// r_end are read from row r_end - 1 (always a valid row) and zeroed on the way to LDS
-__device__ __forceinline__ void wgrad_g2r(uint4 (&v)[WeightGradCfg::kPieces], const half_t* __restrict__ src, int E,
-                                          int r0, int r_end, int c0, int tid) {
-#pragma unroll
-    for (int it = 0; it < WeightGradCfg::kPieces; ++it) {
-        const int pc = tid + kThreads * it;
-        const int r = min(r0 + pc / 16, r_end - 1);
-        v[it] = *reinterpret_cast<const uint4*>(src + (int64_t)r * E + c0 + (pc % 16) * 8);
-    }
+// Column fragment X[8G + e][c0 + i], e = 0..7, of a stage array [32][LD] (LD halves per row, no
+// padding): like col8, with the 32-byte segments of row r stored at segment ^ (r % 4 + 4 (r / 8 % 2)),
+// which spreads the 16 row pieces of a transposing read over all banks.  The rotation depends on
+// the lane's first row only (4 rows further it is the same).
+template <int LD>
+__device__ __forceinline__ h8 col8_rot(const half_t* X, int seg, int lane) {
+    const int s = lane & 15, G = lane >> 4;
+    const int r = 8 * G + (s >> 2);
+    const half_t* p = X + r * LD + (seg ^ ((s >> 2) | ((G & 1) << 2))) * 16 + 4 * (s & 3);
+    const h4 a = tr_read4(p);
+    const h4 b = tr_read4(p + 4 * LD);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-__device__ __forceinline__ void wgrad_r2s(const uint4 (&v)[WeightGradCfg::kPieces], half_t* Xs, int r0, int r_end,
-                                          int tid) {
-#pragma unroll
-    for (int it = 0; it < WeightGradCfg::kPieces; ++it) {
-        const int pc = tid + kThreads * it;
-        const bool keep = r0 + pc / 16 < r_end;
-        uint4 x = v[it];
-        x.x = keep ? x.x : 0u; x.y = keep ? x.y : 0u; x.z = keep ? x.z : 0u; x.w = keep ? x.w : 0u;
-        *reinterpret_cast<uint4*>(Xs + (pc / 16) * WeightGradCfg::LD + (pc % 16) * 8) = x;
-    }
-}
-
-// grid = 8 * ceil(nsplit / 8) * np * (Eo / 128) * (Ei / 128): the workgroups of one split (which
-// share its rows of x and dy) are dealt to one XCD.  rows_per_split is a multiple of 64.
-__global__ __launch_bounds__(kThreads) void k_weight_grad_partial(
+// Workgroup (split s, projection p, tile): a 128 x 128 tile of dW_p over the rows of split s, four waves of
+// 64 x 64, steps of 32 rows through a three-stage ring of direct loads with one barrier per step (the
+// layout and the waits of k_project_phi).  What bounds it is the step itself -- barrier, transposing
+// reads, 16 products -- which two to three workgroups per CU hide in each other; tiles of 256 x 128 spill.
+// Measured with k_weight_grad_reduce, us (before: register-staged loads, two buffers, at least 8 splits):
+// 8192 rows, 512 -> 3 x 512 36.4 -> 25.8; 1024 -> 3 x 1024 94 -> 67 (770 TFLOP/s); 1024 -> 1024 35.3 -> 29.9;
+// 512 -> 512 26.0 -> 23.2; 1000 rows, 384 -> 3 x 384 22.8 -> 14.4.
+// grid = 8 * ceil(work / 8), work = nsplit * np * tiles; each XCD gets a contiguous range of the numbers
+// (split first), so that the workgroups that share rows of x and dy meet in its L2.  rows_per_split is a
+// multiple of 32.
+__global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
     const half_t* __restrict__ x, WeightGradArgs wa, float* __restrict__ part, float* __restrict__ bpart, int R,
     int Eo, int Ei, int np, int nsplit, int rows_per_split) {
     using Cfg = WeightGradCfg;
-    constexpr int LD = Cfg::LD, C = Cfg::C;
+    constexpr int TO = Cfg::TO, TI = Cfg::TI, C = Cfg::C, NO = Cfg::NO, NI = Cfg::NI, STAGES = Cfg::kStages;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, G = lane >> 4;
-    const int wo = wv >> 1, wi = wv & 1;                  // wave -> 64 x 64 quadrant of the tile
+    const int wo = wv >> 1, wi = wv & 1;                  // wave -> quadrant of the tile
 
-    const int tiles_i = Ei / Cfg::TI, tiles_o = Eo / Cfg::TO;
-    const int per_split = np * tiles_o * tiles_i;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int s = xcd + 8 * (slot / per_split);
-    if (s >= nsplit) return;
-    int idx = slot % per_split;
+    const int tiles_i = Ei / TI, tiles_o = Eo / TO;
+    const int work = nsplit * np * tiles_o * tiles_i, per_xcd = (work + kXcds - 1) / kXcds;
+    int idx = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (idx >= work) return;
     const int ti = idx % tiles_i; idx /= tiles_i;
-    const int to = idx % tiles_o;
-    const int p = idx / tiles_o;
+    const int to = idx % tiles_o; idx /= tiles_o;
+    const int p = idx % np, s = idx / np;
     const int r_begin = s * rows_per_split, r_end = min(r_begin + rows_per_split, R);
-    const int o0 = to * Cfg::TO, c0 = ti * Cfg::TI;
-    const half_t* __restrict__ dy = pick3(wa.dy, p);
+    const int o0 = to * TO, c0 = ti * TI;
     const bool with_bias = ti == 0 && wi == 0 && pick3(wa.db, p) != nullptr;   // wave-uniform
 
-    f4 acc[4][4];        // (m = o, n = c) tiles of this wave's quadrant
-    f4 accb[4];          // column sums of dy: every column n holds the same sum
+    f4 acc[NO][NI];      // (m = o, n = c) tiles of this wave's quadrant
+    f4 accb[NO];         // column sums of dy: every column n holds the same sum
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < NO; ++a) {
         accb[a] = f4_zero();
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = f4_zero();
+        for (int b = 0; b < NI; ++b) acc[a][b] = f4_zero();
     }
-    h8 ones;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ones[e] = (half_t)1.0f;
+    const h8 ones = h8_ones();
 
     if (r_begin < r_end) {
-        uint4 yr[Cfg::kPieces], xr[Cfg::kPieces];
-        wgrad_g2r(yr, dy, Eo, r_begin, r_end, o0, tid);
-        wgrad_g2r(xr, x, Ei, r_begin, r_end, c0, tid);
-        wgrad_r2s(yr, smem, r_begin, r_end, tid);
-        wgrad_r2s(xr, smem + Cfg::kTile, r_begin, r_end, tid);
-        __syncthreads();
-        int buf = 0;
-        for (int r0 = r_begin; r0 < r_end; r0 += C) {
-            // branch-free prefetch of the next step (the last one re-reads valid rows and zeroes them)
-            wgrad_g2r(yr, dy, Eo, r0 + C, r_end, o0, tid);
-            wgrad_g2r(xr, x, Ei, r0 + C, r_end, c0, tid);
-            const half_t* Ys = smem + buf * 2 * Cfg::kTile;
-            const half_t* Xs = Ys + Cfg::kTile;
+        // 1 KiB of a stage array per instruction: 512 / LD rows, lane -> (row, 16-byte piece)
+        const half_t* const dyb = pick3(wa.dy, p) + (int64_t)r_begin * Eo + o0;
+        const half_t* const xb = x + (int64_t)r_begin * Ei + c0;
+        const int nrows = r_end - r_begin, nk = (nrows + C - 1) / C;
+        auto rot = [](int r) { return ((r & 3) | ((r >> 1) & 4)) * 2; };
+        // byte offsets inside a step; the rows of the last step past the end read the last row (the dy
+        // operand drops them)
+        unsigned yoff[2][Cfg::YI], xoff[2][Cfg::XI];
 #pragma unroll
-            for (int rs = 0; rs < C / 32; ++rs) {
-                h8 xa[4];
+        for (int last = 0; last < 2; ++last) {
+            const int rmax = last ? nrows - 1 - (nk - 1) * C : C - 1;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) xa[b] = col8(Xs, LD, 32 * rs, 64 * wi + 16 * b, lane);
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const h8 ya = col8(Ys, LD, 32 * rs, 64 * wo + 16 * a, lane);
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) acc[a][b] = mfma32(ya, xa[b], acc[a][b]);
-                    if (with_bias) accb[a] = mfma32(ya, ones, accb[a]);
-                }
+            for (int it = 0; it < Cfg::YI; ++it) {
+                const int r = (wv * Cfg::YI + it) * (512 / TO) + lane / (TO / 8);
+                yoff[last][it] = (unsigned)min(r, rmax) * (unsigned)(Eo * 2) + ((lane % (TO / 8)) ^ rot(r)) * 16;
             }
-            buf ^= 1;
-            wgrad_r2s(yr, smem + buf * 2 * Cfg::kTile, r0 + C, r_end, tid);
-            wgrad_r2s(xr, smem + buf * 2 * Cfg::kTile + Cfg::kTile, r0 + C, r_end, tid);
-            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < Cfg::XI; ++it) {
+                const int r = (wv * Cfg::XI + it) * (512 / TI) + lane / (TI / 8);
+                xoff[last][it] = (unsigned)min(r, rmax) * (unsigned)(Ei * 2) + ((lane % (TI / 8)) ^ rot(r)) * 16;
+            }
+        }
+        auto load_stage = [&](int kk, int buf) {
+            half_t* st = smem + buf * Cfg::kStageHalves;
+            const half_t* yb = dyb + (int64_t)kk * C * Eo;
+            const half_t* xk = xb + (int64_t)kk * C * Ei;
+            const bool last = kk == nk - 1;
+#pragma unroll
+            for (int it = 0; it < Cfg::YI; ++it)
+                dma16_opaque(yb, last ? yoff[1][it] : yoff[0][it], st + (wv * Cfg::YI + it) * 512);
+#pragma unroll
+            for (int it = 0; it < Cfg::XI; ++it)
+                dma16_opaque(xk, last ? xoff[1][it] : xoff[0][it], st + C * TO + (wv * Cfg::XI + it) * 512);
+        };
+#pragma unroll
+        for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
+        int buf = 0;
+        for (int kk = 0; kk < nk; ++kk) {
+            stage_barrier<(STAGES - 2) * (Cfg::YI + Cfg::XI)>();
+            load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
+            const half_t* Ys = smem + buf * Cfg::kStageHalves;
+            const half_t* Xs = Ys + C * TO;
+            h8 xa[NI], ya[NO];
+#pragma unroll
+            for (int b = 0; b < NI; ++b) xa[b] = col8_rot<TI>(Xs, 4 * wi + b, lane);
+#pragma unroll
+            for (int a = 0; a < NO; ++a) ya[a] = col8_rot<TO>(Ys, NO * wo + a, lane);
+            if (kk * C + C > nrows) {                     // the ragged end of the rows
+                const int keep = nrows - kk * C - 8 * G;
+#pragma unroll
+                for (int a = 0; a < NO; ++a)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ya[a][e] = e < keep ? ya[a][e] : (half_t)0.f;
+            }
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int a = 0; a < NO; ++a) {
+#pragma unroll
+                for (int b = 0; b < NI; ++b) acc[a][b] = mfma32(ya[a], xa[b], acc[a][b]);
+            }
+            if (with_bias) {
+#pragma unroll
+                for (int a = 0; a < NO; ++a) accb[a] = mfma32(ya[a], ones, accb[a]);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            buf = buf == STAGES - 1 ? 0 : buf + 1;
         }
     }
-    float* po = part + ((int64_t)(s * np + p) * Eo + o0 + 64 * wo) * Ei + c0 + 64 * wi;
+    float* po = part + ((int64_t)(s * np + p) * Eo + o0 + TO / 2 * wo) * Ei + c0 + 64 * wi;
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NO; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < NI; ++b)
 #pragma unroll
             for (int e = 0; e < 4; ++e) po[(int64_t)(16 * a + 4 * G + e) * Ei + 16 * b + i] = acc[a][b][e];
     if (with_bias && i == 0) {
-        float* pb = bpart + (int64_t)(s * np + p) * Eo + o0 + 64 * wo;
+        float* pb = bpart + (int64_t)(s * np + p) * Eo + o0 + TO / 2 * wo;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) *reinterpret_cast<f4*>(pb + 16 * a + 4 * G) = accb[a];
+        for (int a = 0; a < NO; ++a) *reinterpret_cast<f4*>(pb + 16 * a + 4 * G) = accb[a];
     }
 }
 

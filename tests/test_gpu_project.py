@@ -255,6 +255,20 @@ def test_linear_weight_and_bias_gradients(R, Eo, Ei, n):
         rfa_hip.linear_weight_grad(x[:, :64].contiguous().cuda(), [d.cuda() for d in dys], want_bias)
 
 
+# the ring of 32-row steps: one step (ragged), the ring's depth and one around it, the first row counts with a
+# second split, a last split of a single ragged step
+@pytest.mark.parametrize("R", [1, 31, 32, 33, 64, 95, 97, 1023, 1024, 1025, 1057, 1569])
+def test_linear_weight_gradient_step_edges(R):
+    """dW and db exactly (whole numbers: every product and sum is exact in fp32, every result below 2048)."""
+    from rfa_amd import rfa_hip
+    g = torch.Generator().manual_seed(990 + R)
+    x = torch.randint(-1, 2, (R, 128), generator=g).half()
+    dy = (torch.randint(-1, 2, (R, 256), generator=g)).half()
+    (dw,), (db,) = rfa_hip.linear_weight_grad(x.cuda(), [dy.cuda()], [True])
+    assert torch.equal(dw.double().cpu(), dy.double().t() @ x.double())
+    assert torch.equal(db.double().cpu(), dy.double().sum(0))
+
+
 def test_cross_modules_fused_projections_match_unfused_chain():
     """CrossAttentionProjectLayer + CrossAttention with their projections on the fused launch vs
     the same modules on nn.Linear + random_project: output within 4e-3, gradients within 1e-2."""
