@@ -413,6 +413,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             __builtin_amdgcn_s_setprio(0);
             buf = buf == STAGES - 1 ? 0 : buf + 1;
         }
+        // the last re-requested stages are still on their way into this workgroup's LDS: they land before it ends
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     float* po = part + ((int64_t)(s * np + p) * Eo + o0 + TO / 2 * wo) * Ei + c0 + 64 * wi;
 #pragma unroll
