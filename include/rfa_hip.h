@@ -314,8 +314,12 @@ int rfa_cross_state_backward(const void* phi_k, const void* v, const uint8_t* ke
  *                      Tp = T rounded up to a multiple of 64, padding columns non-zero; may be NULL
  *   attn_mask_t      : its transpose, bytes [T (key), Tp (query)], padded the same way
  *   rsum             : fp32 [T, N] raw row sums (forward: optional output; backward: input)
+ * rfa_pack_mask writes both byte matrices from a [T, T] mask whose entries < 0 are masked
+ * (type 0 fp32, 1 fp16, 2 bf16; strides in elements).
  *   dphi_q, dphi_k, dv : every element written; a padded key gets zero dphi_k and dv.
  * ------------------------------------------------------------------------- */
+int rfa_pack_mask(const void* mask, int type, int64_t stride_row, int64_t stride_col, uint8_t* out, uint8_t* out_t,
+                  int64_t T, int64_t Tp, void* stream);
 int rfa_masked_forward(const void* phi_q, const void* phi_k, const void* v, const uint8_t* key_padding_mask,
                        const uint8_t* attn_mask, void* out, float* rsum, int64_t T, int64_t Tp, int64_t B,
                        int H, int K, int d, void* stream);

@@ -67,6 +67,7 @@ SIGNATURES = {
     "rfa_cross_readout": (c_int, [c_void_p] * 4 + [c_int64, c_int64, c_int, c_int, c_void_p]),
     "rfa_cross_readout_backward": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int, c_int, c_void_p]),
     "rfa_cross_state_backward": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
+    "rfa_pack_mask": (c_int, [c_void_p, c_int, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "rfa_masked_forward": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "rfa_masked_backward_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int]),
     "rfa_masked_backward": (c_int, [c_void_p] * 12 + [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),

@@ -46,14 +46,14 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
                                    "k_masked_fwd", "k_masked_bwd_prep", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
-                                   "k_sliced_bwd", "k_copy_rows_strided"};
+                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -1426,6 +1426,35 @@ static int check_masked(const char* fn, int64_t T, int64_t Tp, int64_t B, int H,
     if (amask && (Tp < T || Tp % 64 != 0))
         return fail(RFA_ERR_BAD_SHAPE, "%s: the attn_mask row stride must be T rounded up to a multiple of 64 (got %lld for T=%lld)",
                     fn, (long long)Tp, (long long)T);
+    return RFA_OK;
+}
+
+int rfa_pack_mask(const void* mask, int type, int64_t stride_row, int64_t stride_col, uint8_t* out, uint8_t* out_t,
+                  int64_t T, int64_t Tp, void* stream) {
+    if (type < 0 || type > 2) return fail(RFA_ERR_UNSUPPORTED, "rfa_pack_mask: type must be 0 (fp32), 1 (fp16) or 2 (bf16), got %d", type);
+    if (T < 0 || Tp < T || Tp % 64 != 0 || Tp - T >= 64)
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_pack_mask: the row stride must be T rounded up to a multiple of 64 (got %lld for T=%lld)",
+                    (long long)Tp, (long long)T);
+    if (T > (int64_t)64 * rfa::kMaxMaskBlocks)
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_pack_mask: at most %d steps (got %lld)", 64 * rfa::kMaxMaskBlocks, (long long)T);
+    if (T == 0) return RFA_OK;
+    if (!mask || !out || !out_t) return fail(RFA_ERR_NULL_POINTER, "rfa_pack_mask: NULL pointer");
+    if (!aligned16(out) || !aligned16(out_t)) return fail(RFA_ERR_ALIGNMENT, "rfa_pack_mask: outputs must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(mask) % (type == 0 ? 4 : 2) != 0)
+        return fail(RFA_ERR_ALIGNMENT, "rfa_pack_mask: mask is not aligned to its type");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid((unsigned)(Tp / 64), (unsigned)(Tp / 64));
+    if (type == 0) {
+        RFA_LAUNCH(PACK_MASK, rfa::k_pack_mask<float>, grid, dim3(256), 0, st, static_cast<const float*>(mask), stride_row,
+                   stride_col, out, out_t, (int)T, (int)Tp);
+    } else if (type == 1) {
+        RFA_LAUNCH(PACK_MASK, rfa::k_pack_mask<rfa::half_t>, grid, dim3(256), 0, st, static_cast<const rfa::half_t*>(mask),
+                   stride_row, stride_col, out, out_t, (int)T, (int)Tp);
+    } else {
+        RFA_LAUNCH(PACK_MASK, rfa::k_pack_mask<rfa::Bf16Bits>, grid, dim3(256), 0, st,
+                   static_cast<const rfa::Bf16Bits*>(mask), stride_row, stride_col, out, out_t, (int)T, (int)Tp);
+    }
+    RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
 

@@ -104,6 +104,45 @@ __device__ __forceinline__ int next_live_block(const unsigned char* skip, int b,
     return b;
 }
 
+// The two byte matrices that the kernels below read, from a mask whose entries < 0 are masked (fp32, fp16 or
+// bf16, any strides): out [T][Tp] and its transpose out_t [T][Tp], columns past T set.  One 64 x 64 tile per
+// workgroup: coalesced reads along the mask's rows, the tile of bytes through LDS, 4-byte stores on both sides.
+// At 512 x 512 the launch bounds it; what it replaces was a chain of six ATen launches (compare, two fills, a
+// conversion, two strided copies), 28 us of device time and the host work of six launches.
+// grid = (Tp / 64, Tp / 64)
+struct Bf16Bits { uint16_t bits; };
+__device__ __forceinline__ bool is_negative(float x) { return x < 0.f; }
+__device__ __forceinline__ bool is_negative(half_t x) { return (float)x < 0.f; }
+__device__ __forceinline__ bool is_negative(Bf16Bits x) { return __uint_as_float((uint32_t)x.bits << 16) < 0.f; }
+
+template <typename M>
+__global__ __launch_bounds__(256) void k_pack_mask(const M* __restrict__ mask, int64_t stride_r, int64_t stride_c,
+                                                   uint8_t* __restrict__ out, uint8_t* __restrict__ out_t, int T,
+                                                   int Tp) {
+    __shared__ uint8_t tile[64][68];       // 17 words a row: both read patterns spread over the banks
+    const int tid = threadIdx.x, r0 = 64 * blockIdx.y, c0 = 64 * blockIdx.x;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int r = 4 * u + (tid >> 6), c = tid & 63;
+        bool set = true;
+        if (r0 + r < T && c0 + c < T) set = is_negative(mask[(r0 + r) * stride_r + (c0 + c) * stride_c]);
+        tile[r][c] = set ? 1 : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int a = 16 * u + (tid >> 4), b = 4 * (tid & 15);
+        if (r0 + a < T) *reinterpret_cast<uint32_t*>(out + (int64_t)(r0 + a) * Tp + c0 + b) =
+            *reinterpret_cast<const uint32_t*>(&tile[a][b]);
+        if (c0 + a < T) {
+            uint32_t word = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) word |= (uint32_t)tile[b + e][a] << (8 * e);
+            *reinterpret_cast<uint32_t*>(out_t + (int64_t)(c0 + a) * Tp + r0 + b) = word;
+        }
+    }
+}
+
 template <int KD, int DH>
 __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
     

@@ -520,6 +520,22 @@ Tensor incremental_qkv(const Tensor& qkv, const Tensor& w, double scale, const T
 }
 
 // ---- quadratic form with explicit masks -------------------------------------------------------
+std::tuple<Tensor, Tensor> pack_negative_mask(const Tensor& mask) {
+    TORCH_CHECK(mask.is_cuda(), "attn_mask must live on a HIP device (got ", mask.device(), ")");
+    TORCH_CHECK_VALUE(mask.dim() == 2 && mask.size(0) == mask.size(1), "attn_mask must be [tgt_len, tgt_len] (got ",
+                      mask.sizes(), ")");
+    const auto t = mask.scalar_type();
+    TORCH_CHECK_TYPE(t == torch::kFloat32 || t == torch::kFloat16 || t == torch::kBFloat16,
+                     "attn_mask must be float32, float16 or bfloat16 (got ", t, ")");
+    const int64_t T = mask.size(0), Tp = (T + 63) / 64 * 64;
+    Tensor m = torch::empty({T, Tp}, mask.options().dtype(torch::kUInt8));
+    Tensor mt = torch::empty_like(m);
+    Launch l(mask);
+    check_rc(rfa_pack_mask(ptr(mask), t == torch::kFloat32 ? 0 : t == torch::kFloat16 ? 1 : 2, mask.stride(0), mask.stride(1),
+                           m.data_ptr<uint8_t>(), mt.data_ptr<uint8_t>(), T, Tp, l.stream));
+    return {m, mt};
+}
+
 std::tuple<Tensor, Tensor> masked_forward(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v, int64_t H,
                                           const c10::optional<Tensor>& pad, const c10::optional<Tensor>& attn_mask_bytes) {
     check_qkv(phi_q, phi_k, v);
@@ -611,6 +627,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("s"), py::arg("z"), py::arg("s_out") = py::none(), py::arg("z_out") = py::none());
     m.def("incremental_qkv", &incremental_qkv, py::arg("qkv"), py::arg("w"), py::arg("scale"), py::arg("s"), py::arg("z"),
           py::arg("s_out") = py::none(), py::arg("z_out") = py::none());
+    m.def("pack_negative_mask", &pack_negative_mask, py::arg("mask"));
     m.def("masked_forward", &masked_forward, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("H"),
           py::arg("key_padding_mask") = py::none(), py::arg("attn_mask_bytes") = py::none());
     m.def("masked_backward", &masked_backward, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("grad_attn"),

@@ -631,6 +631,28 @@ def pack_attn_mask(masked: Tensor):
     return m, mt
 
 
+_MASK_TYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+MASK_DTYPES = tuple(_MASK_TYPES)        # what pack_negative_mask reads as it is
+
+
+def pack_negative_mask(mask: Tensor):
+    """``pack_attn_mask(mask < 0)`` in one launch, for an fp32, fp16 or bf16 mask [T, T] of any strides on
+    a HIP device."""
+    _require(mask.is_cuda, RuntimeError, lambda: f"attn_mask must live on a HIP device (got {mask.device})")
+    _require(mask.dim() == 2 and mask.shape[0] == mask.shape[1], ValueError,
+             lambda: f"attn_mask must be [tgt_len, tgt_len] (got {tuple(mask.shape)})")
+    _require(mask.dtype in _MASK_TYPES, TypeError,
+             lambda: f"attn_mask must be float32, float16 or bfloat16 (got {mask.dtype})")
+    T = mask.shape[0]
+    Tp = (T + 63) // 64 * 64
+    m = torch.empty((T, Tp), dtype=torch.uint8, device=mask.device)
+    mt = torch.empty_like(m)
+    with _on_device(mask.device):
+        _lib.check(_lib.load().rfa_pack_mask(mask.data_ptr(), _MASK_TYPES[mask.dtype], mask.stride(0), mask.stride(1),
+                                             m.data_ptr(), mt.data_ptr(), T, Tp, _stream_ptr(mask.device)))
+    return m, mt
+
+
 def masked_forward(phi_q: Tensor, phi_k: Tensor, v: Tensor, H: int, key_padding_mask=None, attn_mask_bytes=None):
     """(attn [T, N, d], rsum fp32 [T, N]).  phi_q, phi_k fp16 [T, N, K], v fp16 [T, N, d], N = B * H;
     key_padding_mask [B, T] (non-zero = pad) or None; attn_mask_bytes from pack_attn_mask()[0] or None."""
@@ -690,7 +712,7 @@ _BOUND = ("supported", "feature_map_supported", "selftest_layout", "forward", "b
           "feature_map_backward", "feature_map_backward_pair", "feature_map_backward_pair_packed", "project_feature_map", "linear_weight_grad", "cross_state",
           "cross_state_backward", "cross_readout", "cross_readout_backward", "incremental", "incremental_fused",
           "incremental_qkv",
-          "masked_forward", "masked_backward")
+          "pack_negative_mask", "masked_forward", "masked_backward")
 _CTYPES_IMPL = {name: globals()[name] for name in _BOUND}
 _active = "ctypes"
 

@@ -410,3 +410,27 @@ def test_causal_attention_module_quadratic_fallback_matches_scan_module():
         attn = O.masked_rfa(O.random_project(q, w), O.random_project(k, w), v, None, am.cpu())
         want = f(m.out_proj, attn.reshape(T, B, E).cuda())
     assert (y.float() - want).abs().max().item() <= 2e-2
+
+
+@pytest.mark.usefixtures("binding")
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 3, 63, 64, 65, 200])
+def test_pack_negative_mask_matches_the_general_packing(T, dtype):
+    """One launch against compare + pack_attn_mask, byte for byte: values around zero, infinities and
+    NaN, and every stride order a mask may come with."""
+    from rfa_amd import rfa_hip
+    gen = torch.Generator().manual_seed(T)
+    special = torch.tensor([0.0, -0.0, -1e-7, 1e-7, float("-inf"), float("inf"), float("nan"), -1.0, -3e38, 1e-38, -1e-38])
+    base = special[torch.randint(0, len(special), (2 * T, 3 * T), generator=gen)].to(dtype).cuda()
+    print(f"pack_negative_mask T={T} {dtype}", flush=True)
+    row = base[0]
+    for mask in (base[:T, :T].contiguous(), base[:T, :T].t(), base[::2, ::3], base[1:T + 1, T:2 * T] if T > 1 else base[1:2, 1:2],
+                 row[None, :T].expand(T, T), row[:T, None].expand(T, T)):
+        want = rfa_hip.pack_attn_mask(mask < 0.0)
+        got = rfa_hip.pack_negative_mask(mask)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    if T == 3:
+        with pytest.raises((RuntimeError, ValueError)):
+            rfa_hip.pack_negative_mask(base[:2, :3])
+        with pytest.raises((RuntimeError, TypeError)):
+            rfa_hip.pack_negative_mask(base[:3, :3].to(torch.int32))
