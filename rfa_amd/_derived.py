@@ -16,7 +16,7 @@ from torch import Tensor
 
 
 def _state(t: Optional[Tensor]):
-    return None if t is None else (t._version, t.data_ptr(), t.dtype, tuple(t.shape), str(t.device))
+    return None if t is None else (t._version, t.data_ptr(), t.dtype, t.shape, t.device)
 
 
 class _Entry:

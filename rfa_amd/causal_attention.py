@@ -115,6 +115,10 @@ def masked_rfa(*, phi_q: Tensor, phi_k: Tensor, v: Tensor, key_padding_mask: Opt
             mask_bytes, mask_t_bytes = rfa_hip.pack_negative_mask(attn_mask.detach().resolve_neg())
         else:
             mask_bytes, mask_t_bytes = rfa_hip.pack_attn_mask((attn_mask < 0.0).to(phi_q.device))
+    if rfa_hip.native is not None:
+        attn = rfa_hip.native.node_masked(phi_q, phi_k, v, key_padding_mask, mask_bytes, mask_t_bytes)
+        if attn is not None:
+            return attn
     n = bsz * num_heads
     attn = _MaskedRFA.apply(phi_q.contiguous().view(tgt_len, n, feat), phi_k.contiguous().view(tgt_len, n, feat),
                             v.contiguous().view(tgt_len, n, head_dim), num_heads, key_padding_mask, mask_bytes,
@@ -136,6 +140,10 @@ def cuda_causal_rfa(*, phi_q: Tensor, phi_k: Tensor, v: Tensor,
         assert key_padding_mask.size(0) == bsz and key_padding_mask.size(1) == tgt_len
         pad = key_padding_mask.to(torch.bool).transpose(0, 1)[:, :, None, None]
         phi_k = phi_k.masked_fill(pad, 0.0)
+    if rfa_hip.native is not None:
+        attn = rfa_hip.native.node_causal(phi_q, phi_k, v)
+        if attn is not None:
+            return attn
     n = bsz * num_heads
     attn = RFA.apply(phi_q.contiguous().view(tgt_len, n, feat),
                      phi_k.contiguous().view(tgt_len, n, feat),
@@ -250,6 +258,17 @@ class CausalAttention(nn.Module):
         """
         tgt_len, bsz, embed_dim = x.size()
         assert embed_dim == self.embed_dim
+        native = rfa_hip.native
+        if (native is not None and saved_state is None and self.fuse_projections and self.cuda_causal_rfa
+                and _drop_scalar_mask(key_padding_mask) is None and isinstance(self.tau, (int, float))):
+            build = torch.is_grad_enabled()
+            layers = (self.q_proj, self.k_proj, self.v_proj)
+            attn = native.node_causal_layer(
+                x, random_matrices if build else self._scaled_matrices(random_matrices),
+                self.sigma if build and self.reparam_proj else None, self.tau, build, [p.weight for p in layers],
+                [p.bias for p in layers], self.num_heads, SCALE)
+            if attn is not None:
+                return linear_out(attn, self.out_proj)
         w = self._scaled_matrices(random_matrices)
         if saved_state is not None and saved_state.get("prev_s") is not None and self._packed_decode_ok(x):
             # a decoding step without autograd: q, k, v of the token(s) from one stacked projection (one

@@ -87,6 +87,15 @@ class CrossAttentionProjectLayer(nn.Module):
         Returns (s [bsz, heads, 2*proj_dim, head_dim], z [bsz, heads, 2*proj_dim], W', tau)
         (reference cross_attention.py:52-106)."""
         src_len, bsz, _ = encoder_output.size()
+        pad = None
+        if mask is not None:
+            pad = mask.reshape(src_len, bsz).transpose(0, 1).contiguous()   # [bsz, src_len]
+        if rfa_hip.native is not None and self.fuse_projections and isinstance(self.tau, (int, float)):
+            state = rfa_hip.native.node_cross_source(
+                encoder_output, random_matrices, self.sigma if self.reparam_proj else None, self.tau,
+                [self.k_proj.weight, self.v_proj.weight], [self.k_proj.bias, self.v_proj.bias], self.num_heads, SCALE, pad)
+            if state is not None:
+                return (*state, self.tau)
         w = build_random_matrices(random_matrices=random_matrices, tau=self.tau,
                                   sigma=self.sigma if self.reparam_proj else None,
                                   reparam_proj=self.reparam_proj)
@@ -98,9 +107,6 @@ class CrossAttentionProjectLayer(nn.Module):
             k = self.k_proj(encoder_output).contiguous().view(src_len, bsz, self.num_heads, self.head_dim)
             v = self.v_proj(encoder_output).contiguous().view(src_len, bsz, self.num_heads, self.head_dim)
             phi_k = random_project(x=k, random_matrices=w)
-        pad = None
-        if mask is not None:
-            pad = mask.reshape(src_len, bsz).transpose(0, 1).contiguous()   # [bsz, src_len]
         s, z = _CrossState.apply(phi_k, v, pad)
         return s, z, w, self.tau
 
@@ -184,6 +190,11 @@ class CrossAttention(nn.Module):
         s, z, random_matrices, tau = state
         tgt_len, bsz, embed_dim = query.size()
         assert embed_dim == self.embed_dim
+        if rfa_hip.native is not None and self.fuse_projections:
+            attn = rfa_hip.native.node_cross_query(query, random_matrices, self.q_proj.weight, self.q_proj.bias,
+                                                   self.num_heads, SCALE, s, z)
+            if attn is not None:
+                return linear_out(attn, self.out_proj)
         if self.fuse_projections and fused_projection_supported(query, (self.q_proj,), self.num_heads, random_matrices):
             # q projection, the view to heads and phi(q) in one launch
             (phi_q,) = project_heads(query, (self.q_proj,), (True,), self.num_heads, random_matrices, SCALE)

@@ -1,0 +1,473 @@
+// The package's autograd functions as C++ nodes, and the chains of them that one call of a module is.
+//
+// The Python autograd functions (rfa_amd/rfa.py, utils.py, projection.py, causal_attention.py,
+// cross_attention.py) are the general form: any dtype, either binding, tracing, dispatch modes,
+// functorch's errors.  What a training or serving step does -- plain fp16 tensors on one HIP
+// device -- comes here instead: the same launches in the same order, without an interpreter between
+// them.  Each entry point returns nothing when a tensor or the mode is not plain (see plain()), and
+// the caller then goes its general way; errors in shapes are raised by the same checks as there.
+//
+// What bounds a layer without this is the host: 8 heads of 64, 8192 tokens, forward + backward is 215 us
+// of kernels; issued through four Python functions and their backwards it took 456 us, from here 298
+// (128 tokens of 4 heads, the scan alone: 114 -> 68; encoder-decoder layer, 16384 + 8192 rows: 574 -> 430).
+#pragma once
+#include <ATen/ThreadLocalState.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+
+namespace {
+
+using OptTensor = c10::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ---- which calls are plain ------------------------------------------------------------
+// Tracing must record the Python functions, dispatch modes and tensor subclasses must see them, and
+// functorch's wrappers and forward-mode tangents must meet the errors that those raise.
+bool plain_mode() {
+    return !torch::jit::tracer::isTracing() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+bool plain(const Tensor& t, torch::ScalarType type, int64_t dim) {
+    static const c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                          c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Batched,
+                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Negative,
+                                          c10::DispatchKey::Conjugate});
+    return t.defined() && t.is_cuda() && t.scalar_type() == type && t.dim() == dim && t.layout() == c10::kStrided &&
+           !t.key_set().has_any(odd) && !t._fw_grad(0).defined();
+}
+
+bool plain_half(const Tensor& t, int64_t dim) { return plain(t, torch::kFloat16, dim); }
+bool plain_half(const OptTensor& t, int64_t dim) { return !t.has_value() || plain(*t, torch::kFloat16, dim); }
+
+template <typename... T>
+bool wants_grad(const T&... t) {
+    return at::GradMode::is_enabled() && (... || (t.defined() && t.requires_grad()));
+}
+bool wants_grad_opt(const OptTensor& t) { return t.has_value() && t->requires_grad(); }
+
+Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : c10::nullopt; }
+
+// ---- random matrices --------------------------------------------------------------------
+struct BuildNode : public torch::autograd::Function<BuildNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& w, const OptTensor& sigma, double tau) {
+        const Tensor wc = w.contiguous();
+        const OptTensor sg = sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt;
+        ctx->saved_data["tau"] = tau;
+        ctx->saved_data["need_w"] = w.requires_grad();
+        ctx->saved_data["need_sigma"] = wants_grad_opt(sigma);
+        ctx->save_for_backward({wc, opt(sg)});
+        return build_random_matrices(wc, sg, tau);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [dsigma, dw] = build_random_matrices_backward(saved[0], opt(saved[1]), g[0].contiguous(),
+                                                           ctx->saved_data["tau"].toDouble(),
+                                                           ctx->saved_data["need_sigma"].toBool(),
+                                                           ctx->saved_data["need_w"].toBool());
+        return {opt(dw), opt(dsigma), Tensor()};
+    }
+};
+
+Tensor build_matrices(const Tensor& w, const OptTensor& sigma, double tau) {
+    if (at::GradMode::is_enabled() && (w.requires_grad() || wants_grad_opt(sigma))) return BuildNode::apply(w, sigma, tau);
+    return build_random_matrices(w.contiguous(), sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt, tau);
+}
+
+// tau = 0 or matrices that are not fp16 [H, D, d] with sigma [H, 1, d] take the ATen chain
+bool plain_matrices(const Tensor& w, const OptTensor& sigma, double tau) {
+    return plain_half(w, 3) && tau != 0 &&
+           (!sigma.has_value() || (plain_half(*sigma, 3) && sigma->size(0) == w.size(0) && sigma->size(1) == 1 &&
+                                   sigma->size(2) == w.size(2)));
+}
+
+// ---- feature map ------------------------------------------------------------------------
+struct FeatureNode : public torch::autograd::Function<FeatureNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double scale) {
+        const Tensor xc = x.contiguous(), wc = w.contiguous();
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["need_w"] = w.requires_grad();
+        ctx->save_for_backward({xc, wc});
+        return feature_map_forward(xc, wc, scale);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [dx, dw] = feature_map_backward(saved[0], saved[1], g[0].contiguous(), ctx->saved_data["scale"].toDouble(),
+                                             ctx->saved_data["need_w"].toBool());
+        return {dx, dw.has_value() ? dw->to(torch::kFloat16) : Tensor(), Tensor()};
+    }
+};
+
+OptTensor node_random_project(const Tensor& x, const Tensor& w, double scale) {
+    if (!plain_mode() || !plain_half(x, 4) || !plain_half(w, 3)) return c10::nullopt;
+    if (wants_grad(x, w)) return FeatureNode::apply(x, w, scale);
+    return feature_map_forward(x.contiguous(), w.contiguous(), scale);
+}
+
+// ---- projections to heads, with the feature map where a bit of `phi` is set ----------------------
+// The weights and biases of up to three Linear layers over one input; unused places are empty.
+struct Layers {
+    std::vector<Tensor> w;
+    std::vector<OptTensor> b;
+    bool phi[3] = {false, false, false};
+};
+
+std::vector<bool> phi_flags(const Layers& l) { return std::vector<bool>(l.phi, l.phi + l.w.size()); }
+
+// (dW, db) of Linear layers that share the input x2: one row-split launch where the widths allow it
+std::pair<std::vector<Tensor>, std::vector<OptTensor>> param_grads(const Tensor& x2, const std::vector<Tensor>& dys,
+                                                                   const std::vector<bool>& bias) {
+    if (dys[0].size(1) % 128 == 0 && x2.size(1) % 128 == 0) {
+        std::vector<Tensor> c;
+        for (const Tensor& dy : dys) c.push_back(dy.contiguous());
+        auto [dws, dbs] = linear_weight_grad(x2.contiguous(), c, bias);
+        return {dws, dbs};
+    }
+    std::vector<Tensor> dws;
+    std::vector<OptTensor> dbs;
+    for (size_t p = 0; p < dys.size(); ++p) {
+        dws.push_back(at::mm(dys[p].t(), x2));
+        dbs.push_back(bias[p] ? OptTensor(dys[p].sum(0)) : c10::nullopt);
+    }
+    return {dws, dbs};
+}
+
+struct ProjectNode : public torch::autograd::Function<ProjectNode> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& wf, double scale, int64_t heads,
+                                 int64_t phi, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
+                                 const OptTensor& b1, const OptTensor& w2, const OptTensor& b2) {
+        Layers l;
+        for (const auto& [w, b] : {std::pair(&w0, &b0), std::pair(&w1, &b1), std::pair(&w2, &b2)}) {
+            if (!w->has_value()) break;
+            l.phi[l.w.size()] = (phi >> l.w.size()) & 1;
+            l.w.push_back((*w)->contiguous());
+            l.b.push_back(*b);
+        }
+        const OptTensor wfc = wf.has_value() ? OptTensor(wf->contiguous()) : c10::nullopt;
+        auto [ys, phis] = project_feature_map(x.contiguous(), l.w, l.b, phi_flags(l), wfc, heads, scale, true);
+        int64_t bias = 0;
+        variable_list keep{x, opt(wfc)}, out;
+        for (const OptTensor& w : {w0, w1, w2})
+            if (w.has_value()) keep.push_back(*w);
+        for (size_t p = 0; p < l.w.size(); ++p) {
+            bias |= (int64_t)l.b[p].has_value() << p;
+            if (l.phi[p]) keep.push_back(*ys[p]);
+            out.push_back(l.phi[p] ? *phis[p] : *ys[p]);
+        }
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["phi"] = phi;
+        ctx->saved_data["bias"] = bias;
+        ctx->saved_data["n"] = (int64_t)l.w.size();
+        ctx->saved_data["need_x"] = x.requires_grad();
+        ctx->saved_data["need_wf"] = wants_grad_opt(wf);
+        ctx->save_for_backward(keep);
+        return out;
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const int64_t n = ctx->saved_data["n"].toInt(), phi = ctx->saved_data["phi"].toInt();
+        const int64_t bias_bits = ctx->saved_data["bias"].toInt();
+        const double scale = ctx->saved_data["scale"].toDouble();
+        const bool need_x = ctx->saved_data["need_x"].toBool(), need_wf = ctx->saved_data["need_wf"].toBool();
+        const Tensor &x = saved[0], &wf = saved[1];
+        const Tensor* const w = &saved[2];
+        const Tensor* const y = &saved[2 + n];
+        const int64_t rows = x.size(0) * x.size(1);
+        const Tensor x2 = x.reshape({rows, x.size(2)});
+        variable_list out(11);                    // x, wf, scale, heads, phi, w0, b0, w1, b1, w2, b2
+        std::vector<bool> bias;
+        for (int64_t p = 0; p < n; ++p) bias.push_back((bias_bits >> p) & 1);
+        OptTensor dwf;
+        if (n == 3 && phi == 3 && need_x) {
+            // [dy_q | dy_k | dv] side by side, written by the feature-map backward launch itself: one
+            // GEMM for dx and one contraction for the three weight gradients
+            const int64_t e_out = w[0].size(0);
+            Tensor packed;
+            std::tie(packed, dwf) = feature_map_backward_pair_packed(y[0], y[1], wf, g[0].contiguous(), g[1].contiguous(),
+                                                                     g[2].contiguous(), scale, need_wf);
+            out[0] = at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
+            auto [dws, dbs] = param_grads(x2, {packed}, {bias_bits != 0});
+            for (int64_t p = 0; p < n; ++p) {
+                out[5 + 2 * p] = dws[0].narrow(0, p * e_out, e_out);
+                if (bias[p]) out[6 + 2 * p] = dbs[0]->narrow(0, p * e_out, e_out);
+            }
+        } else {
+            std::vector<Tensor> dys(n);
+            if (n >= 2 && (phi & (phi - 1)) != 0 && phi != 7) {          // two of them: one launch
+                const int p0 = (phi & 1) ? 0 : 1, p1 = (phi & 4) ? 2 : 1;
+                std::tie(dys[p0], dys[p1], dwf) = feature_map_backward_pair(y[0], y[1], wf, g[p0].contiguous(),
+                                                                            g[p1].contiguous(), scale, need_wf);
+            }
+            int64_t yi = 0;
+            for (int64_t p = 0; p < n; ++p) {
+                if (!dys[p].defined()) {
+                    dys[p] = g[p].contiguous();
+                    if ((phi >> p) & 1) {
+                        OptTensor dw;
+                        std::tie(dys[p], dw) = feature_map_backward(y[yi++], wf, dys[p], scale, need_wf);
+                        if (dw.has_value()) dwf = dwf.has_value() ? *dwf + *dw : *dw;
+                    }
+                }
+                dys[p] = dys[p].reshape({rows, -1});
+                if (need_x) out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
+            }
+            auto [dws, dbs] = param_grads(x2, dys, bias);
+            for (int64_t p = 0; p < n; ++p) {
+                out[5 + 2 * p] = dws[p];
+                out[6 + 2 * p] = opt(dbs[p]);
+            }
+            if (out[0].defined()) out[0] = out[0].view(x.sizes());
+        }
+        if (dwf.has_value()) out[1] = dwf->to(torch::kFloat16);
+        return out;
+    }
+};
+
+// what the fused launch takes (rfa_amd/projection.py: fused_projection_supported)
+bool plain_layers(const Tensor& x, const OptTensor& wf, const Layers& l, int64_t heads) {
+    if (!plain_half(x, 3)) return false;
+    const Tensor& w0 = l.w[0];
+    for (size_t p = 0; p < l.w.size(); ++p)
+        if (!plain_half(l.w[p], 2) || l.w[p].sizes() != w0.sizes() || !plain_half(l.b[p], 1)) return false;
+    const int64_t out = w0.size(0), in = w0.size(1);
+    if (in != x.size(2) || in % 64 != 0 || out % heads != 0 || (out / heads != 64 && out / heads != 128)) return false;
+    return !wf.has_value() ||
+           (plain_half(*wf, 3) && (wf->size(1) == 32 || wf->size(1) == 64 || wf->size(1) == 128));
+}
+
+std::vector<Tensor> project(const Tensor& x, const OptTensor& wf, double scale, int64_t heads, const Layers& l) {
+    bool grad = x.requires_grad() || wants_grad_opt(wf);
+    int64_t phi = 0;
+    for (size_t p = 0; p < l.w.size(); ++p) {
+        grad = grad || l.w[p].requires_grad() || wants_grad_opt(l.b[p]);
+        phi |= (int64_t)l.phi[p] << p;
+    }
+    auto w = [&](size_t p) { return p < l.w.size() ? OptTensor(l.w[p]) : c10::nullopt; };
+    auto b = [&](size_t p) { return p < l.w.size() ? l.b[p] : c10::nullopt; };
+    if (grad && at::GradMode::is_enabled())
+        return ProjectNode::apply(x, wf, scale, heads, phi, w(0), b(0), w(1), b(1), w(2), b(2));
+    std::vector<Tensor> wc, out;
+    for (const Tensor& t : l.w) wc.push_back(t.contiguous());
+    auto [ys, phis] = project_feature_map(x.contiguous(), wc, l.b, phi_flags(l),
+                                          wf.has_value() ? OptTensor(wf->contiguous()) : c10::nullopt, heads, scale, false);
+    for (size_t p = 0; p < l.w.size(); ++p) out.push_back(l.phi[p] ? *phis[p] : *ys[p]);
+    return out;
+}
+
+// ---- Linear layer on the way out ------------------------------------------------------------
+struct LinearNode : public torch::autograd::Function<LinearNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& b) {
+        ctx->saved_data["bias"] = b.has_value();
+        ctx->saved_data["need_x"] = x.requires_grad();
+        ctx->save_for_backward({x, w});
+        return at::linear(x, w, b);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &w = saved[1];
+        const Tensor dy2 = g[0].reshape({-1, g[0].size(-1)}), x2 = x.reshape({-1, x.size(-1)});
+        Tensor dx;
+        if (ctx->saved_data["need_x"].toBool()) dx = at::mm(dy2, w).view(x.sizes());
+        auto [dws, dbs] = param_grads(x2, {dy2}, {ctx->saved_data["bias"].toBool()});
+        return {dx, dws[0], opt(dbs[0])};
+    }
+};
+
+// for the callers' condition (fp16, grad mode on, widths that are multiples of 128) see linear_out
+OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
+    if (!plain_mode() || !plain_half(x, x.dim()) || !plain_half(w, 2) || !plain_half(b, 1)) return c10::nullopt;
+    return LinearNode::apply(x, w, b);
+}
+
+// ---- causal attention -------------------------------------------------------------------------
+// phi_q, phi_k [T, B, H, K], v [T, B, H, d] -> attn [T, B, H * d], through the saving pair
+struct ScanDims {
+    int64_t T, N;
+    int K, d;
+    explicit ScanDims(const Tensor& q, const Tensor& v)
+        : T(q.size(0)), N(q.size(1) * q.size(2)), K((int)q.size(3)), d((int)v.size(3)) {}
+};
+
+Tensor scan_output(const Tensor& v) { return torch::empty({v.size(0), v.size(1), v.size(2) * v.size(3)}, v.options()); }
+
+struct CausalNode : public torch::autograd::Function<CausalNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& phi_q, const Tensor& phi_k, const Tensor& values) {
+        const Tensor q = phi_q.contiguous(), k = phi_k.contiguous(), v = values.contiguous();
+        const ScanDims n(q, v);
+        Tensor attn = scan_output(v);
+        Launch l(q);
+        const size_t nbytes = rfa_causal_forward_workspace_bytes(n.T, n.N, n.K, n.d);
+        const size_t sbytes = rfa_causal_saved_state_bytes(n.T, n.N, n.K, n.d);
+        Tensor ws = workspace(nbytes, q), state = workspace(sbytes, q);
+        check_rc(rfa_causal_forward_save(ptr(q), ptr(k), ptr(v), ptr(attn), ptr(state), sbytes, n.T, n.N, n.K, n.d, ptr(ws),
+                                         nbytes, l.stream));
+        ctx->save_for_backward({q, k, v, attn, state});
+        return attn;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &state = saved[4];
+        const Tensor attn = saved[3].contiguous(), grad = g[0].contiguous();
+        const ScanDims n(q, v);
+        Tensor dq = torch::empty_like(q), dk = torch::empty_like(k), dv = torch::empty_like(v);
+        Launch l(q);
+        const size_t nbytes = rfa_causal_backward_saved_workspace_bytes(ptr(state), n.T, n.N, n.K, n.d);
+        Tensor ws = workspace(nbytes, q);
+        check_rc(rfa_causal_backward_saved(ptr(q), ptr(k), ptr(v), ptr(grad), ptr(attn), ptr(state), (size_t)state.numel(),
+                                           ptr(dq), ptr(dk), ptr(dv), n.T, n.N, n.K, n.d, ptr(ws), nbytes, l.stream));
+        return {dq, dk, dv};
+    }
+};
+
+bool plain_scan(const Tensor& q, const Tensor& k, const Tensor& v) {
+    return plain_half(q, 4) && plain_half(k, 4) && plain_half(v, 4) && q.sizes() == k.sizes() && v.size(0) == q.size(0) &&
+           v.size(1) == q.size(1) && v.size(2) == q.size(2) && q.device() == k.device() && q.device() == v.device();
+}
+
+Tensor causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& values) {
+    if (wants_grad(phi_q, phi_k, values)) return CausalNode::apply(phi_q, phi_k, values);
+    const Tensor q = phi_q.contiguous(), k = phi_k.contiguous(), v = values.contiguous();
+    const ScanDims n(q, v);
+    Tensor attn = scan_output(v);
+    Launch l(q);
+    const size_t nbytes = rfa_causal_forward_workspace_bytes(n.T, n.N, n.K, n.d);
+    Tensor ws = workspace(nbytes, q);
+    check_rc(rfa_causal_forward(ptr(q), ptr(k), ptr(v), ptr(attn), n.T, n.N, n.K, n.d, ptr(ws), nbytes, l.stream));
+    return attn;
+}
+
+OptTensor node_causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v) {
+    if (!plain_mode() || !plain_scan(phi_q, phi_k, v)) return c10::nullopt;
+    return causal(phi_q, phi_k, v);
+}
+
+// q, k, v projections, phi(q) and phi(k), the scan: x [T, B, E] -> attn [T, B, H * d].  `matrices` is
+// W' itself where `build` is false.
+OptTensor node_causal_layer(const Tensor& x, const Tensor& matrices, const OptTensor& sigma, double tau, bool build,
+                            const std::vector<Tensor>& weights, const std::vector<OptTensor>& biases, int64_t heads,
+                            double scale) {
+    Layers l{weights, biases, {true, true, false}};
+    if (!plain_mode() || weights.size() != 3 || biases.size() != 3 || !plain_layers(x, matrices, l, heads) ||
+        (build && !plain_matrices(matrices, sigma, tau)))
+        return c10::nullopt;
+    const Tensor w = build ? build_matrices(matrices, sigma, tau) : matrices;
+    const auto out = project(x, w, scale, heads, l);
+    return causal(out[0], out[1], out[2]);
+}
+
+// ---- quadratic form with explicit masks ---------------------------------------------------------
+struct MaskedNode : public torch::autograd::Function<MaskedNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& phi_q, const Tensor& phi_k, const Tensor& values,
+                          const OptTensor& pad, const OptTensor& mask, const OptTensor& mask_t) {
+        const Tensor q = phi_q.contiguous(), k = phi_k.contiguous(), v = values.contiguous();
+        auto [out, rsum] = masked_forward(q.flatten(1, 2), k.flatten(1, 2), v.flatten(1, 2), q.size(2), pad, mask);
+        Tensor attn = at::_unsafe_view(out, {v.size(0), v.size(1), v.size(2) * v.size(3)});
+        ctx->saved_data["pad"] = pad;
+        ctx->saved_data["mask"] = mask;
+        ctx->saved_data["mask_t"] = mask_t;
+        ctx->save_for_backward({q, k, v, attn, rsum});
+        return attn;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2];
+        const Tensor v3 = v.flatten(1, 2);
+        auto mask = [&](const char* name) { return ctx->saved_data[name].toOptional<Tensor>(); };
+        auto grads = masked_backward(q.flatten(1, 2), k.flatten(1, 2), v3, g[0].contiguous().view(v3.sizes()),
+                                     saved[3].contiguous().view(v3.sizes()), saved[4], q.size(2), mask("pad"), mask("mask"),
+                                     mask("mask_t"));
+        return {grads[0].view(q.sizes()), grads[1].view(k.sizes()), grads[2].view(v.sizes()), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+OptTensor node_masked(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v, const OptTensor& pad, const OptTensor& mask,
+                      const OptTensor& mask_t) {
+    if (!plain_mode() || !plain_scan(phi_q, phi_k, v) || phi_q.numel() == 0 || !wants_grad(phi_q, phi_k, v))
+        return c10::nullopt;
+    return MaskedNode::apply(phi_q, phi_k, v, pad, mask, mask_t);
+}
+
+// ---- cross attention ------------------------------------------------------------------------------
+struct CrossStateNode : public torch::autograd::Function<CrossStateNode> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& phi_k, const Tensor& values, const OptTensor& pad) {
+        const Tensor k = phi_k.contiguous(), v = values.contiguous();
+        auto [s, z] = cross_state(k, v, pad);
+        ctx->saved_data["pad"] = pad;
+        ctx->save_for_backward({k, v});
+        return {s, z};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        auto [dk, dv] = cross_state_backward(saved[0], saved[1], g[0].contiguous(), g[1].contiguous(),
+                                             ctx->saved_data["pad"].toOptional<Tensor>());
+        return {dk, dv, Tensor()};
+    }
+};
+
+// phi_q [T, B, H, K], s, z -> attn [T, B, H * d]
+struct CrossReadoutNode : public torch::autograd::Function<CrossReadoutNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& phi_q, const Tensor& s, const Tensor& z) {
+        const Tensor q = phi_q.contiguous(), sc = s.contiguous(), zc = z.contiguous();
+        ctx->save_for_backward({q, sc, zc});
+        const Tensor out = cross_readout(q, sc, zc);
+        return at::_unsafe_view(out, {out.size(0), out.size(1), out.size(2) * out.size(3)});
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &s = saved[1];
+        auto [dq, ds, dz] = cross_readout_backward(q, s, saved[2],
+                                                   g[0].contiguous().view({q.size(0), q.size(1), q.size(2), s.size(3)}));
+        return {dq, ds, dz};
+    }
+};
+
+// the source side of a layer: enc [S, B, E], pad [B, S] -> (s, z, W')
+c10::optional<std::tuple<Tensor, Tensor, Tensor>> node_cross_source(
+    const Tensor& enc, const Tensor& matrices, const OptTensor& sigma, double tau, const std::vector<Tensor>& weights,
+    const std::vector<OptTensor>& biases, int64_t heads, double scale, const OptTensor& pad) {
+    Layers l{weights, biases, {true, false, false}};
+    if (!plain_mode() || weights.size() != 2 || biases.size() != 2 || !plain_layers(enc, matrices, l, heads) ||
+        !plain_matrices(matrices, sigma, tau))
+        return c10::nullopt;
+    const Tensor w = build_matrices(matrices, sigma, tau);
+    const auto out = project(enc, w, scale, heads, l);
+    if (wants_grad(out[0], out[1])) {
+        const auto state = CrossStateNode::apply(out[0], out[1], pad);
+        return std::tuple(state[0], state[1], w);
+    }
+    auto [s, z] = cross_state(out[0], out[1], pad);
+    return std::tuple(s, z, w);
+}
+
+// the target side up to the output projection: query [T, B, E] -> attn [T, B, H * d]
+OptTensor node_cross_query(const Tensor& query, const Tensor& w, const Tensor& weight, const OptTensor& bias, int64_t heads,
+                           double scale, const Tensor& s, const Tensor& z) {
+    Layers l{{weight}, {bias}, {true, false, false}};
+    if (!plain_mode() || !plain_layers(query, w, l, heads) || !plain(s, torch::kFloat32, 4) || !plain(z, torch::kFloat32, 3))
+        return c10::nullopt;
+    const auto phi_q = project(query, w, scale, heads, l)[0];
+    if (wants_grad(phi_q, s, z)) return CrossReadoutNode::apply(phi_q, s, z);
+    const Tensor out = cross_readout(phi_q, s.contiguous(), z.contiguous());
+    return out.view({out.size(0), out.size(1), out.size(2) * out.size(3)});
+}
+
+void bind_nodes(pybind11::module_& m) {
+    namespace py = pybind11;
+    // each returns None where the call is not plain: the caller's general path takes it
+    m.def("node_random_project", &node_random_project, py::arg("x"), py::arg("w"), py::arg("scale"));
+    m.def("node_linear", &node_linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
+    m.def("node_causal", &node_causal, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"));
+    m.def("node_causal_layer", &node_causal_layer, py::arg("x"), py::arg("matrices"), py::arg("sigma"), py::arg("tau"),
+          py::arg("build"), py::arg("weights"), py::arg("biases"), py::arg("heads"), py::arg("scale"));
+    m.def("node_masked", &node_masked, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("key_padding_mask"),
+          py::arg("mask"), py::arg("mask_t"));
+    m.def("node_cross_source", &node_cross_source, py::arg("enc"), py::arg("matrices"), py::arg("sigma"), py::arg("tau"),
+          py::arg("weights"), py::arg("biases"), py::arg("heads"), py::arg("scale"), py::arg("key_padding_mask"));
+    m.def("node_cross_query", &node_cross_query, py::arg("query"), py::arg("w"), py::arg("weight"), py::arg("bias"),
+          py::arg("heads"), py::arg("scale"), py::arg("s"), py::arg("z"));
+}
+
+}  // namespace

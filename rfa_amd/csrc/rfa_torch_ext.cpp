@@ -588,6 +588,8 @@ void selftest_layout() {
 
 }  // namespace
 
+#include "rfa_autograd.h"
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "PyTorch-ROCm binding of librfa_hip.so (Random Feature Attention kernels for MI355X)";
     namespace py = pybind11;
@@ -633,4 +635,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("masked_backward", &masked_backward, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("grad_attn"),
           py::arg("out"), py::arg("rsum"), py::arg("H"), py::arg("key_padding_mask") = py::none(),
           py::arg("attn_mask_bytes") = py::none(), py::arg("attn_mask_t_bytes") = py::none());
+    bind_nodes(m);
 }

@@ -192,5 +192,9 @@ def linear_out(x: Tensor, layer: nn.Linear) -> Tensor:
     if (x.is_cuda and x.dtype == torch.float16 and w.dtype == torch.float16 and torch.is_grad_enabled()
             and (w.requires_grad or x.requires_grad) and rfa_hip.linear_weight_grad_supported(*w.shape)
             and (layer.bias is None or layer.bias.dtype == torch.float16)):
+        if rfa_hip.native is not None:
+            y = rfa_hip.native.node_linear(x, w, layer.bias)
+            if y is not None:
+                return y
         return _LinearOut.apply(x, w, layer.bias)
     return layer(x)

@@ -713,8 +713,14 @@ _BOUND = ("supported", "feature_map_supported", "selftest_layout", "forward", "b
           "cross_state_backward", "cross_readout", "cross_readout_backward", "incremental", "incremental_fused",
           "incremental_qkv",
           "pack_negative_mask", "masked_forward", "masked_backward")
+# autograd functions and chains of them as C++ nodes (csrc/rfa_autograd.h): only the binding has them
+_NODES = ("node_random_project", "node_linear", "node_causal", "node_causal_layer", "node_masked", "node_cross_source",
+          "node_cross_query")
 _CTYPES_IMPL = {name: globals()[name] for name in _BOUND}
 _active = "ctypes"
+# the module with the _NODES while the binding is "ext", else None.  Each node answers None where a call
+# is not plain fp16 tensors on a HIP device in an ordinary mode; callers then take their general path.
+native = None
 
 _ext = None
 
@@ -730,7 +736,7 @@ def _resolve_ext():
             mod = importlib.import_module(__package__ + "._rfa_hip_ext")   # built by rfa_amd.build.build_ext
         except ImportError:
             mod = None
-        if mod is not None and not all(hasattr(mod, n) for n in _BOUND):
+        if mod is not None and not all(hasattr(mod, n) for n in _BOUND + _NODES):
             # built from older sources than this file (the build itself imports the package first):
             # unusable until rebuilt, and a rebuilt file needs a fresh process to be loaded
             import warnings
@@ -751,7 +757,7 @@ def binding() -> str:
 
 
 def use_binding(name: str) -> None:
-    global _active
+    global _active, native
     if name == "ext":
         if _resolve_ext() is None:
             raise ImportError("the torch binding _rfa_hip_ext has not been built (python -m rfa_amd.build)")
@@ -761,6 +767,7 @@ def use_binding(name: str) -> None:
     else:
         raise ValueError(f"binding must be 'ext' or 'ctypes' (got {name!r})")
     globals().update(impl)
+    native = _ext if name == "ext" else None
     _active = name
 
 

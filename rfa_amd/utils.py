@@ -170,6 +170,10 @@ def random_project(*, x: Tensor, random_matrices: Tensor, scale: float = SCALE) 
     -> [seq_len, bsz, num_heads, 2 * proj_dim].  ``scale`` defaults to the reference's
     constant 0.1; pass proj_dim ** -0.5 for the variance-normalised map.
     """
+    if rfa_hip.native is not None:
+        phi = rfa_hip.native.node_random_project(x, random_matrices, scale)
+        if phi is not None:
+            return phi
     return _FeatureMap.apply(x, random_matrices, scale)
 
 

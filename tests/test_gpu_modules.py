@@ -434,3 +434,121 @@ def test_pack_negative_mask_matches_the_general_packing(T, dtype):
             rfa_hip.pack_negative_mask(base[:2, :3])
         with pytest.raises((RuntimeError, TypeError)):
             rfa_hip.pack_negative_mask(base[:3, :3].to(torch.int32))
+
+
+def _native_forms(path, form):
+    """(run, leaves) of one path in one form of its inputs; run() -> outputs whose sum of products is differentiated."""
+    from rfa_amd import causal_attention as C, cross_attention as X, utils
+    T, B, H, d, D = 37, 3, 2, 64, 32
+    E = H * d
+    gen = torch.Generator("cuda").manual_seed(5)
+    grad = form != "no_grad"
+
+    def leaf(*shape, scale=None):
+        x = torch.randn(*shape, generator=gen, device="cuda")
+        if scale is not None:           # feature values of one sign: no row sum near zero
+            x = scale * x.abs()
+        if form == "strided":       # every second entry of a wider tensor, batch and time swapped in memory
+            wide = torch.zeros(shape[1], shape[0], *shape[2:-1], 2 * shape[-1], device="cuda", dtype=torch.float16)
+            wide[..., ::2] = x.half().transpose(0, 1)
+            return wide[..., ::2].transpose(0, 1).detach().requires_grad_(grad)
+        return x.half().requires_grad_(grad)
+
+    def layer(cls):
+        torch.manual_seed(7)
+        m = cls(embed_dim=E, num_heads=H, head_dim=d, proj_dim=D).cuda().half()
+        if form == "no_bias":
+            for lin in m.children():
+                lin.bias = None
+        if form == "frozen":
+            for p in m.parameters():
+                p.requires_grad_(False)
+        return m
+
+    W = O.make_w(d, D, H).cuda().half()
+    if path == "random_project":
+        x = leaf(T, B, H, d)
+        w = W.clone().requires_grad_(grad and form != "frozen")
+        return lambda: utils.random_project(x=x, random_matrices=w), [x, w]
+    if path in ("causal", "masked"):
+        q, k, v = leaf(T, B, H, 2 * D, scale=0.1), leaf(T, B, H, 2 * D, scale=0.1), leaf(T, B, H, d)
+        if form == "frozen":
+            k = k.detach()
+        if path == "causal":
+            return lambda: C.cuda_causal_rfa(phi_q=q, phi_k=k, v=v), [q, k, v]
+        pad = torch.zeros(B, T, dtype=torch.bool, device="cuda")
+        pad[0, 30:] = True
+        mask = torch.full((T, T), float("-inf"), device="cuda").triu(1)
+        return lambda: C.masked_rfa(phi_q=q, phi_k=k, v=v, key_padding_mask=pad, attn_mask=mask), [q, k, v]
+    x = leaf(T, B, E)
+    if path == "module":
+        m = layer(C.CausalAttention)
+        return lambda: m(x, W), [x, *m.parameters()]
+    enc = leaf(T + 4, B, E)
+    src, m = layer(X.CrossAttentionProjectLayer), layer(X.CrossAttention)
+    mask = torch.zeros(T + 4, B, 1, 1, dtype=torch.bool, device="cuda")
+    mask[T:, 1] = True
+    return (lambda: m(x, src(encoder_output=enc, random_matrices=W, mask=mask)),
+            [x, enc, *src.parameters(), *m.parameters()])
+
+
+@pytest.mark.parametrize("form", ["plain", "strided", "frozen", "no_bias", "no_grad", "hooks", "twice"])
+@pytest.mark.parametrize("path", ["random_project", "causal", "masked", "module", "cross"])
+def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypatch):
+    """The C++ autograd nodes against the Python autograd functions over the same kernels: outputs and every
+    gradient bit for bit, from strided inputs, with frozen or missing parameters, through saved-tensor
+    hooks, and with two backward passes over one graph."""
+    from rfa_amd import rfa_hip
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    print(f"native nodes: {path} {form}", flush=True)
+    run, leaves = _native_forms(path, form)
+    results = []
+    for native in (rfa_hip.native, None):
+        monkeypatch.setattr(rfa_hip, "native", native)
+        for t in leaves:
+            t.grad = None
+        packed = []
+        if form == "hooks":
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t.clone(), lambda t: t):
+                out = run()
+            assert packed
+        else:
+            with torch.set_grad_enabled(form != "no_grad"):
+                out = run()
+        assert out.is_contiguous() and out.requires_grad == (form != "no_grad")
+        if form != "no_grad":
+            g = torch.randn(out.shape, generator=torch.Generator("cuda").manual_seed(9), device="cuda").half()
+            out.backward(g, retain_graph=form == "twice")
+            if form == "twice":
+                out.backward(g)
+        results.append([out.detach()] + [None if t.grad is None else t.grad.clone() for t in leaves])
+    for a, b in zip(*results):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+def test_native_nodes_leave_odd_calls_to_the_python_functions():
+    """Dispatch modes and tracing see the Python functions, and functorch transforms and forward-mode
+    tangents meet the errors that those raise."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from rfa_amd import rfa_hip
+    from rfa_amd.causal_attention import cuda_causal_rfa
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    q, k, v = (torch.randn(9, 2, 2, n, device="cuda").half().requires_grad_() for n in (64, 64, 64))
+    call = lambda a: cuda_causal_rfa(phi_q=a, phi_k=k, v=v)
+    assert rfa_hip.native.node_causal(q, k, v) is not None
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        assert rfa_hip.native.node_causal(q, k, v) is None
+        call(q)
+    assert rfa_hip.native.node_causal(q.float(), k, v) is None
+    assert rfa_hip.native.node_causal(q.cpu(), k, v) is None
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda a: call(a).float().sum())(q.detach())
+    with pytest.raises(RuntimeError), forward_ad.dual_level():
+        call(forward_ad.make_dual(q.detach(), torch.ones_like(q)))
