@@ -233,6 +233,12 @@ int rfa_feature_map_backward_pair_packed(const void* x0, const void* x1, const v
                                          int64_t R, int H, int D, int d, float scale, void* workspace,
                                          size_t workspace_bytes, void* stream);
 
+/* y = x W^T + b (torch.nn.Linear) for few rows, a decoding step's projections:
+ *   x fp16 [R, E_in], w fp16 [E_out, E_in], bias fp16 [E_out] or NULL, y fp16 [R, E_out];
+ *   fp32 sums, E_in a multiple of 32 and E_out of 16.  Right for any R, meant for R up to a few hundred. */
+int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int64_t R, int e_in, int e_out,
+                    void* stream);
+
 /* ---------------------------------------------------------------------------
  * Linear projections to heads with the feature map in the epilogue.
  *

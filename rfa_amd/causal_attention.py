@@ -20,7 +20,7 @@ from torch.nn import Parameter
 
 from . import rfa_hip
 from ._derived import derived
-from .projection import fused_projection_supported, linear_out, project_heads
+from .projection import fused_projection_supported, linear_out, linear_rows, project_heads
 from .rfa import RFA
 from .utils import (EPS, SCALE, build_random_matrices, random_project, random_project_pair,
                     upgrade_state_dict_named)
@@ -282,7 +282,10 @@ class CausalAttention(nn.Module):
             if not self.decode_inplace and (s is s_in or z is z_in):
                 s_out, z_out = torch.empty_like(s), torch.empty_like(z)
             weight, bias = self._stacked_qkv()
-            rows = F.linear(x, weight, bias).view(tgt_len, bsz, 3, self.num_heads, self.head_dim)
+            rows = linear_rows(x, weight, bias)
+            if rows is None:
+                rows = F.linear(x, weight, bias)
+            rows = rows.view(tgt_len, bsz, 3, self.num_heads, self.head_dim)
             attn = rfa_hip.incremental_qkv(rows, w.to(torch.float16).contiguous(), SCALE, s, z, s_out, z_out)
             if s_out is not None:
                 s, z = s_out, z_out

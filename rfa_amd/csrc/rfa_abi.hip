@@ -46,14 +46,14 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
                                    "k_masked_fwd", "k_masked_bwd_prep", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
-                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask"};
+                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -1830,6 +1830,36 @@ int rfa_project_feature_map(const void* x, const void* const* weights, const voi
     RFA_DISPATCH_FEATURE(D, d, RFA_CALL)
 #undef RFA_CALL
     return fail(RFA_ERR_UNSUPPORTED, "unreachable");
+}
+
+int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int64_t R, int e_in, int e_out, void* stream) {
+    if (R < 0 || R > (1 << 20) || e_in <= 0 || e_out <= 0)
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_rows: bad sizes R=%lld E_in=%d E_out=%d", (long long)R, e_in, e_out);
+    if (e_in % 32 != 0 || e_out % 16 != 0)
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_linear_rows: E_in must be a multiple of 32 and E_out of 16 (got %d, %d)", e_in, e_out);
+    if (R == 0) return RFA_OK;
+    if (!x || !w || !y) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_rows: NULL tensor pointer");
+    if (!aligned16(x) || !aligned16(w) || !aligned16(y))
+        return fail(RFA_ERR_ALIGNMENT, "rfa_linear_rows: tensors must be 16-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto* xh = static_cast<const rfa::half_t*>(x);
+    auto* wh = static_cast<const rfa::half_t*>(w);
+    auto* bh = static_cast<const rfa::half_t*>(bias);
+    auto* yh = static_cast<rfa::half_t*>(y);
+    const int rt = R <= 16 ? 1 : R <= 32 ? 2 : 4;
+    // two tiles of columns per workgroup (half the reads of x) once one tile each would overfill the chip
+    const int64_t row_blocks = (R + 16 * rt - 1) / (16 * rt);
+    const int ct = rt == 4 && row_blocks * (e_out / 16) > device_cus() ? 2 : 1;
+    const dim3 grid((unsigned)((e_out / 16 + ct - 1) / ct), (unsigned)row_blocks);
+#define RFA_ROWS(RT, CT) \
+    RFA_LAUNCH(LINEAR_ROWS, (rfa::k_linear_rows<RT, CT>), grid, dim3(rfa::kThreads), 0, st, xh, wh, bh, yh, (int)R, e_in, e_out)
+    if (rt == 1) { RFA_ROWS(1, 1); }
+    else if (rt == 2) { RFA_ROWS(2, 1); }
+    else if (ct == 1) { RFA_ROWS(4, 1); }
+    else { RFA_ROWS(4, 2); }
+#undef RFA_ROWS
+    RFA_HIP_TRY(hipGetLastError());
+    return RFA_OK;
 }
 
 size_t rfa_linear_weight_grad_workspace_bytes(int64_t R, int E_out, int E_in, int np) {

@@ -11,7 +11,7 @@
 // of kernels; issued through four Python functions and their backwards it took 456 us, from here 298
 // (128 tokens of 4 heads, the scan alone: 114 -> 68; encoder-decoder layer, 16384 + 8192 rows: 574 -> 430).
 #pragma once
-#include <ATen/ThreadLocalState.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -276,10 +276,38 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
     }
 };
 
+// The row kernel costs 4 us of host time, a library product 19; on the device it is ahead or level up to about
+// 96 rows of 1024 -> 3072 (9.2 / 8.9 us) or 256 of 1024 -> 1024 (7.1 / 8.0), and behind past that (160 rows of
+// 1024 -> 3072 12.9 / 8.5) and where a long contraction is split over its four waves only (64 rows of
+// 2048 -> 2048 12.6 / 8.8).
+bool few_rows(int64_t R, int64_t e_in, int64_t e_out) {
+    return R <= 256 && (R <= 32 || e_in <= 1024) && R * e_in * e_out <= (int64_t)300 << 20;
+}
+
 // for the callers' condition (fp16, grad mode on, widths that are multiples of 128) see linear_out
 OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     if (!plain_mode() || !plain_half(x, x.dim()) || !plain_half(w, 2) || !plain_half(b, 1)) return c10::nullopt;
     return LinearNode::apply(x, w, b);
+}
+
+// y = x W^T + b without autograd where the rows are few enough for the row kernel; the library otherwise
+// (and whenever autocast would choose the type).
+OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b) {
+    if (!plain_mode() || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 ||
+        !plain_half(x, x.dim()) || !plain_half(w, 2) || !plain_half(b, 1))
+        return c10::nullopt;
+    const int64_t e_in = w.size(1), e_out = w.size(0), R = e_in ? x.numel() / e_in : 0;
+    auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    if (R < 1 || !few_rows(R, e_in, e_out) || x.size(-1) != e_in || e_in % 32 != 0 || e_out % 16 != 0 || e_out == 0 ||
+        !x.is_contiguous() || !w.is_contiguous() || !aligned(x) || !aligned(w) || w.device() != x.device())
+        return c10::nullopt;
+    if (b.has_value() && (b->size(0) != e_out || !b->is_contiguous() || b->device() != x.device())) return c10::nullopt;
+    auto shape = x.sizes().vec();
+    shape.back() = e_out;
+    Tensor y = torch::empty(shape, x.options());
+    Launch l(x);
+    check_rc(rfa_linear_rows(ptr(x), ptr(w), ptr(b), ptr(y), R, (int)e_in, (int)e_out, l.stream));
+    return y;
 }
 
 // ---- causal attention -------------------------------------------------------------------------
@@ -459,6 +487,7 @@ void bind_nodes(pybind11::module_& m) {
     // each returns None where the call is not plain: the caller's general path takes it
     m.def("node_random_project", &node_random_project, py::arg("x"), py::arg("w"), py::arg("scale"));
     m.def("node_linear", &node_linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
+    m.def("node_linear_rows", &node_linear_rows, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("node_causal", &node_causal, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"));
     m.def("node_causal_layer", &node_causal_layer, py::arg("x"), py::arg("matrices"), py::arg("sigma"), py::arg("tau"),
           py::arg("build"), py::arg("weights"), py::arg("biases"), py::arg("heads"), py::arg("scale"));

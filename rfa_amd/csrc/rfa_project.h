@@ -262,6 +262,78 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
 }
 
 // ---------------------------------------------------------------------------
+// y[r][o] = x[r] . W[o] + b[o] for few rows: the projections of a decoding step.
+//
+// What bounds it is one trip to memory for W and the launch around it, so every byte of W is asked for at
+// once: a workgroup of four waves owns 16 columns (16 rows of W) of up to 64 rows of x, the waves share
+// the contraction, each with its 32-deep steps in flight together, operands straight from memory in the
+// lanes' own order; the four partial sums meet in LDS.  x comes out of the L2: with 64 rows its reads
+// bound the kernel, and 32 columns per workgroup halve them where that still leaves a workgroup per CU.
+// Measured, device us of the kernel / the library's product (which costs 19 us of host time, this 4):
+// 4 rows 512 -> 1536 2.7 / 3.7, 1024 -> 3072 3.7 / 5.9; 64 rows 512 -> 512 4.4 / 5.4, 1024 -> 3072 7.5 / 8.5;
+// 96 rows 1024 -> 3072 9.2 / 8.9; 160 rows 12.9 / 8.5.
+// grid = (ceil(Eo / (16 CT)), ceil(R / (16 RT)));  E % 32 == 0, Eo % 16 == 0
+// ---------------------------------------------------------------------------
+template <int RT, int CT>
+__global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restrict__ x, const half_t* __restrict__ w,
+                                                          const half_t* __restrict__ bias, half_t* __restrict__ y, int R,
+                                                          int E, int Eo) {
+    __shared__ f4 red[4][RT * CT][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int i = lane & 15, G = lane >> 4;
+    const int c0 = 16 * CT * blockIdx.x, r0 = 16 * RT * blockIdx.y;
+    const int nk = E / 32, per_wave = (nk + 3) / 4;
+    const int k_begin = min(wv * per_wave, nk), k_end = min(k_begin + per_wave, nk);
+    const half_t* wp[CT];
+    const half_t* xp[RT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) wp[c] = w + (int64_t)min(c0 + 16 * c + i, Eo - 1) * E + 8 * G;
+#pragma unroll
+    for (int a = 0; a < RT; ++a) xp[a] = x + (int64_t)min(r0 + 16 * a + i, R - 1) * E + 8 * G;
+    f4 acc[RT][CT];      // y^T tiles: lane (i, G) holds columns 4G .. of row i
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[a][c] = f4_zero();
+    constexpr int U = 4;      // steps in flight; 8 only repeat the last step's loads where E = 512
+    for (int k = k_begin; k < k_end; k += U) {
+        h8 wa[U][CT], xb[U][RT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kk = 32 * min(k + u, k_end - 1);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) wa[u][c] = *reinterpret_cast<const h8*>(wp[c] + kk);
+#pragma unroll
+            for (int a = 0; a < RT; ++a) xb[u][a] = *reinterpret_cast<const h8*>(xp[a] + kk);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k + u < k_end) {
+#pragma unroll
+                for (int a = 0; a < RT; ++a)
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) acc[a][c] = mfma32(wa[u][c], xb[u][a], acc[a][c]);
+            }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) red[wv][a * CT + c][lane] = acc[a][c];
+    __syncthreads();
+    for (int t = wv; t < RT * CT; t += 4) {
+        const int r = r0 + 16 * (t / CT) + i, col = c0 + 16 * (t % CT) + 4 * G;
+        const f4 s = (red[0][t][lane] + red[1][t][lane]) + (red[2][t][lane] + red[3][t][lane]);
+        if (r < R && col < Eo) {
+            h4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (half_t)(s[e] + (bias ? (float)bias[col + e] : 0.f));
+            *reinterpret_cast<h4*>(y + (int64_t)r * Eo + col) = o;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Weight and bias gradients of those Linear layers:
 //     dW_p[o][c] = sum_r dy_p[r][o] * x[r][c],      db_p[o] = sum_r dy_p[r][o]
 // (what autograd computes for torch.nn.Linear).  The contraction runs over the R rows, far

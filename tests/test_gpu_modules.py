@@ -502,6 +502,7 @@ def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypa
     if rfa_hip.native is None:
         pytest.skip("the torch binding is not active")
     print(f"native nodes: {path} {form}", flush=True)
+    monkeypatch.setattr("rfa_amd.projection.linear_rows", lambda *a: None)     # another sum than the library's
     run, leaves = _native_forms(path, form)
     results = []
     for native in (rfa_hip.native, None):

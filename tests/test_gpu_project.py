@@ -467,3 +467,48 @@ def test_empty_input():
     assert ys[0].shape == (0, 3, H, d) and phis[0].shape == (0, 3, H, 2 * D) and phis[1] is None
     dws, dbs = rfa_hip.linear_weight_grad(x.view(0, E), [torch.empty(0, H * d, dtype=torch.float16).cuda()], [True])
     assert dws[0].shape == (H * d, E) and (dws[0] == 0).all() and (dbs[0] == 0).all()
+
+
+@pytest.mark.parametrize("e_in,e_out", [(32, 16), (96, 48), (512, 1536), (992, 272), (1024, 3072)])
+@pytest.mark.parametrize("R", [1, 15, 16, 17, 32, 33, 64, 65, 97, 130])
+def test_linear_rows(R, e_in, e_out):
+    """The few-rows product against fp64 at the edges of its row tiles, column tiles and wave splits: fp32
+    sums of exact products, one rounding to fp16 (2^-11 of the value; sums of 1024 terms below 2^-16)."""
+    from rfa_amd import projection, rfa_hip
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    gen = torch.Generator("cuda").manual_seed(R)
+    x = torch.randn(R, e_in, generator=gen, device="cuda").half()
+    w = (torch.randn(e_out, e_in, generator=gen, device="cuda") / e_in ** 0.5).half()
+    b = torch.randn(e_out, generator=gen, device="cuda").half()
+    print(f"linear_rows R={R} {e_in}->{e_out}", flush=True)
+    want = x.double() @ w.double().t()
+    with torch.no_grad():
+        for bias in (b, None):
+            y = projection.linear_rows(x, w, bias)
+            ref = want if bias is None else want + b.double()
+            if R * e_in * e_out > 300 << 20:
+                assert y is None
+                continue
+            assert ((y.double() - ref).abs() <= 2.0 ** -10 * ref.abs() + 2e-5).all()
+        # what the kernel does not read as it is goes to the library
+        assert projection.linear_rows(x.t().contiguous().t() if R > 1 else x.float(), w, b) is None
+        assert projection.linear_rows(x, w[:, :e_in - 8], b) is None and projection.linear_rows(x.float(), w.float(), None) is None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert projection.linear_rows(x, w, b) is None
+    assert projection.linear_rows(x, w, b) is None          # autograd is on
+
+
+def test_output_projection_keeps_its_hooks():
+    """Without autograd the output layer may take the row kernel, but not past hooks or a forward of its own."""
+    from rfa_amd import projection
+    layer = torch.nn.Linear(64, 64).cuda().half()
+    x = torch.randn(3, 64).cuda().half()
+    seen = []
+    with torch.no_grad():
+        plain = projection.linear_out(x, layer)
+        handle = layer.register_forward_hook(lambda *a: seen.append(1))
+        assert torch.allclose(projection.linear_out(x, layer), plain, atol=2e-3) and seen == [1]
+        handle.remove()
+        layer.forward = lambda t: t * 0
+        assert projection.linear_out(x, layer).abs().max().item() == 0
