@@ -300,6 +300,10 @@ int rfa_cross_state(const void* phi_k, const void* v, const uint8_t* key_padding
                     int64_t S_len, int64_t B, int H, int K, int d, void* stream);
 int rfa_cross_readout(const void* phi_q, const float* s, const float* z, void* out, int64_t T, int64_t N,
                       int K, int d, void* stream);
+/* one target step: phi(q) and the readout in one launch; q fp16 [B, H, d] (projected rows), w fp16 [H, D, d],
+ * s, z as above for N = B * H, out fp16 [B, H, d] */
+int rfa_cross_step(const void* q, const void* w, float scale, const float* s, const float* z, void* out, int64_t B,
+                   int H, int D, int d, void* stream);
 int rfa_cross_readout_backward(const void* phi_q, const float* s, const float* z, const void* grad_attn,
                                void* dphi_q, float* ds, float* dz, int64_t T, int64_t N, int K, int d,
                                void* stream);

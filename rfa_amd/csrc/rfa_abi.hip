@@ -46,14 +46,15 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
                                    "k_masked_fwd", "k_masked_bwd_prep", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
-                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows"};
+                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
+                                   "k_cross_step"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -1365,6 +1366,30 @@ int rfa_cross_readout(const void* phi_q, const float* s, const float* z, void* o
     auto* oh = static_cast<rfa::half_t*>(out);
 #define RFA_CALL(KD, DH) launch_cross_readout<KD, DH>(qh, s, z, oh, (int)T, (int)N, st)
     RFA_DISPATCH_KD(K, d, RFA_CALL)
+#undef RFA_CALL
+    return fail(RFA_ERR_UNSUPPORTED, "unreachable");
+}
+
+static int check_feature_dims(const char* fn, int64_t R, int H, int D, int d);
+int rfa_cross_step(const void* q, const void* w, float scale, const float* s, const float* z, void* out, int64_t B, int H,
+                   int D, int d, void* stream) {
+    if (int rc = check_feature_dims("rfa_cross_step", B, H, D, d)) return rc;
+    if (B == 0) return RFA_OK;
+    if (!q || !w || !s || !z || !out) return fail(RFA_ERR_NULL_POINTER, "rfa_cross_step: NULL tensor pointer");
+    if (!aligned16(q) || !aligned16(w) || !aligned16(s) || !aligned16(z) || !aligned16(out))
+        return fail(RFA_ERR_ALIGNMENT, "rfa_cross_step: tensors must be 16-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto* qh = static_cast<const rfa::half_t*>(q);
+    auto* wh = static_cast<const rfa::half_t*>(w);
+    auto* oh = static_cast<rfa::half_t*>(out);
+#define RFA_CALL(KD, DH)                                                                                                \
+    ([&]() -> int {                                                                                                     \
+        RFA_LAUNCH(CROSS_STEP, (rfa::k_cross_step<KD, DH>), dim3((unsigned)(B * H)), dim3(rfa::kThreads), 0, st, qh, wh, \
+                   scale, H, s, z, oh);                                                                                 \
+        RFA_HIP_TRY(hipGetLastError());                                                                                 \
+        return RFA_OK;                                                                                                  \
+    })()
+    RFA_DISPATCH_KD(2 * D, d, RFA_CALL)
 #undef RFA_CALL
     return fail(RFA_ERR_UNSUPPORTED, "unreachable");
 }

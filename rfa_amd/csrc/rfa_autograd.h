@@ -47,6 +47,7 @@ bool wants_grad(const T&... t) {
 }
 bool wants_grad_opt(const OptTensor& t) { return t.has_value() && t->requires_grad(); }
 
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : c10::nullopt; }
 
@@ -297,9 +298,8 @@ OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b)
         !plain_half(x, x.dim()) || !plain_half(w, 2) || !plain_half(b, 1))
         return c10::nullopt;
     const int64_t e_in = w.size(1), e_out = w.size(0), R = e_in ? x.numel() / e_in : 0;
-    auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
     if (R < 1 || !few_rows(R, e_in, e_out) || x.size(-1) != e_in || e_in % 32 != 0 || e_out % 16 != 0 || e_out == 0 ||
-        !x.is_contiguous() || !w.is_contiguous() || !aligned(x) || !aligned(w) || w.device() != x.device())
+        !x.is_contiguous() || !w.is_contiguous() || !aligned16(x) || !aligned16(w) || w.device() != x.device())
         return c10::nullopt;
     if (b.has_value() && (b->size(0) != e_out || !b->is_contiguous() || b->device() != x.device())) return c10::nullopt;
     auto shape = x.sizes().vec();
@@ -476,6 +476,22 @@ OptTensor node_cross_query(const Tensor& query, const Tensor& w, const Tensor& w
     Layers l{{weight}, {bias}, {true, false, false}};
     if (!plain_mode() || !plain_layers(query, w, l, heads) || !plain(s, torch::kFloat32, 4) || !plain(z, torch::kFloat32, 3))
         return c10::nullopt;
+    if (query.size(0) == 1 && !at::GradMode::is_enabled() && s.is_contiguous() && z.is_contiguous() && w.is_contiguous()) {
+        // one step: the row kernel for q, then feature map and readout in one launch
+        const int64_t B = query.size(1), d = weight.size(0) / heads, D = w.size(1);
+        const bool fits = s.size(0) == B && s.size(1) == heads && s.size(2) == 2 * D && s.size(3) == d && z.size(0) == B &&
+                          z.size(1) == heads && z.size(2) == 2 * D && w.size(0) == heads && w.size(2) == d &&
+                          aligned16(s) && aligned16(z) && aligned16(w) && s.device() == query.device() &&
+                          z.device() == query.device() && w.device() == query.device();
+        const OptTensor q = fits ? node_linear_rows(query, weight, bias) : c10::nullopt;
+        if (q.has_value()) {
+            Tensor out = torch::empty_like(*q);
+            Launch g(query);
+            check_rc(rfa_cross_step(ptr(*q), ptr(w), (float)scale, s.data_ptr<float>(), z.data_ptr<float>(), ptr(out), B,
+                                    (int)heads, (int)D, (int)d, g.stream));
+            return out;
+        }
+    }
     const auto phi_q = project(query, w, scale, heads, l)[0];
     if (wants_grad(phi_q, s, z)) return CrossReadoutNode::apply(phi_q, s, z);
     const Tensor out = cross_readout(phi_q, s.contiguous(), z.contiguous());

@@ -453,3 +453,27 @@ def test_incremental_qkv_equals_the_step_on_separate_tensors(B, H, d, D, steps):
     assert torch.equal(torch.cat(rows), want[:len(rows)])
     with pytest.raises(Exception, match="3, heads"):
         rfa_hip.incremental_qkv(qkv[:, :, :2].contiguous(), W, O.SCALE, s2, z2)
+
+
+@pytest.mark.parametrize("B,H,d,D", [(1, 2, 64, 32), (3, 2, 64, 64), (5, 3, 64, 128), (2, 2, 128, 32), (7, 1, 128, 64),
+                                     (4, 2, 128, 128)])
+def test_cross_attention_single_step(B, H, d, D):
+    """One target step without autograd (projection rows, then feature map + readout in one launch) against
+    the oracle chain in fp32, among them denominators on both sides of the clamp and of either sign."""
+    from rfa_amd import CrossAttention, CrossAttentionState
+    torch.manual_seed(B + D)
+    E = H * d
+    m = CrossAttention(embed_dim=E, num_heads=H, head_dim=d, proj_dim=D).cuda().half().eval()
+    W = O.make_w(d, D, H).half().cuda()
+    x = torch.randn(1, B, E).half().cuda()
+    s = torch.randn(B, H, 2 * D, d).cuda()
+    z = 20 * torch.randn(B, H, 2 * D).cuda()
+    print(f"cross step B={B} H={H} d={d} D={D}", flush=True)
+    with torch.no_grad():
+        y = m(x, CrossAttentionState(s, z, W, 1.0))
+        f = lambda lin, t: torch.nn.functional.linear(t.double(), lin.weight.double(), lin.bias.double())
+        q = f(m.q_proj, x).half().double().view(1, B, H, d).cpu()
+        attn = O.cross_readout(O.random_project(q, W.double().cpu()), s.double().cpu(), z.double().cpu())
+        want = f(m.out_proj, attn.reshape(1, B, E).half().cuda())
+    # two roundings to fp16 on the way to an fp16 result
+    assert _rel(y.double().cpu(), want.cpu()) <= 2e-3
