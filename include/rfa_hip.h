@@ -139,6 +139,11 @@ int rfa_causal_backward_saved(const void* q, const void* k, const void* v, const
  * the forward).  rfa_causal_saved_describe copies the 16 header ints to host memory and waits
  * for the stream (a debugging aid).  No counterpart in the reference. */
 size_t rfa_causal_backward_saved_workspace_bytes(const void* saved, int64_t T, int64_t N, int K, int d);
+/* Rows [T, B] of `width` halves (a multiple of 8) with the padded ones zero: a copy of src to dst, or with
+ * src == dst the zeros alone.  pad: bytes, (b, t) at b * stride_b + t * stride_t, non-zero = padded
+ * (phi_k.masked_fill of causal_attention.py:136-138 and its gradient). */
+int rfa_mask_rows(const void* src, void* dst, const uint8_t* pad, int64_t stride_b, int64_t stride_t, int64_t T,
+                  int64_t B, int64_t width, void* stream);
 int rfa_causal_saved_describe(const void* saved, int32_t* words16, void* stream);
 
 /* Number of time segments the causal kernels cut a sequence into for the given

@@ -39,6 +39,7 @@ SIGNATURES = {
     "rfa_tuning_set": (c_int, [c_char_p, c_int]),
     "rfa_tuning_get": (c_int, [c_char_p, POINTER(c_int)]),
     "rfa_causal_backward_saved_workspace_bytes": (c_size_t, [c_void_p, c_int64, c_int64, c_int, c_int]),
+    "rfa_mask_rows": (c_int, [c_void_p] * 3 + [c_int64] * 5 + [c_void_p]),
     "rfa_causal_saved_describe": (c_int, [c_void_p, POINTER(ctypes.c_int32), c_void_p]),
     "rfa_causal_forward_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int, c_int]),
     "rfa_causal_forward": (c_int, [c_void_p] * 4 + [c_int64, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),

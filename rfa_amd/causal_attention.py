@@ -138,12 +138,13 @@ def cuda_causal_rfa(*, phi_q: Tensor, phi_k: Tensor, v: Tensor,
     key_padding_mask = _drop_scalar_mask(key_padding_mask)
     if key_padding_mask is not None:
         assert key_padding_mask.size(0) == bsz and key_padding_mask.size(1) == tgt_len
-        pad = key_padding_mask.to(torch.bool).transpose(0, 1)[:, :, None, None]
-        phi_k = phi_k.masked_fill(pad, 0.0)
     if rfa_hip.native is not None:
-        attn = rfa_hip.native.node_causal(phi_q, phi_k, v)
+        attn = rfa_hip.native.node_causal(phi_q, phi_k, v, key_padding_mask)
         if attn is not None:
             return attn
+    if key_padding_mask is not None:
+        pad = key_padding_mask.to(torch.bool).transpose(0, 1)[:, :, None, None]
+        phi_k = phi_k.masked_fill(pad, 0.0)
     n = bsz * num_heads
     attn = RFA.apply(phi_q.contiguous().view(tgt_len, n, feat),
                      phi_k.contiguous().view(tgt_len, n, feat),

@@ -46,7 +46,7 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
@@ -54,7 +54,7 @@ const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
                                    "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
-                                   "k_cross_step"};
+                                   "k_cross_step", "k_mask_rows"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -1127,6 +1127,22 @@ size_t rfa_causal_backward_saved_workspace_bytes(const void* saved, int64_t T, i
     if (saved_plan(saved, T, N, K, d, &p) != RFA_OK) return 0;
     if (p.layout == LAYOUT_FINAL) return 0;
     return layout_workspace(T, N, K, d, p, true).total;
+}
+
+int rfa_mask_rows(const void* src, void* dst, const uint8_t* pad, int64_t stride_b, int64_t stride_t, int64_t T, int64_t B,
+                  int64_t width, void* stream) {
+    if (T < 0 || B < 0 || width <= 0 || width % 8 != 0 || T > (1 << 30) || B > (1 << 30) || width > (1 << 30))
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_mask_rows: bad sizes T=%lld B=%lld width=%lld (a multiple of 8)", (long long)T,
+                    (long long)B, (long long)width);
+    if (T == 0 || B == 0) return RFA_OK;
+    if (!src || !dst || !pad) return fail(RFA_ERR_NULL_POINTER, "rfa_mask_rows: NULL pointer");
+    if (!aligned16(src) || !aligned16(dst)) return fail(RFA_ERR_ALIGNMENT, "rfa_mask_rows: rows must be 16-byte aligned");
+    const int64_t blocks = (T * B * (width / 8) + rfa::kThreads - 1) / rfa::kThreads;
+    RFA_LAUNCH(MASK_ROWS, rfa::k_mask_rows, dim3((unsigned)std::min<int64_t>(blocks, 8 * (int64_t)device_cus())),
+               dim3(rfa::kThreads), 0, static_cast<hipStream_t>(stream), static_cast<const rfa::half_t*>(src),
+               static_cast<rfa::half_t*>(dst), pad, stride_b, stride_t, T * B, (int)B, (int)width);
+    RFA_HIP_TRY(hipGetLastError());
+    return RFA_OK;
 }
 
 int rfa_causal_saved_describe(const void* saved, int32_t* words16, void* stream) {

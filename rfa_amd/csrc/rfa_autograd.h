@@ -321,9 +321,32 @@ struct ScanDims {
 
 Tensor scan_output(const Tensor& v) { return torch::empty({v.size(0), v.size(1), v.size(2) * v.size(3)}, v.options()); }
 
+// rows of t [T, B, H, K] whose key is padded set to zero: of a copy, or where they are
+void mask_rows(const Tensor& src, const Tensor& dst, const Tensor& pad) {
+    Launch l(src);
+    check_rc(rfa_mask_rows(ptr(src), ptr(dst), static_cast<const uint8_t*>(pad.data_ptr()), pad.stride(0), pad.stride(1),
+                           src.size(0), src.size(1), src.size(2) * src.size(3), l.stream));
+}
+
+Tensor masked_keys(const Tensor& phi_k, const OptTensor& pad) {
+    const Tensor k = phi_k.contiguous();
+    if (!pad.has_value()) return k;
+    Tensor out = torch::empty_like(k);
+    mask_rows(k, out, *pad);
+    return out;
+}
+
+// [B, T] of any type and strides on the tensors' device (bools are read where they are)
+bool plain_pad(const OptTensor& pad, const Tensor& k) {
+    return !pad.has_value() ||
+           (plain(*pad, pad->scalar_type(), 2) && !pad->is_complex() && pad->size(0) == k.size(1) &&
+            pad->size(1) == k.size(0) && pad->device() == k.device() && aligned16(k) && k.size(2) * k.size(3) % 8 == 0);
+}
+
 struct CausalNode : public torch::autograd::Function<CausalNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& phi_q, const Tensor& phi_k, const Tensor& values) {
-        const Tensor q = phi_q.contiguous(), k = phi_k.contiguous(), v = values.contiguous();
+    static Tensor forward(AutogradContext* ctx, const Tensor& phi_q, const Tensor& phi_k, const Tensor& values,
+                          const OptTensor& pad) {
+        const Tensor q = phi_q.contiguous(), k = masked_keys(phi_k, pad), v = values.contiguous();
         const ScanDims n(q, v);
         Tensor attn = scan_output(v);
         Launch l(q);
@@ -332,7 +355,7 @@ struct CausalNode : public torch::autograd::Function<CausalNode> {
         Tensor ws = workspace(nbytes, q), state = workspace(sbytes, q);
         check_rc(rfa_causal_forward_save(ptr(q), ptr(k), ptr(v), ptr(attn), ptr(state), sbytes, n.T, n.N, n.K, n.d, ptr(ws),
                                          nbytes, l.stream));
-        ctx->save_for_backward({q, k, v, attn, state});
+        ctx->save_for_backward({q, k, v, attn, state, opt(pad)});
         return attn;
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
@@ -346,7 +369,8 @@ struct CausalNode : public torch::autograd::Function<CausalNode> {
         Tensor ws = workspace(nbytes, q);
         check_rc(rfa_causal_backward_saved(ptr(q), ptr(k), ptr(v), ptr(grad), ptr(attn), ptr(state), (size_t)state.numel(),
                                            ptr(dq), ptr(dk), ptr(dv), n.T, n.N, n.K, n.d, ptr(ws), nbytes, l.stream));
-        return {dq, dk, dv};
+        if (saved[5].defined()) mask_rows(dk, dk, saved[5]);
+        return {dq, dk, dv, Tensor()};
     }
 };
 
@@ -355,9 +379,9 @@ bool plain_scan(const Tensor& q, const Tensor& k, const Tensor& v) {
            v.size(1) == q.size(1) && v.size(2) == q.size(2) && q.device() == k.device() && q.device() == v.device();
 }
 
-Tensor causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& values) {
-    if (wants_grad(phi_q, phi_k, values)) return CausalNode::apply(phi_q, phi_k, values);
-    const Tensor q = phi_q.contiguous(), k = phi_k.contiguous(), v = values.contiguous();
+Tensor causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& values, const OptTensor& pad) {
+    if (wants_grad(phi_q, phi_k, values)) return CausalNode::apply(phi_q, phi_k, values, pad);
+    const Tensor q = phi_q.contiguous(), k = masked_keys(phi_k, pad), v = values.contiguous();
     const ScanDims n(q, v);
     Tensor attn = scan_output(v);
     Launch l(q);
@@ -367,9 +391,9 @@ Tensor causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& values) {
     return attn;
 }
 
-OptTensor node_causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v) {
-    if (!plain_mode() || !plain_scan(phi_q, phi_k, v)) return c10::nullopt;
-    return causal(phi_q, phi_k, v);
+OptTensor node_causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v, const OptTensor& pad) {
+    if (!plain_mode() || !plain_scan(phi_q, phi_k, v) || !plain_pad(pad, phi_k)) return c10::nullopt;
+    return causal(phi_q, phi_k, v, pad.has_value() ? OptTensor(pad->to(torch::kBool)) : c10::nullopt);
 }
 
 // q, k, v projections, phi(q) and phi(k), the scan: x [T, B, E] -> attn [T, B, H * d].  `matrices` is
@@ -383,7 +407,7 @@ OptTensor node_causal_layer(const Tensor& x, const Tensor& matrices, const OptTe
         return c10::nullopt;
     const Tensor w = build ? build_matrices(matrices, sigma, tau) : matrices;
     const auto out = project(x, w, scale, heads, l);
-    return causal(out[0], out[1], out[2]);
+    return causal(out[0], out[1], out[2], c10::nullopt);
 }
 
 // ---- quadratic form with explicit masks ---------------------------------------------------------
@@ -504,7 +528,8 @@ void bind_nodes(pybind11::module_& m) {
     m.def("node_random_project", &node_random_project, py::arg("x"), py::arg("w"), py::arg("scale"));
     m.def("node_linear", &node_linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("node_linear_rows", &node_linear_rows, py::arg("x"), py::arg("weight"), py::arg("bias"));
-    m.def("node_causal", &node_causal, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"));
+    m.def("node_causal", &node_causal, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"),
+          py::arg("key_padding_mask") = py::none());
     m.def("node_causal_layer", &node_causal_layer, py::arg("x"), py::arg("matrices"), py::arg("sigma"), py::arg("tau"),
           py::arg("build"), py::arg("weights"), py::arg("biases"), py::arg("heads"), py::arg("scale"));
     m.def("node_masked", &node_masked, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("key_padding_mask"),

@@ -371,6 +371,27 @@ __device__ __forceinline__ void chunk_r2s(const ChunkRegs<F, NT>& r, half_t* Xs,
     }
 }
 
+// Rows [T, B] of W halves with the padded ones set to zero: a copy of src, or (src == dst) the zeros alone.
+// pad: byte of (b, t) at b * stride_b + t * stride_t, non-zero = padded.  Bound by memory: 777 x 6 rows of
+// 12 heads, 128 features take 6.6 us in place of a clone and a masked_fill of 17.8, forward and again backward
+// (where only the padded rows are written).   grid-stride over 16-byte pieces; W % 8 == 0
+__global__ __launch_bounds__(kThreads) void k_mask_rows(const half_t* src, half_t* dst, const uint8_t* __restrict__ pad,
+                                                        int64_t stride_b, int64_t stride_t, int64_t rows, int B, int W) {
+    const int ppr = W / 8;
+    const int64_t total = rows * ppr;
+    const bool copy = src != dst;
+    for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < total; p += (int64_t)gridDim.x * kThreads) {
+        const int64_t r = p / ppr;
+        const bool padded = pad[(r % B) * stride_b + (r / B) * stride_t] != 0;
+        uint4 x = {0u, 0u, 0u, 0u};
+        if (copy) {
+            const uint4 y = *reinterpret_cast<const uint4*>(src + p * 8);
+            x.x = padded ? 0u : y.x; x.y = padded ? 0u : y.y; x.z = padded ? 0u : y.z; x.w = padded ? 0u : y.w;
+        }
+        if (copy || padded) *reinterpret_cast<uint4*>(dst + p * 8) = x;
+    }
+}
+
 // 1 / x for x >= 1 (denominators): the hardware approximation and one Newton step, 3 vector
 // instructions where the correctly rounded quotient takes about ten; the result differs from
 // it by at most one unit in the last place, far below the fp16 rounding of whatever it scales.

@@ -470,7 +470,7 @@ def _native_forms(path, form):
         x = leaf(T, B, H, d)
         w = W.clone().requires_grad_(grad and form != "frozen")
         return lambda: utils.random_project(x=x, random_matrices=w), [x, w]
-    if path in ("causal", "masked"):
+    if path in ("causal", "masked", "padded"):
         q, k, v = leaf(T, B, H, 2 * D, scale=0.1), leaf(T, B, H, 2 * D, scale=0.1), leaf(T, B, H, d)
         if form == "frozen":
             k = k.detach()
@@ -478,6 +478,10 @@ def _native_forms(path, form):
             return lambda: C.cuda_causal_rfa(phi_q=q, phi_k=k, v=v), [q, k, v]
         pad = torch.zeros(B, T, dtype=torch.bool, device="cuda")
         pad[0, 30:] = True
+        pad[2, 5] = True
+        if path == "padded":
+            pad = pad.t().contiguous().t() if form == "strided" else pad.byte() * 3 if form == "twice" else pad
+            return lambda: C.cuda_causal_rfa(phi_q=q, phi_k=k, v=v, key_padding_mask=pad), [q, k, v]
         mask = torch.full((T, T), float("-inf"), device="cuda").triu(1)
         return lambda: C.masked_rfa(phi_q=q, phi_k=k, v=v, key_padding_mask=pad, attn_mask=mask), [q, k, v]
     x = leaf(T, B, E)
@@ -493,7 +497,7 @@ def _native_forms(path, form):
 
 
 @pytest.mark.parametrize("form", ["plain", "strided", "frozen", "no_bias", "no_grad", "hooks", "twice"])
-@pytest.mark.parametrize("path", ["random_project", "causal", "masked", "module", "cross"])
+@pytest.mark.parametrize("path", ["random_project", "causal", "padded", "masked", "module", "cross"])
 def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypatch):
     """The C++ autograd nodes against the Python autograd functions over the same kernels: outputs and every
     gradient bit for bit, from strided inputs, with frozen or missing parameters, through saved-tensor
