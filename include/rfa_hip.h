@@ -120,6 +120,12 @@ size_t rfa_causal_saved_state_bytes(int64_t T, int64_t N, int K, int d);
 int rfa_causal_forward_save(const void* q, const void* k, const void* v, void* out, void* saved,
                             size_t saved_bytes, int64_t T, int64_t N, int K, int d, void* workspace,
                             size_t workspace_bytes, void* stream);
+/* rfa_causal_prefill from projected rows: q, k, v fp16 [T, B, H, d], w fp16 [H, D, d]; phi(q) and phi(k)
+ * (rfa_feature_map_forward's values) are formed inside the scan.  s fp32 [B, H, 2D, d], z fp32 [B, H, 2D].
+ * Only where rfa_causal_prefill_rows_supported (N = B * H) answers 1: sequences enough to fill the chip. */
+int rfa_causal_prefill_rows_supported(int64_t T, int64_t N, int D, int d);
+int rfa_causal_prefill_rows(const void* q, const void* k, const void* v, const void* w, float scale, void* out,
+                            float* s, float* z, int64_t T, int64_t B, int H, int D, int d, void* stream);
 int rfa_causal_backward_saved(const void* q, const void* k, const void* v, const void* grad_attn,
                               const void* out, const void* saved, size_t saved_bytes, void* dq, void* dk,
                               void* dv, int64_t T, int64_t N, int K, int d, void* workspace,

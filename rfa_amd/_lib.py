@@ -46,6 +46,8 @@ SIGNATURES = {
     "rfa_static_scratch_bytes": (c_size_t, []),
     "rfa_causal_forward_noalloc": (c_int, [c_void_p] * 4 + [c_int64, c_int64, c_int, c_int, c_void_p]),
     "rfa_causal_prefill": (c_int, [c_void_p] * 6 + [c_int64, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "rfa_causal_prefill_rows_supported": (c_int, [c_int64, c_int64, c_int, c_int]),
+    "rfa_causal_prefill_rows": (c_int, [c_void_p] * 4 + [c_float] + [c_void_p] * 3 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "rfa_causal_backward_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int, c_int]),
     "rfa_causal_backward": (c_int, [c_void_p] * 7 + [c_int64, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rfa_causal_saved_state_bytes": (c_size_t, [c_int64, c_int64, c_int, c_int]),

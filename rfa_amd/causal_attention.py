@@ -310,16 +310,20 @@ class CausalAttention(nn.Module):
             s, z = saved_state.get("prev_s"), saved_state.get("prev_z")
             if s is None and tgt_len > 1:
                 # prefill: one pass of the training kernels over the prompt, final state kept
-                with torch.no_grad():
-                    phi_q, phi_k = random_project_pair(x0=q, x1=k, random_matrices=w)
-                    pad = _drop_scalar_mask(key_padding_mask)
-                    if pad is not None:
-                        phi_k = phi_k.masked_fill(pad.to(torch.bool).transpose(0, 1)[:, :, None, None], 0.0)
-                    n = bsz * self.num_heads
-                    attn, s, z = rfa_hip.prefill(
-                        phi_q.to(torch.float16).contiguous().view(tgt_len, n, feat),
-                        phi_k.to(torch.float16).contiguous().view(tgt_len, n, feat),
-                        v.detach().to(torch.float16).contiguous().view(tgt_len, n, self.head_dim))
+                pad = _drop_scalar_mask(key_padding_mask)
+                prefilled = native.node_prefill(q, k, v, w, SCALE) if native is not None and pad is None else None
+                if prefilled is not None:       # feature maps inside the scan
+                    attn, s, z = prefilled
+                else:
+                    with torch.no_grad():
+                        phi_q, phi_k = random_project_pair(x0=q, x1=k, random_matrices=w)
+                        if pad is not None:
+                            phi_k = phi_k.masked_fill(pad.to(torch.bool).transpose(0, 1)[:, :, None, None], 0.0)
+                        n = bsz * self.num_heads
+                        attn, s, z = rfa_hip.prefill(
+                            phi_q.to(torch.float16).contiguous().view(tgt_len, n, feat),
+                            phi_k.to(torch.float16).contiguous().view(tgt_len, n, feat),
+                            v.detach().to(torch.float16).contiguous().view(tgt_len, n, self.head_dim))
                 s = s.view(bsz, self.num_heads, feat, self.head_dim)
                 z = z.view(bsz, self.num_heads, feat)
             else:

@@ -387,7 +387,7 @@ int launch_forward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t
             if (int rc = set_lds(kern, rfa::FwdPipeCfg<KD, DH>::kLds)) return rc;
             RFA_LAUNCH(CAUSAL_FWD, kern, dim3(N * p.nseg), dim3(512), rfa::FwdPipeCfg<KD, DH>::kLds, st, q, k, v, out,
                        (const float*)nullptr, (const float*)nullptr, savedDen, final_s, final_z, T, N, p.nseg, p.seg_len, 0,
-                       savedHdr, pw, bounds, 0);
+                       savedHdr, pw, bounds, 0, (const rfa::half_t*)nullptr, 1, 0.f);
             RFA_HIP_TRY(hipGetLastError());
             return RFA_OK;
         }
@@ -408,7 +408,8 @@ int launch_forward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t
         if (int rc = set_lds(kern, rfa::FwdPipeCfg<KD, DH>::kLds)) return rc;
         RFA_LAUNCH(CAUSAL_FWD, kern, dim3(N * p.nseg), dim3(512), rfa::FwdPipeCfg<KD, DH>::kLds, st, q, k, v, out,
                            wsS, wsZ, savedDen, final_s, final_z, T, N, p.nseg, p.seg_len, p.prefixed, savedHdr, pw,
-                           rfa::SegBounds{}, (int64_t)rfa::kChunk * N * (KD > DH ? KD : DH) * 2 >= ((int64_t)1 << 32) ? 1 : 0);
+                           rfa::SegBounds{}, (int64_t)rfa::kChunk * N * (KD > DH ? KD : DH) * 2 >= ((int64_t)1 << 32) ? 1 : 0,
+                           (const rfa::half_t*)nullptr, 1, 0.f);
     } else {
         auto kern = rfa::k_causal_fwd<KD, DH, NW, true>;
         if (int rc = set_lds(kern, Cfg::kFwdLds)) return rc;
@@ -417,6 +418,28 @@ int launch_forward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t
     }
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
+}
+
+// A prompt from projected rows, feature maps formed inside the scan (k_causal_fwd_pipe<.., PHI>): one
+// segment per sequence, no workspace.
+template <int KD, int DH>
+constexpr bool fwd_phi_fits() { return rfa::FwdPipeCfg<KD, DH>::kPhiLds <= 160 * 1024; }
+
+template <int KD, int DH>
+int launch_prefill_phi(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t* v, const rfa::half_t* w, float scale,
+                       rfa::half_t* out, float* final_s, float* final_z, int T, int N, int H, hipStream_t st) {
+    if constexpr (fwd_phi_fits<KD, DH>()) {
+        auto kern = rfa::k_causal_fwd_pipe<KD, DH, false, true>;
+        if (int rc = set_lds(kern, rfa::FwdPipeCfg<KD, DH>::kPhiLds)) return rc;
+        RFA_LAUNCH(CAUSAL_FWD, kern, dim3(N), dim3(512), rfa::FwdPipeCfg<KD, DH>::kPhiLds, st, q, k, v, out,
+                   (const float*)nullptr, (const float*)nullptr, (float*)nullptr, final_s, final_z, T, N, 1, T, 0, (int*)nullptr,
+                   rfa::PlanWords{}, rfa::SegBounds{}, (int64_t)rfa::kChunk * N * DH * 2 >= ((int64_t)1 << 32) ? 1 : 0, w, H,
+                   scale);
+        RFA_HIP_TRY(hipGetLastError());
+        return RFA_OK;
+    } else {
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_causal_prefill_rows: no kernel for feature width K=%d, head dim d=%d", KD, DH);
+    }
 }
 
 // The cut into segments the backward sweeps use for a forward plan pf.  Where both sweeps run as two
@@ -1197,6 +1220,41 @@ int rfa_causal_prefill(const void* q, const void* k, const void* v, void* out, f
         return RFA_OK;
     }
     return causal_forward_impl(q, k, v, out, T, N, K, d, nullptr, 0, false, s, z, workspace, workspace_bytes, stream);
+}
+
+// One segment per sequence means that the sequences alone fill the chip; with more, the segments' states would
+// need phi(k) in memory first, and the feature map as a launch of its own is the shorter way.
+int rfa_causal_prefill_rows_supported(int64_t T, int64_t N, int D, int d) {
+    const int K = 2 * D;
+    if (T < 1 || N < 1 || !feature_shape_supported(D, d) || !rfa_shape_supported(K, d) || T > (1 << 30) || N > (1 << 22) ||
+        T * N > (int64_t(1) << 31))
+        return 0;
+    const bool fits = K == 64 ? (d == 64 ? fwd_phi_fits<64, 64>() : fwd_phi_fits<64, 128>())
+                      : K == 128 ? (d == 64 ? fwd_phi_fits<128, 64>() : fwd_phi_fits<128, 128>()) : false;
+    return fits && make_plan(T, N, K, d).nseg == 1;
+}
+
+int rfa_causal_prefill_rows(const void* q, const void* k, const void* v, const void* w, float scale, void* out, float* s,
+                            float* z, int64_t T, int64_t B, int H, int D, int d, void* stream) {
+    if (H <= 0 || B < 0) return fail(RFA_ERR_BAD_SHAPE, "rfa_causal_prefill_rows: bad sizes B=%lld H=%d", (long long)B, H);
+    const int64_t N = B * H;
+    if (int rc = check_causal_dims(T, N, 2 * D, d)) return rc;
+    if (!rfa_causal_prefill_rows_supported(T, N, D, d))
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_causal_prefill_rows: T=%lld, B * H=%lld, D=%d, d=%d takes the feature map and rfa_causal_prefill",
+                    (long long)T, (long long)N, D, d);
+    if (!q || !k || !v || !w || !out || !s || !z) return fail(RFA_ERR_NULL_POINTER, "rfa_causal_prefill_rows: NULL pointer");
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(w) || !aligned16(out) || !aligned16(s) || !aligned16(z))
+        return fail(RFA_ERR_ALIGNMENT, "rfa_causal_prefill_rows: tensors must be 16-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto* qh = static_cast<const rfa::half_t*>(q);
+    auto* kh = static_cast<const rfa::half_t*>(k);
+    auto* vh = static_cast<const rfa::half_t*>(v);
+    auto* wh = static_cast<const rfa::half_t*>(w);
+    auto* oh = static_cast<rfa::half_t*>(out);
+#define RFA_CALL(KD, DH) launch_prefill_phi<KD, DH>(qh, kh, vh, wh, scale, oh, s, z, (int)T, (int)N, H, st)
+    RFA_DISPATCH_KD(2 * D, d, RFA_CALL)
+#undef RFA_CALL
+    return fail(RFA_ERR_UNSUPPORTED, "unreachable");
 }
 
 int rfa_causal_forward_save(const void* q, const void* k, const void* v, void* out, void* saved,

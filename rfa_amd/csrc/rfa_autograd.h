@@ -396,6 +396,24 @@ OptTensor node_causal(const Tensor& phi_q, const Tensor& phi_k, const Tensor& v,
     return causal(phi_q, phi_k, v, pad.has_value() ? OptTensor(pad->to(torch::kBool)) : c10::nullopt);
 }
 
+// A prompt without autograd: q, k, v [T, B, H, d] -> (attn [T, B, H * d], s [B, H, 2D, d], z [B, H, 2D]), the
+// feature maps inside the scan; nothing where the sequences do not fill the chip or a tensor is not plain.
+c10::optional<std::tuple<Tensor, Tensor, Tensor>> node_prefill(const Tensor& q, const Tensor& k, const Tensor& v,
+                                                               const Tensor& w, double scale) {
+    if (!plain_mode() || !plain_scan(q, k, v) || !plain_half(w, 3) || q.size(3) != v.size(3) || w.size(0) != q.size(2) ||
+        w.size(2) != q.size(3) || w.device() != q.device() || !q.is_contiguous() || !k.is_contiguous() || !v.is_contiguous() ||
+        !w.is_contiguous() || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(w))
+        return c10::nullopt;
+    const int64_t T = q.size(0), B = q.size(1), H = q.size(2), d = q.size(3), D = w.size(1);
+    if (!rfa_causal_prefill_rows_supported(T, B * H, (int)D, (int)d)) return c10::nullopt;
+    const auto f32 = q.options().dtype(torch::kFloat32);
+    Tensor attn = scan_output(v), s = torch::empty({B, H, 2 * D, d}, f32), z = torch::empty({B, H, 2 * D}, f32);
+    Launch l(q);
+    check_rc(rfa_causal_prefill_rows(ptr(q), ptr(k), ptr(v), ptr(w), (float)scale, ptr(attn), s.data_ptr<float>(),
+                                     z.data_ptr<float>(), T, B, (int)H, (int)D, (int)d, l.stream));
+    return std::tuple(attn, s, z);
+}
+
 // q, k, v projections, phi(q) and phi(k), the scan: x [T, B, E] -> attn [T, B, H * d].  `matrices` is
 // W' itself where `build` is false.
 OptTensor node_causal_layer(const Tensor& x, const Tensor& matrices, const OptTensor& sigma, double tau, bool build,
@@ -530,6 +548,7 @@ void bind_nodes(pybind11::module_& m) {
     m.def("node_linear_rows", &node_linear_rows, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("node_causal", &node_causal, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"),
           py::arg("key_padding_mask") = py::none());
+    m.def("node_prefill", &node_prefill, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("w"), py::arg("scale"));
     m.def("node_causal_layer", &node_causal_layer, py::arg("x"), py::arg("matrices"), py::arg("sigma"), py::arg("tau"),
           py::arg("build"), py::arg("weights"), py::arg("biases"), py::arg("heads"), py::arg("scale"));
     m.def("node_masked", &node_masked, py::arg("phi_q"), py::arg("phi_k"), py::arg("v"), py::arg("key_padding_mask"),

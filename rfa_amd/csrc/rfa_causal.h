@@ -28,6 +28,7 @@
 //     R += Q^T (G/den);  r += Q^T gz
 #pragma once
 #include "rfa_common.h"
+#include "rfa_featuremap.h"
 
 namespace rfa {
 
@@ -484,6 +485,7 @@ struct FwdPipeCfg {
     static constexpr int kBufHalves = 2 * C * LDQ + C * LDV + C * LDA;
     static constexpr size_t kBufBytes = (size_t)kBufHalves * 2 + C * 4;     // + dens[C]
     static constexpr size_t kLds = 2 * kBufBytes + KD * 4;                   // + zs[KD]
+    static constexpr size_t kPhiLds = kLds + (size_t)(KD / 2) * FeatureCfg<KD / 2, DH>::LDW * 2;    // PHI: + W'
     static_assert(kBufBytes % 16 == 0, "buffer alignment");
 };
 
@@ -504,12 +506,20 @@ struct SegBounds {
     int first[17];      // segment s covers chunks [first[s], first[s + 1])
 };
 
-template <int KD, int DH, bool RECOMPUTE = false>
+//
+// PHI: q and k are the projected rows [T, N, DH] and the tile group forms their feature maps on the way into LDS
+// (W' of the sequence's head beside the buffers; the values k_feature_map_fwd gives, rounded to fp16 alike), so
+// phi never passes through memory: 4 DH halves per step and head in place of 4 DH + 12 D.  Bound as before by
+// the rows that arrive and, level with them, by the tile group's own chain.  A layer taking
+// in 64 prompts of 512 tokens, 16 heads of 64, 64 features: 447 -> 363 us, the feature map's launch (95) gone.
+template <int KD, int DH, bool RECOMPUTE = false, bool PHI = false>
 __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     half_t* __restrict__ out, const float* __restrict__ wsS, const float* __restrict__ wsZ,
     float* __restrict__ den_out, float* __restrict__ final_s, float* __restrict__ final_z, int T, int N,
-    int nseg, int seg_len, int prefixed, int* __restrict__ hdr_out, PlanWords plan, SegBounds bounds, int wide_rows) {
+    int nseg, int seg_len, int prefixed, int* __restrict__ hdr_out, PlanWords plan, SegBounds bounds, int wide_rows,
+    const half_t* __restrict__ wf, int H, float scale) {
+    static_assert(!(PHI && RECOMPUTE), "the state before a segment would need phi(k) as well");
     // wide_rows: 64 rows of a tensor span 4 GiB or more, beyond the 32-bit lane offsets of the
     // full-chunk loads; every chunk then takes the clamped 64-bit row addresses (never with RECOMPUTE)
     plan_write(hdr_out, plan);
@@ -539,11 +549,65 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
     // Both branches run n_prefix iterations with one barrier each and one more barrier (RECOMPUTE),
     // then n_chunks + 1 iterations with exactly two barriers each.
     if (tile_group) {
-        const half_t* qb = q + (int64_t)n * KD;
-        const half_t* kb = k + (int64_t)n * KD;
+        constexpr int QW = PHI ? DH : KD;       // width of a q or k row
+        const half_t* qb = q + (int64_t)n * QW;
+        const half_t* kb = k + (int64_t)n * QW;
         const half_t* vb = v + (int64_t)n * DH;
         ChunkRegs<KD, NT> rq, rk;
         ChunkRegs<DH, NT> rv;
+        // PHI: row 16 w + i of the chunk in the order of a matrix operand, 16 bytes per 32 columns
+        h8 fq[DH / 32], fk[DH / 32];
+        const half_t* const Ws = reinterpret_cast<const half_t*>(zs + KD);
+        auto load_rows = [&](h8 (&f)[DH / 32], const half_t* b, int t0) __attribute__((always_inline)) {
+            const half_t* p = b + (int64_t)min(t0 + 16 * w + row, t_end - 1) * N * DH + 8 * G;
+#pragma unroll
+            for (int c = 0; c < DH / 32; ++c) f[c] = *reinterpret_cast<const h8*>(p + 32 * c);
+        };
+        // phi of the wave's 16 q rows and 16 k rows to LDS; rows past the end are zero
+        auto phi_to_lds = [&](half_t* Qs, half_t* Ks, int t0) __attribute__((always_inline)) {
+            constexpr int D = KD / 2, LDW = FeatureCfg<D, DH>::LDW;
+            const bool valid = t0 + 16 * w + row < t_end;
+            float turns[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float ss = 0.f;
+#pragma unroll
+                for (int c = 0; c < DH / 32; ++c) {
+                    const uint4 x = __builtin_bit_cast(uint4, u ? fk[c] : fq[c]);
+                    ss += dot_h8(x, x);
+                }
+                ss = sum_over_groups(ss);
+                turns[u] = rcp_nr(__builtin_amdgcn_sqrtf(ss) + 1e-3f) * 0.15915494309189535f;
+            }
+#pragma unroll
+            for (int t = 0; t < D / 32; ++t) {
+                f4 u[2][2] = {{f4_zero(), f4_zero()}, {f4_zero(), f4_zero()}};
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int c = 0; c < DH / 32; ++c) {
+                        const h8 a = row8(Ws, LDW, 32 * t + 16 * h + row, 32 * c, G);
+                        u[0][h] = mfma32(a, fq[c], u[0][h]);
+                        u[1][h] = mfma32(a, fk[c], u[1][h]);
+                    }
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    h8 sv, cv;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        float s_, c_;
+                        sincos_turns(u[x][e / 4][e % 4] * turns[x], s_, c_);
+                        sv[e] = valid ? (half_t)(scale * s_) : (half_t)0.f;
+                        cv[e] = valid ? (half_t)(scale * c_) : (half_t)0.f;
+                    }
+                    half_t* dst = (x ? Ks : Qs) + (16 * w + row) * LDQ + 32 * t + 8 * G;
+                    *reinterpret_cast<h8*>(dst) = sv;
+                    *reinterpret_cast<h8*>(dst + D) = cv;
+                }
+            }
+        };
+        if constexpr (PHI)
+            load_w_pair_order<KD / 2, DH, NT>(const_cast<half_t*>(Ws), wf + (int64_t)(n % H) * (KD / 2) * DH, tid);
         // full chunks: wave-uniform base plus one lane offset per tensor; only the last chunk of the
         // sequence can be short and takes the clamped row addresses
         RowPtrs<KD, NT> pq_, pk_;
@@ -552,10 +616,16 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
         pk_.init(kb, k_stride, tid);
         pv_.init(vb, v_stride, tid);
         if (n_chunks > 0) {
-            chunk_g2r<KD, NT>(rq, qb + (int64_t)t_begin * k_stride, k_stride, t_end - t_begin, tid);
-            chunk_g2r<KD, NT>(rk, kb + (int64_t)t_begin * k_stride, k_stride, t_end - t_begin, tid);
+            if constexpr (PHI) {
+                load_rows(fq, qb, t_begin);
+                load_rows(fk, kb, t_begin);
+            } else {
+                chunk_g2r<KD, NT>(rq, qb + (int64_t)t_begin * k_stride, k_stride, t_end - t_begin, tid);
+                chunk_g2r<KD, NT>(rk, kb + (int64_t)t_begin * k_stride, k_stride, t_end - t_begin, tid);
+            }
             chunk_g2r<DH, NT>(rv, vb + (int64_t)t_begin * v_stride, v_stride, t_end - t_begin, tid);
         }
+        if constexpr (PHI) wg_barrier();        // W' in place (the state group joins with a barrier of its own)
         f4 zacc[NKTW];      // z for feature tiles kt = w*NKTW + a, element k = 16kt + 4G + e
 #pragma unroll
         for (int a = 0; a < NKTW; ++a) zacc[a] = f4_zero();
@@ -622,8 +692,12 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
             float* dens = reinterpret_cast<float*>(As + C * LDA);
             const bool live = it < n_chunks;
             if (live) {
-                chunk_r2s<KD, NT>(rq, Qs, LDQ, tid);
-                chunk_r2s<KD, NT>(rk, Ks, LDQ, tid);
+                if constexpr (PHI) {
+                    phi_to_lds(Qs, Ks, t_begin + it * C);
+                } else {
+                    chunk_r2s<KD, NT>(rq, Qs, LDQ, tid);
+                    chunk_r2s<KD, NT>(rk, Ks, LDQ, tid);
+                }
                 chunk_r2s<DH, NT>(rv, Vs, LDV, tid);
                 if (row == 0) {
 #pragma unroll
@@ -637,8 +711,16 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
                 const int t0 = t_begin + it * C;
                 const int rows_next = t_end - t0 - C;
                 const bool fast_rows = rows_next >= C && !wide_rows;
-                if (fast_rows) pq_.load_full(rq, (int64_t)(t0 + C) * k_stride);
-                else if (rows_next > 0) chunk_g2r<KD, NT>(rq, qb + (int64_t)(t0 + C) * k_stride, k_stride, rows_next, tid);
+                if constexpr (PHI) {
+                    if (rows_next > 0) {
+                        load_rows(fq, qb, t0 + C);
+                        load_rows(fk, kb, t0 + C);
+                    }
+                } else if (fast_rows) {
+                    pq_.load_full(rq, (int64_t)(t0 + C) * k_stride);
+                } else if (rows_next > 0) {
+                    chunk_g2r<KD, NT>(rq, qb + (int64_t)(t0 + C) * k_stride, k_stride, rows_next, tid);
+                }
                 RFA_TICK_AT(3, 0);
                 // rows i in [16w, 16w+16) of A as A^T tiles (m=j, n=i), all four j tiles
                 f4 at[4];
@@ -651,10 +733,10 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
                     for (int a = 0; a < 4; ++a) at[a] = mfma32(row8(Ks, LDQ, 16 * a + row, ks * 32, G), bq, at[a]);
                 }
                 if (fast_rows) {              // second part of the next chunk's rows
-                    pk_.load_full(rk, (int64_t)(t0 + C) * k_stride);
+                    if constexpr (!PHI) pk_.load_full(rk, (int64_t)(t0 + C) * k_stride);
                     pv_.load_full(rv, (int64_t)(t0 + C) * v_stride);
                 } else if (rows_next > 0) {
-                    chunk_g2r<KD, NT>(rk, kb + (int64_t)(t0 + C) * k_stride, k_stride, rows_next, tid);
+                    if constexpr (!PHI) chunk_g2r<KD, NT>(rk, kb + (int64_t)(t0 + C) * k_stride, k_stride, rows_next, tid);
                     chunk_g2r<DH, NT>(rv, vb + (int64_t)(t0 + C) * v_stride, v_stride, rows_next, tid);
                 }
                 float part = 0.f;
@@ -713,6 +795,7 @@ __global__ __launch_bounds__(512) void k_causal_fwd_pipe(
         for (int a = 0; a < NKT; ++a)
 #pragma unroll
             for (int b = 0; b < NCT; ++b) S[a][b] = f4_zero();
+        if constexpr (PHI) wg_barrier();
         if constexpr (RECOMPUTE) {
             for (int jc = 0; jc < n_prefix; ++jc) {
                 wg_barrier();

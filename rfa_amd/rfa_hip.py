@@ -714,7 +714,7 @@ _BOUND = ("supported", "feature_map_supported", "selftest_layout", "forward", "b
           "incremental_qkv",
           "pack_negative_mask", "masked_forward", "masked_backward")
 # autograd functions and chains of them as C++ nodes (csrc/rfa_autograd.h): only the binding has them
-_NODES = ("node_random_project", "node_linear", "node_linear_rows", "node_causal", "node_causal_layer", "node_masked", "node_cross_source",
+_NODES = ("node_random_project", "node_linear", "node_linear_rows", "node_causal", "node_prefill", "node_causal_layer", "node_masked", "node_cross_source",
           "node_cross_query")
 _CTYPES_IMPL = {name: globals()[name] for name in _BOUND}
 _active = "ctypes"

@@ -557,3 +557,32 @@ def test_native_nodes_leave_odd_calls_to_the_python_functions():
         torch.func.grad(lambda a: call(a).float().sum())(q.detach())
     with pytest.raises(RuntimeError), forward_ad.dual_level():
         call(forward_ad.make_dual(q.detach(), torch.ones_like(q)))
+
+
+@pytest.mark.parametrize("d,D", [(64, 32), (64, 64), (128, 32), (128, 64)])
+@pytest.mark.parametrize("T", [2, 15, 64, 65, 127, 200])
+def test_prefill_from_projected_rows(T, d, D):
+    """The scan that forms phi(q), phi(k) itself against the feature-map launch followed by the scan,
+    at short last chunks and with rows of zeros.  The formulas are the same; the compiler may contract them
+    differently, which moves a phi value to the neighbouring fp16 value at most (2^-11)."""
+    from rfa_amd import _lib, rfa_hip
+    from rfa_amd.utils import random_project_pair
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    H = 4
+    B = 300 if T > 64 else 3        # sequences enough for one segment each
+    assert _lib.load().rfa_causal_prefill_rows_supported(T, B * H, D, d)
+    gen = torch.Generator("cuda").manual_seed(T)
+    q, k, v = (torch.randn(T, B, H, d, generator=gen, device="cuda").half() for _ in range(3))
+    q[T // 2, 1] = 0
+    k[T - 1, 2] = 0
+    W = O.make_w(d, D, H).half().cuda()
+    print(f"prefill from rows T={T} d={d} D={D}", flush=True)
+    attn, s, z = rfa_hip.native.node_prefill(q, k, v, W, O.SCALE)
+    pq, pk = random_project_pair(x0=q, x1=k, random_matrices=W)
+    want = rfa_hip.prefill(pq.view(T, B * H, 2 * D), pk.view(T, B * H, 2 * D), v.view(T, B * H, d))
+    for got, ref in zip((attn, s, z), want):
+        err = _rel(got.reshape(ref.shape).float().cpu(), ref.float().cpu())
+        print(f"  {err:.2e}", flush=True)
+        assert torch.isfinite(got).all() and err <= 2.0 ** -11
+    assert rfa_hip.native.node_prefill(q[:, :1], k[:, :1], v[:, :1], W, O.SCALE) is None      # not contiguous
