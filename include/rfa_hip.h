@@ -287,6 +287,12 @@ size_t rfa_linear_weight_grad_workspace_bytes(int64_t R, int E_out, int E_in, in
 int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw, void* const* db, int np,
                            int64_t R, int E_out, int E_in, void* workspace, size_t workspace_bytes,
                            void* stream);
+/* dx = sum_p dy_p W_p, the input gradient of those layers: dy_p fp16 [R, E_out] with rows ld elements apart
+ * (ld = 3 E_out for the blocks of a packed gradient), w_p fp16 [E_out, E_in], dx fp16 [R, E_in]; fp32 sums over
+ * all p, one rounding.  E_out a multiple of 32, E_in of 128. */
+int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R,
+                          int E_out, int E_in, void* stream);
+
 
 /* ---------------------------------------------------------------------------
  * Cross attention (encoder -> decoder).  The state is fp32.

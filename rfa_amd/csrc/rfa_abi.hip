@@ -46,7 +46,7 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
@@ -54,7 +54,7 @@ const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
                                    "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
-                                   "k_cross_step", "k_mask_rows"};
+                                   "k_cross_step", "k_mask_rows", "k_input_grad"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -800,6 +800,20 @@ WGradPlan make_wgrad_plan(int64_t R, int Eo, int Ei, int np) {
     p.nsplit = (int)((nsteps + sps - 1) / sps);
     if (p.nsplit < 1) p.nsplit = 1;
     return p;
+}
+
+// ---- input-gradient launcher ----------------------------------------------------------
+template <int BM>
+int launch_input_grad(const rfa::InputGradArgs& ga, rfa::half_t* dx, int R, int Eo, int Ei, int np, int64_t ld,
+                             hipStream_t st) {
+    using Cfg = rfa::InputGradCfg<BM>;
+    auto kern = rfa::k_input_grad<BM>;
+    if (int rc = set_lds(kern, Cfg::kLds)) return rc;
+    const int64_t tiles = (int64_t)((R + BM - 1) / BM) * (Ei / Cfg::BN);
+    RFA_LAUNCH(INPUT_GRAD, kern, dim3((unsigned)(rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds))), dim3(rfa::kThreads),
+               Cfg::kLds, st, ga, dx, R, Eo, Ei, np, ld, (int)tiles);
+    RFA_HIP_TRY(hipGetLastError());
+    return RFA_OK;
 }
 
 // ---- feature map launchers ---------------------------------------------------------
@@ -1965,6 +1979,40 @@ size_t rfa_linear_weight_grad_workspace_bytes(int64_t R, int E_out, int E_in, in
     if (R <= 0 || E_out <= 0 || E_in <= 0 || E_out % 128 || E_in % 128 || np < 1 || np > rfa::kMaxProjections) return 0;
     const WGradPlan pl = make_wgrad_plan(R, E_out, E_in, np);
     return (size_t)pl.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+}
+
+int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R, int E_out,
+                          int E_in, void* stream) {
+    if (R < 0 || E_out <= 0 || E_in <= 0 || R > (int64_t(1) << 30) || ld < E_out || ld > (1 << 22) || E_in > (1 << 22))
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: bad sizes rows=%lld E_out=%d E_in=%d ld=%lld", (long long)R, E_out,
+                    E_in, (long long)ld);
+    if (E_out % 32 || E_in % 128 || ld % 8)
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_linear_input_grad: E_out=%d must be a multiple of 32, E_in=%d of 128 and ld=%lld of 8",
+                    E_out, E_in, (long long)ld);
+    if (np < 1 || np > rfa::kMaxProjections)
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: %d projections (1..%d supported)", np, rfa::kMaxProjections);
+    if (R == 0) return RFA_OK;
+    if (!dy || !w || !dx) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_input_grad: NULL pointer");
+    rfa::InputGradArgs ga{};
+    for (int p = 0; p < np; ++p) {
+        ga.dy[p] = static_cast<const rfa::half_t*>(dy[p]);
+        ga.w[p] = static_cast<const rfa::half_t*>(w[p]);
+        if (!ga.dy[p] || !ga.w[p]) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_input_grad: NULL tensor %d", p);
+        if (!aligned16(ga.dy[p]) || !aligned16(ga.w[p]))
+            return fail(RFA_ERR_ALIGNMENT, "rfa_linear_input_grad: tensors must be 16-byte aligned");
+    }
+    if (!aligned16(dx)) return fail(RFA_ERR_ALIGNMENT, "rfa_linear_input_grad: tensors must be 16-byte aligned");
+    if (((R + 63) / 64) * (E_in / 128) > (int64_t(1) << 30))
+        return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: sizes exceed the supported range");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto* dxh = static_cast<rfa::half_t*>(dx);
+    // rows per tile as launch_project_phi chooses them
+    const int64_t cus = device_cus(), t128 = (R + 127) / 128 * (E_in / 128), t256 = (R + 255) / 256 * (E_in / 128);
+    int rows = t128 < cus ? 64 : 128;
+    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= 3 * ((t128 + cus - 1) / cus)) rows = 256;
+    if (rows == 256) return launch_input_grad<256>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
+    if (rows == 128) return launch_input_grad<128>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
+    return launch_input_grad<64>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
 }
 
 int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw, void* const* db, int np, int64_t R,

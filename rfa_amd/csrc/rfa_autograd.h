@@ -135,6 +135,33 @@ std::pair<std::vector<Tensor>, std::vector<OptTensor>> param_grads(const Tensor&
     return {dws, dbs};
 }
 
+// Products through the framework's own kernels: a library product costs 19 us of host time, these 4 to 5, and
+// two of them in a backward need a second pass over dx, three a stack of the weights.  Up to 7e9
+// multiply-adds they are level on the device, us own / library: 8192 rows of 512 -> 512 11.6 / 12.3 (dx), 10.6 /
+// 11.4 (y); three of them 24.8 / 21.4 + 4.6 for the stack.  Past that the library's larger tiles win (8192
+// rows of 1024 -> 1024 28.9 / 23.6, 28.3 / 24.4; three 69.3 / 57.3 + 7.8), for two layers without a packed
+// gradient, where it takes two products, later (16384 rows of 512 28.1 / 38; of 1024 82.5 / 75).
+bool own_product(int64_t rows, int64_t e_out, int64_t e_in, int64_t n) {
+    return rows > 0 && rows * e_out * e_in * n <= (n == 2 ? (int64_t)1 << 34 : (int64_t)7 << 30);
+}
+
+// dx = sum_p dy_p W_p for dy_p [rows, E_out] that lie ld halves a row from dys[p] on
+bool own_input_grad(int64_t rows, const Tensor* w, int64_t n) {
+    bool ok = own_product(rows, w[0].size(0), w[0].size(1), n) && w[0].size(0) % 32 == 0 && w[0].size(1) % 128 == 0;
+    for (int64_t p = 0; p < n; ++p) ok = ok && w[p].is_contiguous() && aligned16(w[p]);
+    return ok;
+}
+
+Tensor input_grad(const std::vector<const void*>& dys, int64_t ld, const Tensor* w, const Tensor& x) {
+    const int64_t n = (int64_t)dys.size(), e_out = w[0].size(0), e_in = w[0].size(1), rows = x.numel() / e_in;
+    std::array<const void*, 3> wp{};
+    for (int64_t p = 0; p < n; ++p) wp[p] = ptr(w[p]);
+    Tensor dx = torch::empty(x.sizes(), x.options());
+    Launch l(x);
+    check_rc(rfa_linear_input_grad(dys.data(), ld, wp.data(), (int)n, ptr(dx), rows, (int)e_out, (int)e_in, l.stream));
+    return dx;
+}
+
 struct ProjectNode : public torch::autograd::Function<ProjectNode> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& wf, double scale, int64_t heads,
                                  int64_t phi, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
@@ -189,7 +216,10 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             Tensor packed;
             std::tie(packed, dwf) = feature_map_backward_pair_packed(y[0], y[1], wf, g[0].contiguous(), g[1].contiguous(),
                                                                      g[2].contiguous(), scale, need_wf);
-            out[0] = at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
+            const char* base = static_cast<const char*>(packed.data_ptr());
+            out[0] = own_input_grad(rows, w, 3)
+                         ? input_grad({base, base + 2 * e_out, base + 4 * e_out}, 3 * e_out, w, x)
+                         : at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
             auto [dws, dbs] = param_grads(x2, {packed}, {bias_bits != 0});
             for (int64_t p = 0; p < n; ++p) {
                 out[5 + 2 * p] = dws[0].narrow(0, p * e_out, e_out);
@@ -213,7 +243,16 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
                     }
                 }
                 dys[p] = dys[p].reshape({rows, -1});
-                if (need_x) out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
+            }
+            bool own = need_x && own_input_grad(rows, w, n);
+            for (const Tensor& dy : dys) own = own && aligned16(dy);
+            if (own) {
+                std::vector<const void*> dyp;
+                for (Tensor& dy : dys) dyp.push_back(ptr(dy));
+                out[0] = input_grad(dyp, w[0].size(0), w, x);
+            }
+            for (int64_t p = 0; p < n && need_x && !own; ++p) {
+                out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
             }
             auto [dws, dbs] = param_grads(x2, dys, bias);
             for (int64_t p = 0; p < n; ++p) {
@@ -264,14 +303,34 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
         ctx->saved_data["bias"] = b.has_value();
         ctx->saved_data["need_x"] = x.requires_grad();
         ctx->save_for_backward({x, w});
-        return at::linear(x, w, b);
+        const int64_t e_in = w.size(1), e_out = w.size(0), rows = e_in ? x.numel() / e_in : 0;
+        const Tensor bias = opt(b);
+        if (!own_product(rows, e_out, e_in, 1) || e_in % 64 != 0 || e_out % 64 != 0 || x.size(-1) != e_in ||
+            !x.is_contiguous() || !w.is_contiguous() || !aligned16(x) || !aligned16(w) || w.device() != x.device() ||
+            (bias.defined() && (bias.size(0) != e_out || !bias.is_contiguous() || !aligned16(bias) || bias.device() != x.device())))
+            return at::linear(x, w, b);
+        // the projection kernel with no feature map: heads of 64 columns are the plain product
+        auto shape = x.sizes().vec();
+        shape.back() = e_out;
+        Tensor y = torch::empty(shape, x.options());
+        std::array<const void*, 1> wp{ptr(w)}, bp{bias.defined() ? ptr(bias) : nullptr};
+        std::array<void*, 1> yp{ptr(y)};
+        Launch l(x);
+        check_rc(rfa_project_feature_map(ptr(x), wp.data(), bp.data(), yp.data(), nullptr, 1, nullptr, rows, (int)e_in,
+                                         (int)(e_out / 64), 32, 64, 0.f, l.stream));
+        return y;
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &w = saved[1];
         const Tensor dy2 = g[0].reshape({-1, g[0].size(-1)}), x2 = x.reshape({-1, x.size(-1)});
         Tensor dx;
-        if (ctx->saved_data["need_x"].toBool()) dx = at::mm(dy2, w).view(x.sizes());
+        if (ctx->saved_data["need_x"].toBool()) {
+            const Tensor dyc = dy2.contiguous();
+            dx = own_input_grad(dyc.size(0), &w, 1) && aligned16(dyc)
+                     ? input_grad({ptr(dyc)}, w.size(0), &w, x)
+                     : at::mm(dyc, w).view(x.sizes());
+        }
         auto [dws, dbs] = param_grads(x2, {dy2}, {ctx->saved_data["bias"].toBool()});
         return {dx, dws[0], opt(dbs[0])};
     }
@@ -287,7 +346,9 @@ bool few_rows(int64_t R, int64_t e_in, int64_t e_out) {
 
 // for the callers' condition (fp16, grad mode on, widths that are multiples of 128) see linear_out
 OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
-    if (!plain_mode() || !plain_half(x, x.dim()) || !plain_half(w, 2) || !plain_half(b, 1)) return c10::nullopt;
+    if (!plain_mode() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 || !plain_half(x, x.dim()) ||
+        !plain_half(w, 2) || !plain_half(b, 1))
+        return c10::nullopt;
     return LinearNode::apply(x, w, b);
 }
 

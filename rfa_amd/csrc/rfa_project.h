@@ -502,6 +502,115 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Input gradient of those Linear layers: dx[r][c] = sum_p sum_o dy_p[r][o] W_p[o][c], one contraction over the
+// output columns of all of them (fp32 accumulate, one rounding; autograd adds rounded products).
+// Layouts: dy_p [R, Eo] with rows ld halves apart (the thirds of a packed gradient: 3 Eo), W_p [Eo, Ei], dx [R, Ei].
+// ---------------------------------------------------------------------------
+struct InputGradArgs {
+    const half_t* dy[kMaxProjections];
+    const half_t* w[kMaxProjections];
+};
+
+template <int BM_>
+struct InputGradCfg {
+    static constexpr int BM = BM_, BN = 128, BK = 32, kStages = 3;
+    static constexpr int RW = BM / 2, NR = RW / 16, NC = 4;       // a wave: BM / 2 rows x 64 columns
+    static constexpr int YI = BM / 64, WI = 2;                    // 1 KiB pieces of a stage per wave: dy, W
+    static constexpr int kStageHalves = (BM + BN) * BK;
+    static constexpr size_t kLds = (size_t)kStages * kStageHalves * 2;
+};
+
+// A tile of BM rows x 128 columns per workgroup of four waves; stages of 32 output columns through the three-stage
+// ring of k_project_phi (dy rows as its x) with W's rows as k_weight_grad_partial stages them: contracted over
+// their row index, read by the transposing read.  The weights are read where they are, no stack of them is
+// formed.  Bound like k_project_phi, by the step (barrier, operand reads, 16 to 32 products) where a tile has few.
+// Measured, us (the library's products over a stacked weight, which costs another 4.6 to 7.8 to form):
+// 8192 rows, 512 -> 512 11.6 (12.3), three of them 24.8 (21.4); 16384 rows, two 28.1 (24.2; 38 as two
+// products); 1024 -> 1024, three 69.3 (57.3).
+// grid = 8 * ceil(tiles / 8), tiles numbered row tile by row tile; each XCD gets a contiguous range.
+template <int BM_>
+__global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, half_t* __restrict__ dx, int R, int Eo, int Ei,
+                                                            int np, int64_t ld, int tiles) {
+    using Cfg = InputGradCfg<BM_>;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, STAGES = Cfg::kStages, NR = Cfg::NR, NC = Cfg::NC;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    half_t* smem = reinterpret_cast<half_t*>(smem_raw);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, G = lane >> 4;
+    const int wr = wv >> 1, wc = wv & 1;
+
+    const int per_xcd = (tiles + kXcds - 1) / kXcds;
+    const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (tile >= tiles) return;                         // whole workgroup: padding of the grid
+    const int tiles_c = Ei / BN;
+    const int row0 = (tile / tiles_c) * BM, c0 = (tile % tiles_c) * BN;
+
+    unsigned yoff[Cfg::YI], woff[Cfg::WI];
+#pragma unroll
+    for (int it = 0; it < Cfg::YI; ++it) {
+        const int r = (wv * Cfg::YI + it) * 16 + (lane >> 2);
+        yoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(ld * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+    }
+#pragma unroll
+    for (int it = 0; it < Cfg::WI; ++it) {
+        const int r = (wv * Cfg::WI + it) * 4 + (lane >> 4);
+        woff[it] = (unsigned)r * (unsigned)(Ei * 2) + (((lane & 15) ^ (((r & 3) | ((r >> 1) & 4)) * 2)) * 16);
+    }
+    const int per_p = Eo / BK, nk = np * per_p;
+    auto load_stage = [&](int kk, int buf) {
+        const int p = kk >= 2 * per_p ? 2 : (kk >= per_p ? 1 : 0), ko = (kk - p * per_p) * BK;
+        const half_t* yb = pick3(ga.dy, p) + (int64_t)row0 * ld + ko;
+        const half_t* wb = pick3(ga.w, p) + (int64_t)ko * Ei + c0;
+        half_t* st = smem + buf * Cfg::kStageHalves;
+#pragma unroll
+        for (int it = 0; it < Cfg::YI; ++it) dma16_opaque(yb, yoff[it], st + (wv * Cfg::YI + it) * 512);
+#pragma unroll
+        for (int it = 0; it < Cfg::WI; ++it) dma16_opaque(wb, woff[it], st + BM * BK + (wv * Cfg::WI + it) * 512);
+    };
+
+    f4 acc[NR][NC];      // dx^T tiles (m = column, n = row)
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[a][c] = f4_zero();
+    const half_t* const yop = smem + (wr * Cfg::RW + i) * BK + (G ^ ((i >> 2) & 3)) * 8;
+
+#pragma unroll
+    for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
+    int buf = 0;
+    for (int kk = 0; kk < nk; ++kk) {
+        stage_barrier<(STAGES - 2) * (Cfg::YI + Cfg::WI)>();
+        load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
+        const half_t* ys = yop + buf * Cfg::kStageHalves;
+        const half_t* Ws = smem + buf * Cfg::kStageHalves + BM * BK;
+        h8 wa[NC], yb[NR];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) wa[c] = col8_rot<BN>(Ws, NC * wc + c, lane);
+#pragma unroll
+        for (int a = 0; a < NR; ++a) yb[a] = *reinterpret_cast<const h8*>(ys + a * 16 * BK);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int a = 0; a < NR; ++a)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[a][c] = mfma32(wa[c], yb[a], acc[a][c]);
+        __builtin_amdgcn_s_setprio(0);
+        buf = buf == STAGES - 1 ? 0 : buf + 1;
+    }
+    // the last re-requested stages are still on their way into this workgroup's LDS: they land before it ends
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int a = 0; a < NR; ++a) {
+        const int r = row0 + wr * Cfg::RW + 16 * a + i;
+        if (r < R) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                *reinterpret_cast<h4*>(dx + (int64_t)r * Ei + c0 + 64 * wc + 16 * c + 4 * G) = to_h4(acc[a][c]);
+        }
+    }
+}
+
 // dW_p = sum of the partials (4 elements per thread), then db_p; grid = ceil(np * (Eo * Ei + Eo) / 4 / 256)
 __global__ __launch_bounds__(kThreads) void k_weight_grad_reduce(
     const float* __restrict__ part, const float* __restrict__ bpart, WeightGradArgs wa, int Eo, int Ei, int np,

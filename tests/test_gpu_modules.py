@@ -500,7 +500,8 @@ def _native_forms(path, form):
 @pytest.mark.parametrize("path", ["random_project", "causal", "padded", "masked", "module", "cross"])
 def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypatch):
     """The C++ autograd nodes against the Python autograd functions over the same kernels: outputs and every
-    gradient bit for bit, from strided inputs, with frozen or missing parameters, through saved-tensor
+    gradient bit for bit (in the layers, whose Linear products are summed by another kernel and rounded to fp16
+    at other places, within a few roundings), from strided inputs, with frozen or missing parameters, through saved-tensor
     hooks, and with two backward passes over one graph."""
     from rfa_amd import rfa_hip
     if rfa_hip.native is None:
@@ -529,7 +530,11 @@ def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypa
                 out.backward(g)
         results.append([out.detach()] + [None if t.grad is None else t.grad.clone() for t in leaves])
     for a, b in zip(*results):
-        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+        assert (a is None) == (b is None)
+        if a is not None and path in ("module", "cross"):
+            assert _rel(a.double().cpu(), b.double().cpu()) <= 4 * 2.0 ** -11
+        elif a is not None:
+            assert torch.equal(a, b)
 
 
 def test_native_nodes_leave_odd_calls_to_the_python_functions():

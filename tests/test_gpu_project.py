@@ -512,3 +512,25 @@ def test_output_projection_keeps_its_hooks():
         handle.remove()
         layer.forward = lambda t: t * 0
         assert projection.linear_out(x, layer).abs().max().item() == 0
+
+
+@pytest.mark.parametrize("e_out,e_in,n", [(32, 128, 1), (96, 128, 2), (128, 256, 3), (512, 512, 3), (64, 384, 2)])
+@pytest.mark.parametrize("R", [1, 15, 63, 64, 65, 129, 257, 1000, 20000])
+def test_linear_input_grad(R, e_out, e_in, n):
+    """dx = sum_p dy_p W_p over the blocks of a packed gradient, at the edges of its row tiles (64, 128 and
+    256 rows), against fp64: exact products, fp32 sums (a share 2^-20 of the sum of their magnitudes covers
+    the order of up to 1536 of them) and one rounding to fp16."""
+    import ctypes
+    from rfa_amd import _lib
+    gen = torch.Generator("cuda").manual_seed(R + e_out)
+    dy = torch.randn(R, n * e_out, generator=gen, device="cuda").half()
+    ws = [(torch.randn(e_out, e_in, generator=gen, device="cuda") / e_out ** 0.5).half() for _ in range(n)]
+    dx = torch.full((R, e_in), float("nan"), dtype=torch.float16, device="cuda")
+    array = lambda ptrs: (ctypes.c_void_p * n)(*ptrs)
+    print(f"linear_input_grad R={R} {e_out}->{e_in} x {n}", flush=True)
+    _lib.check(_lib.load().rfa_linear_input_grad(array([dy.data_ptr() + 2 * p * e_out for p in range(n)]), n * e_out,
+                                                 array([w.data_ptr() for w in ws]), n, dx.data_ptr(), R, e_out, e_in,
+                                                 torch.cuda.current_stream().cuda_stream))
+    W = torch.cat(ws, 0).double()
+    want, size = dy.double() @ W, dy.double().abs() @ W.abs()
+    assert ((dx.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -20 * size + 2.0 ** -24).all()
