@@ -57,9 +57,12 @@ struct MaskedCfg {
     static constexpr size_t kLds = (size_t)(C * LDQ + C * LDV) * 2 + C * 4;
 };
 
-// four mask bytes (one per accumulator element) -> keep flags; NULL mask keeps everything
-__device__ __forceinline__ uint32_t mask_word(const uint8_t* __restrict__ m, int64_t off) {
-    return m ? *reinterpret_cast<const uint32_t*>(m + off) : 0u;
+// the mask bytes of a lane's four 16-wide tiles of a block, one word per tile; a NULL mask keeps everything.
+// They are requested with the block's rows, a block ahead: loaded where they are used they would be the youngest
+// loads, and waiting for them would wait for the next block's rows, which are meant to stay in flight.
+__device__ __forceinline__ void mask_words(uint32_t (&words)[4], const uint8_t* __restrict__ m, int64_t off) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) words[t] = m ? *reinterpret_cast<const uint32_t*>(m + off + 16 * t) : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -177,8 +180,10 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
     masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
     ChunkRegs<KD> rk;
     ChunkRegs<DH> rv;
+    uint32_t mw_next[4];
     auto prefetch = [&](int jb) {
         const int t0 = jb * C;
+        mask_words(mw_next, attn_mask, (int64_t)tic * Tp + t0 + 4 * G);
         chunk_g2r<KD>(rk, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
         chunk_g2r<DH>(rv, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         if (prow) chunk_mask_rows<KD>(rk, prow + t0, tid);
@@ -194,6 +199,7 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
     while (jb < nblk) {
         chunk_r2s<KD>(rk, Ks, LDQ, tid);
         chunk_r2s<DH>(rv, Vs, LDV, tid);
+        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
         __syncthreads();
         const int jb_next = next_live_block(skip, jb + 1, nblk);
         if (jb_next < nblk) prefetch(jb_next);
@@ -204,7 +210,7 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks)
                 at[jt] = mfma32(row8(Ks, LDQ, 16 * jt + row, 32 * ks, G), bq[ks], at[jt]);
-            const uint32_t mw = mask_word(attn_mask, (int64_t)tic * Tp + jb * C + 16 * jt + 4 * G);
+            const uint32_t mw = mw4[jt];
 #pragma unroll
             for (int e = 0; e < 4; ++e) at[jt][e] = ((mw >> (8 * e)) & 0xffu) ? 0.f : at[jt][e];
             rpart += (at[jt][0] + at[jt][1]) + (at[jt][2] + at[jt][3]);
@@ -306,8 +312,10 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
     masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
     ChunkRegs<KD> rk;
     ChunkRegs<DH> rv;
+    uint32_t mw_next[4];
     auto prefetch = [&](int jb) {
         const int t0 = jb * C;
+        mask_words(mw_next, attn_mask, (int64_t)tic * Tp + t0 + 4 * G);
         chunk_g2r<KD>(rk, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
         chunk_g2r<DH>(rv, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         if (prow) chunk_mask_rows<KD>(rk, prow + t0, tid);
@@ -322,6 +330,7 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
     while (jb < nblk) {
         chunk_r2s<KD>(rk, Ks, LDQ, tid);
         chunk_r2s<DH>(rv, Vs, LDV, tid);
+        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
         __syncthreads();
         const int jb_next = next_live_block(skip, jb + 1, nblk);
         if (jb_next < nblk) prefetch(jb_next);
@@ -332,7 +341,7 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
 #pragma unroll
             for (int cs = 0; cs < NCS; ++cs)
                 pt[jt] = mfma32(row8(Vs, LDV, 16 * jt + row, 32 * cs, G), bg[cs], pt[jt]);
-            const uint32_t mw = mask_word(attn_mask, (int64_t)tic * Tp + jb * C + 16 * jt + 4 * G);
+            const uint32_t mw = mw4[jt];
 #pragma unroll
             for (int e = 0; e < 4; ++e) pt[jt][e] = ((mw >> (8 * e)) & 0xffu) ? 0.f : pt[jt][e] + gzi;
         }
@@ -395,7 +404,9 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
     ChunkRegs<KD> rq;
     ChunkRegs<DH> rg;
     float gz_next;
+    uint32_t mw_next[4];
     auto prefetch = [&](int t0) {
+        mask_words(mw_next, attn_mask_t, (int64_t)tjc * Tp + t0 + 4 * G);
         chunk_g2r<KD>(rq, qb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
         chunk_g2r<DH>(rg, gb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         gz_next = gz[(int64_t)(t0 + min(tid & (C - 1), rg.rows - 1)) * N + n];
@@ -415,6 +426,7 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
         chunk_r2s<KD>(rq, Qs, LDQ, tid);
         chunk_r2s<DH>(rg, Gs, LDV, tid);
         if (tid < C) gzs[tid] = tid < rg.rows ? gz_next : 0.f;
+        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
         __syncthreads();
         const int ib_next = next_live_block(skip, ib + 1, nblk);
         if (ib_next < nblk) prefetch(ib_next * C);
@@ -430,7 +442,7 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
             for (int cs = 0; cs < NCS; ++cs)
                 p_[it] = mfma32(row8(Gs, LDV, 16 * it + row, 32 * cs, G), bv[cs], p_[it]);
             const f4 gzv = *reinterpret_cast<const f4*>(gzs + 16 * it + 4 * G);
-            const uint32_t mw = mask_word(attn_mask_t, (int64_t)tjc * Tp + ib * C + 16 * it + 4 * G);
+            const uint32_t mw = mw4[it];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const bool masked = padded || ((mw >> (8 * e)) & 0xffu);
@@ -467,12 +479,14 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 // nblk - 1 - p of one sequence, one after the other.  With a causal mask block p has p + 1 live
 // column blocks, so every workgroup does the same work (nblk + 1 tiles); without that pairing the
 // last row blocks set the kernel time and skipping the masked tiles would not shorten it.
+// The workgroups of a sequence run on one XCD, whose L2 then serves its rows to all but the first.
 // Without a mask nothing is skipped and grid = N * nblk, one row block per workgroup.
 // ---------------------------------------------------------------------------
 #define RFA_MASKED_PAIR(CALL, PAIRED)                                          \
     const int nblk = (T + kChunk - 1) / kChunk;                                \
     const int per_seq = (PAIRED) ? (nblk + 1) / 2 : nblk;                      \
-    const int n = blockIdx.x / per_seq, p = blockIdx.x % per_seq;              \
+    int n, p;                                                                  \
+    seq_seg_of_block(blockIdx.x, N, per_seq, n, p);                            \
     CALL(p * kChunk);                                                          \
     if ((PAIRED) && nblk - 1 - p != p) {                                       \
         __syncthreads();                                                       \
