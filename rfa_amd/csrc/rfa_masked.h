@@ -57,12 +57,16 @@ struct MaskedCfg {
     static constexpr size_t kLds = (size_t)(C * LDQ + C * LDV) * 2 + C * 4;
 };
 
-// the mask bytes of a lane's four 16-wide tiles of a block, one word per tile; a NULL mask keeps everything.
-// They are requested with the block's rows, a block ahead: loaded where they are used they would be the youngest
-// loads, and waiting for them would wait for the next block's rows, which are meant to stay in flight.
-__device__ __forceinline__ void mask_words(uint32_t (&words)[4], const uint8_t* __restrict__ m, int64_t off) {
+// The mask bytes of a lane's four 16-wide tiles of a block, one word per tile.  They are requested with the
+// block's rows, ahead of their use: loaded where they are used they would be the youngest loads, and waiting
+// for them would wait for the rows that are meant to stay in flight.  For the same reason there is no branch
+// around the loads and no arithmetic on them here (see ChunkRegs): without a mask `any` is read, 64 readable
+// bytes, and the words are dropped where they would be used.
+__device__ __forceinline__ void mask_words(uint32_t (&words)[4], const uint8_t* __restrict__ m, int64_t off,
+                                           const void* __restrict__ any) {
+    const uint8_t* p = m ? m + off : static_cast<const uint8_t*>(any);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) words[t] = m ? *reinterpret_cast<const uint32_t*>(m + off + 16 * t) : 0u;
+    for (int t = 0; t < 4; ++t) words[t] = *reinterpret_cast<const uint32_t*>(p + 16 * t);
 }
 
 // ---------------------------------------------------------------------------
@@ -85,6 +89,8 @@ __device__ __forceinline__ void masked_tile_skip(const uint8_t* __restrict__ m, 
     }
     const int r = r0 + (tid >> 2);
     const uint8_t* mrow = m + (int64_t)min(r, T - 1) * Tp + 16 * (tid & 3);
+    __shared__ unsigned char full_in_wave[4][8];
+    const int lane = tid & 63, wv = tid >> 6;
     for (int b0 = 0; b0 < nblk; b0 += 8) {
         uint4 x[8];
 #pragma unroll
@@ -93,12 +99,15 @@ __device__ __forceinline__ void masked_tile_skip(const uint8_t* __restrict__ m, 
         for (int u = 0; u < 8; ++u) {
             // no zero byte in any of the four words <=> all 16 entries set
             auto full = [](uint32_t v) { return ((v - 0x01010101u) & ~v & 0x80808080u) == 0u; };
-            const bool set = r >= T || (full(x[u].x) && full(x[u].y) && full(x[u].z) && full(x[u].w));
-            const int all = __syncthreads_and(set ? 1 : 0);
-            if (tid == 0 && b0 + u < nblk) skip[b0 + u] = all ? 1 : 0;
+            const bool set = (r >= T) | (full(x[u].x) & full(x[u].y) & full(x[u].z) & full(x[u].w));
+            const bool all = __ballot(set) == ~0ull;
+            if (lane == u) full_in_wave[wv][u] = all ? 1 : 0;
         }
+        __syncthreads();
+        if (tid < 8 && b0 + tid < nblk)
+            skip[b0 + tid] = full_in_wave[0][tid] & full_in_wave[1][tid] & full_in_wave[2][tid] & full_in_wave[3][tid];
+        __syncthreads();
     }
-    __syncthreads();
 }
 
 // first block at or after b that is not skipped (nblk if none); uniform over the workgroup
@@ -178,31 +187,41 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
     }
     __shared__ unsigned char skip[kMaxMaskBlocks];
     masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
-    ChunkRegs<KD> rk;
-    ChunkRegs<DH> rv;
-    uint32_t mw_next[4];
-    auto prefetch = [&](int jb) {
-        const int t0 = jb * C;
-        mask_words(mw_next, attn_mask, (int64_t)tic * Tp + t0 + 4 * G);
-        chunk_g2r<KD>(rk, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
-        chunk_g2r<DH>(rv, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
-        if (prow) chunk_mask_rows<KD>(rk, prow + t0, tid);
+    struct Tile {
+        ChunkRegs<KD> k;
+        ChunkRegs<DH> v;
+        uint32_t mw[4];
     };
-    int jb = next_live_block(skip, 0, nblk);
-    if (jb < nblk) prefetch(jb);
+    auto prefetch = [&](Tile& t, int jb) __attribute__((always_inline)) {
+        const int t0 = min(jb, nblk - 1) * C;       // past the last live block: any block, never used
+        mask_words(t.mw, attn_mask, (int64_t)tic * Tp + t0 + 4 * G, kb);
+        chunk_g2r<KD>(t.k, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
+        chunk_g2r<DH>(t.v, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
+        chunk_mask_rows<KD>(t.k, prow ? prow + t0 : reinterpret_cast<const uint8_t*>(kb), tid);
+    };
+    // two blocks in flight, in two sets of registers that take turns
+    Tile ta, tb;
+    int ja = next_live_block(skip, 0, nblk), jb = next_live_block(skip, ja + 1, nblk);
+    prefetch(ta, ja);
+    prefetch(tb, jb);
 
     f4 acc[NCT];
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) acc[ct] = f4_zero();
     float rpart = 0.f;
 
-    while (jb < nblk) {
-        chunk_r2s<KD>(rk, Ks, LDQ, tid);
-        chunk_r2s<DH>(rv, Vs, LDV, tid);
-        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
+    // the block in t; t then gets the one after `other`
+    auto step = [&](Tile& t, int& j, int other) __attribute__((always_inline)) {
+        uint32_t mw4[4];
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) mw4[jt] = attn_mask ? t.mw[jt] : 0u;
+#pragma unroll
+        for (int it = 0; it < ChunkRegs<KD>::kPieces; ++it) t.k.drop[it] = prow ? t.k.drop[it] : 0;
+        chunk_r2s<KD>(t.k, Ks, LDQ, tid);
+        chunk_r2s<DH>(t.v, Vs, LDV, tid);
         __syncthreads();
-        const int jb_next = next_live_block(skip, jb + 1, nblk);
-        if (jb_next < nblk) prefetch(jb_next);
+        j = next_live_block(skip, other + 1, nblk);
+        prefetch(t, j);
         f4 at[4];   // A^T tiles (m = j, n = i)
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -223,7 +242,11 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
                 acc[ct] = mfma32(col_split8(Vs, LDV, 32 * jp, 16 * ct, lane), ba, acc[ct]);
         }
         __syncthreads();
-        jb = jb_next;
+    };
+    while (ja < nblk) {
+        step(ta, ja, jb);
+        if (jb >= nblk) break;
+        step(tb, jb, ja);
     }
 
     const float r = sum_over_groups(rpart);
@@ -310,30 +333,40 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
     }
     __shared__ unsigned char skip[kMaxMaskBlocks];
     masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
-    ChunkRegs<KD> rk;
-    ChunkRegs<DH> rv;
-    uint32_t mw_next[4];
-    auto prefetch = [&](int jb) {
-        const int t0 = jb * C;
-        mask_words(mw_next, attn_mask, (int64_t)tic * Tp + t0 + 4 * G);
-        chunk_g2r<KD>(rk, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
-        chunk_g2r<DH>(rv, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
-        if (prow) chunk_mask_rows<KD>(rk, prow + t0, tid);
+    struct Tile {
+        ChunkRegs<KD> k;
+        ChunkRegs<DH> v;
+        uint32_t mw[4];
     };
-    int jb = next_live_block(skip, 0, nblk);
-    if (jb < nblk) prefetch(jb);
+    auto prefetch = [&](Tile& t, int jb) __attribute__((always_inline)) {
+        const int t0 = min(jb, nblk - 1) * C;       // past the last live block: any block, never used
+        mask_words(t.mw, attn_mask, (int64_t)tic * Tp + t0 + 4 * G, kb);
+        chunk_g2r<KD>(t.k, kb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
+        chunk_g2r<DH>(t.v, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
+        chunk_mask_rows<KD>(t.k, prow ? prow + t0 : reinterpret_cast<const uint8_t*>(kb), tid);
+    };
+    // two blocks in flight, in two sets of registers that take turns
+    Tile ta, tb;
+    int ja = next_live_block(skip, 0, nblk), jb = next_live_block(skip, ja + 1, nblk);
+    prefetch(ta, ja);
+    prefetch(tb, jb);
 
     f4 acc[NKT];   // dQ^T tiles (m = k, n = i)
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt) acc[kt] = f4_zero();
 
-    while (jb < nblk) {
-        chunk_r2s<KD>(rk, Ks, LDQ, tid);
-        chunk_r2s<DH>(rv, Vs, LDV, tid);
-        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
+    // the block in t; t then gets the one after `other`
+    auto step = [&](Tile& t, int& j, int other) __attribute__((always_inline)) {
+        uint32_t mw4[4];
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) mw4[jt] = attn_mask ? t.mw[jt] : 0u;
+#pragma unroll
+        for (int it = 0; it < ChunkRegs<KD>::kPieces; ++it) t.k.drop[it] = prow ? t.k.drop[it] : 0;
+        chunk_r2s<KD>(t.k, Ks, LDQ, tid);
+        chunk_r2s<DH>(t.v, Vs, LDV, tid);
         __syncthreads();
-        const int jb_next = next_live_block(skip, jb + 1, nblk);
-        if (jb_next < nblk) prefetch(jb_next);
+        j = next_live_block(skip, other + 1, nblk);
+        prefetch(t, j);
         f4 pt[4];   // P^T tiles (m = j, n = i)
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -353,7 +386,11 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
                 acc[kt] = mfma32(col_split8(Ks, LDQ, 32 * jp, 16 * kt, lane), bp, acc[kt]);
         }
         __syncthreads();
-        jb = jb_next;
+    };
+    while (ja < nblk) {
+        step(ta, ja, jb);
+        if (jb >= nblk) break;
+        step(tb, jb, ja);
     }
     if (ti < T) {
         half_t* drow = dq + ((int64_t)ti * N + n) * KD;
@@ -401,20 +438,26 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 #pragma unroll
         for (int cs = 0; cs < NCS; ++cs) bv[cs] = *reinterpret_cast<const h8*>(v + tn * DH + 32 * cs + 8 * G);
     }
-    ChunkRegs<KD> rq;
-    ChunkRegs<DH> rg;
-    float gz_next;
-    uint32_t mw_next[4];
-    auto prefetch = [&](int t0) {
-        mask_words(mw_next, attn_mask_t, (int64_t)tjc * Tp + t0 + 4 * G);
-        chunk_g2r<KD>(rq, qb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
-        chunk_g2r<DH>(rg, gb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
-        gz_next = gz[(int64_t)(t0 + min(tid & (C - 1), rg.rows - 1)) * N + n];
+    struct Tile {
+        ChunkRegs<KD> q;
+        ChunkRegs<DH> g;
+        float gz;
+        uint32_t mw[4];
+    };
+    auto prefetch = [&](Tile& t, int ib) __attribute__((always_inline)) {
+        const int t0 = min(ib, nblk - 1) * C;       // past the last live block: any block, never used
+        mask_words(t.mw, attn_mask_t, (int64_t)tjc * Tp + t0 + 4 * G, qb);
+        chunk_g2r<KD>(t.q, qb + (int64_t)t0 * k_stride, k_stride, T - t0, tid);
+        chunk_g2r<DH>(t.g, gb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
+        t.gz = gz[(int64_t)(t0 + min(tid & (C - 1), t.g.rows - 1)) * N + n];
     };
     __shared__ unsigned char skip[kMaxMaskBlocks];
     masked_tile_skip(attn_mask_t, j0, T, Tp, nblk, skip, tid);
-    int ib = next_live_block(skip, 0, nblk);
-    if (ib < nblk) prefetch(ib * C);
+    // two blocks in flight, in two sets of registers that take turns
+    Tile ta, tb;
+    int ia = next_live_block(skip, 0, nblk), ib = next_live_block(skip, ia + 1, nblk);
+    prefetch(ta, ia);
+    prefetch(tb, ib);
 
     f4 acck[NKT], accv[NCT];   // dK^T (m = k, n = s), dV^T (m = c, n = s)
 #pragma unroll
@@ -422,14 +465,17 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) accv[ct] = f4_zero();
 
-    while (ib < nblk) {
-        chunk_r2s<KD>(rq, Qs, LDQ, tid);
-        chunk_r2s<DH>(rg, Gs, LDV, tid);
-        if (tid < C) gzs[tid] = tid < rg.rows ? gz_next : 0.f;
-        uint32_t mw4[4] = {mw_next[0], mw_next[1], mw_next[2], mw_next[3]};
+    // the block in t; t then gets the one after `other`
+    auto step = [&](Tile& t, int& i, int other) __attribute__((always_inline)) {
+        chunk_r2s<KD>(t.q, Qs, LDQ, tid);
+        chunk_r2s<DH>(t.g, Gs, LDV, tid);
+        if (tid < C) gzs[tid] = tid < t.g.rows ? t.gz : 0.f;
+        uint32_t mw4[4];
+#pragma unroll
+        for (int it = 0; it < 4; ++it) mw4[it] = attn_mask_t ? t.mw[it] : 0u;
         __syncthreads();
-        const int ib_next = next_live_block(skip, ib + 1, nblk);
-        if (ib_next < nblk) prefetch(ib_next * C);
+        i = next_live_block(skip, other + 1, nblk);
+        prefetch(t, i);
         f4 a_[4], p_[4];   // tiles (m = t, n = s)
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
@@ -462,7 +508,11 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
                 acck[kt] = mfma32(col_split8(Qs, LDQ, 32 * ip, 16 * kt, lane), bp, acck[kt]);
         }
         __syncthreads();
-        ib = ib_next;
+    };
+    while (ia < nblk) {
+        step(ta, ia, ib);
+        if (ib >= nblk) break;
+        step(tb, ib, ia);
     }
     if (tj < T) {
         half_t* krow = dk + ((int64_t)tj * N + n) * KD;
