@@ -244,6 +244,13 @@ int rfa_feature_map_backward_pair_packed(const void* x0, const void* x1, const v
                                          int64_t R, int H, int D, int d, float scale, void* workspace,
                                          size_t workspace_bytes, void* stream);
 
+/* The three backward entry points with dw in fp16 [H, D, d] (the fp32 sums rounded once): x1 NULL takes one
+ * tensor (workspace as rfa_feature_map_backward), packed non-NULL stands in place of dx0 and dx1. */
+int rfa_feature_map_backward_half(const void* x0, const void* x1, const void* w, const void* grad_phi0,
+                                  const void* grad_phi1, const void* third, void* dx0, void* dx1, void* packed,
+                                  void* dw, int64_t R, int H, int D, int d, float scale, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
 /* y = x W^T + b (torch.nn.Linear) for few rows, a decoding step's projections:
  *   x fp16 [R, E_in], w fp16 [E_out, E_in], bias fp16 [E_out] or NULL, y fp16 [R, E_out];
  *   fp32 sums, E_in a multiple of 32 and E_out of 16.  Right for any R, meant for R up to a few hundred. */

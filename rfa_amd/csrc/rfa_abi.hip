@@ -862,7 +862,8 @@ template <int D, int DH>
 int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::half_t* gphi, rfa::half_t* dx,
                        const rfa::half_t* x1, const rfa::half_t* gphi1, rfa::half_t* dx1,
                        float* dw, float* part, int R, int H, float scale, hipStream_t st,
-                       int64_t dx_rs = 0, const rfa::half_t* copy_src = nullptr, rfa::half_t* copy_dst = nullptr) {
+                       int64_t dx_rs = 0, const rfa::half_t* copy_src = nullptr, rfa::half_t* copy_dst = nullptr,
+                       rfa::half_t* dw16 = nullptr) {
     const int ntens = x1 ? 2 : 1;       // two tensors through the same w: one launch, one reduction
     if (dx_rs == 0) dx_rs = (int64_t)H * DH;
     int nblk;
@@ -889,14 +890,14 @@ int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::ha
         RFA_LAUNCH(COPY_ROWS, rfa::k_copy_rows_strided, dim3(blocks), dim3(rfa::kThreads), 0, st, copy_src, copy_dst, (int64_t)R,
                    H * DH, dx_rs);
     }
-    if (!dw) {                  // dx only: the kernels got no place for partial sums and formed none
+    if (!dw && !dw16) {         // dx only: the kernels got no place for partial sums and formed none
         RFA_HIP_TRY(hipGetLastError());
         return RFA_OK;
     }
     const int64_t elems = (int64_t)H * D * DH;
     static_assert((D * DH) % 256 == 0, "dw reduce works on blocks of 256 elements");
     RFA_LAUNCH(FEATURE_DW_REDUCE, rfa::k_feature_map_dw_reduce, dim3((unsigned)(elems / 256)), dim3(rfa::kThreads), 0, st,
-                       part, dw, ntens * nblk, elems);
+                       part, dw, dw16, ntens * nblk, elems);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
@@ -1901,6 +1902,46 @@ int rfa_feature_map_backward_pair_packed(const void* x0, const void* x1, const v
                                static_cast<const rfa::half_t*>(x1), static_cast<const rfa::half_t*>(grad_phi1),   \
                                pk + E, dw, part, (int)R, H, scale, st, 3 * E,                                     \
                                static_cast<const rfa::half_t*>(third), pk + 2 * E)
+    RFA_DISPATCH_FEATURE(D, d, RFA_CALL)
+#undef RFA_CALL
+    return fail(RFA_ERR_UNSUPPORTED, "unreachable");
+}
+
+// The three forms above with dW' in fp16: x1 NULL takes one tensor; packed non-NULL takes the place of dx0, dx1.
+int rfa_feature_map_backward_half(const void* x0, const void* x1, const void* w, const void* grad_phi0,
+                                  const void* grad_phi1, const void* third, void* dx0, void* dx1, void* packed, void* dw,
+                                  int64_t R, int H, int D, int d, float scale, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+    const char* fn = "rfa_feature_map_backward_half";
+    if (int rc = check_feature_dims(fn, R, H, D, d)) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!dw) return fail(RFA_ERR_NULL_POINTER, "%s: NULL dw (the other entry points form dx alone)", fn);
+    if (!aligned16(dw)) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+    const int64_t E = (int64_t)H * d;
+    if (R == 0) {
+        zero_f32(static_cast<float*>(dw), (int64_t)H * D * d / 2, st);
+        return RFA_OK;
+    }
+    auto* pk = static_cast<rfa::half_t*>(packed);
+    if (pk && !x1) return fail(RFA_ERR_NULL_POINTER, "%s: a packed gradient holds two tensors", fn);
+    if (pk) { dx0 = pk; dx1 = pk + E; }
+    if (!x0 || !w || !grad_phi0 || !dx0 || (x1 && (!grad_phi1 || !dx1)))
+        return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor pointer", fn);
+    if (!aligned16(x0) || !aligned16(x1) || !aligned16(w) || !aligned16(grad_phi0) || !aligned16(grad_phi1) || !aligned16(third) ||
+        !aligned16(dx0) || !aligned16(dx1))
+        return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+    if (R * 3 * E >= ((int64_t)1 << 40)) return fail(RFA_ERR_BAD_SHAPE, "%s: sizes exceed the supported range", fn);
+    const size_t need = x1 ? rfa_feature_map_backward_pair_workspace_bytes(R, H, D, d)
+                           : rfa_feature_map_backward_workspace_bytes(R, H, D, d);
+    if (!workspace || workspace_bytes < need || !aligned16(workspace))
+        return fail(RFA_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", fn, need, workspace ? workspace_bytes : (size_t)0);
+#define RFA_CALL(DD, DH)                                                                                          \
+    launch_feature_bwd<DD, DH>(static_cast<const rfa::half_t*>(x0), static_cast<const rfa::half_t*>(w),            \
+                               static_cast<const rfa::half_t*>(grad_phi0), static_cast<rfa::half_t*>(dx0),         \
+                               static_cast<const rfa::half_t*>(x1), static_cast<const rfa::half_t*>(grad_phi1),    \
+                               static_cast<rfa::half_t*>(dx1), nullptr, static_cast<float*>(workspace), (int)R, H, \
+                               scale, st, pk ? 3 * E : 0, pk ? static_cast<const rfa::half_t*>(third) : nullptr,   \
+                               pk ? pk + 2 * E : nullptr, static_cast<rfa::half_t*>(dw))
     RFA_DISPATCH_FEATURE(D, d, RFA_CALL)
 #undef RFA_CALL
     return fail(RFA_ERR_UNSUPPORTED, "unreachable");

@@ -85,6 +85,41 @@ bool plain_matrices(const Tensor& w, const OptTensor& sigma, double tau) {
 }
 
 // ---- feature map ------------------------------------------------------------------------
+// dx of one or two tensors through the same w, or the packed gradient [dx0 | dx1 | third] in `packed`; returns dW'
+// in fp16, undefined where w takes no gradient
+Tensor feature_grads(const Tensor& x0, const Tensor* x1, const Tensor& w, const Tensor& g0, const Tensor* g1,
+                     const Tensor* third, Tensor& dx0, Tensor* dx1, bool packed, double scale, bool need_dw) {
+    if (!need_dw) {
+        if (packed) dx0 = std::get<0>(feature_map_backward_pair_packed(x0, *x1, w, g0, *g1, opt(*third), scale, false));
+        else if (x1) std::tie(dx0, *dx1, std::ignore) = feature_map_backward_pair(x0, *x1, w, g0, *g1, scale, false);
+        else dx0 = std::get<0>(feature_map_backward(x0, w, g0, scale, false));
+        return Tensor();
+    }
+    const int64_t R = x0.size(0) * x0.size(1);
+    const int H = (int)x0.size(2), d = (int)x0.size(3), D = (int)w.size(1);
+    auto check = [&](const Tensor& x, const Tensor& g) {
+        check_feature_args(x, w);
+        check_half("grad_phi", g, 4);
+        TORCH_CHECK_VALUE(x.sizes() == x0.sizes() && g.size(0) == x0.size(0) && g.size(1) == x0.size(1) && g.size(2) == H &&
+                              g.size(3) == 2 * D, "grad_phi ", g.sizes(), " does not fit x ", x0.sizes(), " and ", D, " features");
+    };
+    check(x0, g0);
+    if (x1) check(*x1, *g1);
+    if (third) TORCH_CHECK_VALUE(third->numel() == x0.numel() && third->is_contiguous(), "third must hold the rows of x");
+    dx0 = packed ? torch::empty({R, 3 * (int64_t)H * d}, x0.options()) : torch::empty_like(x0);
+    if (x1 && !packed) *dx1 = torch::empty_like(*x1);
+    Tensor dw = torch::empty({H, D, d}, x0.options());
+    Launch l(x0);
+    const size_t nbytes = x1 ? rfa_feature_map_backward_pair_workspace_bytes(R, H, D, d)
+                             : rfa_feature_map_backward_workspace_bytes(R, H, D, d);
+    Tensor ws = workspace(nbytes, x0);
+    check_rc(rfa_feature_map_backward_half(ptr(x0), x1 ? ptr(*x1) : nullptr, ptr(w), ptr(g0), g1 ? ptr(*g1) : nullptr,
+                                           third ? ptr(*third) : nullptr, packed ? nullptr : ptr(dx0),
+                                           x1 && !packed ? ptr(*dx1) : nullptr, packed ? ptr(dx0) : nullptr, ptr(dw), R, H, D,
+                                           d, (float)scale, ptr(ws), nbytes, l.stream));
+    return dw;
+}
+
 struct FeatureNode : public torch::autograd::Function<FeatureNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double scale) {
         const Tensor xc = x.contiguous(), wc = w.contiguous();
@@ -95,9 +130,10 @@ struct FeatureNode : public torch::autograd::Function<FeatureNode> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        auto [dx, dw] = feature_map_backward(saved[0], saved[1], g[0].contiguous(), ctx->saved_data["scale"].toDouble(),
-                                             ctx->saved_data["need_w"].toBool());
-        return {dx, dw.has_value() ? dw->to(torch::kFloat16) : Tensor(), Tensor()};
+        Tensor dx;
+        const Tensor dw = feature_grads(saved[0], nullptr, saved[1], g[0].contiguous(), nullptr, nullptr, dx, nullptr, false,
+                                        ctx->saved_data["scale"].toDouble(), ctx->saved_data["need_w"].toBool());
+        return {dx, dw, Tensor()};
     }
 };
 
@@ -108,7 +144,8 @@ OptTensor node_random_project(const Tensor& x, const Tensor& w, double scale) {
 }
 
 // ---- projections to heads, with the feature map where a bit of `phi` is set ----------------------
-// The weights and biases of up to three Linear layers over one input; unused places are empty.
+// The weights and biases of up to three Linear layers over one input; the first, or the first two, through the
+// feature map.
 struct Layers {
     std::vector<Tensor> w;
     std::vector<OptTensor> b;
@@ -208,14 +245,14 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
         variable_list out(11);                    // x, wf, scale, heads, phi, w0, b0, w1, b1, w2, b2
         std::vector<bool> bias;
         for (int64_t p = 0; p < n; ++p) bias.push_back((bias_bits >> p) & 1);
-        OptTensor dwf;
+        Tensor dwf;
         if (n == 3 && phi == 3 && need_x) {
             // [dy_q | dy_k | dv] side by side, written by the feature-map backward launch itself: one
             // GEMM for dx and one contraction for the three weight gradients
             const int64_t e_out = w[0].size(0);
             Tensor packed;
-            std::tie(packed, dwf) = feature_map_backward_pair_packed(y[0], y[1], wf, g[0].contiguous(), g[1].contiguous(),
-                                                                     g[2].contiguous(), scale, need_wf);
+            const Tensor g0 = g[0].contiguous(), g1 = g[1].contiguous(), g2 = g[2].contiguous();
+            dwf = feature_grads(y[0], &y[1], wf, g0, &g1, &g2, packed, nullptr, true, scale, need_wf);
             const char* base = static_cast<const char*>(packed.data_ptr());
             out[0] = own_input_grad(rows, w, 3)
                          ? input_grad({base, base + 2 * e_out, base + 4 * e_out}, 3 * e_out, w, x)
@@ -227,19 +264,16 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             }
         } else {
             std::vector<Tensor> dys(n);
-            if (n >= 2 && (phi & (phi - 1)) != 0 && phi != 7) {          // two of them: one launch
-                const int p0 = (phi & 1) ? 0 : 1, p1 = (phi & 4) ? 2 : 1;
-                std::tie(dys[p0], dys[p1], dwf) = feature_map_backward_pair(y[0], y[1], wf, g[p0].contiguous(),
-                                                                            g[p1].contiguous(), scale, need_wf);
+            if (phi == 3) {              // two of them: one launch
+                const Tensor g0 = g[0].contiguous(), g1 = g[1].contiguous();
+                dwf = feature_grads(y[0], &y[1], wf, g0, &g1, nullptr, dys[0], &dys[1], false, scale, need_wf);
             }
-            int64_t yi = 0;
             for (int64_t p = 0; p < n; ++p) {
                 if (!dys[p].defined()) {
                     dys[p] = g[p].contiguous();
-                    if ((phi >> p) & 1) {
-                        OptTensor dw;
-                        std::tie(dys[p], dw) = feature_map_backward(y[yi++], wf, dys[p], scale, need_wf);
-                        if (dw.has_value()) dwf = dwf.has_value() ? *dwf + *dw : *dw;
+                    if ((phi >> p) & 1) {        // the only one
+                        const Tensor gp = dys[p];
+                        dwf = feature_grads(y[0], nullptr, wf, gp, nullptr, nullptr, dys[p], nullptr, false, scale, need_wf);
                     }
                 }
                 dys[p] = dys[p].reshape({rows, -1});
@@ -261,7 +295,7 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             }
             if (out[0].defined()) out[0] = out[0].view(x.sizes());
         }
-        if (dwf.has_value()) out[1] = dwf->to(torch::kFloat16);
+        out[1] = dwf;
         return out;
     }
 };
