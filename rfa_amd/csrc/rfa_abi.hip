@@ -666,6 +666,10 @@ int launch_cross_state_bwd(const rfa::half_t* k, const rfa::half_t* v, const uin
 
 
 // ---- quadratic form with explicit masks ---------------------------------------------------
+// Row blocks in pairs (rfa_masked.h): above three blocks per CU, and where one block alone may be a chain of
+// more than 32 tiles (T 4096, 8 sequences, 64 blocks each: 97 us forward in pairs, 104 singly; 16 each 51 / 42).
+bool masked_paired(int N, int nblk) { return (int64_t)N * nblk > 3 * (int64_t)device_cus() || nblk > 32; }
+
 template <int KD, int DH>
 int launch_masked_fwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t* v, const uint8_t* pad,
                       const uint8_t* amask, rfa::half_t* out, float* rsum, int T, int Tp, int N, int H,
@@ -674,7 +678,8 @@ int launch_masked_fwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::hal
     auto kern = rfa::k_masked_fwd<KD, DH>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     const int nblk = (T + rfa::kChunk - 1) / rfa::kChunk;
-    RFA_LAUNCH(MASKED_FWD, kern, dim3(N * (amask ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, pad, amask, out, rsum, T, Tp, N, H);
+    const int paired = amask && masked_paired(N, nblk) ? 1 : 0;
+    RFA_LAUNCH(MASKED_FWD, kern, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, pad, amask, out, rsum, T, Tp, N, H, paired);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
@@ -686,18 +691,19 @@ int launch_masked_bwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::hal
                       rfa::half_t* ghat, float* gz, int T, int Tp, int N, int H, hipStream_t st) {
     using Cfg = rfa::MaskedCfg<KD, DH>;
     const int nblk = (T + rfa::kChunk - 1) / rfa::kChunk;
+    const int paired = amask && masked_paired(N, nblk) ? 1 : 0;
     const int64_t rows = (int64_t)T * N;
     const int64_t pieces = rows * (DH / 8);
     RFA_LAUNCH(MASKED_PREP, rfa::k_masked_bwd_prep<DH>, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, g, out,
                rsum, ghat, gz, rows);
     auto kq = rfa::k_masked_dq<KD, DH>;
     if (int rc = set_lds(kq, Cfg::kLds)) return rc;
-    RFA_LAUNCH(MASKED_DQ, kq, dim3(N * (amask ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, (const rfa::half_t*)ghat, (const float*)gz, k,
-               v, pad, amask, dq, T, Tp, N, H);
+    RFA_LAUNCH(MASKED_DQ, kq, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, (const rfa::half_t*)ghat, (const float*)gz, k,
+               v, pad, amask, dq, T, Tp, N, H, paired);
     auto kk = rfa::k_masked_dkdv<KD, DH>;
     if (int rc = set_lds(kk, Cfg::kLds)) return rc;
-    RFA_LAUNCH(MASKED_DKDV, kk, dim3(N * (amask_t ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, (const rfa::half_t*)ghat,
-               (const float*)gz, pad, amask_t, dk, dv, T, Tp, N, H);
+    RFA_LAUNCH(MASKED_DKDV, kk, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, (const rfa::half_t*)ghat,
+               (const float*)gz, pad, amask_t, dk, dv, T, Tp, N, H, paired);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }

@@ -525,31 +525,46 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 }
 
 // ---------------------------------------------------------------------------
-// Kernels.  With an attention mask, grid = N * ceil(nblk / 2): a workgroup takes row blocks p and
-// nblk - 1 - p of one sequence, one after the other.  With a causal mask block p has p + 1 live
-// column blocks, so every workgroup does the same work (nblk + 1 tiles); without that pairing the
-// last row blocks set the kernel time and skipping the masked tiles would not shorten it.
-// The workgroups of a sequence run on one XCD, whose L2 then serves its rows to all but the first.
-// Without a mask nothing is skipped and grid = N * nblk, one row block per workgroup.
+// Kernels.  A workgroup takes one row block of a sequence (grid = N * nblk), or two (`paired`, grid = N * ceil(nblk /
+// 2)).  With a causal mask block p has p + 1 live column blocks; a pair p, nblk - 1 - p is the same work for every
+// workgroup, where single blocks leave the CUs to the last long ones.  But while the single blocks are few enough
+// to be on the chip at once (26 KB of LDS each at K = 128), several to a CU, they hide each other's round trips:
+// the launcher pairs above three per CU.  Measured, single / paired, causal, fwd and bwd us: T 512, 64 sequences
+// (512 blocks) 18.5 / 21.5, 49 / 54; T 300, 128 (640) 19.0 / 21.1, 52 / 58; T 1024, 16, K 256, d 128 (256)
+// 41.6 / 50.7, 127 / 146; T 1024, 64 (1024) 58.4 / 49.3, 151 / 120.  Before the two register sets and the shared
+// barrier of the flags, paired: 27.0, 69.1; 24.2, 64.9; 58.8, 161; 59.8, 145.
+// The workgroups of a sequence run on one XCD, whose L2 then serves its rows to all but the first; single blocks
+// of the sequences of every second round of workgroups over an XCD's 32 CUs are dealt in reverse, so that a CU
+// gets long and short ones.
 // ---------------------------------------------------------------------------
-#define RFA_MASKED_PAIR(CALL, PAIRED)                                          \
-    const int nblk = (T + kChunk - 1) / kChunk;                                \
-    const int per_seq = (PAIRED) ? (nblk + 1) / 2 : nblk;                      \
-    int n, p;                                                                  \
-    seq_seg_of_block(blockIdx.x, N, per_seq, n, p);                            \
-    CALL(p * kChunk);                                                          \
-    if ((PAIRED) && nblk - 1 - p != p) {                                       \
-        __syncthreads();                                                       \
-        CALL((nblk - 1 - p) * kChunk);                                         \
+struct MaskedBlocks {
+    int n, first, second;      // sequence, row blocks (second < 0: one only)
+    __device__ __forceinline__ MaskedBlocks(int b, int N, int T, bool paired) {
+        const int nblk = (T + kChunk - 1) / kChunk;
+        int p;
+        seq_seg_of_block(b, N, paired ? (nblk + 1) / 2 : nblk, n, p);
+        const bool reverse = !paired && ((((n >> 3) * nblk) >> 5) & 1) != 0;      // the same for all blocks of a sequence
+        first = reverse ? nblk - 1 - p : p;
+        second = paired && nblk - 1 - p != p ? nblk - 1 - p : -1;
+    }
+};
+
+// CALL for each of the workgroup's row blocks
+#define RFA_MASKED_BLOCKS(CALL)                                       \
+    const MaskedBlocks mb(blockIdx.x, N, T, paired != 0);             \
+    for (int p = mb.first;; p = mb.second) {                          \
+        CALL(mb.n, p * kChunk);                                       \
+        if (p == mb.second || mb.second < 0) break;                   \
+        __syncthreads();                                              \
     }
 
 template <int KD, int DH>
 __global__ __launch_bounds__(256) void k_masked_fwd(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     const uint8_t* __restrict__ pad_mask, const uint8_t* __restrict__ attn_mask, half_t* __restrict__ out,
-    float* __restrict__ rsum, int T, int Tp, int N, int H) {
-#define RFA_CALL_BLOCK(R0) masked_fwd_block<KD, DH>(n, R0, q, k, v, pad_mask, attn_mask, out, rsum, T, Tp, N, H)
-    RFA_MASKED_PAIR(RFA_CALL_BLOCK, attn_mask != nullptr)
+    float* __restrict__ rsum, int T, int Tp, int N, int H, int paired) {
+#define RFA_CALL_BLOCK(n, row0) masked_fwd_block<KD, DH>(n, row0, q, k, v, pad_mask, attn_mask, out, rsum, T, Tp, N, H)
+    RFA_MASKED_BLOCKS(RFA_CALL_BLOCK)
 #undef RFA_CALL_BLOCK
 }
 
@@ -557,9 +572,9 @@ template <int KD, int DH>
 __global__ __launch_bounds__(256) void k_masked_dq(
     const half_t* __restrict__ ghat, const float* __restrict__ gz, const half_t* __restrict__ k,
     const half_t* __restrict__ v, const uint8_t* __restrict__ pad_mask, const uint8_t* __restrict__ attn_mask,
-    half_t* __restrict__ dq, int T, int Tp, int N, int H) {
-#define RFA_CALL_BLOCK(R0) masked_dq_block<KD, DH>(n, R0, ghat, gz, k, v, pad_mask, attn_mask, dq, T, Tp, N, H)
-    RFA_MASKED_PAIR(RFA_CALL_BLOCK, attn_mask != nullptr)
+    half_t* __restrict__ dq, int T, int Tp, int N, int H, int paired) {
+#define RFA_CALL_BLOCK(n, row0) masked_dq_block<KD, DH>(n, row0, ghat, gz, k, v, pad_mask, attn_mask, dq, T, Tp, N, H)
+    RFA_MASKED_BLOCKS(RFA_CALL_BLOCK)
 #undef RFA_CALL_BLOCK
 }
 
@@ -568,11 +583,12 @@ __global__ __launch_bounds__(256) void k_masked_dkdv(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     const half_t* __restrict__ ghat, const float* __restrict__ gz, const uint8_t* __restrict__ pad_mask,
     const uint8_t* __restrict__ attn_mask_t, half_t* __restrict__ dk, half_t* __restrict__ dv, int T, int Tp,
-    int N, int H) {
-#define RFA_CALL_BLOCK(R0) masked_dkdv_block<KD, DH>(n, R0, q, k, v, ghat, gz, pad_mask, attn_mask_t, dk, dv, T, Tp, N, H)
-    RFA_MASKED_PAIR(RFA_CALL_BLOCK, attn_mask_t != nullptr)
+    int N, int H, int paired) {
+#define RFA_CALL_BLOCK(n, row0) masked_dkdv_block<KD, DH>(n, row0, q, k, v, ghat, gz, pad_mask, attn_mask_t, dk, dv, T, Tp, N, H)
+    RFA_MASKED_BLOCKS(RFA_CALL_BLOCK)
 #undef RFA_CALL_BLOCK
 }
-#undef RFA_MASKED_PAIR
+
+#undef RFA_MASKED_BLOCKS
 
 }  // namespace rfa

@@ -591,3 +591,30 @@ def test_prefill_from_projected_rows(T, d, D):
         print(f"  {err:.2e}", flush=True)
         assert torch.isfinite(got).all() and err <= 2.0 ** -11
     assert rfa_hip.native.node_prefill(q[:, :1], k[:, :1], v[:, :1], W, O.SCALE) is None      # not contiguous
+
+
+@pytest.mark.parametrize("T", [64, 65, 130, 300])
+@pytest.mark.parametrize("with_mask", [True, False])
+def test_masked_rfa_blocks_dealt_singly_and_in_pairs(T, with_mask):
+    """Many sequences (row blocks dealt in pairs under a mask) give the bits of the same sequences a few
+    at a time (dealt singly, every second round in reverse): the order of a row's sums does not depend on it."""
+    from rfa_amd import rfa_hip
+    H, d, D = 4, 64, 32
+    B = -(-1000 // (H * -(-T // 64)))
+    gen = torch.Generator("cuda").manual_seed(T)
+    q, k = (torch.rand(T, B * H, 2 * D, generator=gen, device="cuda").half() for _ in range(2))
+    v, g = (torch.randn(T, B * H, d, generator=gen, device="cuda").half() for _ in range(2))
+    m = mt = None
+    if with_mask:
+        m, mt = rfa_hip.pack_attn_mask(torch.ones(T, T, dtype=torch.bool, device="cuda").triu(1))
+    print(f"masked blocks T={T} N={B * H} mask={with_mask}", flush=True)
+
+    def run(b0, b1):
+        cut = lambda t: t[:, b0 * H:b1 * H].contiguous()
+        out, rsum = rfa_hip.masked_forward(cut(q), cut(k), cut(v), H, None, m)
+        return [out, rsum, *rfa_hip.masked_backward(cut(q), cut(k), cut(v), cut(g), out, rsum, H, None, m, mt)]
+
+    whole = run(0, B)
+    for b0 in (0, B // 2, B - 17):
+        for a, b in zip(whole, run(b0, b0 + 17)):
+            assert torch.isfinite(b).all() and torch.equal(a[:, b0 * H:(b0 + 17) * H], b)
