@@ -20,7 +20,7 @@ from torch.nn import Parameter
 
 from . import rfa_hip
 from ._derived import derived
-from .projection import fused_projection_supported, linear_out, linear_rows, project_heads
+from .projection import fused_projection_supported, linear_no_grad, linear_out, linear_rows, project_heads
 from .rfa import RFA
 from .utils import (EPS, SCALE, build_random_matrices, random_project, random_project_pair,
                     upgrade_state_dict_named)
@@ -302,9 +302,7 @@ class CausalAttention(nn.Module):
                 attn = masked_rfa(phi_q=phi_q, phi_k=phi_k, v=v, attn_mask=attn_mask,
                                   key_padding_mask=key_padding_mask)
             return linear_out(attn, self.out_proj)
-        q = self._heads(self.q_proj(x), tgt_len, bsz)
-        k = self._heads(self.k_proj(x), tgt_len, bsz)
-        v = self._heads(self.v_proj(x), tgt_len, bsz)
+        q, k, v = (self._heads(linear_no_grad(x, layer), tgt_len, bsz) for layer in qkv)
         if saved_state is not None:
             feat = 2 * self.proj_dim
             s, z = saved_state.get("prev_s"), saved_state.get("prev_z")

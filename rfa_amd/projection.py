@@ -186,8 +186,8 @@ class _LinearOut(torch.autograd.Function):
 
 
 def linear_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor]) -> Optional[Tensor]:
-    """x W^T + b without autograd by the row kernel, None where it does not apply (many rows, odd widths, other
-    types): a library product of a decoding step's size costs 20 us of host time, four times the launch."""
+    """x W^T + b without autograd by the row kernel or the projection kernel, None where neither applies (the
+    largest products, odd widths, other types): a library product costs 19 us of host time, four times the launch."""
     return None if rfa_hip.native is None else rfa_hip.native.node_linear_rows(x, weight, bias)
 
 
@@ -201,13 +201,18 @@ def _is_bare_linear(layer: nn.Module) -> bool:
             and "forward" not in layer.__dict__ and not any(_GLOBAL_HOOKS))
 
 
+def linear_no_grad(x: Tensor, layer: nn.Linear) -> Tensor:
+    """``layer(x)``, without autograd by the framework's own kernels where they apply."""
+    y = linear_rows(x, layer.weight, layer.bias) if not torch.is_grad_enabled() and _is_bare_linear(layer) else None
+    return layer(x) if y is None else y
+
+
 def linear_out(x: Tensor, layer: nn.Linear) -> Tensor:
     """``layer(x)`` (the modules' out_proj, causal_attention.py:278, cross_attention.py:298); fp16 HIP
     tensors with widths that are multiples of 128 take the row-split gradient kernel in backward."""
     w = layer.weight
     if not torch.is_grad_enabled():
-        y = linear_rows(x, w, layer.bias) if _is_bare_linear(layer) else None
-        return layer(x) if y is None else y
+        return linear_no_grad(x, layer)
     if (x.is_cuda and x.dtype == torch.float16 and w.dtype == torch.float16
             and (w.requires_grad or x.requires_grad) and rfa_hip.linear_weight_grad_supported(*w.shape)
             and (layer.bias is None or layer.bias.dtype == torch.float16)):

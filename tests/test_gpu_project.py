@@ -470,9 +470,10 @@ def test_empty_input():
 
 
 @pytest.mark.parametrize("e_in,e_out", [(32, 16), (96, 48), (512, 1536), (992, 272), (1024, 3072)])
-@pytest.mark.parametrize("R", [1, 15, 16, 17, 32, 33, 64, 65, 97, 130])
+@pytest.mark.parametrize("R", [1, 15, 16, 17, 32, 33, 64, 65, 97, 130, 700, 3000])
 def test_linear_rows(R, e_in, e_out):
-    """The few-rows product against fp64 at the edges of its row tiles, column tiles and wave splits: fp32
+    """The products without autograd against fp64, few rows at the edges of the row tiles, column tiles and wave
+    splits of their kernel, more by the projection kernel: fp32
     sums of exact products, one rounding to fp16 (2^-11 of the value; sums of 1024 terms below 2^-16)."""
     from rfa_amd import projection, rfa_hip
     if rfa_hip.native is None:
@@ -487,8 +488,8 @@ def test_linear_rows(R, e_in, e_out):
         for bias in (b, None):
             y = projection.linear_rows(x, w, bias)
             ref = want if bias is None else want + b.double()
-            if R * e_in * e_out > 300 << 20:
-                assert y is None
+            if R * e_in * e_out > 1 << 31 or ((R > 256 or R * e_in * e_out > 300 << 20) and (e_in % 64 or e_out % 64)):
+                assert y is None        # the library's
                 continue
             assert ((y.double() - ref).abs() <= 2.0 ** -10 * ref.abs() + 2e-5).all()
         # what the kernel does not read as it is goes to the library
