@@ -48,6 +48,13 @@ bool wants_grad(const T&... t) {
 bool wants_grad_opt(const OptTensor& t) { return t.has_value() && t->requires_grad(); }
 
 bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+// A saved tensor comes back through the hooks that the program may have set.  Other strides are theirs to choose, and
+// a hook may get type or device wrong: all three are looked at again before a pointer is used.
+void check_saved(const char* name, const Tensor& t, const Tensor& like) {
+    TORCH_CHECK(t.is_cuda() && t.device() == like.device(), name, " must be on ", like.device(), " (got ", t.device(), ")");
+    TORCH_CHECK_TYPE(t.scalar_type() == torch::kFloat16, name, " must be float16 (got ", t.scalar_type(), ")");
+}
+
 Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : c10::nullopt; }
 
@@ -240,6 +247,10 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
         const Tensor &x = saved[0], &wf = saved[1];
         const Tensor* const w = &saved[2];
         const Tensor* const y = &saved[2 + n];
+        check_saved("x", x, g[0]);
+        for (int64_t p = 0; p < n; ++p) check_saved("weight", w[p], g[0]);
+        for (int64_t p = 0, i = 0; p < n; ++p)
+            if ((phi >> p) & 1) check_saved("y", y[i++], g[0]);
         const int64_t rows = x.size(0) * x.size(1);
         const Tensor x2 = x.reshape({rows, x.size(2)});
         variable_list out(11);                    // x, wf, scale, heads, phi, w0, b0, w1, b1, w2, b2
@@ -365,6 +376,8 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &w = saved[1];
+        check_saved("x", x, g[0]);
+        check_saved("weight", w, g[0]);
         const Tensor dy2 = g[0].reshape({-1, g[0].size(-1)}), x2 = x.reshape({-1, x.size(-1)});
         Tensor dx;
         if (ctx->saved_data["need_x"].toBool()) {
@@ -468,16 +481,29 @@ struct CausalNode : public torch::autograd::Function<CausalNode> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &state = saved[4];
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &state = saved[4], &pad = saved[5];
         const Tensor attn = saved[3].contiguous(), grad = g[0].contiguous();
+        check_half("q", q, 4);
+        check_half("k", k, 4);
+        check_half("v", v, 4);
+        check_half("out", attn, 3);
+        for (const Tensor* t : {&k, &v, &attn, &grad}) check_saved("a saved tensor", *t, q);
         const ScanDims n(q, v);
+        TORCH_CHECK_VALUE(k.sizes() == q.sizes() && v.size(0) == n.T && v.size(1) == q.size(1) && v.size(2) == q.size(2) &&
+                              attn.numel() == v.numel() && grad.numel() == v.numel(),
+                          "saved q ", q.sizes(), ", k ", k.sizes(), ", v ", v.sizes(), ", out ", attn.sizes(), " do not fit");
+        TORCH_CHECK_TYPE(state.is_cuda() && state.device() == q.device() && state.scalar_type() == torch::kUInt8 &&
+                             state.is_contiguous(), "saved must be the byte buffer of the forward");
+        if (pad.defined())
+            TORCH_CHECK_VALUE(pad.device() == q.device() && pad.scalar_type() == torch::kBool && pad.dim() == 2 &&
+                                  pad.size(0) == q.size(1) && pad.size(1) == n.T, "saved key_padding_mask does not fit");
         Tensor dq = torch::empty_like(q), dk = torch::empty_like(k), dv = torch::empty_like(v);
         Launch l(q);
         const size_t nbytes = rfa_causal_backward_saved_workspace_bytes(ptr(state), n.T, n.N, n.K, n.d);
         Tensor ws = workspace(nbytes, q);
         check_rc(rfa_causal_backward_saved(ptr(q), ptr(k), ptr(v), ptr(grad), ptr(attn), ptr(state), (size_t)state.numel(),
                                            ptr(dq), ptr(dk), ptr(dv), n.T, n.N, n.K, n.d, ptr(ws), nbytes, l.stream));
-        if (saved[5].defined()) mask_rows(dk, dk, saved[5]);
+        if (pad.defined()) mask_rows(dk, dk, pad);
         return {dq, dk, dv, Tensor()};
     }
 };

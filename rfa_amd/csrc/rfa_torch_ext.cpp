@@ -176,6 +176,11 @@ std::tuple<c10::optional<Tensor>, c10::optional<Tensor>> build_random_matrices_b
     check_half("grad_out", grad_out, 3);
     TORCH_CHECK_VALUE(grad_out.sizes() == w.sizes(), "grad_out must have the shape of random_matrices");
     const int H = (int)w.size(0), D = (int)w.size(1), d = (int)w.size(2);
+    if (sigma.has_value()) {
+        check_half("sigma", *sigma, 3);
+        TORCH_CHECK_VALUE(sigma->size(0) == H && sigma->size(1) == 1 && sigma->size(2) == d && sigma->device() == w.device(),
+                          "sigma must be [", H, ", 1, ", d, "] on the matrices' device (got ", sigma->sizes(), ")");
+    }
     want_dsigma = want_dsigma && sigma.has_value();
     c10::optional<Tensor> dsigma, dw;
     if (want_dsigma) dsigma = torch::empty({H, 1, d}, w.options());

@@ -537,6 +537,46 @@ def test_native_nodes_give_the_bits_of_the_python_functions(path, form, monkeypa
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("path", ["random_project", "causal", "padded", "masked", "module", "cross"])
+def test_native_nodes_check_what_saved_tensor_hooks_return(path):
+    """Each saved tensor in turn comes back with other strides (same values: what a hook may do), another type or
+    another device.  The backward pass gives the gradients of the run without hooks (in the layers within the
+    roundings of another product kernel) or raises; for another type or device it raises."""
+    from rfa_amd import rfa_hip
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    run, leaves = _native_forms(path, "plain")
+
+    def gradients(change=None, which=-1):
+        count = [0]
+
+        def pack(t):
+            count[0] += 1
+            return t if count[0] - 1 != which else change(t)
+        for t in leaves:
+            t.grad = None
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+            out = run()
+        out.backward(torch.randn(out.shape, generator=torch.Generator("cuda").manual_seed(9), device="cuda").half())
+        return [t.grad.clone() for t in leaves], count[0]
+
+    want, saved = gradients()
+    refused = {"strides": 0, "type": 0, "device": 0}
+    for which in range(saved):
+        for name, change in (("strides", lambda t: t.transpose(0, 1).contiguous().transpose(0, 1) if t.dim() > 1 else t),
+                             ("type", lambda t: t.double()), ("device", lambda t: t.cpu())):
+            print(f"saved tensor {which} of {path}: other {name}", flush=True)
+            try:
+                got, _ = gradients(change, which)
+            except (RuntimeError, ValueError, TypeError):
+                refused[name] += 1
+                continue
+            assert name == "strides"
+            for a, b in zip(got, want):
+                assert _rel(a.double().cpu(), b.double().cpu()) <= (4 * 2.0 ** -11 if path in ("module", "cross") else 0)
+    assert refused["type"] == refused["device"] == saved
+
+
 def test_native_nodes_leave_odd_calls_to_the_python_functions():
     """Dispatch modes and tracing see the Python functions, and functorch transforms and forward-mode
     tangents meet the errors that those raise."""
