@@ -111,7 +111,7 @@ def masked_rfa(*, phi_q: Tensor, phi_k: Tensor, v: Tensor, key_padding_mask: Opt
     if attn_mask is not None:
         assert attn_mask.size(0) == tgt_len and attn_mask.size(1) == tgt_len
         if (attn_mask.is_cuda and attn_mask.device == phi_q.device and attn_mask.dim() == 2
-                and attn_mask.dtype in rfa_hip.MASK_DTYPES):
+                and attn_mask.dtype in rfa_hip.MASK_DTYPES and rfa_hip.plain_call(attn_mask)):
             mask_bytes, mask_t_bytes = rfa_hip.pack_negative_mask(attn_mask.detach().resolve_neg())
         else:
             mask_bytes, mask_t_bytes = rfa_hip.pack_attn_mask((attn_mask < 0.0).to(phi_q.device))

@@ -38,6 +38,8 @@ bool plain(const Tensor& t, torch::ScalarType type, int64_t dim) {
            !t.key_set().has_any(odd) && !t._fw_grad(0).defined();
 }
 
+bool node_plain(const Tensor& t) { return plain_mode() && plain(t, t.scalar_type(), t.dim()); }
+
 bool plain_half(const Tensor& t, int64_t dim) { return plain(t, torch::kFloat16, dim); }
 bool plain_half(const OptTensor& t, int64_t dim) { return !t.has_value() || plain(*t, torch::kFloat16, dim); }
 
@@ -676,7 +678,8 @@ OptTensor node_cross_query(const Tensor& query, const Tensor& w, const Tensor& w
 
 void bind_nodes(pybind11::module_& m) {
     namespace py = pybind11;
-    // each returns None where the call is not plain: the caller's general path takes it
+    m.def("node_plain", &node_plain, py::arg("t"));
+    // each of the others returns None where the call is not plain: the caller's general path takes it
     m.def("node_random_project", &node_random_project, py::arg("x"), py::arg("w"), py::arg("scale"));
     m.def("node_linear", &node_linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("node_linear_rows", &node_linear_rows, py::arg("x"), py::arg("weight"), py::arg("bias"));

@@ -20,6 +20,7 @@ from typing import List, Optional
 
 import torch
 from torch import Tensor
+from torch.utils import _python_dispatch
 
 from . import _lib
 
@@ -635,6 +636,15 @@ _MASK_TYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 MASK_DTYPES = tuple(_MASK_TYPES)        # what pack_negative_mask reads as it is
 
 
+def plain_call(t: Tensor) -> bool:
+    """Whether a launch on t's memory may stand where tensor operations on t would: not while they are traced,
+    seen by a dispatch mode or a functorch transform, and not for subclasses and wrappers."""
+    if native is not None:
+        return native.node_plain(t)
+    return (type(t) in (Tensor, torch.nn.Parameter) and not torch.jit.is_tracing()
+            and _python_dispatch._get_current_dispatch_mode() is None)
+
+
 def pack_negative_mask(mask: Tensor):
     """``pack_attn_mask(mask < 0)`` in one launch, for an fp32, fp16 or bf16 mask [T, T] of any strides on
     a HIP device."""
@@ -714,7 +724,7 @@ _BOUND = ("supported", "feature_map_supported", "selftest_layout", "forward", "b
           "incremental_qkv",
           "pack_negative_mask", "masked_forward", "masked_backward")
 # autograd functions and chains of them as C++ nodes (csrc/rfa_autograd.h): only the binding has them
-_NODES = ("node_random_project", "node_linear", "node_linear_rows", "node_causal", "node_prefill", "node_causal_layer", "node_masked", "node_cross_source",
+_NODES = ("node_plain", "node_random_project", "node_linear", "node_linear_rows", "node_causal", "node_prefill", "node_causal_layer", "node_masked", "node_cross_source",
           "node_cross_query")
 _CTYPES_IMPL = {name: globals()[name] for name in _BOUND}
 _active = "ctypes"

@@ -436,6 +436,21 @@ def test_pack_negative_mask_matches_the_general_packing(T, dtype):
             rfa_hip.pack_negative_mask(base[:3, :3].to(torch.int32))
 
 
+@pytest.mark.usefixtures("binding")
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_traced_masked_rfa_follows_its_mask(dtype):
+    """A traced call packs the mask that it is given, not the one that it was traced with."""
+    from rfa_amd.causal_attention import masked_rfa
+    T, B, H, d = 70, 2, 2, 64
+    q, k = (0.2 * torch.rand(T, B, H, 64, device="cuda").half() for _ in range(2))
+    v = torch.randn(T, B, H, d, device="cuda").half()
+    masks = [torch.full((T, T), float("-inf"), device="cuda", dtype=dtype).triu(n) for n in (1, 9)]
+    call = lambda q, k, v, m: masked_rfa(phi_q=q, phi_k=k, v=v, attn_mask=m)
+    traced = torch.jit.trace(call, (q, k, v, masks[0]), check_trace=False)
+    for m in masks:
+        assert torch.equal(traced(q, k, v, m), call(q, k, v, m))
+
+
 def _native_forms(path, form):
     """(run, leaves) of one path in one form of its inputs; run() -> outputs whose sum of products is differentiated."""
     from rfa_amd import causal_attention as C, cross_attention as X, utils
