@@ -191,9 +191,11 @@ bool own_product(int64_t rows, int64_t e_out, int64_t e_in, int64_t n) {
     return rows > 0 && rows * e_out * e_in * n <= (n == 2 ? (int64_t)1 << 34 : (int64_t)7 << 30);
 }
 
-// dx = sum_p dy_p W_p for dy_p [rows, E_out] that lie ld halves a row from dys[p] on
+// dx = sum_p dy_p W_p for dy_p [rows, E_out] that lie ld halves a row from dys[p] on.  Not where the backward pass
+// itself is recorded (create_graph): the library's products are differentiable, a launch is not.
 bool own_input_grad(int64_t rows, const Tensor* w, int64_t n) {
-    bool ok = own_product(rows, w[0].size(0), w[0].size(1), n) && w[0].size(0) % 32 == 0 && w[0].size(1) % 128 == 0;
+    bool ok = !at::GradMode::is_enabled() && own_product(rows, w[0].size(0), w[0].size(1), n) && w[0].size(0) % 32 == 0 &&
+              w[0].size(1) % 128 == 0;
     for (int64_t p = 0; p < n; ++p) ok = ok && w[p].is_contiguous() && aligned16(w[p]);
     return ok;
 }

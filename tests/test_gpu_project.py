@@ -31,6 +31,10 @@ def _inputs(L, B, E, H, d, seed, n):
     return x, ws, bs
 
 
+def _rel(a, b):
+    return ((a - b).norm() / b.norm()).item()
+
+
 def _linear64(x, w, b, H, d):
     y = x.double() @ w.double().t()
     if b is not None:
@@ -498,6 +502,29 @@ def test_linear_rows(R, e_in, e_out):
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert projection.linear_rows(x, w, b) is None
     assert projection.linear_rows(x, w, b) is None          # autograd is on
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_output_projection_differentiated_twice(bias):
+    """The input gradient of the output layer under create_graph is itself differentiable (a gradient penalty):
+    d/dW and d/dx of the sum of dx . r, where dx is the gradient of |x W^T + b|^2 / 2, against fp64."""
+    from rfa_amd import projection
+    torch.manual_seed(3)
+    layer = torch.nn.Linear(128, 256, bias=bias).cuda().half()
+    x, r = (torch.randn(37, 128, device="cuda").half() for _ in range(2))
+
+    def second(x, weight, b, forward):
+        x = x.detach().requires_grad_()
+        y = forward(x)
+        (dx,) = torch.autograd.grad(y, x, y, create_graph=True)
+        return [dx] + list(torch.autograd.grad((dx * r.to(dx.dtype)).sum(), [weight, x]))
+
+    got = second(x, layer.weight, layer.bias, lambda t: projection.linear_out(t, layer))
+    w = layer.weight.detach().double().requires_grad_()
+    b = layer.bias.detach().double() if bias else None
+    want = second(x.double(), w, b, lambda t: torch.nn.functional.linear(t, w, b))
+    for a, ref in zip(got, want):       # a few roundings to fp16, sums of up to 256 products of such terms
+        assert _rel(a.double(), ref) <= 4 * 2.0 ** -11
 
 
 def test_output_projection_keeps_its_hooks():
