@@ -265,7 +265,7 @@ int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int
  * random_project on the q and k projections
  *   (random_feature_attention/causal_attention.py:228-247; cross_attention.py:66-76 for the
  *    k / v projections of the encoder output, :279-283 for the q projection; utils.py:100-120).
- *   x        : fp16 [R, E]      R = seq_len * bsz rows, E a multiple of 64
+ *   x        : fp16 [R, E]      R = seq_len * bsz rows, E a multiple of 64, at most 2^25
  *   weights  : np pointers (1 <= np <= 3) to fp16 [H*d, E], torch.nn.Linear.weight layout
  *   biases   : np pointers to fp16 [H*d] (8-byte aligned); the array or any entry may be NULL
  *   y        : np pointers to fp16 [R, H, d]   y_p = x W_p^T + b_p (the backward of the feature
@@ -296,7 +296,7 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
                            void* stream);
 /* dx = sum_p dy_p W_p, the input gradient of those layers: dy_p fp16 [R, E_out] with rows ld elements apart
  * (ld = 3 E_out for the blocks of a packed gradient), w_p fp16 [E_out, E_in], dx fp16 [R, E_in]; fp32 sums over
- * all p, one rounding.  E_out a multiple of 32, E_in of 128. */
+ * all p, one rounding.  E_out a multiple of 32, E_in of 128, E_in and ld at most 2^22. */
 int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R,
                           int E_out, int E_in, void* stream);
 

@@ -194,8 +194,9 @@ bool own_product(int64_t rows, int64_t e_out, int64_t e_in, int64_t n) {
 // dx = sum_p dy_p W_p for dy_p [rows, E_out] that lie ld halves a row from dys[p] on.  Not where the backward pass
 // itself is recorded (create_graph): the library's products are differentiable, a launch is not.
 bool own_input_grad(int64_t rows, const Tensor* w, int64_t n) {
+    const int64_t widest = (int64_t)1 << 22;      // what the launch addresses
     bool ok = !at::GradMode::is_enabled() && own_product(rows, w[0].size(0), w[0].size(1), n) && w[0].size(0) % 32 == 0 &&
-              w[0].size(1) % 128 == 0;
+              w[0].size(1) % 128 == 0 && w[0].size(1) <= widest && n * w[0].size(0) <= widest;
     for (int64_t p = 0; p < n; ++p) ok = ok && w[p].is_contiguous() && aligned16(w[p]);
     return ok;
 }
@@ -315,6 +316,8 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
     }
 };
 
+constexpr int64_t kMaxProjectWidth = (int64_t)1 << 25;       // rfa_project_feature_map: 32-bit offsets within a row tile
+
 // what the fused launch takes (rfa_amd/projection.py: fused_projection_supported)
 bool plain_layers(const Tensor& x, const OptTensor& wf, const Layers& l, int64_t heads) {
     if (!plain_half(x, 3)) return false;
@@ -322,7 +325,7 @@ bool plain_layers(const Tensor& x, const OptTensor& wf, const Layers& l, int64_t
     for (size_t p = 0; p < l.w.size(); ++p)
         if (!plain_half(l.w[p], 2) || l.w[p].sizes() != w0.sizes() || !plain_half(l.b[p], 1)) return false;
     const int64_t out = w0.size(0), in = w0.size(1);
-    if (in != x.size(2) || in % 64 != 0 || out % heads != 0 || (out / heads != 64 && out / heads != 128)) return false;
+    if (in != x.size(2) || in % 64 != 0 || in > kMaxProjectWidth || out % heads != 0 || (out / heads != 64 && out / heads != 128)) return false;
     return !wf.has_value() ||
            (plain_half(*wf, 3) && (wf->size(1) == 32 || wf->size(1) == 64 || wf->size(1) == 128));
 }
@@ -350,7 +353,7 @@ std::vector<Tensor> project(const Tensor& x, const OptTensor& wf, double scale, 
 // heads of 64 columns and no feature map: the plain product
 bool own_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     const int64_t e_in = w.size(1), e_out = w.size(0), rows = e_in ? x.numel() / e_in : 0;
-    return own_product(rows, e_out, e_in, 1) && e_in % 64 == 0 && e_out % 64 == 0 && e_in > 0 && e_out > 0 &&
+    return own_product(rows, e_out, e_in, 1) && e_in <= kMaxProjectWidth && e_in % 64 == 0 && e_out % 64 == 0 && e_in > 0 && e_out > 0 &&
            x.size(-1) == e_in && x.is_contiguous() && w.is_contiguous() && aligned16(x) && aligned16(w) &&
            w.device() == x.device() &&
            (!b.has_value() || (b->size(0) == e_out && b->is_contiguous() && aligned16(*b) && b->device() == x.device()));

@@ -133,12 +133,13 @@ class _ProjectHeads(torch.autograd.Function):
 def fused_projection_supported(x: Tensor, layers: Sequence[nn.Linear], heads: int,
                                w_feat: Optional[Tensor] = None) -> bool:
     """True when the fused launch can stand in for ``[layer(x) for layer in layers]``: fp16 HIP
-    tensors, a common [out, in] weight shape with ``in`` a multiple of 64 and a head width of
+    tensors, a common [out, in] weight shape with ``in`` a multiple of 64 up to 2^25 and a head width of
     64 or 128 (and a supported proj_dim if a feature map is asked for)."""
     if not (x.is_cuda and x.dtype == torch.float16 and x.dim() == 3 and 1 <= len(layers) <= 3):
         return False
     out_dim, in_dim = layers[0].weight.shape
-    if in_dim != x.shape[-1] or in_dim % 64 != 0 or out_dim % heads != 0 or out_dim // heads not in (64, 128):
+    if (in_dim != x.shape[-1] or in_dim % 64 != 0 or in_dim > 1 << 25 or out_dim % heads != 0
+            or out_dim // heads not in (64, 128)):
         return False
     for layer in layers:
         if tuple(layer.weight.shape) != (out_dim, in_dim) or layer.weight.dtype != torch.float16:

@@ -504,6 +504,27 @@ def test_linear_rows(R, e_in, e_out):
     assert projection.linear_rows(x, w, b) is None          # autograd is on
 
 
+@pytest.mark.parametrize("e_in", [(1 << 22) + 128, (1 << 25) + 128])
+def test_output_projection_wider_than_the_kernels_address(e_in):
+    """Widths that the input-gradient launch (2^22) and the projection launch (2^25) refuse go to the library."""
+    from rfa_amd import projection
+    layer = torch.nn.Linear(128, 128, device="cuda", dtype=torch.float16)
+    layer.weight = torch.nn.Parameter(torch.randn(128, e_in, device="cuda", dtype=torch.float16).mul_(e_in ** -0.5))
+    x = torch.randn(1, e_in, device="cuda", dtype=torch.float16).requires_grad_()
+    print(f"linear_out {e_in} -> 128", flush=True)
+    y = projection.linear_out(x, layer)
+    cut = [slice(c, c + (1 << 22)) for c in range(0, e_in, 1 << 22)]
+    want = sum(x.detach()[:, c].double() @ layer.weight.detach()[:, c].double().t() for c in cut) + layer.bias.detach().double()
+    assert _rel(y.detach().double(), want) <= 2.0 ** -10      # one rounding, fp32 sums of 2^25 terms of either sign
+    if e_in < 1 << 25:
+        dy = torch.randn_like(y)
+        y.backward(dy)
+        assert _rel(x.grad.double(), dy.double() @ layer.weight.detach().double()) <= 2.0 ** -11
+    odd = torch.nn.Linear(64, 64, device="cuda", dtype=torch.float16)
+    odd.weight = torch.nn.Parameter(torch.zeros(1, e_in - 64, device="cuda", dtype=torch.float16).expand(64, e_in - 64))
+    assert projection.fused_projection_supported(x.detach()[None, :, 64:], [odd], 1) == (e_in - 64 <= 1 << 25)
+
+
 @pytest.mark.parametrize("bias", [True, False])
 def test_output_projection_differentiated_twice(bias):
     """The input gradient of the output layer under create_graph is itself differentiable (a gradient penalty):
