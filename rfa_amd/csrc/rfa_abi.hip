@@ -666,9 +666,39 @@ int launch_cross_state_bwd(const rfa::half_t* k, const rfa::half_t* v, const uin
 
 
 // ---- quadratic form with explicit masks ---------------------------------------------------
-// Row blocks in pairs (rfa_masked.h): above three blocks per CU, and where one block alone may be a chain of
-// more than 32 tiles (T 4096, 8 sequences, 64 blocks each: 97 us forward in pairs, 104 singly; 16 each 51 / 42).
-bool masked_paired(int N, int nblk) { return (int64_t)N * nblk > 3 * (int64_t)device_cus() || nblk > 32; }
+// Workgroups of a kernel that one CU of the current device holds; asked once per kernel and device.
+template <auto kKernel>
+int resident_blocks(int threads, size_t lds) {
+    constexpr int kMaxDev = 64;
+    static std::atomic<int> cache[kMaxDev];
+    int dev = 0, blocks = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) dev = 0;
+    blocks = cache[dev].load(std::memory_order_relaxed);
+    if (blocks <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kKernel, threads, lds) != hipSuccess || blocks <= 0) {
+            (void)hipGetLastError();
+            blocks = 1;
+        }
+        cache[dev].store(blocks, std::memory_order_relaxed);
+    }
+    return blocks;
+}
+
+// Whether a workgroup takes row blocks in pairs (rfa_masked.h), from the tiles of a causal mask that the busiest CU
+// walks through, with `resident` workgroups to a CU: pairs are nblk + 1 tiles each, in rounds; single blocks, while
+// all are on the chip at once, end with the longest (nblk), else they are dealt as CUs come free and the last ones
+// trail (by 0.8 of the longest: between 0.5 and 1 fits).  Chains of more than 32 tiles go in pairs as soon as
+// two share a CU.  Measured, single / paired, causal, forward us: K 128, d 64 (3 to a CU), T 512, 64 sequences
+// 16.3 / 18.1; 128, 31.2 / 26.0; 640, 123 / 119; T 1024, 64, 50.3 / 40.3; T 4096, 4 sequences 99 / 102, 12, 157 / 139;
+// K 256, d 128 (2), T 1024, 16, 36.5 / 43.0; 32, 41.1 / 45.0; 320, 352 / 333; K 256, d 64 (2), T 300, 256, 39.8 / 44.9.
+bool masked_paired(int64_t N, int64_t nblk, int resident) {
+    const int64_t cus = device_cus(), slots = resident * cus, pairs = N * ((nblk + 1) / 2);
+    if (N * nblk <= cus) return false;
+    if (nblk > 32) return true;
+    const int64_t paired = (pairs + slots - 1) / slots * (nblk + 1);
+    const double single = N * nblk <= slots ? nblk : 0.8 * nblk + 0.5 * (double)(N * nblk) * (nblk + 1) / slots;
+    return single > paired;
+}
 
 template <int KD, int DH>
 int launch_masked_fwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t* v, const uint8_t* pad,
@@ -678,7 +708,7 @@ int launch_masked_fwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::hal
     auto kern = rfa::k_masked_fwd<KD, DH>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     const int nblk = (T + rfa::kChunk - 1) / rfa::kChunk;
-    const int paired = amask && masked_paired(N, nblk) ? 1 : 0;
+    const int paired = amask && masked_paired(N, nblk, resident_blocks<rfa::k_masked_fwd<KD, DH>>(256, Cfg::kLds)) ? 1 : 0;
     RFA_LAUNCH(MASKED_FWD, kern, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, pad, amask, out, rsum, T, Tp, N, H, paired);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
@@ -691,17 +721,18 @@ int launch_masked_bwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::hal
                       rfa::half_t* ghat, float* gz, int T, int Tp, int N, int H, hipStream_t st) {
     using Cfg = rfa::MaskedCfg<KD, DH>;
     const int nblk = (T + rfa::kChunk - 1) / rfa::kChunk;
-    const int paired = amask && masked_paired(N, nblk) ? 1 : 0;
     const int64_t rows = (int64_t)T * N;
     const int64_t pieces = rows * (DH / 8);
     RFA_LAUNCH(MASKED_PREP, rfa::k_masked_bwd_prep<DH>, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, g, out,
                rsum, ghat, gz, rows);
     auto kq = rfa::k_masked_dq<KD, DH>;
     if (int rc = set_lds(kq, Cfg::kLds)) return rc;
+    int paired = amask && masked_paired(N, nblk, resident_blocks<rfa::k_masked_dq<KD, DH>>(256, Cfg::kLds)) ? 1 : 0;
     RFA_LAUNCH(MASKED_DQ, kq, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, (const rfa::half_t*)ghat, (const float*)gz, k,
                v, pad, amask, dq, T, Tp, N, H, paired);
     auto kk = rfa::k_masked_dkdv<KD, DH>;
     if (int rc = set_lds(kk, Cfg::kLds)) return rc;
+    paired = amask && masked_paired(N, nblk, resident_blocks<rfa::k_masked_dkdv<KD, DH>>(256, Cfg::kLds)) ? 1 : 0;
     RFA_LAUNCH(MASKED_DKDV, kk, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, q, k, v, (const rfa::half_t*)ghat,
                (const float*)gz, pad, amask_t, dk, dv, T, Tp, N, H, paired);
     RFA_HIP_TRY(hipGetLastError());

@@ -199,19 +199,16 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
         chunk_g2r<DH>(t.v, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         chunk_mask_rows<KD>(t.k, prow ? prow + t0 : reinterpret_cast<const uint8_t*>(kb), tid);
     };
-    // two blocks in flight, in two sets of registers that take turns
-    Tile ta, tb;
-    int ja = next_live_block(skip, 0, nblk), jb = next_live_block(skip, ja + 1, nblk);
-    prefetch(ta, ja);
-    prefetch(tb, jb);
+    Tile t;
+    int jb = next_live_block(skip, 0, nblk);
+    prefetch(t, jb);
 
     f4 acc[NCT];
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) acc[ct] = f4_zero();
     float rpart = 0.f;
 
-    // the block in t; t then gets the one after `other`
-    auto step = [&](Tile& t, int& j, int other) __attribute__((always_inline)) {
+    while (jb < nblk) {
         uint32_t mw4[4];
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) mw4[jt] = attn_mask ? t.mw[jt] : 0u;
@@ -220,8 +217,8 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
         chunk_r2s<KD>(t.k, Ks, LDQ, tid);
         chunk_r2s<DH>(t.v, Vs, LDV, tid);
         __syncthreads();
-        j = next_live_block(skip, other + 1, nblk);
-        prefetch(t, j);
+        jb = next_live_block(skip, jb + 1, nblk);
+        prefetch(t, jb);
         f4 at[4];   // A^T tiles (m = j, n = i)
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -242,11 +239,6 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
                 acc[ct] = mfma32(col_split8(Vs, LDV, 32 * jp, 16 * ct, lane), ba, acc[ct]);
         }
         __syncthreads();
-    };
-    while (ja < nblk) {
-        step(ta, ja, jb);
-        if (jb >= nblk) break;
-        step(tb, jb, ja);
     }
 
     const float r = sum_over_groups(rpart);
@@ -345,18 +337,15 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
         chunk_g2r<DH>(t.v, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         chunk_mask_rows<KD>(t.k, prow ? prow + t0 : reinterpret_cast<const uint8_t*>(kb), tid);
     };
-    // two blocks in flight, in two sets of registers that take turns
-    Tile ta, tb;
-    int ja = next_live_block(skip, 0, nblk), jb = next_live_block(skip, ja + 1, nblk);
-    prefetch(ta, ja);
-    prefetch(tb, jb);
+    Tile t;
+    int jb = next_live_block(skip, 0, nblk);
+    prefetch(t, jb);
 
     f4 acc[NKT];   // dQ^T tiles (m = k, n = i)
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt) acc[kt] = f4_zero();
 
-    // the block in t; t then gets the one after `other`
-    auto step = [&](Tile& t, int& j, int other) __attribute__((always_inline)) {
+    while (jb < nblk) {
         uint32_t mw4[4];
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) mw4[jt] = attn_mask ? t.mw[jt] : 0u;
@@ -365,8 +354,8 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
         chunk_r2s<KD>(t.k, Ks, LDQ, tid);
         chunk_r2s<DH>(t.v, Vs, LDV, tid);
         __syncthreads();
-        j = next_live_block(skip, other + 1, nblk);
-        prefetch(t, j);
+        jb = next_live_block(skip, jb + 1, nblk);
+        prefetch(t, jb);
         f4 pt[4];   // P^T tiles (m = j, n = i)
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -386,11 +375,6 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
                 acc[kt] = mfma32(col_split8(Ks, LDQ, 32 * jp, 16 * kt, lane), bp, acc[kt]);
         }
         __syncthreads();
-    };
-    while (ja < nblk) {
-        step(ta, ja, jb);
-        if (jb >= nblk) break;
-        step(tb, jb, ja);
     }
     if (ti < T) {
         half_t* drow = dq + ((int64_t)ti * N + n) * KD;
@@ -453,11 +437,9 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
     };
     __shared__ unsigned char skip[kMaxMaskBlocks];
     masked_tile_skip(attn_mask_t, j0, T, Tp, nblk, skip, tid);
-    // two blocks in flight, in two sets of registers that take turns
-    Tile ta, tb;
-    int ia = next_live_block(skip, 0, nblk), ib = next_live_block(skip, ia + 1, nblk);
-    prefetch(ta, ia);
-    prefetch(tb, ib);
+    Tile t;
+    int ib = next_live_block(skip, 0, nblk);
+    prefetch(t, ib);
 
     f4 acck[NKT], accv[NCT];   // dK^T (m = k, n = s), dV^T (m = c, n = s)
 #pragma unroll
@@ -465,8 +447,9 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) accv[ct] = f4_zero();
 
-    // the block in t; t then gets the one after `other`
-    auto step = [&](Tile& t, int& i, int other) __attribute__((always_inline)) {
+    // the block in t; t then gets the one after j (written into the loop itself this takes two more registers,
+    // which at K = 256, d = 64 are not there)
+    auto step = [&](Tile& t, int& i, int j) __attribute__((always_inline)) {
         chunk_r2s<KD>(t.q, Qs, LDQ, tid);
         chunk_r2s<DH>(t.g, Gs, LDV, tid);
         if (tid < C) gzs[tid] = tid < t.g.rows ? t.gz : 0.f;
@@ -474,7 +457,7 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 #pragma unroll
         for (int it = 0; it < 4; ++it) mw4[it] = attn_mask_t ? t.mw[it] : 0u;
         __syncthreads();
-        i = next_live_block(skip, other + 1, nblk);
+        i = next_live_block(skip, j + 1, nblk);
         prefetch(t, i);
         f4 a_[4], p_[4];   // tiles (m = t, n = s)
 #pragma unroll
@@ -509,11 +492,7 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
         }
         __syncthreads();
     };
-    while (ia < nblk) {
-        step(ta, ia, ib);
-        if (ib >= nblk) break;
-        step(tb, ib, ia);
-    }
+    while (ib < nblk) step(t, ib, ib);
     if (tj < T) {
         half_t* krow = dk + ((int64_t)tj * N + n) * KD;
         half_t* vrow = dv + ((int64_t)tj * N + n) * DH;
@@ -528,11 +507,13 @@ __device__ __forceinline__ void masked_dkdv_block(const int n, const int j0,
 // Kernels.  A workgroup takes one row block of a sequence (grid = N * nblk), or two (`paired`, grid = N * ceil(nblk /
 // 2)).  With a causal mask block p has p + 1 live column blocks; a pair p, nblk - 1 - p is the same work for every
 // workgroup, where single blocks leave the CUs to the last long ones.  But while the single blocks are few enough
-// to be on the chip at once (26 KB of LDS each at K = 128), several to a CU, they hide each other's round trips:
-// the launcher pairs above three per CU.  Measured, single / paired, causal, fwd and bwd us: T 512, 64 sequences
-// (512 blocks) 18.5 / 21.5, 49 / 54; T 300, 128 (640) 19.0 / 21.1, 52 / 58; T 1024, 16, K 256, d 128 (256)
-// 41.6 / 50.7, 127 / 146; T 1024, 64 (1024) 58.4 / 49.3, 151 / 120.  Before the two register sets and the shared
-// barrier of the flags, paired: 27.0, 69.1; 24.2, 64.9; 58.8, 161; 59.8, 145.
+// to be on the chip at once, several to a CU, they hide each other's round trips.  How many a CU holds is a matter
+// of registers (4 at K = 64, d = 64; 3, dK/dV 2, at K = 128; 2 at K = 256, dK/dV with d = 128 1), and the launcher
+// asks for it.  One block is in flight in registers while the one before it is worked on: a second set of registers
+// for a block more cost a resident workgroup or two everywhere and was slower at every size but the smallest.
+// Measured, causal, fwd + dQ + dK/dV, us, before the prefetched mask words and the shared barrier of the flags / two
+// register sets and three blocks to a CU / now: K 128, d 64, T 512, 64 sequences 86 / 59 / 57; 640 sequences 468 / 484 /
+// 425; T 1024, 64, 193 / 153 / 138; K 128, d 128, T 512, 96, 125 / 136 / 95; K 256, d 128, T 1024, 32, 231 / 284 / 143.
 // The workgroups of a sequence run on one XCD, whose L2 then serves its rows to all but the first; single blocks
 // of the sequences of every second round of workgroups over an XCD's 32 CUs are dealt in reverse, so that a CU
 // gets long and short ones.
@@ -579,7 +560,7 @@ __global__ __launch_bounds__(256) void k_masked_dq(
 }
 
 template <int KD, int DH>
-__global__ __launch_bounds__(256) void k_masked_dkdv(
+__global__ __launch_bounds__(256, KD == 256 && DH == 128 ? 1 : 2) void k_masked_dkdv(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     const half_t* __restrict__ ghat, const float* __restrict__ gz, const uint8_t* __restrict__ pad_mask,
     const uint8_t* __restrict__ attn_mask_t, half_t* __restrict__ dk, half_t* __restrict__ dv, int T, int Tp,

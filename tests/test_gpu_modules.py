@@ -673,3 +673,37 @@ def test_masked_rfa_blocks_dealt_singly_and_in_pairs(T, with_mask):
     for b0 in (0, B // 2, B - 17):
         for a, b in zip(whole, run(b0, b0 + 17)):
             assert torch.isfinite(b).all() and torch.equal(a[:, b0 * H:(b0 + 17) * H], b)
+
+
+@pytest.mark.parametrize("d,D", [(64, 32), (64, 64), (64, 128), (128, 32), (128, 64), (128, 128)])
+def test_masked_rfa_blocks_dealt_singly_and_in_pairs_at_every_width(d, D):
+    """384 sequences of 4 row blocks go in pairs whatever a CU holds (one to four workgroups), 16 of them singly: the
+    same bits, and 4 of them against the oracle in fp64 with a padded key and a row that keeps one key only."""
+    from rfa_amd import rfa_hip
+    T, H, B, few = 200, 4, 96, 4
+    gen = torch.Generator("cuda").manual_seed(D)
+    q, k = (torch.rand(T, B * H, 2 * D, generator=gen, device="cuda").half() / D ** 0.5 for _ in range(2))
+    v, g = (torch.randn(T, B * H, d, generator=gen, device="cuda").half() for _ in range(2))
+    masked = torch.ones(T, T, dtype=torch.bool, device="cuda").triu(1)
+    masked[70] = True
+    masked[70, 3] = False
+    m, mt = rfa_hip.pack_attn_mask(masked)
+    pad = torch.zeros(B, T, dtype=torch.bool, device="cuda")
+    pad[0, 190:] = True
+    print(f"masked blocks at every width d={d} D={D}", flush=True)
+
+    def run(b0, b1):
+        cut = lambda t: t[:, b0 * H:b1 * H].contiguous()
+        out, rsum = rfa_hip.masked_forward(cut(q), cut(k), cut(v), H, pad[b0:b1], m)
+        return [out, rsum, *rfa_hip.masked_backward(cut(q), cut(k), cut(v), cut(g), out, rsum, H, pad[b0:b1], m, mt)]
+
+    whole = run(0, B)
+    for b0 in (0, B - few):
+        for a, b in zip(whole, run(b0, b0 + few)):
+            assert torch.isfinite(b).all() and torch.equal(a[:, b0 * H:(b0 + few) * H], b)
+    wide = lambda t: t[:, :H].reshape(T, 1, H, -1).double().cpu().requires_grad_()
+    q64, k64, v64 = wide(q), wide(k), wide(v)
+    ref = O.masked_rfa(q64, k64, v64, pad[:1].cpu(), torch.zeros(T, T).masked_fill(masked.cpu(), float("-inf")).double())
+    ref.backward(g[:, :H].reshape(ref.shape).double().cpu())
+    for got, want in zip([whole[0]] + whole[2:], [ref.detach(), q64.grad, k64.grad, v64.grad]):
+        assert _rel(got[:, :H].double().cpu().reshape(want.shape), want) <= 4 * 2.0 ** -11      # fp16 tiles and results
