@@ -6,6 +6,7 @@
 #include <hip/hip_ext.h>
 
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -821,14 +822,19 @@ struct WGradPlan {
     int rows_per_split;    // multiple of 32
 };
 
-// Two workgroups per CU, but at least 16 steps of 32 rows each: every split writes and re-reads an fp32
-// copy of dW, and its ring has to fill first.  Measured (us, 8192 rows) for 4 / 8 / 10 / 16 / 32 splits:
+// Up to two workgroups per CU.  Every split writes and re-reads an fp32 copy of dW and its ring has to fill first, so
+// that beyond some 4096 rows a split has at least 16 steps of 32; a few hundred rows of a small dW are a chain of
+// steps (0.3 us each) with next to no copies beside it, and the least of steps / splits + splits * tiles lies at a root.
+// Measured (us, 8192 rows) for 4 / 8 / 10 / 16 / 32 splits:
 // 512 -> 3 x 512 (48 tiles) 34.8 / 27.0 / 25.8 / 29.5 / 40.8; 1024 -> 1024 (64) 36.3 / 29.9 / 34.1 / 37.0 /
 // 50.1; 512 -> 512 (16) 32.4 / 23.9 / 22.7 / 23.2 / 24.9; 1000 rows, 384 -> 3 x 384 (27): 4 -> 14.0, 16 -> 22.6.
+// 512 rows for 1 / 2 / 4 / 8 splits: 128 -> 128 (1) 11.7 / 8.9 / 8.0 / 8.3; 512 -> 512 11.9 / 9.8 / 9.7 / 11.9;
+// 1024 rows for 2 / 4 / 8: 256 -> 256 (4) 12.1 / 9.7 / 9.7; 1024 -> 1024 16.9 / 18.4 / 24.0.
 WGradPlan make_wgrad_plan(int64_t R, int Eo, int Ei, int np) {
     const int64_t tiles = (int64_t)np * (Eo / 128) * (Ei / 128);
     const int64_t nsteps = (R + 31) / 32;
-    int64_t want = std::min<int64_t>(2 * (int64_t)device_cus() / tiles, nsteps / 16);
+    const int64_t root = (int64_t)(std::sqrt(16.0 * nsteps / (tiles + 16)) + 0.3);
+    int64_t want = std::min<int64_t>(2 * (int64_t)device_cus() / tiles, std::max<int64_t>(nsteps / 16, root));
     if (want > 64) want = 64;
     if (want < 1) want = 1;
     const int64_t sps = (nsteps + want - 1) / want;

@@ -273,6 +273,21 @@ def test_linear_weight_gradient_step_edges(R):
     assert torch.equal(db.double().cpu(), dy.double().sum(0))
 
 
+@pytest.mark.parametrize("R", [98, 128, 129, 257, 449, 600, 2000])
+@pytest.mark.parametrize("e_out,e_in,n", [(128, 128, 1), (256, 384, 2), (512, 512, 3)])
+def test_linear_weight_gradient_of_few_rows(R, e_out, e_in, n):
+    """A few hundred rows split by the root of their steps, down to two steps and a last one of a single row: dW and
+    db exactly (whole numbers)."""
+    from rfa_amd import rfa_hip
+    g = torch.Generator().manual_seed(R + n)
+    x = torch.randint(-1, 2, (R, e_in), generator=g).half()
+    dys = [torch.randint(-1, 2, (R, e_out), generator=g).half() for _ in range(n)]
+    dws, dbs = rfa_hip.linear_weight_grad(x.cuda(), [dy.cuda() for dy in dys], [True] * n)
+    for dy, dw, db in zip(dys, dws, dbs):
+        assert torch.equal(dw.double().cpu(), dy.double().t() @ x.double())
+        assert torch.equal(db.double().cpu(), dy.double().sum(0))
+
+
 def test_cross_modules_fused_projections_match_unfused_chain():
     """CrossAttentionProjectLayer + CrossAttention with their projections on the fused launch vs
     the same modules on nn.Linear + random_project: output within 4e-3, gradients within 1e-2."""
