@@ -12,6 +12,7 @@
 // (128 tokens of 4 heads, the scan alone: 114 -> 68; encoder-decoder layer, 16384 + 8192 rows: 574 -> 430).
 #pragma once
 #include <ATen/autocast_mode.h>
+#include <ATen/hip/HIPContextLight.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -182,11 +183,14 @@ std::pair<std::vector<Tensor>, std::vector<OptTensor>> param_grads(const Tensor&
 }
 
 // Products through the framework's own kernels: a library product costs 19 us of host time, these 4 to 5, and
-// two of them in a backward need a second pass over dx, three a stack of the weights.  Up to 7e9
-// multiply-adds they are level on the device, us own / library: 8192 rows of 512 -> 512 11.6 / 12.3 (dx), 10.6 /
-// 11.4 (y); three of them 24.8 / 21.4 + 4.6 for the stack.  Past that the library's larger tiles win (8192
-// rows of 1024 -> 1024 28.9 / 23.6, 28.3 / 24.4; three 69.3 / 57.3 + 7.8), for two layers without a packed
-// gradient, where it takes two products, later (16384 rows of 512 28.1 / 38; of 1024 82.5 / 75).
+// two of them in a backward need a second pass over dx, three a stack of the weights.  Up to 7 * 2^30
+// multiply-adds they are level on the device where there are rows enough, us own / library: 8192 rows of 512 -> 512
+// 11.6 / 12.3 (dx), 10.3 / 11.3 (y); three of them 25 / 21.5 + 3.0 for the stack.  Past that the library's larger tiles
+// win (8192 rows of 1024 -> 1024 28.5 / 23.4, 26.7 / 22.6; three 69 / 57 + 7.8), for two layers without a packed
+// gradient, where it takes two products, later (16384 rows of 512 28.4 / 35.6; of 1024 82.5 / 75).  Few rows of a
+// wide layer lose device time to it (the contraction is walked by one workgroup per tile: 512 rows of 1024 -> 1024
+// 12.6 / 8.0 dx, 10.8 / 8.6 y; three 32 / 16.5 + 4.5), which is given for the host time: a step of that size waits
+// for the host by far.
 bool own_product(int64_t rows, int64_t e_out, int64_t e_in, int64_t n) {
     return rows > 0 && rows * e_out * e_in * n <= (n == 2 ? (int64_t)1 << 34 : (int64_t)7 << 30);
 }
@@ -398,13 +402,29 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
     }
 };
 
-// The row kernel costs 4 us of host time, a library product 19; on the device it is ahead or level up to about
-// 96 rows of 1024 -> 3072 (9.2 / 8.9 us) or 256 of 1024 -> 1024 (7.1 / 8.0), and behind past that (160 rows of
-// 1024 -> 3072 12.9 / 8.5) and where a long contraction is split over its four waves only (64 rows of
-// 2048 -> 2048 12.6 / 8.8).
-bool few_rows(int64_t R, int64_t e_in, int64_t e_out) {
-    return R <= 256 && (R <= 32 || e_in <= 1024) && R * e_in * e_out <= (int64_t)300 << 20;
+// Without autograd the row kernel takes up to 512 rows while its workgroups (64 rows x 32 columns) are at most one to
+// a CU and the contraction is short (four waves share E_in), or a few rows of anything up to 192 M products.
+// Device us there, row kernel / library: 512 -> 512 64 rows 4.4 / 5.6, 512 rows 4.7 / 5.2; 1024 -> 3072 64 rows 7.1 / 8.3,
+// 128 rows 8.9 / 9.2; at worst 768 -> 2304 96 rows 7.9 / 6.3, 1024 -> 1024 320 rows 8.4 / 6.5; 2048 -> 2048 32 rows 7.7 /
+// 8.4.  Past it two rounds of workgroups: 1024 -> 1024 768 rows 14.0 / 8.7; rows of x that every column tile reads again,
+// from other XCDs' caches where they were just written (a layer's forward over 1024 rows of 512: 26.9 with the output
+// projection by it, 25.0 by the projection kernel); a long contraction: 2048 -> 2048 64 rows 11.2 / 8.9.
+// Widths that the projection kernel does not take stay with the library past 256 rows.
+bool few_rows(int64_t R, int64_t e_in, int64_t e_out, int64_t cus) {
+    if (R <= 32 && R * e_in * e_out <= (int64_t)192 << 20) return true;
+    return e_in <= 1024 && R <= (e_in % 64 == 0 && e_out % 64 == 0 ? 512 : 256) &&
+           (R + 63) / 64 * ((e_out + 31) / 32) <= cus;
 }
+
+// More rows go to the projection kernel, up to E_in = 1024 and 2^31 products, beyond that to the library: its tiles walk
+// the contraction alone, 0.27 us per 32 columns of E_in however few they are.  Device us, projection kernel /
+// library: 512 -> 512 2048 rows 7.3 / 7.2, 8192 10.3 / 11.3; 768 -> 768 768 rows 9.0 / 6.7, 2048 9.4 / 9.1; 1024 -> 1024 768
+// rows 10.8 / 8.7, 2048 11.5 / 10.7; not taken: 1536 -> 1536 512 rows 15.2 / 9.4; 2048 -> 2048 64 rows 17.5 / 8.9, 512
+// rows 19.0 / 11.3.  Both kernels may lose up to 2.4 us on the device to the library, for the 15 us of host time that
+// each saves: a layer taking in one prompt of 512 tokens, E 1024, takes 63 us eagerly (130 through the library)
+// and 53 from a replayed graph (51), 1024 tokens 66 (133) and 66 (58); a token for each of 64 sequences at E 2048, on
+// the projection kernel 81 and 83, on the library 68 and 65.
+constexpr int64_t kWidestOwnProjection = 1024;
 
 // for the callers' condition (fp16, grad mode on, widths that are multiples of 128) see linear_out
 OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
@@ -422,10 +442,9 @@ OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b)
         return c10::nullopt;
     const int64_t e_in = w.size(1), e_out = w.size(0), R = e_in ? x.numel() / e_in : 0;
     if (R < 1 || x.size(-1) != e_in) return c10::nullopt;
-    // a prompt is bound by the device sooner than a training step: up to 2^31, where the projection kernel is level
-    // or ahead there too (8192 rows of 512 -> 512 10.6 / 11.4 us; 4662 of 768 -> 768 14.4 / 12.0, 16384 of 512 17.1 / 16.1)
-    if (!few_rows(R, e_in, e_out))
-        return R * e_in * e_out <= (int64_t)1 << 31 && own_linear(x, w, b) ? OptTensor(projection(x, w, b)) : c10::nullopt;
+    if (!few_rows(R, e_in, e_out, at::cuda::getDeviceProperties(x.get_device())->multiProcessorCount))
+        return e_in <= kWidestOwnProjection && R * e_in * e_out <= (int64_t)1 << 31 && own_linear(x, w, b)
+                   ? OptTensor(projection(x, w, b)) : c10::nullopt;
     if (e_in % 32 != 0 || e_out % 16 != 0 || e_out == 0 ||
         !x.is_contiguous() || !w.is_contiguous() || !aligned16(x) || !aligned16(w) || w.device() != x.device())
         return c10::nullopt;

@@ -198,6 +198,13 @@ __device__ __forceinline__ h4 h4_zero() {
     h4 r; r[0] = (half_t)0.f; r[1] = (half_t)0.f; r[2] = (half_t)0.f; r[3] = (half_t)0.f; return r;
 }
 
+__device__ __forceinline__ h8 h8_zero() {
+    h8 r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = (half_t)0.f;
+    return r;
+}
+
 __device__ __forceinline__ h8 h8_ones() {
     h8 r;
 #pragma unroll

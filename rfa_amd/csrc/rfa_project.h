@@ -264,14 +264,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
 // ---------------------------------------------------------------------------
 // y[r][o] = x[r] . W[o] + b[o] for few rows: the projections of a decoding step.
 //
-// What bounds it is one trip to memory for W and the launch around it, so every byte of W is asked for at
-// once: a workgroup of four waves owns 16 columns (16 rows of W) of up to 64 rows of x, the waves share
-// the contraction, each with its 32-deep steps in flight together, operands straight from memory in the
-// lanes' own order; the four partial sums meet in LDS.  x comes out of the L2: with 64 rows its reads
-// bound the kernel, and 32 columns per workgroup halve them where that still leaves a workgroup per CU.
-// Measured, device us of the kernel / the library's product (which costs 19 us of host time, this 4):
-// 4 rows 512 -> 1536 2.7 / 3.7, 1024 -> 3072 3.7 / 5.9; 64 rows 512 -> 512 4.4 / 5.4, 1024 -> 3072 7.5 / 8.5;
-// 96 rows 1024 -> 3072 9.2 / 8.9; 160 rows 12.9 / 8.5.
+// What bounds it is the trips to memory and the launch around them: a workgroup of four waves owns 16 columns (16 rows of
+// W) of up to 64 rows of x, the waves share the contraction, each with four 32-deep steps in flight together (the
+// loads of a batch before its first product, no branch between them), operands straight from memory in the
+// lanes' own order; the four partial sums meet in LDS.  A lane's 16 bytes lie a whole row from its neighbour's, so
+// a load asks for 16 lines, and x is read again for every 16 columns: from 64 rows on these reads bound the kernel,
+// and 32 columns per workgroup halve them where that still leaves a workgroup per CU.
+// Measured, device us with the loads of a batch one behind the other / now / the library's product (which costs 19 us
+// of host time, this 4): 4 rows 512 -> 1536 2.9 / 2.8 / 3.9, 1024 -> 3072 4.2 / 3.8 / 5.7; 64 rows 512 -> 512 4.6 /
+// 4.4 / 5.6, 768 -> 768 6.8 / 6.1 / 5.7, 1024 -> 3072 7.7 / 7.1 / 8.3; 320 rows 1024 -> 1024 9.1 / 8.4 / 6.5.
 // grid = (ceil(Eo / (16 CT)), ceil(R / (16 RT)));  E % 32 == 0, Eo % 16 == 0
 // ---------------------------------------------------------------------------
 template <int RT, int CT>
@@ -279,7 +280,8 @@ __global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restri
                                                           const half_t* __restrict__ bias, half_t* __restrict__ y, int R,
                                                           int E, int Eo) {
     __shared__ f4 red[4][RT * CT][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // the wave's bounds are scalar: no lane masks
     const int i = lane & 15, G = lane >> 4;
     const int c0 = 16 * CT * blockIdx.x, r0 = 16 * RT * blockIdx.y;
     const int nk = E / 32, per_wave = (nk + 3) / 4;
@@ -296,26 +298,36 @@ __global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restri
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[a][c] = f4_zero();
     constexpr int U = 4;      // steps in flight; 8 only repeat the last step's loads where E = 512
-    for (int k = k_begin; k < k_end; k += U) {
+    // steps k .. k + U - 1, no branch between the loads; steps from `end` on (none unless `ragged`) count as zeros
+    auto batch = [&](int k, int end, auto ragged) __attribute__((always_inline)) {
         h8 wa[U][CT], xb[U][RT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int kk = 32 * min(k + u, k_end - 1);
+            const int kk = 32 * (ragged ? min(k + u, end - 1) : k + u);
 #pragma unroll
             for (int c = 0; c < CT; ++c) wa[u][c] = *reinterpret_cast<const h8*>(wp[c] + kk);
 #pragma unroll
             for (int a = 0; a < RT; ++a) xb[u][a] = *reinterpret_cast<const h8*>(xp[a] + kk);
         }
+        __builtin_amdgcn_sched_barrier(0);      // all loads of the batch before its first product
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (k + u < k_end) {
+            if (ragged) {
+                const bool live = k + u < end;
 #pragma unroll
-                for (int a = 0; a < RT; ++a)
+                for (int c = 0; c < CT; ++c) wa[u][c] = live ? wa[u][c] : h8_zero();
 #pragma unroll
-                    for (int c = 0; c < CT; ++c) acc[a][c] = mfma32(wa[u][c], xb[u][a], acc[a][c]);
+                for (int a = 0; a < RT; ++a) xb[u][a] = live ? xb[u][a] : h8_zero();
             }
+#pragma unroll
+            for (int a = 0; a < RT; ++a)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[a][c] = mfma32(wa[u][c], xb[u][a], acc[a][c]);
         }
-    }
+    };
+    int k = k_begin;
+    for (; k + U <= k_end; k += U) batch(k, k_end, std::false_type{});
+    if (k < k_end) batch(k, k_end, std::true_type{});
 #pragma unroll
     for (int a = 0; a < RT; ++a)
 #pragma unroll

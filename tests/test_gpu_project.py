@@ -519,6 +519,30 @@ def test_linear_rows(R, e_in, e_out):
     assert projection.linear_rows(x, w, b) is None          # autograd is on
 
 
+@pytest.mark.parametrize("R,e_in,e_out", [(1024, 512, 512), (1025, 512, 512), (320, 512, 1536), (321, 512, 1536), (512, 1024, 1024),
+                                          (513, 1024, 1024), (129, 1024, 3072), (16, 2048, 6144), (32, 2080, 48), (33, 2048, 2048),
+                                          (7, 160, 16), (19, 288, 32), (64, 992, 272)])
+def test_linear_rows_where_the_choice_changes(R, e_in, e_out):
+    """Both sides of one workgroup per CU and of the widest contraction, and contractions that end in a ragged batch of
+    steps for one or more of the four waves, whose columns of W past the end are not numbers: against fp64."""
+    from rfa_amd import projection, rfa_hip
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    gen = torch.Generator("cuda").manual_seed(R)
+    x = torch.randn(R, e_in, generator=gen, device="cuda").half()
+    w = torch.full((e_out + 1, e_in), float("nan"), device="cuda", dtype=torch.float16)[:e_out]
+    w.copy_(torch.randn(e_out, e_in, generator=gen, device="cuda") / e_in ** 0.5)
+    b = torch.randn(e_out, generator=gen, device="cuda").half()
+    print(f"linear_rows where the choice changes R={R} {e_in}->{e_out}", flush=True)
+    with torch.no_grad():
+        y = projection.linear_rows(x, w, b)
+    if R > 32 and e_in > 1024:
+        assert y is None        # the library's
+        return
+    want = x.double() @ w.double().t() + b.double()
+    assert ((y.double() - want).abs() <= 2.0 ** -10 * want.abs() + 2e-5).all()
+
+
 @pytest.mark.parametrize("e_in", [(1 << 22) + 128, (1 << 25) + 128])
 def test_output_projection_wider_than_the_kernels_address(e_in):
     """Widths that the input-gradient launch (2^22) and the projection launch (2^25) refuse go to the library."""
