@@ -204,8 +204,14 @@ def _is_bare_linear(layer: nn.Module) -> bool:
 
 def linear_no_grad(x: Tensor, layer: nn.Linear) -> Tensor:
     """``layer(x)``, without autograd by the framework's own kernels where they apply."""
-    y = linear_rows(x, layer.weight, layer.bias) if not torch.is_grad_enabled() and _is_bare_linear(layer) else None
-    return layer(x) if y is None else y
+    if torch.is_grad_enabled() or not _is_bare_linear(layer):
+        return layer(x)
+    weight, bias = layer.weight, layer.bias
+    y = linear_rows(x, weight, bias)
+    if y is not None:
+        return y
+    # the library's: what the call comes to, without its 1.5 us of hook handling (a trace records the call itself)
+    return layer(x) if torch.jit.is_tracing() else nn.functional.linear(x, weight, bias)
 
 
 def linear_out(x: Tensor, layer: nn.Linear) -> Tensor:
