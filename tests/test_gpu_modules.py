@@ -619,6 +619,85 @@ def test_native_nodes_leave_odd_calls_to_the_python_functions():
         call(forward_ad.make_dual(q.detach(), torch.ones_like(q)))
 
 
+def test_traced_scan_follows_its_inputs():
+    """While a call is traced the nodes step aside, so that the trace holds the Python functions."""
+    from rfa_amd import rfa_hip
+    from rfa_amd.causal_attention import cuda_causal_rfa
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    aside = []
+
+    def call(q, k, v):
+        if torch.jit.is_tracing():
+            aside.append(rfa_hip.native.node_causal(q, k, v) is None)
+        return cuda_causal_rfa(phi_q=q, phi_k=k, v=v)
+    first, second = ([0.1 * torch.rand(70, 2, 2, 64, device="cuda").half() for _ in range(3)] for _ in range(2))
+    traced = torch.jit.trace(call, tuple(first), check_trace=False)
+    assert aside == [True]
+    assert torch.equal(traced(*second), call(*second))
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("T,B,H,d", [(70, 3, 3, 64), (205, 40, 8, 128)])
+@pytest.mark.parametrize("path", ["module", "cross"])
+def test_layer_gradients_where_the_library_multiplies(path, T, B, H, d, bias):
+    """The nodes' other branches: widths that are no multiple of 128 (library products for every gradient, the stack
+    of three weights) and rows above the own kernels' limits (library products for dx and y), outputs and every
+    gradient against the formulas in fp64.  fp16 at some eight places on the way to each: 8 x 2^-11 / sqrt(3)."""
+    from rfa_amd import causal_attention as C, cross_attention as X
+    D, E = 32, H * d
+    gen = torch.Generator("cuda").manual_seed(T)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    W = rand(H, D, d).half()
+
+    def layer(cls):
+        m = cls(embed_dim=E, num_heads=H, head_dim=d, proj_dim=D).cuda().half()
+        with torch.no_grad():
+            for name, p in m.named_parameters():
+                p.copy_(1 + 0.1 * rand(*p.shape) if name == "sigma" else rand(*p.shape) / (2 * E) ** 0.5)
+        if not bias:
+            for lin in m.children():
+                lin.bias = None
+        return m, {n: p.detach().double().requires_grad_() for n, p in m.named_parameters()}
+
+    leaf = lambda t: t.half().requires_grad_()
+    lin = lambda p, name, t: t @ p[name + ".weight"].t() + p.get(name + ".bias", 0.0)
+    heads = lambda t: t.view(*t.shape[:2], H, d)
+    x, g = leaf(rand(T, B, E)), rand(T, B, E).half()
+    x64 = x.detach().double().requires_grad_()
+    print(f"layer gradients {path} T={T} B={B} H={H} d={d} bias={bias}", flush=True)
+    if path == "module":
+        m, p = layer(C.CausalAttention)
+        out = m(x, W)
+        w = W.double() * p["sigma"]
+        q, k, v = (heads(lin(p, n, x64)) for n in ("q_proj", "k_proj", "v_proj"))
+        rows = lambda t: t.reshape(T, B * H, -1)
+        attn = O.causal_forward_cumsum(rows(O.random_project(q, w)), rows(O.random_project(k, w)), rows(v))
+        leaves, leaves64 = [x, *m.parameters()], [x64, *p.values()]
+    else:
+        src, ps = layer(X.CrossAttentionProjectLayer)
+        m, p = layer(X.CrossAttention)
+        enc = leaf(rand(T, B, E))
+        enc64 = enc.detach().double().requires_grad_()
+        pad = torch.zeros(T, B, 1, 1, dtype=torch.bool, device="cuda")
+        pad[T - 9:, 1] = True
+        out = m(x, src(encoder_output=enc, random_matrices=W, mask=pad))
+        w = W.double() * ps["sigma"]
+        k, v = (heads(lin(ps, n, enc64)) for n in ("k_proj", "v_proj"))
+        phi_k = O.random_project(k, w).masked_fill(pad, 0.0)
+        attn = O.cross_readout(O.random_project(heads(lin(p, "q_proj", x64)), w),
+                               torch.einsum("tbhk,tbhd->bhkd", phi_k, v), phi_k.sum(0))
+        leaves = [x, enc, *src.parameters(), *m.parameters()]
+        leaves64 = [x64, enc64, *ps.values(), *p.values()]
+    want = lin(p, "out_proj", attn.reshape(T, B, E))
+    out.backward(g)
+    want.backward(g.double())
+    for a, b in [(out.detach(), want.detach())] + [(s.grad, t.grad) for s, t in zip(leaves, leaves64)]:
+        err = _rel(a.double(), b)
+        print(f"  {tuple(a.shape)} {err:.2e}", flush=True)
+        assert err <= 8 * 2.0 ** -11 / 3 ** 0.5
+
+
 @pytest.mark.parametrize("d,D", [(64, 32), (64, 64), (128, 32), (128, 64)])
 @pytest.mark.parametrize("T", [2, 15, 64, 65, 127, 200])
 def test_prefill_from_projected_rows(T, d, D):
