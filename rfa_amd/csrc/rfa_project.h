@@ -435,8 +435,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
         const half_t* const xb = x + (int64_t)r_begin * Ei + c0;
         const int nrows = r_end - r_begin, nk = (nrows + C - 1) / C;
         auto rot = [](int r) { return ((r & 3) | ((r >> 1) & 4)) * 2; };
-        // byte offsets inside a step; the rows of the last step past the end read the last row (the dy
-        // operand drops them)
+        // byte offsets inside a step; the rows of the last step past the end read the last row (both operands
+        // drop them: that row may hold an infinity, and 0 times it is not a number)
         unsigned yoff[2][Cfg::YI], xoff[2][Cfg::XI];
 #pragma unroll
         for (int last = 0; last < 2; ++last) {
@@ -480,9 +480,12 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             if (kk * C + C > nrows) {                     // the ragged end of the rows
                 const int keep = nrows - kk * C - 8 * G;
 #pragma unroll
-                for (int a = 0; a < NO; ++a)
+                for (int e = 0; e < 8; ++e) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) ya[a][e] = e < keep ? ya[a][e] : (half_t)0.f;
+                    for (int a = 0; a < NO; ++a) ya[a][e] = e < keep ? ya[a][e] : (half_t)0.f;
+#pragma unroll
+                    for (int b = 0; b < NI; ++b) xa[b][e] = e < keep ? xa[b][e] : (half_t)0.f;
+                }
             }
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll

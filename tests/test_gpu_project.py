@@ -273,6 +273,21 @@ def test_linear_weight_gradient_step_edges(R):
     assert torch.equal(db.double().cpu(), dy.double().sum(0))
 
 
+@pytest.mark.parametrize("R", [1, 31, 33, 98, 1025, 8191])
+def test_linear_weight_gradient_of_an_infinity_in_the_last_row(R):
+    """Rows past the ragged end count for nothing, also where the last row, which stands in for them, holds an infinity:
+    its column of dW is infinite with the sign of dy, as the product gives it, and the others are exact."""
+    from rfa_amd import rfa_hip
+    g = torch.Generator().manual_seed(R)
+    x = torch.randint(-1, 2, (R, 128), generator=g).half()
+    dy = (2 * torch.randint(0, 2, (R, 128), generator=g) - 1).half()
+    want = dy.double().t() @ x.double()
+    x[-1, 5], x[-1, 77] = float("inf"), float("-inf")
+    want[:, 5], want[:, 77] = dy[-1].double() * float("inf"), dy[-1].double() * float("-inf")
+    (dw,), _ = rfa_hip.linear_weight_grad(x.cuda(), [dy.cuda()], [False])
+    assert torch.equal(dw.double().cpu(), want)
+
+
 @pytest.mark.parametrize("R", [98, 128, 129, 257, 449, 600, 2000])
 @pytest.mark.parametrize("e_out,e_in,n", [(128, 128, 1), (256, 384, 2), (512, 512, 3)])
 def test_linear_weight_gradient_of_few_rows(R, e_out, e_in, n):
