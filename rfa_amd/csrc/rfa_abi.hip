@@ -2130,7 +2130,7 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
     const int64_t work = (int64_t)pl.nsplit * np * (E_out / 128) * (E_in / 128);
     if (work > (int64_t(1) << 30)) return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_weight_grad: sizes exceed the supported range");
     const unsigned grid = (unsigned)(rfa::kXcds * ((work + rfa::kXcds - 1) / rfa::kXcds));
-    auto kern = rfa::k_weight_grad_partial;
+    auto kern = std::max(E_out, E_in) > (1 << 26) ? rfa::k_weight_grad_partial<true> : rfa::k_weight_grad_partial<false>;
     if (int rc = set_lds(kern, rfa::WeightGradCfg::kLds)) return rc;
     // R = 0: every split is empty and the partials come out as zeros
     RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3(grid), dim3(rfa::kThreads), rfa::WeightGradCfg::kLds, st,

@@ -394,7 +394,8 @@ __device__ __forceinline__ h8 col8_rot(const half_t* X, int seg, int lane) {
 // 512 -> 512 26.0 -> 23.2; 1000 rows, 384 -> 3 x 384 22.8 -> 14.4.
 // grid = 8 * ceil(work / 8), work = nsplit * np * tiles; each XCD gets a contiguous range of the numbers
 // (split first), so that the workgroups that share rows of x and dy meet in its L2.  rows_per_split is a
-// multiple of 32.
+// multiple of 32.  WIDE: rows of more than 2^26 halves, 32 of which lie beyond a 32-bit byte offset.
+template <bool WIDE>
 __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
     const half_t* __restrict__ x, WeightGradArgs wa, float* __restrict__ part, float* __restrict__ bpart, int R,
     int Eo, int Ei, int np, int nsplit, int rows_per_split) {
@@ -437,21 +438,26 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
         auto rot = [](int r) { return ((r & 3) | ((r >> 1) & 4)) * 2; };
         // byte offsets inside a step; the rows of the last step past the end read the last row (both operands
         // drop them: that row may hold an infinity, and 0 times it is not a number)
-        unsigned yoff[2][Cfg::YI], xoff[2][Cfg::XI];
+        using Offset = std::conditional_t<WIDE, int64_t, unsigned>;
+        Offset yoff[2][Cfg::YI], xoff[2][Cfg::XI];
 #pragma unroll
         for (int last = 0; last < 2; ++last) {
             const int rmax = last ? nrows - 1 - (nk - 1) * C : C - 1;
 #pragma unroll
             for (int it = 0; it < Cfg::YI; ++it) {
                 const int r = (wv * Cfg::YI + it) * (512 / TO) + lane / (TO / 8);
-                yoff[last][it] = (unsigned)min(r, rmax) * (unsigned)(Eo * 2) + ((lane % (TO / 8)) ^ rot(r)) * 16;
+                yoff[last][it] = (Offset)min(r, rmax) * ((Offset)Eo * 2) + ((lane % (TO / 8)) ^ rot(r)) * 16;
             }
 #pragma unroll
             for (int it = 0; it < Cfg::XI; ++it) {
                 const int r = (wv * Cfg::XI + it) * (512 / TI) + lane / (TI / 8);
-                xoff[last][it] = (unsigned)min(r, rmax) * (unsigned)(Ei * 2) + ((lane % (TI / 8)) ^ rot(r)) * 16;
+                xoff[last][it] = (Offset)min(r, rmax) * ((Offset)Ei * 2) + ((lane % (TI / 8)) ^ rot(r)) * 16;
             }
         }
+        auto dma = [](const half_t* base, Offset off, half_t* lds) __attribute__((always_inline)) {
+            if constexpr (WIDE) dma16(reinterpret_cast<const char*>(base) + off, lds);
+            else dma16_opaque(base, off, lds);
+        };
         auto load_stage = [&](int kk, int buf) {
             half_t* st = smem + buf * Cfg::kStageHalves;
             const half_t* yb = dyb + (int64_t)kk * C * Eo;
@@ -459,10 +465,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             const bool last = kk == nk - 1;
 #pragma unroll
             for (int it = 0; it < Cfg::YI; ++it)
-                dma16_opaque(yb, last ? yoff[1][it] : yoff[0][it], st + (wv * Cfg::YI + it) * 512);
+                dma(yb, last ? yoff[1][it] : yoff[0][it], st + (wv * Cfg::YI + it) * 512);
 #pragma unroll
             for (int it = 0; it < Cfg::XI; ++it)
-                dma16_opaque(xk, last ? xoff[1][it] : xoff[0][it], st + C * TO + (wv * Cfg::XI + it) * 512);
+                dma(xk, last ? xoff[1][it] : xoff[0][it], st + C * TO + (wv * Cfg::XI + it) * 512);
         };
 #pragma unroll
         for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);

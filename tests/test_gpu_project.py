@@ -288,6 +288,26 @@ def test_linear_weight_gradient_of_an_infinity_in_the_last_row(R):
     assert torch.equal(dw.double().cpu(), want)
 
 
+@pytest.mark.parametrize("wide_input", [True, False])
+def test_linear_weight_gradient_wider_than_32_bit_offsets(wide_input):
+    """The rows of a step (32) of a matrix 69 * 2^20 wide span more than 4 GiB: dW and db exactly (whole numbers)."""
+    from rfa_amd import rfa_hip
+    E, R = 69 << 20, 33
+    gen = torch.Generator("cuda").manual_seed(69)
+    print(f"wide weight gradient, wide_input={wide_input}", flush=True)
+    big = torch.randint(-1, 2, (R, E), generator=gen, device="cuda", dtype=torch.int8).half()
+    small = torch.randint(-1, 2, (R, 128), generator=gen, device="cuda", dtype=torch.int8).half()
+    x, dy = (big, small) if wide_input else (small, big)
+    (dw,), (db,) = rfa_hip.linear_weight_grad(x, [dy], [True])
+    assert torch.equal(db, dy.float().sum(0).half())
+    for c in range(0, E, 3 << 20):
+        cut = slice(c, c + (3 << 20))
+        if wide_input:
+            assert torch.equal(dw[:, cut], (dy.float().t() @ x[:, cut].float()).half())
+        else:
+            assert torch.equal(dw[cut], (dy[:, cut].t().float() @ x.float()).half())
+
+
 @pytest.mark.parametrize("R", [98, 128, 129, 257, 449, 600, 2000])
 @pytest.mark.parametrize("e_out,e_in,n", [(128, 128, 1), (256, 384, 2), (512, 512, 3)])
 def test_linear_weight_gradient_of_few_rows(R, e_out, e_in, n):
