@@ -162,6 +162,7 @@ int rfa_causal_num_segments(int64_t T, int64_t N, int K, int d);
  *   "nseg_same"  1: the K = 256, d = 128 backward keeps the forward's segment length
  *   "free_wg"  workgroups the cross-attention readout and state backward aim for
  *   "project_streaming"  rows per tile of rfa_project_feature_map for every shape: 0 -> 64, 1 -> 256, 2 -> 128
+ *             (the name is older than the meaning: it chose between two kernels, of which one is left)
  *   "sliced"  1/0: rfa_causal_forward_save writes the final-state layout, whose backward is one
  *             launch that walks whole sequences by state slices (K <= 128; taken by itself at
  *             d = 64 when the slices cover 45 % of the compute units, at d = 128 only with K = 128

@@ -542,7 +542,7 @@ def test_linear_rows(R, e_in, e_out):
         for bias in (b, None):
             y = projection.linear_rows(x, w, bias)
             ref = want if bias is None else want + b.double()
-            if R * e_in * e_out > 1 << 31 or ((R > 256 or R * e_in * e_out > 300 << 20) and (e_in % 64 or e_out % 64)):
+            if R * e_in * e_out > 1 << 31 or (R > 256 and (e_in % 64 or e_out % 64)):
                 assert y is None        # the library's
                 continue
             assert ((y.double() - ref).abs() <= 2.0 ** -10 * ref.abs() + 2e-5).all()
