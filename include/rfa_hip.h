@@ -161,7 +161,8 @@ int rfa_causal_num_segments(int64_t T, int64_t N, int K, int d);
  *   "prefix"  1/0: consumers read pre-scanned segment totals / add the totals up themselves
  *   "nseg_same"  1: the K = 256, d = 128 backward keeps the forward's segment length
  *   "free_wg"  workgroups the cross-attention readout and state backward aim for
- *   "project_streaming"  rows per tile of rfa_project_feature_map for every shape: 0 -> 64, 1 -> 256, 2 -> 128
+ *   "project_streaming"  rows per tile of rfa_project_feature_map for every shape: 0 -> 64, 1 -> 256, 2 -> 128, 3 -> 128
+ *             with two groups of waves that share the tile's contraction (0 has two as well)
  *             (the name is older than the meaning: it chose between two kernels, of which one is left)
  *   "sliced"  1/0: rfa_causal_forward_save writes the final-state layout, whose backward is one
  *             launch that walks whole sequences by state slices (K <= 128; taken by itself at

@@ -778,42 +778,54 @@ int launch_decode(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t*
 }
 
 // ---- projection launcher -----------------------------------------------------------
-template <int D, int DH, int BM>
+// Rows of a tile and the groups of waves that share its contraction, for the kernels that walk `steps` of 32 per tile of
+// `rows` x 128.  While every CU has at most one tile, a step is a chain of a barrier, operand reads and products that
+// nothing else on the CU hides: two groups of waves that walk half the steps each do (four where the contraction is
+// long enough for their sum at the end and the tile low enough for their registers).  With more tiles than CUs, two or
+// three workgroups per CU hide each other's steps, and one group reads the fewest operand bytes.
+struct TileShape { int rows, groups; };
+
+template <int D, int DH, int BM, int KG>
 int launch_project_tiles(const rfa::half_t* x, const rfa::ProjectArgs& pa, const rfa::half_t* wf, int R, int E, int H,
                          int np, float scale, hipStream_t st) {
-    using Cfg = rfa::ProjectCfg<D, DH, BM>;
-    auto kern = rfa::k_project_phi<D, DH, BM>;
+    using Cfg = rfa::ProjectCfg<D, DH, BM, KG>;
+    auto kern = rfa::k_project_phi<D, DH, BM, KG>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     const int tiles_c = (H * np + Cfg::PPT - 1) / Cfg::PPT;
     const int64_t tiles = (int64_t)((R + BM - 1) / BM) * tiles_c;
     const int64_t grid = rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds);
-    RFA_LAUNCH(PROJECT_PHI, kern, dim3((unsigned)grid), dim3(rfa::kThreads), Cfg::kLds, st, x, pa, wf, R, E, H, np, tiles_c,
+    RFA_LAUNCH(PROJECT_PHI, kern, dim3((unsigned)grid), dim3(rfa::kThreads * KG), Cfg::kLds, st, x, pa, wf, R, E, H, np, tiles_c,
                (int)tiles, scale);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
 
-// Rows per tile.  256 rows read the fewest operand bytes per product; a lower tile has more workgroups
-// and a shorter epilogue, but stages w' for fewer rows: 64 until 128 gives every CU a tile, then 128
-// until the busiest CU would have 5/3 as many tiles of 128 as of 256 (5/4 where w' is the larger
-// operand, D > d).  Measured, us for 256 / 128 / 64 rows (tiles of 256 in brackets):
-// 8192 x 512 -> 3 x 512 (384) 30.1 / 28.2 / 35; 16384 x 512 -> 2 x 512 (512) 33.3 / 36.7 / 43;
-// 8192 x 1024 -> 3 x 1024 (768) 82.6 / 88 / 121; 4096 x 768 -> 3 x 768, D 128 (288) 35.2 / 39.7 / 49;
-// 8192 x 512 -> 512 (128) 19.9 / 14.3 / 14.4; 1024 x 1024 -> 3 x 1024 (96) 28.2 / 20.4 / 19.6;
-// 512 x 512 -> 3 x 512 (24) 18.0 / 12.1 / 9.6; 160 x 512 -> 512 (4) 17.0 / 11.3 / 8.5.
+// 64 rows by two groups while those tiles are at most one to a CU, then 128 by two groups likewise; then 128 rows
+// until the busiest CU would have 5/3 as many tiles of 128 as of 256 (5/4 where w' is the larger operand, D > d).
+// Measured, us (tiles of 64 rows in brackets) for 64 rows, one group / 64, two / 128, one / 128, two / 256:
+// 512 x 512 -> 3 x 512 (96) 8.8 / 7.5 / 11.6 / 10.5 / 17.8; 2048 x 512 -> 3 x 512 (384) 12.9 / 12.7 / 13.5 / 12.5 / 19.5;
+// 4096 x 512 -> 512 (256) 7.4 / 6.6 / 9.4 / 8.7 / 13.5; 8192 x 512 -> 512 (512) 10.5 / 9.9 / 10.3 / 9.7 / 14.5;
+// 4096 x 1024 -> 1024 (512) 17.5 / 15.3 / 16.2 / 13.9 / 23.2; 512 x 1024 -> 3 x 1024, D 128 (192) 16.0 / 13.5 / 18.9 / 15.3 /
+// 26.9; 8192 x 512 -> 3 x 512 (1536) 39.3 / 32.5 / 29.9 / 34.1 / 32.0; 8192 x 1024 -> 3 x 1024 (3072) 117 / 111 / 88 / 95 / 78.
+TileShape project_shape(int64_t R, int E, int64_t tiles_c, bool wide_features) {
+    const int knob = tune::get(tune::PROJECT_STREAMING);
+    if (E > (1 << 23)) return {64, 2};      // the rows of a tile are addressed with 32-bit byte offsets
+    if (knob >= 0) return knob == 0 ? TileShape{64, 2} : knob == 1 ? TileShape{256, 1} : knob == 2 ? TileShape{128, 1} : TileShape{128, 2};
+    const int64_t cus = device_cus(), t64 = (R + 63) / 64 * tiles_c, t128 = (R + 127) / 128 * tiles_c, t256 = (R + 255) / 256 * tiles_c;
+    if (t64 <= cus) return {64, 2};
+    if (t128 <= cus) return {128, 2};
+    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= (wide_features ? 4 : 3) * ((t128 + cus - 1) / cus)) return {256, 1};
+    return {128, 1};
+}
+
 template <int D, int DH>
 int launch_project_phi(const rfa::half_t* x, const rfa::ProjectArgs& pa, const rfa::half_t* wf, int R, int E, int H,
                        int np, float scale, hipStream_t st) {
-    const int knob = tune::get(tune::PROJECT_STREAMING);
-    const int64_t tiles_c = ((int64_t)H * np * DH + 127) / 128;
-    const int64_t cus = device_cus(), t128 = (int64_t)((R + 127) / 128) * tiles_c, t256 = (int64_t)((R + 255) / 256) * tiles_c;
-    int rows = t128 < cus ? 64 : 128;
-    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= (D > DH ? 4 : 3) * ((t128 + cus - 1) / cus)) rows = 256;
-    if (knob >= 0) rows = knob == 0 ? 64 : (knob == 1 ? 256 : 128);
-    if (E > (1 << 23)) rows = 64;      // the rows of a tile are addressed with 32-bit byte offsets
-    if (rows == 256) return launch_project_tiles<D, DH, 256>(x, pa, wf, R, E, H, np, scale, st);
-    if (rows == 128) return launch_project_tiles<D, DH, 128>(x, pa, wf, R, E, H, np, scale, st);
-    return launch_project_tiles<D, DH, 64>(x, pa, wf, R, E, H, np, scale, st);
+    const TileShape t = project_shape(R, E, ((int64_t)H * np * DH + 127) / 128, D > DH);
+    if (t.rows == 256) return launch_project_tiles<D, DH, 256, 1>(x, pa, wf, R, E, H, np, scale, st);
+    if (t.rows == 64) return launch_project_tiles<D, DH, 64, 2>(x, pa, wf, R, E, H, np, scale, st);
+    if (t.groups == 2) return launch_project_tiles<D, DH, 128, 2>(x, pa, wf, R, E, H, np, scale, st);
+    return launch_project_tiles<D, DH, 128, 1>(x, pa, wf, R, E, H, np, scale, st);
 }
 
 // ---- weight-gradient plan -------------------------------------------------------------
@@ -846,17 +858,32 @@ WGradPlan make_wgrad_plan(int64_t R, int Eo, int Ei, int np) {
 }
 
 // ---- input-gradient launcher ----------------------------------------------------------
-template <int BM>
+template <int BM, int KG>
 int launch_input_grad(const rfa::InputGradArgs& ga, rfa::half_t* dx, int R, int Eo, int Ei, int np, int64_t ld,
-                             hipStream_t st) {
-    using Cfg = rfa::InputGradCfg<BM>;
-    auto kern = rfa::k_input_grad<BM>;
+                      hipStream_t st) {
+    using Cfg = rfa::InputGradCfg<BM, KG>;
+    auto kern = rfa::k_input_grad<BM, KG>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     const int64_t tiles = (int64_t)((R + BM - 1) / BM) * (Ei / Cfg::BN);
-    RFA_LAUNCH(INPUT_GRAD, kern, dim3((unsigned)(rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds))), dim3(rfa::kThreads),
-               Cfg::kLds, st, ga, dx, R, Eo, Ei, np, ld, (int)tiles);
+    RFA_LAUNCH(INPUT_GRAD, kern, dim3((unsigned)(rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds))),
+               dim3(rfa::kThreads * KG), Cfg::kLds, st, ga, dx, R, Eo, Ei, np, ld, (int)tiles);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
+}
+
+// As the projections, with four groups for 64 rows where the contraction is 768 or longer; a group's columns divide each
+// layer's E_out.  Measured, us for 64 rows by one group / two / four, 128 by one / two, 256:
+// 512 rows of 512 -> 512 7.8 / 6.8 / 7.0 / 10.2 / 8.9 / 14.8; 512 of 3 x 512 17.5 / 12.9 / 11.6 / 22.5 / 16.7 / 32.2; 2048 of
+// 3 x 1024 32.7 / 23.9 / 21.9 / 41.4 / 29.6 / 58.6; 4096 of 3 x 768 31.9 / 27.5 / 31.7 / 33.5 / 25.4 / 46.0; 8192 of 512 11.2 /
+// 11.7 / 14.7 / 11.8 / 10.6 / 16.4, of 3 x 512 25.1 / 23.0 / 25.6 / 25.1 / 19.9 / 34.3, of 3 x 1024 80 / 72 / 83 / 63 / 67 / 67.
+TileShape input_grad_shape(int64_t R, int Eo, int Ei, int np) {
+    const int64_t cus = device_cus(), tiles_c = Ei / 128;
+    const int64_t t64 = (R + 63) / 64 * tiles_c, t128 = (R + 127) / 128 * tiles_c, t256 = (R + 255) / 256 * tiles_c;
+    if (Eo % 64 != 0 && t128 < cus) return {64, 1};
+    if (t64 <= cus) return {64, Eo % 128 == 0 && np * Eo >= 768 ? 4 : 2};
+    if (t128 <= cus && Eo % 64 == 0) return {128, 2};
+    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= 3 * ((t128 + cus - 1) / cus)) return {256, 1};
+    return {128, 1};
 }
 
 // ---- feature map launchers ---------------------------------------------------------
@@ -2090,13 +2117,17 @@ int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* 
         return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: sizes exceed the supported range");
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto* dxh = static_cast<rfa::half_t*>(dx);
-    // rows per tile as launch_project_phi chooses them
-    const int64_t cus = device_cus(), t128 = (R + 127) / 128 * (E_in / 128), t256 = (R + 255) / 256 * (E_in / 128);
-    int rows = t128 < cus ? 64 : 128;
-    if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= 3 * ((t128 + cus - 1) / cus)) rows = 256;
-    if (rows == 256) return launch_input_grad<256>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
-    if (rows == 128) return launch_input_grad<128>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
-    return launch_input_grad<64>(ga, dxh, (int)R, E_out, E_in, np, ld, st);
+    const TileShape t = input_grad_shape(R, E_out, E_in, np);
+#define RFA_DX(BM, KG) \
+    if (t.rows == BM && t.groups == KG) return launch_input_grad<BM, KG>(ga, dxh, (int)R, E_out, E_in, np, ld, st)
+    RFA_DX(64, 1);
+    RFA_DX(64, 2);
+    RFA_DX(64, 4);
+    RFA_DX(128, 1);
+    RFA_DX(128, 2);
+    RFA_DX(256, 1);
+#undef RFA_DX
+    return fail(RFA_ERR_UNSUPPORTED, "unreachable");
 }
 
 int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw, void* const* db, int np, int64_t R,

@@ -35,24 +35,84 @@ __device__ __forceinline__ T pick3(T const (&a)[kMaxProjections], int p) {
     return p == 0 ? a[0] : (p == 1 ? a[1] : a[2]);
 }
 
-template <int D, int DH, int BM_>
+// A stage array whose rows are 32 KG halves of the contraction (KG groups of waves side by side), stored without
+// padding (a direct load writes 1 KiB in lane order): the 16-byte pieces of row r are stored rotated, piece c at slot
+// c ^ (r's number within 256 bytes' worth of rows), which spreads a wave's operand read (16 rows x 16 bytes per 16 lanes)
+// over all banks.  slot() is its own inverse.
+template <int KG>
+struct StageRows {
+    static constexpr int kSlots = 4 * KG;
+    static __device__ __forceinline__ int slot(int r, int c) { return c ^ ((r / (4 / KG)) % kSlots); }
+};
+
+// Sums of one tile over KG groups of four waves, each of which walked its own share of the contraction: wave w of every
+// group holds the same tiles acc[NR][NC].  Group g < kFin leaves with own[l] = the sum of acc[kFin l + g] over all groups
+// (its own first, then the others in order); the rest have nothing left to do.  One workgroup barrier, all groups call.
+template <int NR, int NC, int KG>
+struct GroupSum {
+    static constexpr int kFin = KG > 1 && NR % 2 == 0 ? 2 : 1;
+    static constexpr int kOwn = NR / kFin;
+    static constexpr size_t kLds = (size_t)(KG - 1) * NR * NC * kThreads * 16;
+    static __device__ __forceinline__ void run(const f4 (&acc)[NR][NC], f4 (&own)[kOwn][NC], unsigned char* lds, int kg, int tid) {
+        if constexpr (KG == 1) {
+#pragma unroll
+            for (int a = 0; a < NR; ++a)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) own[a][c] = acc[a][c];
+        } else {
+            // [finishing group][other group, in order][tile][thread]
+            f4* const red = reinterpret_cast<f4*>(lds) + tid;
+            auto slot = [&](int fin, int g) { return red + (fin * (KG - 1) + (g < fin ? g : g - 1)) * (kOwn * NC * kThreads); };
+#pragma unroll
+            for (int o = 0; o < kFin; ++o) {
+                if (kg == o) continue;
+                f4* const to = slot(o, kg);
+#pragma unroll
+                for (int l = 0; l < kOwn; ++l)
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) to[(l * NC + c) * kThreads] = acc[kFin * l + o][c];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int l = 0; l < kOwn; ++l)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const f4 first = acc[kFin * l][c], second = acc[kFin * l + kFin - 1][c];     // values: no indexed registers
+                    own[l][c] = kg == 1 ? second : first;
+                }
+            if (kg < kFin) {
+                const f4* const from = red + kg * (KG - 1) * (kOwn * NC * kThreads);
+#pragma unroll
+                for (int j = 0; j < KG - 1; ++j)
+#pragma unroll
+                    for (int l = 0; l < kOwn; ++l)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) own[l][c] += from[(j * kOwn * NC + l * NC + c) * kThreads];
+            }
+        }
+    }
+};
+
+template <int D, int DH, int BM_, int KG_ = 1>
 struct ProjectCfg {
     static_assert(D % 32 == 0 && (DH == 64 || DH == 128), "D multiple of 32, DH 64 or 128");
     static constexpr int BM = BM_;                 // rows of x per workgroup
     static constexpr int BN = 128;                 // output columns: one head of 128 or two of 64
     static constexpr int BK = 32;                  // contraction step: one MFMA deep
-    static constexpr int kStages = 3;              // 4 to 6 measured no faster at any size
+    static constexpr int kStages = 3;              // 4 to 6 measured no faster at any size, with any number of groups
     static constexpr int PPT = BN / DH;            // heads per tile
     static constexpr int WR = 4 / PPT;             // waves along the rows; a wave owns whole heads
     static constexpr int RW = BM / WR;             // rows of a wave
     static constexpr int NR = RW / 16, NC = DH / 16;
     static constexpr int XI = BM / 64, WI = BN / 64;    // 1 KiB pieces of a stage per wave: x, W
+    static constexpr int KG = KG_;                 // groups of four waves that share a tile's contraction
     static constexpr int kStageHalves = (BM + BN) * BK;
     static constexpr int LDW = DH + lds_pad(DH);   // rows of w'
-    static constexpr size_t kLoopLds = (size_t)kStages * kStageHalves * 2;
-    static constexpr size_t kEpiLds = (size_t)PPT * D * LDW * 2;
+    using Sum = GroupSum<NR, NC, KG>;
+    static constexpr size_t kLoopLds = (size_t)kStages * KG * kStageHalves * 2;
+    static constexpr size_t kEpiLds = Sum::kLds + (size_t)PPT * D * LDW * 2;
     static constexpr size_t kLds = kLoopLds > kEpiLds ? kLoopLds : kEpiLds;
-    static_assert(kLds <= 80 * 1024, "two workgroups per CU");
+    static_assert(kLds <= (KG == 1 ? 80 : 160) * 1024, "two workgroups per CU, one of several groups");
 };
 
 // 64 lanes x 16 bytes, global -> LDS without registers: lane l's bytes land at lds + 16 l
@@ -84,32 +144,36 @@ __device__ __forceinline__ void stage_barrier() {
 // ring, one barrier per step; two (256 rows) or three (128) workgroups share a CU, so that one's
 // epilogue runs under another's products.  A wave owns BM / 2 rows x 64 columns (or BM / 4 x 128):
 // with 256 rows 12 operand reads for 32 MFMAs, 48 KB of LDS traffic per 512 clocks of the matrix pipes.
+// Where there is at most one tile to a CU nothing hides a step (0.3 us at 64 rows: barrier, direct loads of 18 bytes a
+// clock, operand reads, products, one after the other), so KG = 2 groups of four waves take 32 columns each of a stage of
+// 64: whole 128-byte lines, half the steps, 26 bytes a clock; the groups' sums meet in LDS.
 //
 // Measured (us; q, k, v projections with phi(q), phi(k); before: rows of x in registers for E <= 512,
 // a register-staged two-buffer loop otherwise):
 //   8192 rows, E 512, 8 heads of 64, D 64       42.1 -> 28.2      8192, 1024, 8 of 128, D 128   112 -> 83
-//   32768, 1024, 16 of 64, D 64                  964 -> 304 (678 TFLOP/s)      512, 512   12.4 -> 9.6
+//   32768, 1024, 16 of 64, D 64                  964 -> 304 (678 TFLOP/s)      512, 512   12.4 -> 9.6 -> 7.5 (two groups)
+//   one projection without phi: 4096, 512 7.4 -> 6.6; 2048, 1024 11.3 -> 9.1 (two groups)
 //
-// LDS stage: x tile [BM][32], then W tile [128][32] halves, no padding (a direct load writes 1 KiB
-// in lane order); the four 16-byte pieces of row r are stored rotated, piece c at c ^ ((r >> 2) & 3),
-// which spreads a wave's operand read (16 rows x 16 bytes per 16 lanes) over all banks.  The rows of
+// LDS stage: x tile [BM][32 KG], then W tile [128][32 KG] halves (StageRows).  The rows of
 // W sit in pair order (pair_pos), so that accumulator tiles 2p, 2p + 1 give lane (i, G) the 8
 // consecutive columns 32 p + 8 G of row i: y goes out in 16-byte pieces, is the operand of the
 // feature product as it stands, and phi goes out the same way; nothing passes through LDS again.
 //
 // Tiles are numbered row tile by row tile; each XCD gets a contiguous range of numbers, so that
 // the tiles that share rows of x meet in its L2.   grid = 8 * ceil(tiles / 8).
-template <int D, int DH, int BM_>
-__global__ __launch_bounds__(kThreads, 2) void k_project_phi(
+template <int D, int DH, int BM_, int KG>
+__global__ __launch_bounds__(kThreads * KG, 2) void k_project_phi(
     const half_t* __restrict__ x, ProjectArgs pa, const half_t* __restrict__ wf, int R, int E, int H, int np,
     int tiles_c, int tiles, float scale) {
-    using Cfg = ProjectCfg<D, DH, BM_>;
+    using Cfg = ProjectCfg<D, DH, BM_, KG>;
+    using Sum = typename Cfg::Sum;
     constexpr int BM = Cfg::BM, BK = Cfg::BK, STAGES = Cfg::kStages, NR = Cfg::NR, NC = Cfg::NC, LDW = Cfg::LDW;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);      // wave inside its group
+    half_t* const smem = reinterpret_cast<half_t*>(smem_raw);
     const int i = lane & 15, G = lane >> 4;
 
     const int per_xcd = (tiles + kXcds - 1) / kXcds;
@@ -119,33 +183,39 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
     const int hp0 = (tile % tiles_c) * Cfg::PPT;       // (projection, head) pairs: hp -> hp / H, hp % H
     const int pairs = H * np;
 
-    // ---- direct-load addresses: wave-uniform base + 32-bit lane offset, set up once
+    // ---- direct-load addresses: wave-uniform base + 32-bit lane offset, set up once.  A load covers 64 / kSlots rows.
+    using Rows = StageRows<KG>;
+    constexpr int SK = BK * KG, RPL = 64 / Rows::kSlots;      // columns of a stage; rows of one load
+    const int wave = kg * 4 + wv;
     const char* xbase = reinterpret_cast<const char*>(x + (int64_t)row0 * E);
     unsigned xoff[Cfg::XI], woff[Cfg::WI];
 #pragma unroll
     for (int it = 0; it < Cfg::XI; ++it) {
-        const int r = (wv * Cfg::XI + it) * 16 + (lane >> 2);
-        xoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(E * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+        const int r = (wave * Cfg::XI + it) * RPL + lane / Rows::kSlots;
+        xoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(E * 2) + Rows::slot(r, lane % Rows::kSlots) * 16;
     }
-    // W rows 32 wv .. of the tile: 32-row groups never straddle a head
-    const int hp_ld = min(hp0 + 32 * wv / DH, pairs - 1);
+    // W rows of this wave: 32 / KG of them, never across a 32-row group or a head
+    constexpr int WRW = 32 / KG;
+    const int wrow0 = WRW * wave / 32 * 32;            // first row of the 32-row group
+    const int hp_ld = min(hp0 + wrow0 / DH, pairs - 1);
     const char* wbase = reinterpret_cast<const char*>(
-        pick3(pa.w, hp_ld / H) + ((int64_t)(hp_ld % H) * DH + (32 * wv) % DH) * E);
+        pick3(pa.w, hp_ld / H) + ((int64_t)(hp_ld % H) * DH + wrow0 % DH) * E);
 #pragma unroll
     for (int it = 0; it < Cfg::WI; ++it) {
-        const int r = it * 16 + (lane >> 2);           // LDS row within the group; it holds column pair_inv
+        const int r = WRW * wave - wrow0 + it * RPL + lane / Rows::kSlots;      // LDS row within the group; it holds column pair_inv
         const int c = (r & 3) | ((r & 16) >> 2) | ((r & 12) << 1);
-        woff[it] = (unsigned)c * (unsigned)(E * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+        woff[it] = (unsigned)c * (unsigned)(E * 2) + Rows::slot(wrow0 + r, lane % Rows::kSlots) * 16;
     }
-    half_t* const xdst = smem + wv * Cfg::XI * 512;
-    half_t* const wdst = smem + BM * BK + wv * Cfg::WI * 512;
-    auto load_stage = [&](int kk, int buf) {
-        const char* xb = xbase + (int64_t)kk * (BK * 2);
-        const char* wb = wbase + (int64_t)kk * (BK * 2);
+    half_t* const xdst = smem + wave * Cfg::XI * 512;
+    half_t* const wdst = smem + BM * SK + wave * Cfg::WI * 512;
+    constexpr int kRing = KG * Cfg::kStageHalves;      // halves from one stage to the next
+    auto load_stage = [&](int step, int buf) {
+        const char* xb = xbase + (int64_t)step * (SK * 2);
+        const char* wb = wbase + (int64_t)step * (SK * 2);
 #pragma unroll
-        for (int it = 0; it < Cfg::XI; ++it) dma16(xb + xoff[it], xdst + buf * Cfg::kStageHalves + it * 512);
+        for (int it = 0; it < Cfg::XI; ++it) dma16(xb + xoff[it], xdst + buf * kRing + it * 512);
 #pragma unroll
-        for (int it = 0; it < Cfg::WI; ++it) dma16(wb + woff[it], wdst + buf * Cfg::kStageHalves + it * 512);
+        for (int it = 0; it < Cfg::WI; ++it) dma16(wb + woff[it], wdst + buf * kRing + it * 512);
     };
     constexpr int kPerStage = Cfg::XI + Cfg::WI;
 
@@ -157,12 +227,12 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[a][c] = f4_zero();
 
-    // operand rows of this lane inside a stage: row (16 t + i), piece G
-    const int piece = (G ^ ((i >> 2) & 3)) * 8;
-    const half_t* const xop = smem + (wr * Cfg::RW + i) * BK + piece;
-    const half_t* const wop = smem + BM * BK + (wc * DH + i) * BK + piece;
+    // operand rows of this lane inside a stage: row (16 t + i), piece G of its group's columns
+    const int piece = Rows::slot(i, 4 * kg + G) * 8;
+    const half_t* const xop = smem + (wr * Cfg::RW + i) * SK + piece;
+    const half_t* const wop = smem + BM * SK + (wc * DH + i) * SK + piece;
 
-    const int nk = E / BK;
+    const int nk = E / (BK * KG);       // KG divides the steps
 #pragma unroll
     for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
     int buf = 0;
@@ -171,13 +241,13 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
         stage_barrier<(STAGES - 2) * kPerStage>();
         // the last steps re-request the last stage's columns into buffers nobody reads again
         load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
-        const half_t* xs = xop + buf * Cfg::kStageHalves;
-        const half_t* wsm = wop + buf * Cfg::kStageHalves;
+        const half_t* xs = xop + buf * kRing;
+        const half_t* wsm = wop + buf * kRing;
         h8 wa[NC], xb[NR];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) wa[c] = *reinterpret_cast<const h8*>(wsm + c * 16 * BK);
+        for (int c = 0; c < NC; ++c) wa[c] = *reinterpret_cast<const h8*>(wsm + c * 16 * SK);
 #pragma unroll
-        for (int a = 0; a < NR; ++a) xb[a] = *reinterpret_cast<const h8*>(xs + a * 16 * BK);
+        for (int a = 0; a < NR; ++a) xb[a] = *reinterpret_cast<const h8*>(xs + a * 16 * SK);
         __builtin_amdgcn_s_setprio(1);      // the other workgroup's loads and epilogue give way: 2 % at full size
 #pragma unroll
         for (int a = 0; a < NR; ++a)
@@ -187,8 +257,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
         buf = buf == STAGES - 1 ? 0 : buf + 1;
     }
 
-    // ---- epilogue: the ring becomes the place of w' (rows in pair order)
+    // ---- epilogue: the ring becomes the place of the groups' sums and of w' (rows in pair order)
     stage_barrier<0>();
+    half_t* const wfs = reinterpret_cast<half_t*>(smem_raw + Sum::kLds);
     const int hp = hp0 + wc;
     const bool live = hp < pairs;                      // an odd number of 64-wide heads leaves half a tile
     const int hpc = live ? hp : pairs - 1;
@@ -201,7 +272,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
         for (int u = 0; u < Cfg::PPT; ++u) {
             const int hu = min(hp0 + u, pairs - 1);
             if (pick3(pa.phi, hu / H))
-                load_w_pair_order<D, DH, kThreads>(smem + u * D * LDW, wf + (int64_t)(hu % H) * D * DH, tid);
+                load_w_pair_order<D, DH, kThreads * KG>(wfs + u * D * LDW, wf + (int64_t)(hu % H) * D * DH, tid);
         }
     }
     h8 bv[NC / 2];
@@ -214,19 +285,21 @@ __global__ __launch_bounds__(kThreads, 2) void k_project_phi(
             bv[c] = __builtin_shufflevector(b4[0], b4[1], 0, 1, 2, 3, 4, 5, 6, 7);
         }
     }
-    __syncthreads();
-    if (!live) return;
-    const half_t* const Wfs = smem + wc * D * LDW;
+    f4 own[Sum::kOwn][NC];
+    Sum::run(acc, own, smem_raw, kg, tid & (kThreads - 1));
+    if (KG == 1) __syncthreads();
+    if (!live || kg >= Sum::kFin) return;
+    const half_t* const Wfs = wfs + wc * D * LDW;
 #pragma unroll
-    for (int a = 0; a < NR; ++a) {
-        const int r = row0 + wr * Cfg::RW + 16 * a + i;
+    for (int a = 0; a < Sum::kOwn; ++a) {
+        const int r = row0 + wr * Cfg::RW + 16 * (Sum::kFin * a + kg) + i;
         const int64_t at = (int64_t)r * H + h;
         h8 op[NC / 2];       // the rounded row pieces: y as stored, and the operand of the feature product
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < NC / 2; ++c) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) op[c][e] = (half_t)(acc[a][2 * c + e / 4][e % 4] + (float)bv[c][e]);
+            for (int e = 0; e < 8; ++e) op[c][e] = (half_t)(own[a][2 * c + e / 4][e % 4] + (float)bv[c][e]);
             ss += dot_h8(__builtin_bit_cast(uint4, op[c]), __builtin_bit_cast(uint4, op[c]));
         }
         if (y && r < R) {    // NULL: the caller keeps only phi(y) (no backward pass will ask for y)
@@ -533,32 +606,40 @@ struct InputGradArgs {
     const half_t* w[kMaxProjections];
 };
 
-template <int BM_>
+template <int BM_, int KG_ = 1>
 struct InputGradCfg {
     static constexpr int BM = BM_, BN = 128, BK = 32, kStages = 3;
     static constexpr int RW = BM / 2, NR = RW / 16, NC = 4;       // a wave: BM / 2 rows x 64 columns
     static constexpr int YI = BM / 64, WI = 2;                    // 1 KiB pieces of a stage per wave: dy, W
+    static constexpr int KG = KG_;
     static constexpr int kStageHalves = (BM + BN) * BK;
-    static constexpr size_t kLds = (size_t)kStages * kStageHalves * 2;
+    using Sum = GroupSum<NR, NC, KG>;
+    static constexpr size_t kLoopLds = (size_t)kStages * KG * kStageHalves * 2;
+    static constexpr size_t kLds = kLoopLds > Sum::kLds ? kLoopLds : Sum::kLds;
 };
 
 // A tile of BM rows x 128 columns per workgroup of four waves; stages of 32 output columns through the three-stage
 // ring of k_project_phi (dy rows as its x) with W's rows as k_weight_grad_partial stages them: contracted over
 // their row index, read by the transposing read.  The weights are read where they are, no stack of them is
-// formed.  Bound like k_project_phi, by the step (barrier, operand reads, 16 to 32 products) where a tile has few.
-// Measured, us (the library's products over a stacked weight, which costs another 4.6 to 7.8 to form):
-// 8192 rows, 512 -> 512 11.6 (12.3), three of them 24.8 (21.4); 16384 rows, two 28.1 (24.2; 38 as two
-// products); 1024 -> 1024, three 69.3 (57.3).
+// formed.  Bound like k_project_phi, by the step (barrier, operand reads, 16 to 32 products) where a tile has few, by the
+// direct loads (12 TB/s over the chip with 128 x 128 tiles) where 256 of them fill it; KG groups as there.
+// Measured, us, one group -> as chosen (the library's products over a stacked weight, another 4.6 to 7.8 to form):
+// 8192 rows, 512 -> 512 11.8 -> 10.6 (12.3), three of them 25.1 -> 19.9 (21.4); 2048 rows, three of 768 25.3 -> 16.8; 512
+// rows, three of 1024 31.3 -> 19.4 (16.5); 16384 rows, two of 512 28.1 (24.2; 38 as two products); 1024 -> 1024, three 69.3 (57.3).
 // grid = 8 * ceil(tiles / 8), tiles numbered row tile by row tile; each XCD gets a contiguous range.
-template <int BM_>
-__global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, half_t* __restrict__ dx, int R, int Eo, int Ei,
-                                                            int np, int64_t ld, int tiles) {
-    using Cfg = InputGradCfg<BM_>;
+template <int BM_, int KG>
+__global__ __launch_bounds__(kThreads * KG, 2) void k_input_grad(InputGradArgs ga, half_t* __restrict__ dx, int R, int Eo,
+                                                                 int Ei, int np, int64_t ld, int tiles) {
+    using Cfg = InputGradCfg<BM_, KG>;
+    using Sum = typename Cfg::Sum;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, STAGES = Cfg::kStages, NR = Cfg::NR, NC = Cfg::NC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    half_t* smem = reinterpret_cast<half_t*>(smem_raw);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);      // wave inside its group
+    half_t* const smem = reinterpret_cast<half_t*>(smem_raw);
+    constexpr int kRing = KG * Cfg::kStageHalves, SK = BK * KG;      // halves of a stage, its columns of dy
+    using Rows = StageRows<KG>;
     const int i = lane & 15, G = lane >> 4;
     const int wr = wv >> 1, wc = wv & 1;
 
@@ -571,24 +652,24 @@ __global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, ha
     unsigned yoff[Cfg::YI], woff[Cfg::WI];
 #pragma unroll
     for (int it = 0; it < Cfg::YI; ++it) {
-        const int r = (wv * Cfg::YI + it) * 16 + (lane >> 2);
-        yoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(ld * 2) + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+        const int r = ((kg * 4 + wv) * Cfg::YI + it) * (64 / Rows::kSlots) + lane / Rows::kSlots;
+        yoff[it] = (unsigned)min(r, R - 1 - row0) * (unsigned)(ld * 2) + Rows::slot(r, lane % Rows::kSlots) * 16;
     }
 #pragma unroll
     for (int it = 0; it < Cfg::WI; ++it) {
         const int r = (wv * Cfg::WI + it) * 4 + (lane >> 4);
         woff[it] = (unsigned)r * (unsigned)(Ei * 2) + (((lane & 15) ^ (((r & 3) | ((r >> 1) & 4)) * 2)) * 16);
     }
-    const int per_p = Eo / BK, nk = np * per_p;
+    const int per_p = Eo / SK, nk = np * per_p;      // SK divides Eo
     auto load_stage = [&](int kk, int buf) {
-        const int p = kk >= 2 * per_p ? 2 : (kk >= per_p ? 1 : 0), ko = (kk - p * per_p) * BK;
+        const int p = kk >= 2 * per_p ? 2 : (kk >= per_p ? 1 : 0), ko = (kk - p * per_p) * SK;
         const half_t* yb = pick3(ga.dy, p) + (int64_t)row0 * ld + ko;
-        const half_t* wb = pick3(ga.w, p) + (int64_t)ko * Ei + c0;
-        half_t* st = smem + buf * Cfg::kStageHalves;
+        const half_t* wb = pick3(ga.w, p) + (int64_t)(ko + BK * kg) * Ei + c0;
+        half_t* st = smem + buf * kRing;
 #pragma unroll
-        for (int it = 0; it < Cfg::YI; ++it) dma16_opaque(yb, yoff[it], st + (wv * Cfg::YI + it) * 512);
+        for (int it = 0; it < Cfg::YI; ++it) dma16_opaque(yb, yoff[it], st + ((kg * 4 + wv) * Cfg::YI + it) * 512);
 #pragma unroll
-        for (int it = 0; it < Cfg::WI; ++it) dma16_opaque(wb, woff[it], st + BM * BK + (wv * Cfg::WI + it) * 512);
+        for (int it = 0; it < Cfg::WI; ++it) dma16_opaque(wb, woff[it], st + BM * SK + ((kg * 4 + wv) * Cfg::WI + it) * 512);
     };
 
     f4 acc[NR][NC];      // dx^T tiles (m = column, n = row)
@@ -596,7 +677,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, ha
     for (int a = 0; a < NR; ++a)
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[a][c] = f4_zero();
-    const half_t* const yop = smem + (wr * Cfg::RW + i) * BK + (G ^ ((i >> 2) & 3)) * 8;
+    const half_t* const yop = smem + (wr * Cfg::RW + i) * SK + Rows::slot(i, 4 * kg + G) * 8;
 
 #pragma unroll
     for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
@@ -604,13 +685,13 @@ __global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, ha
     for (int kk = 0; kk < nk; ++kk) {
         stage_barrier<(STAGES - 2) * (Cfg::YI + Cfg::WI)>();
         load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
-        const half_t* ys = yop + buf * Cfg::kStageHalves;
-        const half_t* Ws = smem + buf * Cfg::kStageHalves + BM * BK;
+        const half_t* ys = yop + buf * kRing;
+        const half_t* Ws = smem + buf * kRing + BM * SK + kg * BK * BN;
         h8 wa[NC], yb[NR];
 #pragma unroll
         for (int c = 0; c < NC; ++c) wa[c] = col8_rot<BN>(Ws, NC * wc + c, lane);
 #pragma unroll
-        for (int a = 0; a < NR; ++a) yb[a] = *reinterpret_cast<const h8*>(ys + a * 16 * BK);
+        for (int a = 0; a < NR; ++a) yb[a] = *reinterpret_cast<const h8*>(ys + a * 16 * SK);
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int a = 0; a < NR; ++a)
@@ -620,14 +701,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_input_grad(InputGradArgs ga, ha
         buf = buf == STAGES - 1 ? 0 : buf + 1;
     }
     // the last re-requested stages are still on their way into this workgroup's LDS: they land before it ends
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    stage_barrier<0>();
+    f4 own[Sum::kOwn][NC];
+    Sum::run(acc, own, smem_raw, kg, tid & (kThreads - 1));
+    if (kg >= Sum::kFin) return;
 #pragma unroll
-    for (int a = 0; a < NR; ++a) {
-        const int r = row0 + wr * Cfg::RW + 16 * a + i;
+    for (int a = 0; a < Sum::kOwn; ++a) {
+        const int r = row0 + wr * Cfg::RW + 16 * (Sum::kFin * a + kg) + i;
         if (r < R) {
 #pragma unroll
             for (int c = 0; c < NC; ++c)
-                *reinterpret_cast<h4*>(dx + (int64_t)r * Ei + c0 + 64 * wc + 16 * c + 4 * G) = to_h4(acc[a][c]);
+                *reinterpret_cast<h4*>(dx + (int64_t)r * Ei + c0 + 64 * wc + 16 * c + 4 * G) = to_h4(own[a][c]);
         }
     }
 }

@@ -90,6 +90,14 @@ def test_projection_tile_edges(R, E, H, d, D, n, rows_knob, knobs):
             assert (phis[p].float().cpu() - own).abs().max().item() <= 2e-3
 
 
+# the same edges with two groups of waves to a tile: one stage of 64 columns, two, an odd number, more than the ring holds
+@pytest.mark.parametrize("rows_knob", [0, 3])
+@pytest.mark.parametrize("R,E,H,d,D,n", [(1, 64, 1, 64, 32, 1), (65, 128, 3, 64, 128, 3), (127, 192, 1, 128, 128, 2), (129, 64, 2, 128, 64, 1),
+                                         (257, 320, 5, 64, 64, 2), (500, 512, 2, 128, 32, 3)])
+def test_projection_by_two_groups(R, E, H, d, D, n, rows_knob, knobs):
+    test_projection_tile_edges(R, E, H, d, D, n, rows_knob, knobs)
+
+
 @pytest.mark.parametrize("streaming", [False, True])
 def test_projection_without_keeping_y(streaming, knobs):
     """keep_y=False (what the modules ask for when nothing requires a gradient): phi and the plain
