@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -106,6 +107,7 @@ const char* const kEnv[COUNT] = {"RFA_HIP_NSEG", "RFA_HIP_PREFIX", "RFA_HIP_NSEG
                                  "RFA_HIP_PROJECT_STREAMING", "RFA_HIP_SLICED", "RFA_HIP_RECOMPUTE",
                                  "RFA_HIP_PREFIX_COST", "RFA_HIP_FEATURE_WG"};
 std::atomic<int> value[COUNT];
+std::atomic<unsigned> changes{0};      // rfa_tuning_set calls: what was derived from the knobs before is stale
 std::once_flag once;
 
 void init() {
@@ -171,16 +173,19 @@ enum SavedLayout { LAYOUT_SEGMENTS = 0, LAYOUT_FINAL = 1 };
 
 bool sliced_supported(int K, int d) { return (K == 64 || K == 128) && (d == 64 || d == 128); }
 
+// a kernel exists, and its loader addresses the 64 rows of a chunk with 32-bit byte offsets
+bool sliced_addressable(int64_t N, int K, int d) {
+    return sliced_supported(K, d) && (int64_t)rfa::kChunk * N * (K > d ? K : d) * 2 < ((int64_t)1 << 32);
+}
+
 // The sliced backward has N * (K / 64 + d / 64) workgroups that never wait for each other, each
-// walking a whole sequence.  Taken when they cover enough of the compute units ("sliced" knob: 0
+// walking a whole sequence.  For long sequences it is taken when they cover enough of the compute units ("sliced" knob: 0
 // never, 1 whenever a kernel exists).  Measured against the two time-segmented sweeps at T = 1024:
 // d = 64, K = 128 wins from 120 workgroups on (N = 40: 34.8 vs 37.3 us, N = 64: 34 vs 43, N = 512:
 // 262 vs 285); d = 128 wins with K = 128 at 256 workgroups (60 vs 67 us) and loses with K = 64 at
 // 192 (54 vs 50 us).
 int choose_saved_layout(int64_t N, int K, int d) {
-    if (!sliced_supported(K, d)) return LAYOUT_SEGMENTS;
-    // its loader addresses the 64 rows of a chunk with 32-bit byte offsets
-    if ((int64_t)rfa::kChunk * N * (K > d ? K : d) * 2 >= ((int64_t)1 << 32)) return LAYOUT_SEGMENTS;
+    if (!sliced_addressable(N, K, d)) return LAYOUT_SEGMENTS;
     const int knob = tune::get(tune::SLICED);
     if (knob >= 0) return knob ? LAYOUT_FINAL : LAYOUT_SEGMENTS;
     const int64_t wgs = N * (K / rfa::kSliceWidth + d / rfa::kSliceWidth), cus = device_cus();
@@ -198,29 +203,161 @@ bool use_scanned_totals(int nseg, int K, int d) {
     return (int64_t)(nseg - 1) * K * d * 2 >= 128 * 1024;
 }
 
-// Enough (sequence, segment) workgroups to cover the compute units, at least two
-// chunks per segment, at most 16 segments (the consumer sums the totals of all
-// earlier segments).
-ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
+// The cut into `want` segments or the nearest number that the chunks allow.
+void cut_segments(ScanPlan* p, int64_t T, int64_t want, int K, int d) {
+    const int64_t nchunks = (T + rfa::kChunk - 1) / rfa::kChunk;
+    if (want > rfa::kMaxSegments) want = rfa::kMaxSegments;
+    if (want > nchunks) want = nchunks;
+    if (want < 1) want = 1;
+    const int64_t cps = (nchunks + want - 1) / want;
+    p->nseg = (int)((nchunks + cps - 1) / cps);
+    p->seg_len = (int)(cps * rfa::kChunk);
+    p->prefixed = use_scanned_totals(p->nseg, K, d) ? 1 : 0;
+}
+
+// Enough (sequence, segment) workgroups to cover the compute units, at least two chunks per segment, at most 16 segments:
+// what the pair without a saved buffer and the forward on static memory run with (their buffers are sized by it), and
+// where the choice of make_plan starts.
+ScanPlan cover_plan(int64_t T, int64_t N, int K, int d) {
     ScanPlan p{1, rfa::kChunk, 0, LAYOUT_SEGMENTS};
     if (T <= 0 || N <= 0) return p;
     p.layout = choose_saved_layout(N, K, d);
     const int64_t nchunks = (T + rfa::kChunk - 1) / rfa::kChunk;
     int64_t want = (device_cus() + N - 1) / N;
     const int knob = tune::get(tune::NSEG);
-    if (knob >= 1) {
-        want = knob;
-    } else {
-        if (want > nchunks / 2) want = nchunks / 2;
-    }
-    if (want > rfa::kMaxSegments) want = rfa::kMaxSegments;
-    if (want > nchunks) want = nchunks;
-    if (want < 1) want = 1;
-    const int64_t cps = (nchunks + want - 1) / want;
-    p.nseg = (int)((nchunks + cps - 1) / cps);
-    p.seg_len = (int)(cps * rfa::kChunk);
-    p.prefixed = use_scanned_totals(p.nseg, K, d) ? 1 : 0;
+    if (knob >= 1) want = knob;
+    else if (want > nchunks / 2) want = nchunks / 2;
+    cut_segments(&p, T, want, K, d);
     return p;
+}
+
+// The forward without segment totals (k_causal_fwd_pipe<.., RECOMPUTE>): every workgroup rebuilds
+// the state at its segment's first step from the k, v rows before it.  A prefix chunk costs
+// about an eighth of a scan chunk ("prefix_cost" knob, percent; measured at T = 1024, N = 64:
+// 10 and 15 give 18.8 us, 20 to 30 give 19.0 to 19.2), so segment s gets
+// u - cost * first[s] chunks, with u the smallest figure whose segments cover the sequence:
+// prefix plus scan then take every workgroup about equally long.  Pays while a sequence has few
+// segments (the last one streams nearly the whole sequence): up to 4 ("recompute" knob: 0 never,
+// 1 whenever the kernel exists).  Returns u, or 0 if no such cut exists.
+double recompute_bounds(int64_t T, int nseg, rfa::SegBounds* b) {
+    const int knob = tune::get(tune::RECOMPUTE);
+    if (knob == 0 || nseg < 2 || nseg > rfa::kMaxSegments || (knob < 0 && nseg > 4)) return 0;
+    const int nch = (int)((T + rfa::kChunk - 1) / rfa::kChunk);
+    const int cost_knob = tune::get(tune::PREFIX_COST);
+    const double cost = (cost_knob >= 0 ? cost_knob : 12) / 100.0;
+    double u = (double)nch / nseg;
+    if (cost > 0 && cost < 1 && nch > 64) {
+        // uncut, the segments add up to u (1 - (1 - cost)^nseg) / cost: no smaller u covers the sequence (segments of
+        // a chunk or more)
+        const double least = nch * cost / (1 - std::pow(1 - cost, nseg));
+        if (least > u && least * std::pow(1 - cost, nseg - 1) > 2) u += 0.25 * std::floor((least - u) / 0.25);
+    }
+    for (; u <= nch; u += 0.25) {
+        b->first[0] = 0;
+        for (int s_ = 0; s_ < nseg; ++s_) {
+            int len = (int)(u - cost * b->first[s_] + 1e-9);
+            if (len < 1) len = 1;
+            b->first[s_ + 1] = b->first[s_] + len;
+        }
+        if (b->first[nseg] < nch) continue;
+        if (b->first[nseg - 1] >= nch) return 0;        // the cut leaves a segment empty
+        b->first[nseg] = nch;
+        for (int s_ = nseg + 1; s_ <= rfa::kMaxSegments; ++s_) b->first[s_] = nch;
+        return u;
+    }
+    return 0;
+}
+
+// What a forward + backward of the saving pair takes with a given plan, us: every launch is a number of rounds of workgroups,
+// one to a CU (two of K = d = 64), each a start plus its chunks of 64 steps, and none is faster than its bytes at
+// 3.5 TB/s (2.5 in the sliced backward).  A workgroup of segment totals costs `totals` + `totals_chunk` a chunk, one of
+// the forward scan `scan` + `scan_chunk` a chunk + `slot` for each state that it adds up, of the sliced backward
+// `slices` + `slices_chunk` a chunk, of the two sweeps together `sweeps` + `sweeps_chunk` a chunk + `sweeps_slot` a state;
+// scanning the totals costs 5 us forward, 9 in both directions.  Fitted to 6000 measurements (T 64 .. 16384, 2 to 512
+// sequences, every number of segments, both layouts): typically 6 % off, and the plan that it picks is 1 to 5 % off
+// the best one.
+struct ScanCost {
+    double scan, scan_chunk, totals, totals_chunk, slot, slices, slices_chunk, sweeps, sweeps_chunk, sweeps_slot;
+};
+
+ScanCost scan_cost(int K, int d) {
+    if (d == 64) return K == 64 ? ScanCost{3.8, 1.45, 2.8, 0.45, 0.0, 4.6, 1.75, 7.0, 4.8, 0.6}
+                      : K == 128 ? ScanCost{4.1, 2.2, 3.2, 0.6, 0.15, 3.6, 1.8, 6.6, 6.3, 1.1}
+                                 : ScanCost{3.0, 5.2, 7.8, 1.3, 2.8, 0, 0, 7.4, 8.2, 6.6};
+    return K == 64 ? ScanCost{4.5, 1.9, 2.8, 0.5, 0.1, 3.6, 2.5, 6.9, 7.3, 0.9}
+         : K == 128 ? ScanCost{5.0, 2.7, 4.0, 0.7, 0.0, 4.1, 2.7, 8.1, 9.2, 3.1}
+                    : ScanCost{2.9, 5.4, 4.0, 1.5, 8.0, 0, 0, 6.0, 9.1, 15.0};
+}
+
+ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool have_saved, int* s_ratio);
+
+double estimate_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cus) {
+    const ScanCost c = scan_cost(K, d);
+    const double nch = (double)((T + rfa::kChunk - 1) / rfa::kChunk), rows = (double)T * N, gap = 1.5;
+    auto rounds = [&](double wgs) {
+        const double full = std::max(1.0, std::ceil(wgs / cus));
+        return K == 64 && d == 64 ? 1.5 * std::floor(full / 2) + std::fmod(full, 2.0) : full;
+    };
+    double fwd, moved = rows * (K + d) * 4;
+    rfa::SegBounds b;
+    const double u = p.layout == LAYOUT_FINAL ? recompute_bounds(T, p.nseg, &b) : 0;
+    if (p.nseg == 1) {
+        fwd = rounds((double)N) * (c.scan + c.scan_chunk * nch);
+    } else if (u > 0) {
+        fwd = rounds((double)N * p.nseg) * (c.scan + c.scan_chunk * u);
+    } else {
+        const double cps = p.seg_len / rfa::kChunk;
+        fwd = gap + rounds((double)N * (p.nseg - 1)) * (c.totals + c.totals_chunk * cps) + (p.prefixed ? 5 : 0) +
+              rounds((double)N * p.nseg) * (c.scan + c.scan_chunk * cps + c.slot * (p.prefixed ? 1 : p.nseg - 1));
+        moved *= 1.5;
+    }
+    fwd = std::max(fwd, moved / 3.5e6);
+    if (p.layout == LAYOUT_FINAL)
+        return fwd + std::max(rounds((double)N * (K + d) / rfa::kSliceWidth) * (c.slices + c.slices_chunk * nch), rows * (8 * K + 10 * d) / 2.5e6);
+    int ratio;
+    const ScanPlan pb = backward_plan(p, K, d, true, &ratio);
+    const int split = K >= 256 && d >= 128 ? 2 : 1;      // workgroups of a sweep to a segment
+    const double slots = pb.nseg > 1 ? (p.prefixed ? 1 : pb.nseg - 1) : 0;
+    return fwd + std::max(gap + (pb.prefixed ? 9 : 0) + rounds((double)N * pb.nseg * split) *
+                                    (c.sweeps + c.sweeps_chunk * (pb.seg_len / rfa::kChunk) + c.sweeps_slot * slots),
+                          rows * 12 * (K + d) / 3.5e6);
+}
+
+// Layout and segments of a forward (with or without a saved buffer: the same bits) and of the backward that follows it:
+// cover_plan (always that with the "nseg" or "sliced" knob), unless another is estimated more than 8 % shorter.  What that finds, us forward + backward at
+// K = 128, d = 64, before / after: segments that spill into a second round of workgroups (T 1024, 72 sequences, 4 segments
+// -> 3) 67.1 / 55.1, raw (777, 72) 58.5 / 45.8; short sequences, where the sliced backward's one launch and the forward
+// without totals beat four launches however few CUs they cover (T 256, 16 sequences) 38.3 / 20.9; (512, 8) 41.3 / 27.6;
+// single chunks as segments (1024, 4) 49.2 / 41.2; fewer, longer segments (4096, 24) 141 / 108.
+ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
+    const ScanPlan base = cover_plan(T, N, K, d);
+    if (T <= 0 || N <= 0 || tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0) return base;
+    // called several times for one operation: the last answer of this thread, by all that goes into it
+    struct Memo { int64_t T, N; int K, d, cus; unsigned knobs; ScanPlan plan; };
+    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, base};
+    const int cus = device_cus();
+    const unsigned knobs = tune::changes.load(std::memory_order_acquire);
+    if (memo.T == T && memo.N == N && memo.K == K && memo.d == d && memo.cus == cus && memo.knobs == knobs) return memo.plan;
+    const int64_t nchunks = (T + rfa::kChunk - 1) / rfa::kChunk;
+    ScanPlan best = base;
+    const double start = estimate_us(base, T, N, K, d, cus);
+    double least = start;
+    for (int layout : {LAYOUT_SEGMENTS, LAYOUT_FINAL}) {
+        if (layout == LAYOUT_FINAL && !sliced_addressable(N, K, d)) continue;
+        // with the final state alone in the saved buffer, segments are for the forward that rebuilds their states
+        const int most = layout == LAYOUT_FINAL ? 4 : rfa::kMaxSegments;
+        int last = 0;
+        for (int64_t want = 1; want <= most && want <= nchunks; ++want) {
+            ScanPlan p{1, rfa::kChunk, 0, layout};
+            cut_segments(&p, T, want, K, d);
+            if (p.nseg == last) continue;
+            last = p.nseg;
+            const double us = estimate_us(p, T, N, K, d, cus);
+            if (us < least) { least = us; best = p; }
+        }
+    }
+    memo = Memo{T, N, K, d, cus, knobs, least * 1.08 < start ? best : base};
+    return memo.plan;
 }
 
 // ---- description of a saved-state buffer ---------------------------------------------
@@ -335,36 +472,6 @@ void launch_totals_scan(float* a, int64_t Ma, float* b, int64_t Mb, int N, int n
                dim3(rfa::kThreads), 0, st, a, Ma, b, Mb, nseg);
 }
 
-// The forward without segment totals (k_causal_fwd_pipe<.., RECOMPUTE>): every workgroup rebuilds
-// the state at its segment's first step from the k, v rows before it.  A prefix chunk costs
-// about an eighth of a scan chunk ("prefix_cost" knob, percent; measured at T = 1024, N = 64:
-// 10 and 15 give 18.8 us, 20 to 30 give 19.0 to 19.2), so segment s gets
-// u - cost * first[s] chunks, with u the smallest figure whose segments cover the sequence:
-// prefix plus scan then take every workgroup about equally long.  Pays while a sequence has few
-// segments (the last one streams nearly the whole sequence): up to 4 ("recompute" knob: 0 never,
-// 1 whenever the kernel exists).  False if no such cut exists.
-bool recompute_bounds(int64_t T, int nseg, rfa::SegBounds* b) {
-    const int knob = tune::get(tune::RECOMPUTE);
-    if (knob == 0 || nseg < 2 || nseg > rfa::kMaxSegments || (knob < 0 && nseg > 4)) return false;
-    const int nch = (int)((T + rfa::kChunk - 1) / rfa::kChunk);
-    const int cost_knob = tune::get(tune::PREFIX_COST);
-    const double cost = (cost_knob >= 0 ? cost_knob : 12) / 100.0;
-    for (double u = (double)nch / nseg; u <= nch; u += 0.25) {
-        b->first[0] = 0;
-        for (int s_ = 0; s_ < nseg; ++s_) {
-            int len = (int)(u - cost * b->first[s_] + 1e-9);
-            if (len < 1) len = 1;
-            b->first[s_ + 1] = b->first[s_] + len;
-        }
-        if (b->first[nseg] < nch) continue;
-        if (b->first[nseg - 1] >= nch) return false;        // the cut leaves a segment empty
-        b->first[nseg] = nch;
-        for (int s_ = nseg + 1; s_ <= rfa::kMaxSegments; ++s_) b->first[s_] = nch;
-        return true;
-    }
-    return false;
-}
-
 template <int KD, int DH>
 int launch_forward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t* v, rfa::half_t* out,
                    int T, int N, const ScanPlan& p, char* ws, const Workspace& wl, int* savedHdr, float* savedS,
@@ -382,7 +489,7 @@ int launch_forward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_t
         // nobody else reads the totals (the saved pair of this layout keeps only the final state):
         // one launch that needs none
         rfa::SegBounds bounds{};
-        if (allow_recompute && !savedS && recompute_bounds(T, p.nseg, &bounds) &&
+        if (allow_recompute && !savedS && recompute_bounds(T, p.nseg, &bounds) > 0 &&
             (int64_t)rfa::kChunk * N * (KD > DH ? KD : DH) * 2 < ((int64_t)1 << 32)) {
             auto kern = rfa::k_causal_fwd_pipe<KD, DH, true>;
             if (int rc = set_lds(kern, rfa::FwdPipeCfg<KD, DH>::kLds)) return rc;
@@ -1127,6 +1234,7 @@ int rfa_tuning_set(const char* name, int value) {
     if (value < -1 || value > (1 << 20)) return fail(RFA_ERR_BAD_SHAPE, "rfa_tuning_set: value %d out of range", value);
     (void)tune::get((tune::Key)k);      // the environment is read before the first store
     tune::value[k].store(value, std::memory_order_relaxed);
+    tune::changes.fetch_add(1, std::memory_order_release);
     return RFA_OK;
 }
 
@@ -1166,12 +1274,16 @@ int rfa_selftest_mfma_rate(int waves_per_simd, int iters, float* sink, double* f
 
 size_t rfa_causal_forward_workspace_bytes(int64_t T, int64_t N, int K, int d) {
     if (T <= 0 || N <= 0 || !rfa_shape_supported(K, d)) return 0;
-    return layout_workspace(T, N, K, d, make_plan(T, N, K, d), false).total;
+    // of the forward that takes it and of the one on static memory
+    return std::max(layout_workspace(T, N, K, d, make_plan(T, N, K, d), false).total,
+                    layout_workspace(T, N, K, d, cover_plan(T, N, K, d), false).total);
 }
 
 size_t rfa_causal_backward_workspace_bytes(int64_t T, int64_t N, int K, int d) {
     if (T <= 0 || N <= 0 || !rfa_shape_supported(K, d)) return 0;
-    return layout_workspace(T, N, K, d, make_plan(T, N, K, d), true).total;
+    // of the backward without a saved buffer and of the one with it
+    return std::max(layout_workspace(T, N, K, d, make_plan(T, N, K, d), true).total,
+                    layout_workspace(T, N, K, d, cover_plan(T, N, K, d), true).total);
 }
 
 // RFA_ONLY_KD=<K>,<d> (a development build: python -m rfa_amd.build --only K,d): kernels of one
@@ -1265,6 +1377,7 @@ static int causal_forward_impl(const void* q, const void* k, const void* v, void
                                int K, int d, void* saved, size_t saved_bytes, bool want_saved, float* final_s,
                                float* final_z, void* workspace, size_t workspace_bytes, void* stream,
                                bool allow_recompute = true);
+static ScanPlan noalloc_plan(int64_t T, int64_t N, int K, int d);
 
 int rfa_causal_forward(const void* q, const void* k, const void* v, void* out, int64_t T, int64_t N,
                        int K, int d, void* workspace, size_t workspace_bytes, void* stream) {
@@ -1274,11 +1387,17 @@ int rfa_causal_forward(const void* q, const void* k, const void* v, void* out, i
 
 size_t rfa_static_scratch_bytes(void) { return kStaticScratchBytes; }
 
+// the plan (and the bits) of rfa_causal_forward where its totals fit the static array
+static ScanPlan noalloc_plan(int64_t T, int64_t N, int K, int d) {
+    const ScanPlan p = make_plan(T, N, K, d);
+    return layout_workspace(T, N, K, d, p, false).total <= kStaticScratchBytes ? p : cover_plan(T, N, K, d);
+}
+
 int rfa_causal_forward_noalloc(const void* q, const void* k, const void* v, void* out, int64_t T, int64_t N,
                                int K, int d, void* stream) {
     if (int rc = check_causal_dims(T, N, K, d)) return rc;
     if (T == 0 || N == 0) return RFA_OK;
-    const size_t need = rfa_causal_forward_workspace_bytes(T, N, K, d);
+    const size_t need = layout_workspace(T, N, K, d, noalloc_plan(T, N, K, d), false).total;
     if (need > kStaticScratchBytes)
         return fail(RFA_ERR_WORKSPACE,
                     "rfa_causal_forward_noalloc: this shape needs %zu bytes of segment totals, the static scratch "
@@ -1316,7 +1435,7 @@ int rfa_causal_prefill_rows_supported(int64_t T, int64_t N, int D, int d) {
         return 0;
     const bool fits = K == 64 ? (d == 64 ? fwd_phi_fits<64, 64>() : fwd_phi_fits<64, 128>())
                       : K == 128 ? (d == 64 ? fwd_phi_fits<128, 64>() : fwd_phi_fits<128, 128>()) : false;
-    return fits && make_plan(T, N, K, d).nseg == 1;
+    return fits && cover_plan(T, N, K, d).nseg == 1;
 }
 
 int rfa_causal_prefill_rows(const void* q, const void* k, const void* v, const void* w, float scale, void* out, float* s,
@@ -1355,7 +1474,7 @@ static int causal_forward_impl(const void* q, const void* k, const void* v, void
                                bool allow_recompute) {
     if (int rc = check_causal_dims(T, N, K, d)) return rc;
     if (T == 0 || N == 0) return RFA_OK;
-    const ScanPlan p = make_plan(T, N, K, d);
+    const ScanPlan p = allow_recompute ? make_plan(T, N, K, d) : noalloc_plan(T, N, K, d);
     int* savedHdr = nullptr;
     float* savedS = nullptr;
     float* savedZ = nullptr;
@@ -1429,7 +1548,7 @@ static int causal_backward_impl(const void* q, const void* k, const void* v, con
                                 size_t workspace_bytes, void* stream) {
     if (int rc = check_causal_dims(T, N, K, d)) return rc;
     if (T == 0 || N == 0) return RFA_OK;
-    ScanPlan p = make_plan(T, N, K, d);
+    ScanPlan p = cover_plan(T, N, K, d);
     const int* savedHdr = nullptr;
     const float* savedS = nullptr;
     const float* savedZ = nullptr;

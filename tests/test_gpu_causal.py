@@ -113,6 +113,29 @@ def test_saved_pair_matches_oracle(T, B, H, d, D):
     assert _rel(got[2], plain[2].float().cpu()) <= 2e-3
 
 
+@pytest.mark.parametrize("T,B,H,d,D", SHAPES[:-4] + [(100, 2, 1, 64, 64), (300, 1, 2, 128, 64), (257, 1, 9, 128, 32), (512, 2, 2, 64, 32)])
+def test_saved_pair_by_segments_matches_oracle(T, B, H, d, D, knobs):
+    """Short sequences take the final-state layout by themselves: the two sweeps over segments on the same shapes."""
+    from rfa_amd import rfa_hip
+    knobs(sliced=0)
+    cpu = _features(T, B, H, d, D, seed=3000 + T)
+    pq, pk, v, g = (t.cuda() for t in cpu)
+    print(f"causal saved pair by segments T={T} N={B*H} K={2*D} d={d}", flush=True)
+    out, saved = rfa_hip.forward_save(pq, pk, v)
+    assert (out.float().cpu() - _oracle_fwd(*cpu[:3])).abs().max().item() <= OUT_ATOL
+    got = [t.float().cpu() for t in rfa_hip.backward_saved(pq, pk, v, g, out, saved)]
+    for name, a, b in zip(("dq", "dk", "dv"), got, _oracle_bwd(*cpu)):
+        assert _rel(a, b) <= GRAD_RTOL, (name, _rel(a, b))
+
+
+# a second round of workgroups avoided (3 segments of 72 sequences), the last chunk a single step, single chunks as
+# segments, the sliced backward of few short sequences at every width
+@pytest.mark.parametrize("T,B,H,d,D", [(777, 6, 12, 64, 64), (449, 9, 8, 64, 32), (1024, 1, 4, 64, 64), (65, 1, 1, 128, 32),
+                                       (256, 2, 8, 128, 64), (321, 3, 5, 64, 64)])
+def test_saved_pair_on_chosen_plans(T, B, H, d, D):
+    test_saved_pair_matches_oracle(T, B, H, d, D)
+
+
 def test_saved_pair_clamped_and_unclamped_rows():
     """Rows with den_raw <= 1 take gz = 0 (strict >, cuda/utils.cu:31-40); rows above take
     -(g . out) / den.  Scaling phi_k moves every row across the clamp."""

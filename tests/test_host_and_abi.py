@@ -163,6 +163,32 @@ def test_load_random_matrices_leaves_the_global_numpy_generator_alone():
     assert torch.equal(mats, torch.tensor(want, dtype=torch.half))
 
 
+@pytest.mark.parametrize("K,d", [(64, 64), (128, 64), (256, 64), (64, 128), (128, 128), (256, 128)])
+def test_causal_plans(K, d):
+    """Every shape has a plan: 1 to 16 segments, none without a chunk, the same answer however often it is asked (other
+    shapes between), buffers for every plan that a call may run with; a knob overrides it and gives it back."""
+    from rfa_amd import _lib
+    lib = _lib.load()
+    shapes = [(T, N) for T in (1, 64, 65, 128, 300, 777, 1024, 4095, 16384, 100000) for N in (1, 3, 16, 40, 72, 96, 192, 300, 1000)]
+    ask = lambda T, N: (lib.rfa_causal_num_segments(T, N, K, d), lib.rfa_causal_forward_workspace_bytes(T, N, K, d),
+                        lib.rfa_causal_backward_workspace_bytes(T, N, K, d), lib.rfa_causal_saved_state_bytes(T, N, K, d))
+    first = {s: ask(*s) for s in shapes}
+    for (T, N), got in first.items():
+        nseg, fwd, bwd, saved = got
+        chunks = (T + 63) // 64
+        assert 1 <= nseg <= min(16, chunks) and -(-chunks // -(-chunks // nseg)) == nseg
+        state = 4 * N * (K * d + K)
+        assert fwd >= (nseg * state if nseg > 1 else 0) and bwd >= (2 * nseg * state if nseg > 1 else 0) + 8 * T * N
+        assert saved >= 256 + state + 4 * T * N
+        assert ask(T, N) == got
+    lib.rfa_tuning_set(b"nseg", 2)
+    try:
+        assert lib.rfa_causal_num_segments(1024, 64, K, d) == 2
+    finally:
+        lib.rfa_tuning_set(b"nseg", -1)
+    assert {s: ask(*s) for s in shapes} == first
+
+
 def test_masked_rfa_has_no_cpu_path():
     """masked_rfa runs on the quadratic-form HIP kernels only: CPU tensors raise."""
     from rfa_amd.causal_attention import masked_rfa
