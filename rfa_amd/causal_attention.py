@@ -246,6 +246,30 @@ class CausalAttention(nn.Module):
                 and all(layer.weight.dtype == torch.float16 for layer in layers)
                 and (all(with_bias) or not any(with_bias)))
 
+    def _native_step(self, native, x: Tensor, random_matrices: Tensor, saved_state) -> Optional[Tensor]:
+        """A decoding step whose caches, stacked projection and new state tensors come from one native call;
+        None where a tensor, a layer or the mode is not plain (the caller's general path takes it)."""
+        s, z = saved_state["prev_s"], saved_state.get("prev_z")
+        tau, params = self.tau, self._parameters
+        sigma = params.get("sigma") if self.reparam_proj else None
+        if z is None or type(tau) not in (int, float) or (self.reparam_proj and sigma is None):
+            return None
+        layers = [self._modules.get(name) for name in ("q_proj", "k_proj", "v_proj", "out_proj")]
+        if None in layers:
+            return None
+        q, k, v = (layer._parameters for layer in layers[:3])
+        cache = self.__dict__.setdefault("_inference_cache", {})
+        if "step" not in cache:
+            cache["step"] = native.DecodeCache()
+        rows = cache["step"].rows(x, random_matrices, sigma, tau, q.get("weight"), q.get("bias"), k.get("weight"), k.get("bias"),
+                                  v.get("weight"), v.get("bias"), self.num_heads, s, z, self.decode_inplace)
+        if rows is None:
+            return None
+        rows, w, s_out, z_out = rows
+        attn = rfa_hip.incremental_qkv(rows, w, SCALE, s, z, s_out, z_out)
+        saved_state["prev_s"], saved_state["prev_z"] = (s, z) if s_out is None else (s_out, z_out)
+        return linear_no_grad(attn.view(x.shape), layers[3])
+
     def forward(self, x: Tensor, random_matrices: Tensor, key_padding_mask: Optional[Tensor] = None,
                 attn_mask: Optional[Tensor] = None,
                 saved_state: Optional[Dict[str, Optional[Tensor]]] = None) -> Tensor:
@@ -270,6 +294,11 @@ class CausalAttention(nn.Module):
                 [p.bias for p in layers], self.num_heads, SCALE)
             if attn is not None:
                 return linear_out(attn, self.out_proj)
+        if (native is not None and saved_state is not None and saved_state.get("prev_s") is not None
+                and not torch.is_grad_enabled()):
+            y = self._native_step(native, x, random_matrices, saved_state)
+            if y is not None:
+                return y
         w = self._scaled_matrices(random_matrices)
         if saved_state is not None and saved_state.get("prev_s") is not None and self._packed_decode_ok(x):
             # a decoding step without autograd: q, k, v of the token(s) from one stacked projection (one

@@ -10,7 +10,7 @@
 // What bounds a layer without this is the host.  The Python functions over the same kernels (input gradients by the
 // library there) / these nodes, us: a layer of 8 heads of 64, 8192 tokens, forward + backward, 212 of kernels, 487 / 237;
 // 128 tokens of 4 heads, the scan alone, 125 / 75; an encoder-decoder layer, 16384 + 8192 rows, 611 / 324; a decoding step of
-// 64 sequences 71 / 37.
+// 64 sequences 71 / 28.
 #pragma once
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContextLight.h>
@@ -458,6 +458,94 @@ OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b)
     return y;
 }
 
+// ---- what decoding keeps between calls --------------------------------------------------------
+// Tensors that a value was made from, as rfa_amd/_derived.py remembers them: the very same objects (a weak reference
+// keeps another from taking a dead one's place) in the very same state.
+class Sources {
+    struct Source {
+        c10::weak_intrusive_ptr<at::TensorImpl> impl;
+        uint32_t version;
+        const void* data;
+        std::vector<int64_t> sizes;
+        at::ScalarType type;
+        at::Device device;
+    };
+    std::vector<c10::optional<Source>> sources_;
+    double extra_ = 0;
+
+public:
+    using List = std::vector<const OptTensor*>;
+    static bool can_remember(const List& tensors) {      // inference tensors count no versions
+        for (const OptTensor* t : tensors)
+            if (t->has_value() && ((*t)->is_inference() || !(*t)->has_storage())) return false;
+        return true;
+    }
+    bool same(const List& tensors, double extra) const {
+        if (sources_.size() != tensors.size() || extra != extra_) return false;
+        for (size_t i = 0; i < tensors.size(); ++i) {
+            const auto& k = sources_[i];
+            const OptTensor& t = *tensors[i];
+            if (k.has_value() != t.has_value()) return false;
+            if (k.has_value() && !(k->impl._unsafe_get_target() == t->unsafeGetTensorImpl() && k->version == t->_version() &&
+                                   k->data == t->data_ptr() && k->sizes == t->sizes() && k->type == t->scalar_type() &&
+                                   k->device == t->device()))
+                return false;
+        }
+        return true;
+    }
+    void remember(const List& tensors, double extra) {
+        sources_.clear();
+        for (const OptTensor* t : tensors) {
+            if (!t->has_value()) sources_.emplace_back(c10::nullopt);
+            else
+                sources_.emplace_back(Source{c10::weak_intrusive_ptr<at::TensorImpl>((*t)->getIntrusivePtr()), (uint32_t)(*t)->_version(),
+                                             (*t)->data_ptr(), (*t)->sizes().vec(), (*t)->scalar_type(), (*t)->device()});
+        }
+        extra_ = extra;
+    }
+};
+
+// The scaled matrices W' and the stacked q, k, v layer of one CausalAttention, and with them the first half of a decoding
+// step: rows [T, B, 3, H, d] of all three projections, W' and the tensors that the step writes its state to (none where it
+// stays in place).  In Python this half costs 16 us of a step whose kernels take 11 (four sequences of 8 heads).
+class DecodeCache {
+    Sources matrix_sources_, layer_sources_;
+    Tensor w_, weight_;
+    OptTensor bias_;
+
+public:
+    using Rows = std::tuple<Tensor, Tensor, OptTensor, OptTensor>;
+    c10::optional<Rows> rows(const Tensor& x, const Tensor& matrices, const OptTensor& sigma, double tau, const OptTensor& wq,
+                             const OptTensor& bq, const OptTensor& wk, const OptTensor& bk, const OptTensor& wv,
+                             const OptTensor& bv, int64_t heads, const Tensor& s, const Tensor& z, bool in_place) {
+        if (!plain_mode() || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || !plain_half(x, 3) ||
+            !plain_matrices(matrices, sigma, tau) || !plain(s, torch::kFloat32, 4) || !plain(z, torch::kFloat32, 3) ||
+            !s.is_contiguous() || !z.is_contiguous())
+            return c10::nullopt;
+        const int64_t E = x.size(2);
+        for (const OptTensor* w : {&wq, &wk, &wv})
+            if (!w->has_value() || !plain_half(**w, 2) || (*w)->size(0) != E || (*w)->size(1) != E) return c10::nullopt;
+        for (const OptTensor* b : {&bq, &bk, &bv})
+            if (b->has_value() != bq.has_value() || !plain_half(*b, 1)) return c10::nullopt;
+        const OptTensor m(matrices);
+        const Sources::List ms{&m, &sigma}, ls{&wq, &bq, &wk, &bk, &wv, &bv};
+        if (heads < 1 || E % heads != 0 || !Sources::can_remember(ms) || !Sources::can_remember(ls)) return c10::nullopt;
+        if (!matrix_sources_.same(ms, tau)) {
+            w_ = build_random_matrices(matrices.contiguous(), sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt, tau);
+            matrix_sources_.remember(ms, tau);
+        }
+        if (!layer_sources_.same(ls, 0)) {
+            weight_ = at::cat({*wq, *wk, *wv}, 0);
+            bias_ = bq.has_value() ? OptTensor(at::cat({*bq, *bk, *bv}, 0)) : c10::nullopt;
+            layer_sources_.remember(ls, 0);
+        }
+        const OptTensor own = node_linear_rows(x, weight_, bias_);
+        const Tensor y = own.has_value() ? *own : at::linear(x, weight_, bias_);
+        auto fresh = [&](const Tensor& t) { return in_place ? c10::nullopt : OptTensor(torch::empty_like(t)); };
+        return Rows{y.view({x.size(0), x.size(1), 3, heads, E / heads}), w_, fresh(s), fresh(z)};
+    }
+};
+
 // ---- causal attention -------------------------------------------------------------------------
 // phi_q, phi_k [T, B, H, K], v [T, B, H, d] -> attn [T, B, H * d], through the saving pair
 struct ScanDims {
@@ -704,6 +792,7 @@ OptTensor node_cross_query(const Tensor& query, const Tensor& w, const Tensor& w
 void bind_nodes(pybind11::module_& m) {
     namespace py = pybind11;
     m.def("node_plain", &node_plain, py::arg("t"));
+    py::class_<DecodeCache>(m, "DecodeCache").def(py::init<>()).def("rows", &DecodeCache::rows);
     // each of the others returns None where the call is not plain: the caller's general path takes it
     m.def("node_random_project", &node_random_project, py::arg("x"), py::arg("w"), py::arg("scale"));
     m.def("node_linear", &node_linear, py::arg("x"), py::arg("weight"), py::arg("bias"));

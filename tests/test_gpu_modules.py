@@ -204,6 +204,60 @@ def test_causal_module_decode_from_one_stacked_projection():
         rfa_hip.incremental_qkv = real
 
 
+@pytest.mark.parametrize("change", ["none", "replaced", "data", "in_place", "no_bias", "mixed_bias", "matrices", "tau", "sigma", "hook",
+                                    "steps", "strided"])
+def test_decode_step_sees_every_change(change):
+    """A decoding step after one that filled the caches gives what a module without caches gives, whatever changed
+    in between; the layers it is compared with run under autograd (nothing cached, three projections: a rounding of
+    fp16 apart)."""
+    import copy
+    from rfa_amd import CausalAttention
+    torch.manual_seed(11)
+    B, H, d, D = 3, 2, 64, 64
+    E = H * d
+    m = CausalAttention(embed_dim=E, num_heads=H, head_dim=d, proj_dim=D).cuda().half().eval()
+    W, x = O.make_w(d, D, H).cuda().half(), torch.randn(4, B, E).cuda().half()
+    with torch.no_grad():
+        first = {}
+        m(x[:2], W, saved_state=first)
+        m(x[2:3], W, saved_state=dict(first))                       # fills the caches
+    seen, now = [], x[3:4]
+    with torch.no_grad():
+        if change == "replaced":
+            m.k_proj = copy.deepcopy(m.k_proj)
+            m.k_proj.weight.mul_(0.5)
+        elif change == "data":
+            m.v_proj.weight.data = m.v_proj.weight.data * 0.5
+        elif change == "in_place":
+            m.q_proj.bias.add_(0.5)
+        elif change in ("no_bias", "mixed_bias"):
+            for layer in (m.q_proj, m.k_proj, m.v_proj)[:3 if change == "no_bias" else 1]:
+                layer.bias = None
+        elif change == "matrices":
+            W = W * 0.5
+        elif change == "tau":
+            m.tau = 2
+        elif change == "sigma":
+            m.sigma.mul_(0.7)
+        elif change == "hook":
+            m.out_proj.register_forward_hook(lambda mod, args, out: seen.append(1) or out * 2)
+        elif change == "steps":
+            now = x[2:4]
+        elif change == "strided":
+            now = torch.randn(1, E, B).cuda().half().transpose(1, 2)
+        got_state, ref_state = dict(first), dict(first)
+        got = m(now, W, saved_state=got_state)
+    m.requires_grad_(True)
+    with torch.enable_grad():
+        want = m(now, W, saved_state=ref_state).detach()
+    if change == "hook":            # called without autograd; a layer in training is one node
+        assert len(seen) == 1
+        got = got / 2
+    assert (got.float() - want.float()).abs().max().item() <= 4e-3
+    for key in ("prev_s", "prev_z"):
+        assert _rel(got_state[key], ref_state[key]) <= 2e-3, key
+
+
 def test_causal_module_training_step_runs_and_matches_oracle():
     from rfa_amd import CausalAttention
     torch.manual_seed(1)
