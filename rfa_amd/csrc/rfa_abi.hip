@@ -47,12 +47,12 @@ int fail(int code, const char* fmt, ...) {
 // ---- optional per-kernel timing with HIP events ------------------------------------
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
-          CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_PREP, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
+          CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
           SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
-                                   "k_masked_fwd", "k_masked_bwd_prep", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
+                                   "k_masked_fwd", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
                                    "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
@@ -829,15 +829,11 @@ int launch_masked_bwd(const rfa::half_t* q, const rfa::half_t* k, const rfa::hal
                       rfa::half_t* ghat, float* gz, int T, int Tp, int N, int H, hipStream_t st) {
     using Cfg = rfa::MaskedCfg<KD, DH>;
     const int nblk = (T + rfa::kChunk - 1) / rfa::kChunk;
-    const int64_t rows = (int64_t)T * N;
-    const int64_t pieces = rows * (DH / 8);
-    RFA_LAUNCH(MASKED_PREP, rfa::k_masked_bwd_prep<DH>, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, g, out,
-               rsum, ghat, gz, rows);
     auto kq = rfa::k_masked_dq<KD, DH>;
     if (int rc = set_lds(kq, Cfg::kLds)) return rc;
     int paired = amask && masked_paired(N, nblk, resident_blocks<rfa::k_masked_dq<KD, DH>>(256, Cfg::kLds)) ? 1 : 0;
-    RFA_LAUNCH(MASKED_DQ, kq, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, (const rfa::half_t*)ghat, (const float*)gz, k,
-               v, pad, amask, dq, T, Tp, N, H, paired);
+    RFA_LAUNCH(MASKED_DQ, kq, dim3(N * (paired ? (nblk + 1) / 2 : nblk)), dim3(256), Cfg::kLds, st, g, out, rsum, k,
+               v, pad, amask, dq, ghat, gz, T, Tp, N, H, paired);
     auto kk = rfa::k_masked_dkdv<KD, DH>;
     if (int rc = set_lds(kk, Cfg::kLds)) return rc;
     paired = amask && masked_paired(N, nblk, resident_blocks<rfa::k_masked_dkdv<KD, DH>>(256, Cfg::kLds)) ? 1 : 0;

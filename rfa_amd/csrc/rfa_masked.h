@@ -120,7 +120,8 @@ __device__ __forceinline__ int next_live_block(const unsigned char* skip, int b,
 // bf16, any strides): out [T][Tp] and its transpose out_t [T][Tp], columns past T set.  One 64 x 64 tile per
 // workgroup: coalesced reads along the mask's rows, the tile of bytes through LDS, 4-byte stores on both sides.
 // At 512 x 512 the launch bounds it; what it replaces was a chain of six ATen launches (compare, two fills, a
-// conversion, two strided copies), 28 us of device time and the host work of six launches; this takes 7.2.
+// conversion, two strided copies), 28 us of device time and the host work of six launches; with a thread's sixteen
+// loads behind branches, one after the other, it took 7.2, with all in flight 3.7.
 // grid = (Tp / 64, Tp / 64)
 struct Bf16Bits { uint16_t bits; };
 __device__ __forceinline__ bool is_negative(float x) { return x < 0.f; }
@@ -133,12 +134,15 @@ __global__ __launch_bounds__(256) void k_pack_mask(const M* __restrict__ mask, i
                                                    int Tp) {
     __shared__ uint8_t tile[64][68];       // 17 words a row: both read patterns spread over the banks
     const int tid = threadIdx.x, r0 = 64 * blockIdx.y, c0 = 64 * blockIdx.x;
+    M x[16];      // all requested before the first is looked at; past the end the last entry, which then counts as set
+    const int c = tid & 63;
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+        x[u] = mask[min(r0 + 4 * u + (tid >> 6), T - 1) * stride_r + min(c0 + c, T - 1) * stride_c];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-        const int r = 4 * u + (tid >> 6), c = tid & 63;
-        bool set = true;
-        if (r0 + r < T && c0 + c < T) set = is_negative(mask[(r0 + r) * stride_r + (c0 + c) * stride_c]);
-        tile[r][c] = set ? 1 : 0;
+        const int r = 4 * u + (tid >> 6);
+        tile[r][c] = r0 + r >= T || c0 + c >= T || is_negative(x[u]) ? 1 : 0;
     }
     __syncthreads();
 #pragma unroll
@@ -256,47 +260,17 @@ __device__ __forceinline__ void masked_fwd_block(const int n, const int i0,
 }
 
 // ---------------------------------------------------------------------------
-// backward pre-pass, one thread group per row:  ghat = g / n,  gz as in the header.
-// grid = ceil(T * N / (256 / (DH/8))), 256 threads; DH/8 adjacent lanes share one row.
-// ---------------------------------------------------------------------------
-template <int DH>
-__global__ __launch_bounds__(256) void k_masked_bwd_prep(const half_t* __restrict__ g, const half_t* __restrict__ o,
-                                                         const float* __restrict__ rsum, half_t* __restrict__ ghat,
-                                                         float* __restrict__ gz, int64_t rows) {
-    constexpr int PPR = DH / 8;
-    const int64_t piece = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t r_ = piece / PPR;
-    const int c8 = (int)(piece % PPR);
-    const bool valid = r_ < rows;
-    const int64_t rc = valid ? r_ : rows - 1;
-    union { uint4 u; h8 h; } xg, xo;
-    xg.u = *reinterpret_cast<const uint4*>(g + rc * DH + c8 * 8);
-    xo.u = *reinterpret_cast<const uint4*>(o + rc * DH + c8 * 8);
-    float dot = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) dot += (float)xg.h[e] * (float)xo.h[e];
-#pragma unroll
-    for (int m = 1; m < PPR; m <<= 1) dot += __shfl_xor(dot, m, 64);
-    const float r = rsum[rc];
-    const float inv = 1.0f / fmaxf(fabsf(r), kQuadEps);
-    if (!valid) return;
-    h8 y;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = (half_t)((float)xg.h[e] * inv);
-    *reinterpret_cast<h8*>(ghat + r_ * DH + c8 * 8) = y;
-    if (c8 == 0) gz[r_] = (fabsf(r) >= kQuadEps) ? (r > 0.f ? -dot * inv : dot * inv) : 0.f;
-}
-
-// ---------------------------------------------------------------------------
 // dphi_q.  Same structure as the forward with (G^, V, K) in the roles of (Q, K, V).  Padded
 // keys need no mask here: their phi_k rows are read as zero, so they add nothing to dphi_q.
+// Every row is one lane group's own here, which forms G^ and gz from g, out and r as it loads them and leaves them
+// for the dK/dV kernel (a pass of its own over the rows took 4.6 us of 69 at T 512, 64 sequences of 64).
 // ---------------------------------------------------------------------------
 template <int KD, int DH>
 __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
     
-    const half_t* __restrict__ ghat, const float* __restrict__ gz, const half_t* __restrict__ k,
+    const half_t* __restrict__ g, const half_t* __restrict__ o, const float* __restrict__ rsum, const half_t* __restrict__ k,
     const half_t* __restrict__ v, const uint8_t* __restrict__ pad_mask, const uint8_t* __restrict__ attn_mask,
-    half_t* __restrict__ dq, int T, int Tp, int N, int H) {
+    half_t* __restrict__ dq, half_t* __restrict__ ghat, float* __restrict__ gz, int T, int Tp, int N, int H) {
     using Cfg = MaskedCfg<KD, DH>;
     constexpr int C = Cfg::C, LDQ = Cfg::LDQ, LDV = Cfg::LDV;
     constexpr int NCS = DH / 32, NKT = KD / 16;
@@ -315,16 +289,15 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
 
     const int ti = i0 + 16 * w + row;
     const int tic = min(ti, T - 1);
-    h8 bg[NCS];
-    float gzi;
-    {
-        const int64_t tn = (int64_t)tic * N + n;
+    const int64_t tn = (int64_t)tic * N + n;
+    h8 bg[NCS], bo[NCS];
 #pragma unroll
-        for (int cs = 0; cs < NCS; ++cs) bg[cs] = *reinterpret_cast<const h8*>(ghat + tn * DH + 32 * cs + 8 * G);
-        gzi = gz[tn];
+    for (int cs = 0; cs < NCS; ++cs) {
+        bg[cs] = *reinterpret_cast<const h8*>(g + tn * DH + 32 * cs + 8 * G);
+        bo[cs] = *reinterpret_cast<const h8*>(o + tn * DH + 32 * cs + 8 * G);
     }
+    const float r = rsum[tn];
     __shared__ unsigned char skip[kMaxMaskBlocks];
-    masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
     struct Tile {
         ChunkRegs<KD> k;
         ChunkRegs<DH> v;
@@ -337,6 +310,26 @@ __device__ __forceinline__ void masked_dq_block(const int n, const int i0,
         chunk_g2r<DH>(t.v, vb + (int64_t)t0 * v_stride, v_stride, T - t0, tid);
         chunk_mask_rows<KD>(t.k, prow ? prow + t0 : reinterpret_cast<const uint8_t*>(kb), tid);
     };
+    masked_tile_skip(attn_mask, i0, T, Tp, nblk, skip, tid);
+    float gzi = 0.f;
+    {
+        const float inv = 1.0f / fmaxf(fabsf(r), kQuadEps);
+        float dot = 0.f;
+#pragma unroll
+        for (int cs = 0; cs < NCS; ++cs)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                dot += (float)bg[cs][e] * (float)bo[cs][e];
+                bg[cs][e] = (half_t)((float)bg[cs][e] * inv);
+            }
+        dot = sum_over_groups(dot);
+        if (fabsf(r) >= kQuadEps) gzi = r > 0.f ? -dot * inv : dot * inv;
+        if (ti < T) {
+#pragma unroll
+            for (int cs = 0; cs < NCS; ++cs) *reinterpret_cast<h8*>(ghat + tn * DH + 32 * cs + 8 * G) = bg[cs];
+            if (G == 0) gz[tn] = gzi;
+        }
+    }
     Tile t;
     int jb = next_live_block(skip, 0, nblk);
     prefetch(t, jb);
@@ -551,10 +544,10 @@ __global__ __launch_bounds__(256) void k_masked_fwd(
 
 template <int KD, int DH>
 __global__ __launch_bounds__(256) void k_masked_dq(
-    const half_t* __restrict__ ghat, const float* __restrict__ gz, const half_t* __restrict__ k,
+    const half_t* __restrict__ g, const half_t* __restrict__ o, const float* __restrict__ rsum, const half_t* __restrict__ k,
     const half_t* __restrict__ v, const uint8_t* __restrict__ pad_mask, const uint8_t* __restrict__ attn_mask,
-    half_t* __restrict__ dq, int T, int Tp, int N, int H, int paired) {
-#define RFA_CALL_BLOCK(n, row0) masked_dq_block<KD, DH>(n, row0, ghat, gz, k, v, pad_mask, attn_mask, dq, T, Tp, N, H)
+    half_t* __restrict__ dq, half_t* __restrict__ ghat, float* __restrict__ gz, int T, int Tp, int N, int H, int paired) {
+#define RFA_CALL_BLOCK(n, row0) masked_dq_block<KD, DH>(n, row0, g, o, rsum, k, v, pad_mask, attn_mask, dq, ghat, gz, T, Tp, N, H)
     RFA_MASKED_BLOCKS(RFA_CALL_BLOCK)
 #undef RFA_CALL_BLOCK
 }
