@@ -302,6 +302,14 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
 int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R,
                           int E_out, int E_in, void* stream);
 
+/* Both of those gradients in one launch (and its reduction): arguments as above, dy_p [R, E_out] with rows ld halves
+ * apart for both.  Where rfa_linear_grads_workspace_bytes answers 0 the two calls above are to be used: E_out or E_in no
+ * multiple of 128, beyond 2^22, or so many rows that either fills the chip by itself. */
+size_t rfa_linear_grads_workspace_bytes(int64_t R, int E_out, int E_in, int np);
+int rfa_linear_grads(const void* x, const void* const* dy, int64_t ld, const void* const* w, int np, void* dx,
+                     void* const* dw, void* const* db, int64_t R, int E_out, int E_in, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 
 /* ---------------------------------------------------------------------------
  * Cross attention (encoder -> decoder).  The state is fp32.

@@ -48,7 +48,7 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, LINEAR_GRADS, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
@@ -56,7 +56,7 @@ const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
                                    "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
-                                   "k_cross_step", "k_mask_rows", "k_input_grad"};
+                                   "k_cross_step", "k_mask_rows", "k_input_grad", "k_linear_grads"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
 bool enabled = false;
@@ -987,6 +987,63 @@ TileShape input_grad_shape(int64_t R, int Eo, int Ei, int np) {
     if (t128 <= cus && Eo % 64 == 0) return {128, 2};
     if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= 3 * ((t128 + cus - 1) / cus)) return {256, 1};
     return {128, 1};
+}
+
+// ---- both gradients of Linear layers ----------------------------------------------------
+struct LinearGradsPlan {
+    TileShape t;      // tiles of dx
+    WGradPlan w;      // row splits of dW
+};
+
+// One launch for dx and the partials of dW: either alone is a launch that fills and drains the chip, and while either
+// leaves CUs idle both together take little more than the longer one.  Two groups of waves to a tile, one workgroup to a
+// CU, where all tiles of both are at most one to a CU (64 rows a tile of dx, then 128); beyond that one group, 128 rows,
+// up to three workgroups to a CU.  dW's rows are split so that its workgroups walk about as many steps as dx's, as far as
+// the workgroups stay within those numbers.  Measured with the reduction, us, as two launches (and theirs) / here:
+// 512 rows of 512 -> 512 16.4 / 10.1, of 3 x 512 23.8 / 16.9; 2048 of 512 21.0 / 14.0, of 3 x 512 31.5 / 18.9, of 1024 31.9 /
+// 20.3; 4096 of 512 25.0 / 17.4, of 1024 40.1 / 29.4; 8192 of 512 33.5 / 24.0, of 3 x 512 47.2 / 40.0; 16384 of 2 x 512 59.5 /
+// 52.1; 8192 of 2 x 1024 96.7 / 87.2.
+bool make_linear_grads_plan(int64_t R, int Eo, int Ei, int np, LinearGradsPlan* p) {
+    if (R <= 0 || R > (1 << 30) || Eo <= 0 || Ei <= 0 || Eo % 128 || Ei % 128 || Eo > (1 << 22) || Ei > (1 << 22) || np < 1 ||
+        np > rfa::kMaxProjections)
+        return false;
+    const int64_t cus = device_cus(), tiles_c = Ei / 128, t64 = (R + 63) / 64 * tiles_c, t128 = (R + 127) / 128 * tiles_c;
+    const int64_t tiles_w = (int64_t)np * (Eo / 128) * tiles_c;
+    const int64_t even = std::max<int64_t>(1, (R + (int64_t)np * Eo / 2) / ((int64_t)np * Eo));      // splits for equal chains
+    int64_t splits;
+    if (t64 + even * tiles_w <= cus) { p->t = {64, 2}; splits = even; }
+    else if (t128 + even * tiles_w <= cus) { p->t = {128, 2}; splits = even; }
+    else if (t128 + tiles_w <= 3 * cus) { p->t = {128, 1}; splits = std::min(even, (3 * cus - t128) / tiles_w); }
+    else return false;
+    const int64_t step = 32 * p->t.groups, nsteps = (R + step - 1) / step;
+    splits = std::min<int64_t>({splits, nsteps, 64});
+    const int64_t sps = (nsteps + splits - 1) / splits;
+    p->w.rows_per_split = (int)(sps * step);
+    p->w.nsplit = (int)((nsteps + sps - 1) / sps);
+    return true;
+}
+
+template <int BM, int KG>
+int launch_linear_grads(const rfa::InputGradArgs& ga, rfa::half_t* dx, const rfa::half_t* x, const rfa::WeightGradArgs& wa,
+                        float* part, float* bpart, int R, int Eo, int Ei, int np, int64_t ld, const WGradPlan& pl, hipStream_t st) {
+    constexpr size_t lds = std::max(rfa::InputGradCfg<BM, KG>::kLds, rfa::WeightGradCfg::kLds<KG>);
+    auto kern = rfa::k_linear_grads<BM, KG>;
+    if (int rc = set_lds(kern, lds)) return rc;
+    const int64_t tiles = (int64_t)((R + BM - 1) / BM) * (Ei / 128), work = (int64_t)pl.nsplit * np * (Eo / 128) * (Ei / 128);
+    const int64_t grid = rfa::kXcds * ((tiles + rfa::kXcds - 1) / rfa::kXcds + (work + rfa::kXcds - 1) / rfa::kXcds);
+    RFA_LAUNCH(LINEAR_GRADS, kern, dim3((unsigned)grid), dim3(rfa::kThreads * KG), lds, st, ga, dx, x, wa, part, bpart, R, Eo, Ei,
+               np, ld, (int)tiles, (int)work, pl.rows_per_split);
+    RFA_HIP_TRY(hipGetLastError());
+    return RFA_OK;
+}
+
+int launch_weight_grad_reduce(const float* part, const float* bpart, const rfa::WeightGradArgs& wa, int Eo, int Ei, int np,
+                              int nsplit, hipStream_t st) {
+    const int64_t threads = (int64_t)np * ((int64_t)Eo * Ei + Eo) / 4;
+    RFA_LAUNCH(WGRAD_REDUCE, rfa::k_weight_grad_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(rfa::kThreads), 0, st, part,
+               bpart, wa, Eo, Ei, np, nsplit);
+    RFA_HIP_TRY(hipGetLastError());
+    return RFA_OK;
 }
 
 // ---- feature map launchers ---------------------------------------------------------
@@ -2277,15 +2334,55 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
     if (work > (int64_t(1) << 30)) return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_weight_grad: sizes exceed the supported range");
     const unsigned grid = (unsigned)(rfa::kXcds * ((work + rfa::kXcds - 1) / rfa::kXcds));
     auto kern = std::max(E_out, E_in) > (1 << 26) ? rfa::k_weight_grad_partial<true> : rfa::k_weight_grad_partial<false>;
-    if (int rc = set_lds(kern, rfa::WeightGradCfg::kLds)) return rc;
+    constexpr size_t lds = rfa::WeightGradCfg::kLds<1>;
+    if (int rc = set_lds(kern, lds)) return rc;
     // R = 0: every split is empty and the partials come out as zeros
-    RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3(grid), dim3(rfa::kThreads), rfa::WeightGradCfg::kLds, st,
-               static_cast<const rfa::half_t*>(x), wa, part, bpart, (int)R, E_out, E_in, np, pl.nsplit, pl.rows_per_split);
-    const int64_t threads = (int64_t)np * ((int64_t)E_out * E_in + E_out) / 4;
-    RFA_LAUNCH(WGRAD_REDUCE, rfa::k_weight_grad_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(rfa::kThreads), 0, st,
-               (const float*)part, (const float*)bpart, wa, E_out, E_in, np, pl.nsplit);
-    RFA_HIP_TRY(hipGetLastError());
-    return RFA_OK;
+    RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3(grid), dim3(rfa::kThreads), lds, st, static_cast<const rfa::half_t*>(x), wa,
+               (int64_t)E_out, part, bpart, (int)R, E_out, E_in, np, pl.nsplit, pl.rows_per_split);
+    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.nsplit, st);
+}
+
+size_t rfa_linear_grads_workspace_bytes(int64_t R, int E_out, int E_in, int np) {
+    LinearGradsPlan pl;
+    if (!make_linear_grads_plan(R, E_out, E_in, np, &pl)) return 0;
+    return (size_t)pl.w.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+}
+
+int rfa_linear_grads(const void* x, const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, void* const* dw,
+                     void* const* db, int64_t R, int E_out, int E_in, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "rfa_linear_grads";
+    LinearGradsPlan pl;
+    if (!make_linear_grads_plan(R, E_out, E_in, np, &pl))
+        return fail(RFA_ERR_UNSUPPORTED, "%s: rows=%lld E_out=%d E_in=%d, %d layers are for rfa_linear_input_grad and rfa_linear_weight_grad",
+                    fn, (long long)R, E_out, E_in, np);
+    if (ld < E_out || ld > (1 << 22) || ld % 8) return fail(RFA_ERR_BAD_SHAPE, "%s: bad row distance ld=%lld for E_out=%d", fn, (long long)ld, E_out);
+    if (!x || !dy || !w || !dx || !dw) return fail(RFA_ERR_NULL_POINTER, "%s: NULL pointer", fn);
+    rfa::InputGradArgs ga{};
+    rfa::WeightGradArgs wa{};
+    for (int p = 0; p < np; ++p) {
+        ga.dy[p] = wa.dy[p] = static_cast<const rfa::half_t*>(dy[p]);
+        ga.w[p] = static_cast<const rfa::half_t*>(w[p]);
+        wa.dw[p] = static_cast<rfa::half_t*>(dw[p]);
+        wa.db[p] = db ? static_cast<rfa::half_t*>(db[p]) : nullptr;
+        if (!ga.dy[p] || !ga.w[p] || !wa.dw[p]) return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor %d", fn, p);
+        if (!aligned16(ga.dy[p]) || !aligned16(ga.w[p]) || !aligned16(wa.dw[p]) || (reinterpret_cast<uintptr_t>(wa.db[p]) & 7u))
+            return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned (bias gradient: 8)", fn);
+    }
+    if (!aligned16(x) || !aligned16(dx)) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+    const size_t need = (size_t)pl.w.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+    if (!workspace || workspace_bytes < need || !aligned16(workspace))
+        return fail(RFA_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", fn, need, workspace ? workspace_bytes : (size_t)0);
+    float* part = static_cast<float*>(workspace);
+    float* bpart = part + (size_t)pl.w.nsplit * np * E_out * E_in;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto* xh = static_cast<const rfa::half_t*>(x);
+    auto* dxh = static_cast<rfa::half_t*>(dx);
+    int rc;
+    if (pl.t.groups == 1) rc = launch_linear_grads<128, 1>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    else if (pl.t.rows == 64) rc = launch_linear_grads<64, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    else rc = launch_linear_grads<128, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    if (rc) return rc;
+    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.w.nsplit, st);
 }
 
 // ---- profiling ----------------------------------------------------------------------

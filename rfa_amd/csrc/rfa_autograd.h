@@ -216,6 +216,32 @@ Tensor input_grad(const std::vector<const void*>& dys, int64_t ld, const Tensor*
     return dx;
 }
 
+// dx (of x's shape), dW and db of layers over one input in one launch where the library takes them so.  dys as for
+// input_grad; `dw` and `db` [n] get the gradients, db those whose flag is set.
+bool linear_grads(const std::vector<const void*>& dys, int64_t ld, const Tensor* w, const Tensor& x, const Tensor& x2,
+                  const std::vector<bool>& bias, Tensor& dx, std::vector<Tensor>& dw, std::vector<OptTensor>& db) {
+    const int64_t n = (int64_t)dys.size(), e_out = w[0].size(0), e_in = w[0].size(1), rows = x2.size(0);
+    const size_t nbytes = rfa_linear_grads_workspace_bytes(rows, (int)e_out, (int)e_in, (int)n);
+    if (nbytes == 0) return false;
+    const Tensor xc = x2.contiguous();
+    if (!aligned16(xc)) return false;
+    std::array<const void*, 3> wp{};
+    std::array<void*, 3> dwp{}, dbp{};
+    for (int64_t p = 0; p < n; ++p) {
+        wp[p] = ptr(w[p]);
+        dw.push_back(torch::empty({e_out, e_in}, x.options()));
+        db.push_back(bias[p] ? OptTensor(torch::empty({e_out}, x.options())) : c10::nullopt);
+        dwp[p] = ptr(dw[p]);
+        dbp[p] = ptr(db[p]);
+    }
+    dx = torch::empty(x.sizes(), x.options());
+    Launch l(x);
+    Tensor ws = workspace(nbytes, x);
+    check_rc(rfa_linear_grads(ptr(xc), dys.data(), ld, wp.data(), (int)n, ptr(dx), dwp.data(), dbp.data(), rows, (int)e_out,
+                              (int)e_in, ptr(ws), nbytes, l.stream));
+    return true;
+}
+
 struct ProjectNode : public torch::autograd::Function<ProjectNode> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& wf, double scale, int64_t heads,
                                  int64_t phi, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
@@ -275,9 +301,19 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             const Tensor g0 = g[0].contiguous(), g1 = g[1].contiguous(), g2 = g[2].contiguous();
             dwf = feature_grads(y[0], &y[1], wf, g0, &g1, &g2, packed, nullptr, true, scale, need_wf);
             const char* base = static_cast<const char*>(packed.data_ptr());
-            out[0] = own_input_grad(rows, w, 3)
-                         ? input_grad({base, base + 2 * e_out, base + 4 * e_out}, 3 * e_out, w, x)
-                         : at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
+            const std::vector<const void*> dyp{base, base + 2 * e_out, base + 4 * e_out};
+            const bool own = own_input_grad(rows, w, 3);
+            std::vector<Tensor> dw;
+            std::vector<OptTensor> db;
+            if (own && linear_grads(dyp, 3 * e_out, w, x, x2, bias, out[0], dw, db)) {
+                for (int64_t p = 0; p < n; ++p) {
+                    out[5 + 2 * p] = dw[p];
+                    out[6 + 2 * p] = opt(db[p]);
+                }
+                out[1] = dwf;
+                return out;
+            }
+            out[0] = own ? input_grad(dyp, 3 * e_out, w, x) : at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
             auto [dws, dbs] = param_grads(x2, {packed}, {bias_bits != 0});
             for (int64_t p = 0; p < n; ++p) {
                 out[5 + 2 * p] = dws[0].narrow(0, p * e_out, e_out);
@@ -301,15 +337,17 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             }
             bool own = need_x && own_input_grad(rows, w, n);
             for (const Tensor& dy : dys) own = own && aligned16(dy);
-            if (own) {
-                std::vector<const void*> dyp;
-                for (Tensor& dy : dys) dyp.push_back(ptr(dy));
-                out[0] = input_grad(dyp, w[0].size(0), w, x);
+            std::vector<Tensor> dws;
+            std::vector<OptTensor> dbs;
+            std::vector<const void*> dyp;
+            for (Tensor& dy : dys) dyp.push_back(ptr(dy));
+            if (!own || !linear_grads(dyp, w[0].size(0), w, x, x2, bias, out[0], dws, dbs)) {
+                if (own) out[0] = input_grad(dyp, w[0].size(0), w, x);
+                for (int64_t p = 0; p < n && need_x && !own; ++p) {
+                    out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
+                }
+                std::tie(dws, dbs) = param_grads(x2, dys, bias);
             }
-            for (int64_t p = 0; p < n && need_x && !own; ++p) {
-                out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
-            }
-            auto [dws, dbs] = param_grads(x2, dys, bias);
             for (int64_t p = 0; p < n; ++p) {
                 out[5 + 2 * p] = dws[p];
                 out[6 + 2 * p] = opt(dbs[p]);
@@ -392,13 +430,16 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
         check_saved("weight", w, g[0]);
         const Tensor dy2 = g[0].reshape({-1, g[0].size(-1)}), x2 = x.reshape({-1, x.size(-1)});
         Tensor dx;
+        const std::vector<bool> bias{ctx->saved_data["bias"].toBool()};
         if (ctx->saved_data["need_x"].toBool()) {
             const Tensor dyc = dy2.contiguous();
-            dx = own_input_grad(dyc.size(0), &w, 1) && aligned16(dyc)
-                     ? input_grad({ptr(dyc)}, w.size(0), &w, x)
-                     : at::mm(dyc, w).view(x.sizes());
+            const bool own = own_input_grad(dyc.size(0), &w, 1) && aligned16(dyc);
+            std::vector<Tensor> dw;
+            std::vector<OptTensor> db;
+            if (own && linear_grads({ptr(dyc)}, w.size(0), &w, x, x2, bias, dx, dw, db)) return {dx, dw[0], opt(db[0])};
+            dx = own ? input_grad({ptr(dyc)}, w.size(0), &w, x) : at::mm(dyc, w).view(x.sizes());
         }
-        auto [dws, dbs] = param_grads(x2, {dy2}, {ctx->saved_data["bias"].toBool()});
+        auto [dws, dbs] = param_grads(x2, {dy2}, bias);
         return {dx, dws[0], opt(dbs[0])};
     }
 };

@@ -440,7 +440,9 @@ struct WeightGradCfg {
     static constexpr int kStages = 3;                      // 4 and 5 measured the same
     static constexpr int NO = TO / 32, NI = TI / 32;       // 16-wide tiles of a wave: 64 x 64
     static constexpr int kStageHalves = C * (TO + TI);
-    static constexpr size_t kLds = (size_t)kStages * kStageHalves * 2;
+    template <int KG> using Sum = GroupSum<NO, NI + 1, KG>;
+    template <int KG> static constexpr size_t kLds =
+        (size_t)kStages * KG * kStageHalves * 2 > Sum<KG>::kLds ? (size_t)kStages * KG * kStageHalves * 2 : Sum<KG>::kLds;
     static constexpr int YI = C * TO / 2048, XI = C * TI / 2048;   // 1 KiB pieces of a stage per wave
 };
 
@@ -468,24 +470,23 @@ __device__ __forceinline__ h8 col8_rot(const half_t* X, int seg, int lane) {
 // grid = 8 * ceil(work / 8), work = nsplit * np * tiles; each XCD gets a contiguous range of the numbers
 // (split first), so that the workgroups that share rows of x and dy meet in its L2.  rows_per_split is a
 // multiple of 32.  WIDE: rows of more than 2^26 halves, 32 of which lie beyond a 32-bit byte offset.
-template <bool WIDE>
-__global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
-    const half_t* __restrict__ x, WeightGradArgs wa, float* __restrict__ part, float* __restrict__ bpart, int R,
-    int Eo, int Ei, int np, int nsplit, int rows_per_split) {
+template <bool WIDE, int KG>
+__device__ __forceinline__ void weight_grad_tile(unsigned char* smem_raw, int idx, const half_t* __restrict__ x,
+                                                 const WeightGradArgs& wa, int64_t ld, float* __restrict__ part,
+                                                 float* __restrict__ bpart, int R, int Eo, int Ei, int np, int rows_per_split) {
     using Cfg = WeightGradCfg;
+    using Sum = typename Cfg::template Sum<KG>;
     constexpr int TO = Cfg::TO, TI = Cfg::TI, C = Cfg::C, NO = Cfg::NO, NI = Cfg::NI, STAGES = Cfg::kStages;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    half_t* smem = reinterpret_cast<half_t*>(smem_raw);
+    constexpr int kRing = KG * Cfg::kStageHalves;
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);      // wave inside its group
+    half_t* const smem = reinterpret_cast<half_t*>(smem_raw) + kg * Cfg::kStageHalves;      // the group's part of a stage
     const int i = lane & 15, G = lane >> 4;
     const int wo = wv >> 1, wi = wv & 1;                  // wave -> quadrant of the tile
 
     const int tiles_i = Ei / TI, tiles_o = Eo / TO;
-    const int work = nsplit * np * tiles_o * tiles_i, per_xcd = (work + kXcds - 1) / kXcds;
-    int idx = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-    if (idx >= work) return;
     const int ti = idx % tiles_i; idx /= tiles_i;
     const int to = idx % tiles_o; idx /= tiles_o;
     const int p = idx % np, s = idx / np;
@@ -493,19 +494,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
     const int o0 = to * TO, c0 = ti * TI;
     const bool with_bias = ti == 0 && wi == 0 && pick3(wa.db, p) != nullptr;   // wave-uniform
 
-    f4 acc[NO][NI];      // (m = o, n = c) tiles of this wave's quadrant
-    f4 accb[NO];         // column sums of dy: every column n holds the same sum
+    // (m = o, n = c) tiles of this wave's quadrant; the last of a row: column sums of dy, the same in every column n
+    f4 acc[NO][NI + 1];
 #pragma unroll
-    for (int a = 0; a < NO; ++a) {
-        accb[a] = f4_zero();
+    for (int a = 0; a < NO; ++a)
 #pragma unroll
-        for (int b = 0; b < NI; ++b) acc[a][b] = f4_zero();
-    }
+        for (int b = 0; b <= NI; ++b) acc[a][b] = f4_zero();
     const h8 ones = h8_ones();
 
     if (r_begin < r_end) {
         // 1 KiB of a stage array per instruction: 512 / LD rows, lane -> (row, 16-byte piece)
-        const half_t* const dyb = pick3(wa.dy, p) + (int64_t)r_begin * Eo + o0;
+        const half_t* const dyb = pick3(wa.dy, p) + (int64_t)r_begin * ld + o0;
         const half_t* const xb = x + (int64_t)r_begin * Ei + c0;
         const int nrows = r_end - r_begin, nk = (nrows + C - 1) / C;
         auto rot = [](int r) { return ((r & 3) | ((r >> 1) & 4)) * 2; };
@@ -519,7 +518,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
 #pragma unroll
             for (int it = 0; it < Cfg::YI; ++it) {
                 const int r = (wv * Cfg::YI + it) * (512 / TO) + lane / (TO / 8);
-                yoff[last][it] = (Offset)min(r, rmax) * ((Offset)Eo * 2) + ((lane % (TO / 8)) ^ rot(r)) * 16;
+                yoff[last][it] = (Offset)min(r, rmax) * ((Offset)ld * 2) + ((lane % (TO / 8)) ^ rot(r)) * 16;
             }
 #pragma unroll
             for (int it = 0; it < Cfg::XI; ++it) {
@@ -531,9 +530,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             if constexpr (WIDE) dma16(reinterpret_cast<const char*>(base) + off, lds);
             else dma16_opaque(base, off, lds);
         };
-        auto load_stage = [&](int kk, int buf) {
-            half_t* st = smem + buf * Cfg::kStageHalves;
-            const half_t* yb = dyb + (int64_t)kk * C * Eo;
+        auto load_stage = [&](int step, int buf) {
+            const int kk = min(step * KG + kg, nk - 1);
+            half_t* st = smem + buf * kRing;
+            const half_t* yb = dyb + (int64_t)kk * C * ld;
             const half_t* xk = xb + (int64_t)kk * C * Ei;
             const bool last = kk == nk - 1;
 #pragma unroll
@@ -543,13 +543,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             for (int it = 0; it < Cfg::XI; ++it)
                 dma(xk, last ? xoff[1][it] : xoff[0][it], st + C * TO + (wv * Cfg::XI + it) * 512);
         };
+        const int nsteps = (nk + KG - 1) / KG;
 #pragma unroll
-        for (int k = 0; k < STAGES - 1; ++k) load_stage(min(k, nk - 1), k);
+        for (int k = 0; k < STAGES - 1; ++k) load_stage(k, k);
         int buf = 0;
-        for (int kk = 0; kk < nk; ++kk) {
+        for (int step = 0; step < nsteps; ++step) {
+            const int kk = step * KG + kg;      // past nk in the last step: nothing is kept
             stage_barrier<(STAGES - 2) * (Cfg::YI + Cfg::XI)>();
-            load_stage(min(kk + STAGES - 1, nk - 1), buf == 0 ? STAGES - 1 : buf - 1);
-            const half_t* Ys = smem + buf * Cfg::kStageHalves;
+            load_stage(step + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
+            const half_t* Ys = smem + buf * kRing;
             const half_t* Xs = Ys + C * TO;
             h8 xa[NI], ya[NO];
 #pragma unroll
@@ -574,26 +576,45 @@ __global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
             }
             if (with_bias) {
 #pragma unroll
-                for (int a = 0; a < NO; ++a) accb[a] = mfma32(ya[a], ones, accb[a]);
+                for (int a = 0; a < NO; ++a) acc[a][NI] = mfma32(ya[a], ones, acc[a][NI]);
             }
             __builtin_amdgcn_s_setprio(0);
             buf = buf == STAGES - 1 ? 0 : buf + 1;
         }
         // the last re-requested stages are still on their way into this workgroup's LDS: they land before it ends
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        stage_barrier<0>();
     }
+    f4 own[Sum::kOwn][NI + 1];
+    Sum::run(acc, own, smem_raw, kg, tid & (kThreads - 1));
+    if (kg >= Sum::kFin) return;
     float* po = part + ((int64_t)(s * np + p) * Eo + o0 + TO / 2 * wo) * Ei + c0 + 64 * wi;
 #pragma unroll
-    for (int a = 0; a < NO; ++a)
+    for (int l = 0; l < Sum::kOwn; ++l) {
+        const int o = 16 * (Sum::kFin * l + kg) + 4 * G;
 #pragma unroll
         for (int b = 0; b < NI; ++b)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) po[(int64_t)(16 * a + 4 * G + e) * Ei + 16 * b + i] = acc[a][b][e];
+            for (int e = 0; e < 4; ++e) po[(int64_t)(o + e) * Ei + 16 * b + i] = own[l][b][e];
+    }
     if (with_bias && i == 0) {
         float* pb = bpart + (int64_t)(s * np + p) * Eo + o0 + TO / 2 * wo;
 #pragma unroll
-        for (int a = 0; a < NO; ++a) *reinterpret_cast<f4*>(pb + 16 * a + 4 * G) = accb[a];
+        for (int l = 0; l < Sum::kOwn; ++l) *reinterpret_cast<f4*>(pb + 16 * (Sum::kFin * l + kg) + 4 * G) = own[l][NI];
     }
+}
+
+// work number of this workgroup: each XCD gets a contiguous range (grid = 8 * ceil(work / 8)); >= work: none
+__device__ __forceinline__ int xcd_range(int block, int work) {
+    return (block % kXcds) * ((work + kXcds - 1) / kXcds) + block / kXcds;
+}
+
+template <bool WIDE>
+__global__ __launch_bounds__(kThreads, 2) void k_weight_grad_partial(
+    const half_t* __restrict__ x, WeightGradArgs wa, int64_t ld, float* __restrict__ part, float* __restrict__ bpart, int R,
+    int Eo, int Ei, int np, int nsplit, int rows_per_split) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int work = nsplit * np * (Eo / WeightGradCfg::TO) * (Ei / WeightGradCfg::TI), idx = xcd_range(blockIdx.x, work);
+    if (idx < work) weight_grad_tile<WIDE, 1>(smem_raw, idx, x, wa, ld, part, bpart, R, Eo, Ei, np, rows_per_split);
 }
 
 // ---------------------------------------------------------------------------
@@ -628,12 +649,11 @@ struct InputGradCfg {
 // rows, three of 1024 31.3 -> 19.4 (16.5); 16384 rows, two of 512 28.1 (24.2; 38 as two products); 1024 -> 1024, three 69.3 (57.3).
 // grid = 8 * ceil(tiles / 8), tiles numbered row tile by row tile; each XCD gets a contiguous range.
 template <int BM_, int KG>
-__global__ __launch_bounds__(kThreads * KG, 2) void k_input_grad(InputGradArgs ga, half_t* __restrict__ dx, int R, int Eo,
-                                                                 int Ei, int np, int64_t ld, int tiles) {
+__device__ __forceinline__ void input_grad_tile(unsigned char* smem_raw, int tile, const InputGradArgs& ga,
+                                                half_t* __restrict__ dx, int R, int Eo, int Ei, int np, int64_t ld) {
     using Cfg = InputGradCfg<BM_, KG>;
     using Sum = typename Cfg::Sum;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, STAGES = Cfg::kStages, NR = Cfg::NR, NC = Cfg::NC;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
     const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);      // wave inside its group
@@ -643,9 +663,6 @@ __global__ __launch_bounds__(kThreads * KG, 2) void k_input_grad(InputGradArgs g
     const int i = lane & 15, G = lane >> 4;
     const int wr = wv >> 1, wc = wv & 1;
 
-    const int per_xcd = (tiles + kXcds - 1) / kXcds;
-    const int tile = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-    if (tile >= tiles) return;                         // whole workgroup: padding of the grid
     const int tiles_c = Ei / BN;
     const int row0 = (tile / tiles_c) * BM, c0 = (tile % tiles_c) * BN;
 
@@ -713,6 +730,38 @@ __global__ __launch_bounds__(kThreads * KG, 2) void k_input_grad(InputGradArgs g
             for (int c = 0; c < NC; ++c)
                 *reinterpret_cast<h4*>(dx + (int64_t)r * Ei + c0 + 64 * wc + 16 * c + 4 * G) = to_h4(own[a][c]);
         }
+    }
+}
+
+template <int BM_, int KG>
+__global__ __launch_bounds__(kThreads * KG, 2) void k_input_grad(InputGradArgs ga, half_t* __restrict__ dx, int R, int Eo,
+                                                                 int Ei, int np, int64_t ld, int tiles) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int tile = xcd_range(blockIdx.x, tiles);
+    if (tile < tiles) input_grad_tile<BM_, KG>(smem_raw, tile, ga, dx, R, Eo, Ei, np, ld);
+}
+
+// Input gradient and weight-gradient partials of the same layers in one launch.  Either alone leaves the CUs half empty at
+// its start and its end, and both read dy: an XCD's workgroups take the same range of rows, a tile of dx and one of dW in
+// turn.  Bound by the operands' way from L2 to LDS, as both are.  Measured with the reduction: 8192 rows, 512 -> 512
+// 33.5 us as two launches, 24.0 here; three of 512 47.2 and 40.0; 512 rows, 512 -> 512 16.4 and 10.1.
+// grid = 8 * (ceil(tiles / 8) + ceil(work / 8))
+template <int BM_, int KG>
+__global__ __launch_bounds__(kThreads * KG, 2) void k_linear_grads(
+    InputGradArgs ga, half_t* __restrict__ dx, const half_t* __restrict__ x, WeightGradArgs wa, float* __restrict__ part,
+    float* __restrict__ bpart, int R, int Eo, int Ei, int np, int64_t ld, int tiles, int work, int rows_per_split) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int xcd = blockIdx.x % kXcds, l = blockIdx.x / kXcds;
+    const int nt = (tiles + kXcds - 1) / kXcds, nw = (work + kXcds - 1) / kXcds;      // per XCD
+    const int both = 2 * min(nt, nw);
+    const bool is_dx = l < both ? (l & 1) == 0 : nt > nw;
+    const int at = l < both ? l >> 1 : l - both / 2;
+    if (is_dx) {
+        const int tile = xcd * nt + at;
+        if (at < nt && tile < tiles) input_grad_tile<BM_, KG>(smem_raw, tile, ga, dx, R, Eo, Ei, np, ld);
+    } else {
+        const int idx = xcd * nw + at;
+        if (at < nw && idx < work) weight_grad_tile<false, KG>(smem_raw, idx, x, wa, ld, part, bpart, R, Eo, Ei, np, rows_per_split);
     }
 }
 

@@ -665,3 +665,43 @@ def test_linear_input_grad(R, e_out, e_in, n):
     W = torch.cat(ws, 0).double()
     want, size = dy.double() @ W, dy.double().abs() @ W.abs()
     assert ((dx.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -20 * size + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("e_out,e_in,n", [(128, 128, 1), (128, 256, 3), (384, 128, 2), (512, 512, 3), (1024, 1024, 1)])
+@pytest.mark.parametrize("R", [1, 31, 33, 64, 65, 200, 1000, 2049, 9000])
+def test_linear_grads(R, e_out, e_in, n):
+    """dx, dW and db from one launch over the blocks of a packed gradient, in every tile shape that the plan takes, against
+    fp64: exact products, fp32 sums (a share 2^-20 of the sum of their magnitudes covers the order) and one rounding to
+    fp16.  The last row holds an infinity in x: where rows past the end read it, nothing of it may show up."""
+    import ctypes
+    from rfa_amd import _lib
+    lib = _lib.load()
+    need = lib.rfa_linear_grads_workspace_bytes(R, e_out, e_in, n)
+    assert need > 0
+    gen = torch.Generator("cuda").manual_seed(R + e_out)
+    x = torch.randn(R, e_in, generator=gen, device="cuda").half()
+    x[-1, 5] = float("inf")
+    dy = torch.randn(R, n * e_out, generator=gen, device="cuda").half()
+    ws = [(torch.randn(e_out, e_in, generator=gen, device="cuda") / e_out ** 0.5).half() for _ in range(n)]
+    new = lambda *shape: torch.full(shape, float("nan"), dtype=torch.float16, device="cuda")
+    dx, dw, db = new(R, e_in), [new(e_out, e_in) for _ in range(n)], [new(e_out) for _ in range(n)]
+    work = torch.empty(need, dtype=torch.uint8, device="cuda")
+    array = lambda ptrs: (ctypes.c_void_p * n)(*ptrs)
+    args = (x.data_ptr(), array([dy.data_ptr() + 2 * p * e_out for p in range(n)]), n * e_out, array([w.data_ptr() for w in ws]), n,
+            dx.data_ptr(), array([w.data_ptr() for w in dw]), array([b.data_ptr() for b in db]), R, e_out, e_in, work.data_ptr())
+    stream = torch.cuda.current_stream().cuda_stream
+    print(f"linear_grads R={R} {e_out}->{e_in} x {n}", flush=True)
+    _lib.check(lib.rfa_linear_grads(*args, need, stream))
+    near = lambda got, want, size: ((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -20 * size + 2.0 ** -24).all()
+    W = torch.cat(ws, 0).double()
+    assert near(dx, dy.double() @ W, dy.double().abs() @ W.abs())
+    keep = torch.arange(e_in, device="cuda") != 5
+    for p in range(n):
+        g = dy[:, p * e_out:(p + 1) * e_out].double()
+        xk = x[:, keep].double()
+        assert near(dw[p][:, keep], g.t() @ xk, g.t().abs() @ xk.abs()), p
+        assert torch.isinf(dw[p][:, 5]).all() and (torch.sign(dw[p][:, 5]) == torch.sign(dy[-1, p * e_out:(p + 1) * e_out])).all()
+        assert near(db[p], g.sum(0), g.abs().sum(0)), p
+    assert lib.rfa_linear_grads(*args, need - 1, stream) == -5              # the workspace is checked
+    assert lib.rfa_linear_grads_workspace_bytes(R, e_out + 64, e_in, n) == 0
+    assert lib.rfa_linear_grads_workspace_bytes(1 << 20, e_out, e_in, n) == 0
