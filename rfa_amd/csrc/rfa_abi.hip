@@ -48,14 +48,14 @@ int fail(int code, const char* fmt, ...) {
 namespace prof {
 enum Id { SEG_STATE, CAUSAL_FWD, CAUSAL_BWD_DQ, CAUSAL_BWD_DKDV, CROSS_READOUT, CROSS_READOUT_BWD,
           CROSS_STATE_BWD, DECODE_STEP, FEATURE_FWD, FEATURE_BWD, FEATURE_DW_REDUCE, MASKED_FWD, MASKED_DQ, MASKED_DKDV, PROJECT_PHI, WGRAD_PARTIAL, WGRAD_REDUCE, TOTALS_SCAN, ZERO_FILL,
-          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, COPY_ROWS, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, LINEAR_GRADS, COUNT };
+          SELFTEST, BUILD_W, DECODE_TOUCH, CAUSAL_BWD_SLICED, PACK_MASK, LINEAR_ROWS, CROSS_STEP, MASK_ROWS, INPUT_GRAD, LINEAR_GRADS, COUNT };
 const char* const kNames[COUNT] = {"k_segment_state", "k_causal_fwd", "k_causal_bwd_dq", "k_causal_bwd_dkdv",
                                    "k_cross_readout", "k_cross_readout_bwd", "k_cross_state_bwd", "k_decode_step",
                                    "k_feature_map_fwd", "k_feature_map_bwd", "k_feature_map_dw_reduce",
                                    "k_masked_fwd", "k_masked_dq", "k_masked_dkdv", "k_project_phi",
                                    "k_weight_grad_partial", "k_weight_grad_reduce", "k_totals_scan",
                                    "k_zero_f32", "k_selftest", "k_build_random_matrices", "k_touch_rows",
-                                   "k_sliced_bwd", "k_copy_rows_strided", "k_pack_mask", "k_linear_rows",
+                                   "k_sliced_bwd", "k_pack_mask", "k_linear_rows",
                                    "k_cross_step", "k_mask_rows", "k_input_grad", "k_linear_grads"};
 struct Rec { int id; hipEvent_t a, b; };
 std::mutex mu;
@@ -1086,8 +1086,8 @@ int launch_feature_fwd(const rfa::half_t* x, const rfa::half_t* w, rfa::half_t* 
 }
 
 // dx_rs: halves between consecutive rows of dx / dx1 (H * DH for tensors of their own).  copy_src
-// [R, H * DH] (or NULL) is copied to rows of copy_dst of the same pitch: the third block of a
-// packed gradient, by a third set of workgroups of the same launch where the kernel has that job.
+// [R, H * DH] (or NULL; only with two tensors) is copied to rows of copy_dst of the same pitch: the third block of a
+// packed gradient, half by the workgroups of either tensor.
 template <int D, int DH>
 int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::half_t* gphi, rfa::half_t* dx,
                        const rfa::half_t* x1, const rfa::half_t* gphi1, rfa::half_t* dx1,
@@ -1096,30 +1096,12 @@ int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::ha
                        rfa::half_t* dw16 = nullptr) {
     const int ntens = x1 ? 2 : 1;       // two tensors through the same w: one launch, one reduction
     if (dx_rs == 0) dx_rs = (int64_t)H * DH;
-    int nblk;
-    if constexpr (rfa::FeatureStreamCfg<D, DH>::kFits) {
-        using Cfg = rfa::FeatureStreamCfg<D, DH>;
-        nblk = feature_stream_blocks(R, H, ntens, rfa::kFeatureBwdWaves);      // never more than feature_bwd_blocks, which sized the workspace
-        auto kern = rfa::k_feature_map_bwd_stream<D, DH>;
-        if (int rc = set_lds(kern, Cfg::kLds)) return rc;
-        const bool copy_job = copy_src && ntens == 2;
-        RFA_LAUNCH(FEATURE_BWD, kern, dim3(nblk, H, ntens + (copy_job ? 1 : 0)), dim3(rfa::kFeatureBwdThreads), Cfg::kLds, st,
-                   x, w, gphi, dx, x1, gphi1, dx1, part, R, H, scale, dx_rs, copy_src, copy_dst);
-        if (copy_job) copy_src = nullptr;
-    } else {
-        using Cfg = rfa::FeatureCfg<D, DH>;
-        nblk = feature_bwd_blocks(R, H, ntens);
-        auto kern = rfa::k_feature_map_bwd<D, DH>;
-        if (int rc = set_lds(kern, Cfg::kBwdLds)) return rc;
-        RFA_LAUNCH(FEATURE_BWD, kern, dim3(nblk, H, ntens), dim3(rfa::kThreads), Cfg::kBwdLds, st, x, w, gphi, dx, x1, gphi1,
-                   dx1, part, R, H, scale, dx_rs);
-    }
-    if (copy_src) {
-        const int64_t pieces = (int64_t)R * H * DH / 8;
-        const unsigned blocks = (unsigned)std::min<int64_t>((pieces + rfa::kThreads - 1) / rfa::kThreads, 4 * (int64_t)device_cus());
-        RFA_LAUNCH(COPY_ROWS, rfa::k_copy_rows_strided, dim3(blocks), dim3(rfa::kThreads), 0, st, copy_src, copy_dst, (int64_t)R,
-                   H * DH, dx_rs);
-    }
+    using Cfg = rfa::FeatureBwdCfg<D, DH>;
+    const int nblk = feature_stream_blocks(R, H, ntens, rfa::kFeatureBwdWaves);      // never more than feature_bwd_blocks, which sized the workspace
+    auto kern = rfa::k_feature_map_bwd<D, DH>;
+    if (int rc = set_lds(kern, Cfg::kLds)) return rc;
+    RFA_LAUNCH(FEATURE_BWD, kern, dim3(nblk, H, ntens), dim3(rfa::kFeatureBwdThreads), Cfg::kLds, st,
+               x, w, gphi, dx, x1, gphi1, dx1, (dw || dw16) ? part : nullptr, R, H, scale, dx_rs, copy_src, copy_dst);
     if (!dw && !dw16) {         // dx only: the kernels got no place for partial sums and formed none
         RFA_HIP_TRY(hipGetLastError());
         return RFA_OK;

@@ -210,6 +210,37 @@ def test_feature_map_waves_that_walk_many_row_groups(L, B, H, d, D, wgs, knobs):
     assert _rel(sw.cpu(), rw0) <= GRAD_RTOL
 
 
+@pytest.mark.parametrize("d,D", [(128, 64), (64, 128), (128, 128), (64, 64)])
+@pytest.mark.parametrize("R,wgs", [(1, 0), (15, 0), (127, 1), (128, 1), (129, 1), (257, 2), (1031, 4), (1040, 6)])
+def test_feature_map_backward_where_waves_share_rows(R, wgs, d, D, knobs):
+    """The eight waves' 128 rows contracted together, at row counts around a full round and with workgroups that walk
+    several rounds, some waves of the last one past the end: against the float64 derivative (float16 rounding of du, of
+    the operands and of dx: 1e-2 as above), and the third block of a packed gradient and its dx bit for bit."""
+    from rfa_amd import rfa_hip
+    H = 2
+    x0 = (_randn(R, 1, H, d, seed=60 + R) * 1.2).half()
+    x1 = (_randn(R, 1, H, d, seed=61 + R) * 0.6).half()
+    if R > 1:
+        x0[R // 2] = 0
+    w = (_randn(H, D, d, seed=62) * 0.9).half()
+    g0, g1 = _randn(R, 1, H, 2 * D, seed=63).half(), _randn(R, 1, H, 2 * D, seed=64).half()
+    third = _randn(R, 1, H, d, seed=65).half().cuda()
+    if wgs:
+        knobs(feature_wg=wgs)
+    print(f"phi bwd shared R={R} wgs={wgs} d={d} D={D}", flush=True)
+    dev = [t.cuda() for t in (x0, x1, w, g0, g1)]
+    dx0, dx1, dw = rfa_hip.feature_map_backward_pair(*dev, O.SCALE)
+    sx, sw = rfa_hip.feature_map_backward(dev[0], dev[2], dev[3], O.SCALE)
+    packed, pw = rfa_hip.feature_map_backward_pair_packed(*dev, third, O.SCALE)
+    r0, rw0 = O.random_project_backward(x0.double(), w.double(), g0.double())
+    r1, rw1 = O.random_project_backward(x1.double(), w.double(), g1.double())
+    assert _rel(dx0.double().cpu(), r0) <= GRAD_RTOL and _rel(dx1.double().cpu(), r1) <= GRAD_RTOL
+    assert torch.equal(sx, dx0) and _rel(sw.double().cpu(), rw0) <= GRAD_RTOL
+    assert _rel(dw.double().cpu(), rw0 + rw1) <= GRAD_RTOL
+    E = H * d
+    assert torch.equal(packed, torch.cat([t.view(R, E) for t in (dx0, dx1, third)], 1)) and torch.equal(pw, dw)
+
+
 @pytest.mark.parametrize("H,D,d,tau,with_sigma", [(8, 64, 64, 1.0, True), (3, 32, 128, 0.7, True),
                                                    (2, 128, 64, 2.0, False), (1, 5, 24, 1.3, True)])
 def test_build_random_matrices_matches_the_aten_chain(H, D, d, tau, with_sigma):
