@@ -310,6 +310,16 @@ int rfa_linear_grads(const void* x, const void* const* dy, int64_t ld, const voi
                      void* const* dw, void* const* db, int64_t R, int E_out, int E_in, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* Backward of np layers over x, the first nphi (1 or 2) of which the feature map followed: grad[p] for p < nphi is the gradient
+ * of phi_p (fp16 [R, H, 2D]) and y[p] the layer's output, else grad[p] is that of the output itself (fp16 [R, H * d]).  dx, dw,
+ * db as above with E_out = H * d; dwf (fp16 [H, D, d], or NULL: not wanted) the gradient of wf.  Three launches: the feature
+ * map's, the layers', one reduction of both's partial sums.  Where rfa_project_grads_workspace_bytes answers 0 (see
+ * rfa_linear_grads_workspace_bytes, rfa_feature_map_supported) rfa_feature_map_backward_half and the calls above do the same. */
+size_t rfa_project_grads_workspace_bytes(int64_t R, int H, int D, int d, int E_in, int np, int nphi);
+int rfa_project_grads(const void* x, const void* const* y, const void* wf, const void* const* grad, const void* const* w,
+                      int np, int nphi, void* dx, void* const* dw, void* const* db, void* dwf, int64_t R, int H, int D, int d,
+                      int E_in, float scale, void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* ---------------------------------------------------------------------------
  * Cross attention (encoder -> decoder).  The state is fp32.

@@ -72,6 +72,9 @@ SIGNATURES = {
     "rfa_linear_grads_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
     "rfa_linear_grads": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                  c_int, c_void_p, c_size_t, c_void_p]),
+    "rfa_project_grads_workspace_bytes": (c_size_t, [c_int64] + [c_int] * 6),
+    "rfa_project_grads": (c_int, [c_void_p] * 5 + [c_int, c_int] + [c_void_p] * 4 + [c_int64] + [c_int] * 4 +
+                          [c_float, c_void_p, c_size_t, c_void_p]),
     "rfa_cross_state": (c_int, [c_void_p] * 5 + [c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "rfa_cross_readout": (c_int, [c_void_p] * 4 + [c_int64, c_int64, c_int, c_int, c_void_p]),
     "rfa_cross_step": (c_int, [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),

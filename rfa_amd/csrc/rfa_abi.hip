@@ -1038,10 +1038,10 @@ int launch_linear_grads(const rfa::InputGradArgs& ga, rfa::half_t* dx, const rfa
 }
 
 int launch_weight_grad_reduce(const float* part, const float* bpart, const rfa::WeightGradArgs& wa, int Eo, int Ei, int np,
-                              int nsplit, hipStream_t st) {
+                              int nsplit, const rfa::FeatureSum& fs, hipStream_t st) {
     const int64_t threads = (int64_t)np * ((int64_t)Eo * Ei + Eo) / 4;
-    RFA_LAUNCH(WGRAD_REDUCE, rfa::k_weight_grad_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(rfa::kThreads), 0, st, part,
-               bpart, wa, Eo, Ei, np, nsplit);
+    RFA_LAUNCH(WGRAD_REDUCE, rfa::k_weight_grad_reduce, dim3((unsigned)(fs.blocks + (threads + 255) / 256)), dim3(rfa::kThreads), 0,
+               st, part, bpart, wa, Eo, Ei, np, nsplit, fs);
     RFA_HIP_TRY(hipGetLastError());
     return RFA_OK;
 }
@@ -1087,13 +1087,14 @@ int launch_feature_fwd(const rfa::half_t* x, const rfa::half_t* w, rfa::half_t* 
 
 // dx_rs: halves between consecutive rows of dx / dx1 (H * DH for tensors of their own).  copy_src
 // [R, H * DH] (or NULL; only with two tensors) is copied to rows of copy_dst of the same pitch: the third block of a
-// packed gradient, half by the workgroups of either tensor.
+// packed gradient, half by the workgroups of either tensor.  With `shares` the partial sums are left to the caller to add
+// up: it gets their number.
 template <int D, int DH>
 int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::half_t* gphi, rfa::half_t* dx,
                        const rfa::half_t* x1, const rfa::half_t* gphi1, rfa::half_t* dx1,
                        float* dw, float* part, int R, int H, float scale, hipStream_t st,
                        int64_t dx_rs = 0, const rfa::half_t* copy_src = nullptr, rfa::half_t* copy_dst = nullptr,
-                       rfa::half_t* dw16 = nullptr) {
+                       rfa::half_t* dw16 = nullptr, int* shares = nullptr) {
     const int ntens = x1 ? 2 : 1;       // two tensors through the same w: one launch, one reduction
     if (dx_rs == 0) dx_rs = (int64_t)H * DH;
     using Cfg = rfa::FeatureBwdCfg<D, DH>;
@@ -1101,8 +1102,9 @@ int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::ha
     auto kern = rfa::k_feature_map_bwd<D, DH>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     RFA_LAUNCH(FEATURE_BWD, kern, dim3(nblk, H, ntens), dim3(rfa::kFeatureBwdThreads), Cfg::kLds, st,
-               x, w, gphi, dx, x1, gphi1, dx1, (dw || dw16) ? part : nullptr, R, H, scale, dx_rs, copy_src, copy_dst);
-    if (!dw && !dw16) {         // dx only: the kernels got no place for partial sums and formed none
+               x, w, gphi, dx, x1, gphi1, dx1, (dw || dw16 || shares) ? part : nullptr, R, H, scale, dx_rs, copy_src, copy_dst);
+    if (shares) *shares = ntens * nblk;
+    if (!dw && !dw16) {         // dx only: the kernel got no place for partial sums and formed none; or they stay as they are
         RFA_HIP_TRY(hipGetLastError());
         return RFA_OK;
     }
@@ -2321,13 +2323,52 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
     // R = 0: every split is empty and the partials come out as zeros
     RFA_LAUNCH(WGRAD_PARTIAL, kern, dim3(grid), dim3(rfa::kThreads), lds, st, static_cast<const rfa::half_t*>(x), wa,
                (int64_t)E_out, part, bpart, (int)R, E_out, E_in, np, pl.nsplit, pl.rows_per_split);
-    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.nsplit, st);
+    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.nsplit, {}, st);
 }
 
 size_t rfa_linear_grads_workspace_bytes(int64_t R, int E_out, int E_in, int np) {
     LinearGradsPlan pl;
     if (!make_linear_grads_plan(R, E_out, E_in, np, &pl)) return 0;
     return (size_t)pl.w.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+}
+
+static int linear_grads(const void* x, const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, void* const* dw,
+                        void* const* db, int64_t R, int E_out, int E_in, const LinearGradsPlan& pl, float* part,
+                        const rfa::FeatureSum& fs, hipStream_t st) {
+    rfa::InputGradArgs ga{};
+    rfa::WeightGradArgs wa{};
+    for (int p = 0; p < np; ++p) {
+        ga.dy[p] = wa.dy[p] = static_cast<const rfa::half_t*>(dy[p]);
+        ga.w[p] = static_cast<const rfa::half_t*>(w[p]);
+        wa.dw[p] = static_cast<rfa::half_t*>(dw[p]);
+        wa.db[p] = db ? static_cast<rfa::half_t*>(db[p]) : nullptr;
+    }
+    float* bpart = part + (size_t)pl.w.nsplit * np * E_out * E_in;
+    auto* xh = static_cast<const rfa::half_t*>(x);
+    auto* dxh = static_cast<rfa::half_t*>(dx);
+    int rc;
+    if (pl.t.groups == 1) rc = launch_linear_grads<128, 1>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    else if (pl.t.rows == 64) rc = launch_linear_grads<64, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    else rc = launch_linear_grads<128, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
+    if (rc) return rc;
+    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.w.nsplit, fs, st);
+}
+
+static size_t linear_grads_bytes(const LinearGradsPlan& pl, int np, int E_out, int E_in) {
+    return (size_t)pl.w.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+}
+
+static int check_linear_grads(const char* fn, const void* x, const void* const* dy, const void* const* w, int np, const void* dx,
+                              void* const* dw, void* const* db) {
+    if (!x || !dy || !w || !dx || !dw) return fail(RFA_ERR_NULL_POINTER, "%s: NULL pointer", fn);
+    for (int p = 0; p < np; ++p) {
+        if (!dy[p] || !w[p] || !dw[p]) return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor %d", fn, p);
+        if (!aligned16(dy[p]) || !aligned16(w[p]) || !aligned16(dw[p]) ||
+            (db && (reinterpret_cast<uintptr_t>(db[p]) & 7u)))
+            return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned (bias gradient: 8)", fn);
+    }
+    if (!aligned16(x) || !aligned16(dx)) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+    return RFA_OK;
 }
 
 int rfa_linear_grads(const void* x, const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, void* const* dw,
@@ -2338,33 +2379,73 @@ int rfa_linear_grads(const void* x, const void* const* dy, int64_t ld, const voi
         return fail(RFA_ERR_UNSUPPORTED, "%s: rows=%lld E_out=%d E_in=%d, %d layers are for rfa_linear_input_grad and rfa_linear_weight_grad",
                     fn, (long long)R, E_out, E_in, np);
     if (ld < E_out || ld > (1 << 22) || ld % 8) return fail(RFA_ERR_BAD_SHAPE, "%s: bad row distance ld=%lld for E_out=%d", fn, (long long)ld, E_out);
-    if (!x || !dy || !w || !dx || !dw) return fail(RFA_ERR_NULL_POINTER, "%s: NULL pointer", fn);
-    rfa::InputGradArgs ga{};
-    rfa::WeightGradArgs wa{};
-    for (int p = 0; p < np; ++p) {
-        ga.dy[p] = wa.dy[p] = static_cast<const rfa::half_t*>(dy[p]);
-        ga.w[p] = static_cast<const rfa::half_t*>(w[p]);
-        wa.dw[p] = static_cast<rfa::half_t*>(dw[p]);
-        wa.db[p] = db ? static_cast<rfa::half_t*>(db[p]) : nullptr;
-        if (!ga.dy[p] || !ga.w[p] || !wa.dw[p]) return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor %d", fn, p);
-        if (!aligned16(ga.dy[p]) || !aligned16(ga.w[p]) || !aligned16(wa.dw[p]) || (reinterpret_cast<uintptr_t>(wa.db[p]) & 7u))
-            return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned (bias gradient: 8)", fn);
-    }
-    if (!aligned16(x) || !aligned16(dx)) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
-    const size_t need = (size_t)pl.w.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
+    if (int rc = check_linear_grads(fn, x, dy, w, np, dx, dw, db)) return rc;
+    const size_t need = linear_grads_bytes(pl, np, E_out, E_in);
     if (!workspace || workspace_bytes < need || !aligned16(workspace))
         return fail(RFA_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", fn, need, workspace ? workspace_bytes : (size_t)0);
-    float* part = static_cast<float*>(workspace);
-    float* bpart = part + (size_t)pl.w.nsplit * np * E_out * E_in;
+    return linear_grads(x, dy, ld, w, np, dx, dw, db, R, E_out, E_in, pl, static_cast<float*>(workspace), {},
+                        static_cast<hipStream_t>(stream));
+}
+
+// ---- layers and the feature map behind the first of them --------------------------------
+struct ProjectGradsPlan {
+    LinearGradsPlan linear;
+    size_t dy, feature, bytes;      // workspace: a dy for each mapped layer, the shares of dW', those of the layers
+};
+
+static bool make_project_grads_plan(int64_t R, int H, int D, int d, int Ei, int np, int nphi, ProjectGradsPlan* p) {
+    if (H <= 0 || d <= 0 || H > (1 << 22) / d || !feature_shape_supported(D, d) || nphi < 1 || nphi > 2 || nphi > np ||
+        !make_linear_grads_plan(R, H * d, Ei, np, &p->linear))
+        return false;
+    const auto round = [](size_t n) { return (n + 255) / 256 * 256; };
+    p->dy = round((size_t)R * H * d * 2);
+    p->feature = round((size_t)nphi * rfa_feature_map_backward_workspace_bytes(R, H, D, d));
+    p->bytes = nphi * p->dy + p->feature + linear_grads_bytes(p->linear, np, H * d, Ei);
+    return true;
+}
+
+size_t rfa_project_grads_workspace_bytes(int64_t R, int H, int D, int d, int E_in, int np, int nphi) {
+    ProjectGradsPlan pl;
+    return make_project_grads_plan(R, H, D, d, E_in, np, nphi, &pl) ? pl.bytes : 0;
+}
+
+int rfa_project_grads(const void* x, const void* const* y, const void* wf, const void* const* grad, const void* const* w, int np,
+                      int nphi, void* dx, void* const* dw, void* const* db, void* dwf, int64_t R, int H, int D, int d, int E_in,
+                      float scale, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "rfa_project_grads";
+    ProjectGradsPlan pl;
+    if (!make_project_grads_plan(R, H, D, d, E_in, np, nphi, &pl))
+        return fail(RFA_ERR_UNSUPPORTED, "%s: rows=%lld H=%d D=%d d=%d E_in=%d, %d layers, %d through the feature map are for the calls of its parts",
+                    fn, (long long)R, H, D, d, E_in, np, nphi);
+    if (int rc = check_linear_grads(fn, x, grad, w, np, dx, dw, db)) return rc;
+    if (!y || !y[0] || !y[nphi - 1] || !wf) return fail(RFA_ERR_NULL_POINTER, "%s: NULL pointer", fn);
+    if (!aligned16(y[0]) || !aligned16(y[nphi - 1]) || !aligned16(wf) || !aligned16(dwf))
+        return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+    if (!workspace || workspace_bytes < pl.bytes || !aligned16(workspace))
+        return fail(RFA_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", fn, pl.bytes, workspace ? workspace_bytes : (size_t)0);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    auto* xh = static_cast<const rfa::half_t*>(x);
-    auto* dxh = static_cast<rfa::half_t*>(dx);
-    int rc;
-    if (pl.t.groups == 1) rc = launch_linear_grads<128, 1>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
-    else if (pl.t.rows == 64) rc = launch_linear_grads<64, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
-    else rc = launch_linear_grads<128, 2>(ga, dxh, xh, wa, part, bpart, (int)R, E_out, E_in, np, ld, pl.w, st);
-    if (rc) return rc;
-    return launch_weight_grad_reduce(part, bpart, wa, E_out, E_in, np, pl.w.nsplit, st);
+    auto* base = static_cast<unsigned char*>(workspace);
+    void* dy0 = base;
+    void* dy1 = nphi > 1 ? base + pl.dy : nullptr;
+    auto* fpart = reinterpret_cast<float*>(base + nphi * pl.dy);
+    auto half = [](const void* p) { return static_cast<const rfa::half_t*>(p); };
+    auto features = [&](int* shares) {
+#define RFA_CALL(DD, DH)                                                                                                        \
+        launch_feature_bwd<DD, DH>(half(y[0]), half(wf), half(grad[0]), static_cast<rfa::half_t*>(dy0), nphi > 1 ? half(y[1]) : nullptr, \
+                                   nphi > 1 ? half(grad[1]) : nullptr, static_cast<rfa::half_t*>(dy1), nullptr, fpart, (int)R, H, scale, st,  \
+                                   0, nullptr, nullptr, nullptr, shares)
+        RFA_DISPATCH_FEATURE(D, d, RFA_CALL)
+#undef RFA_CALL
+        return fail(RFA_ERR_UNSUPPORTED, "unreachable");
+    };
+    int shares = 0;
+    if (int rc = features(dwf ? &shares : nullptr)) return rc;
+    const void* dy[rfa::kMaxProjections] = {};
+    for (int p = 0; p < np; ++p) dy[p] = p == 0 ? dy0 : p < nphi ? dy1 : grad[p];
+    rfa::FeatureSum fs{};
+    if (dwf) fs = {fpart, static_cast<rfa::half_t*>(dwf), H * D * d / 256, shares};
+    return linear_grads(x, dy, H * d, w, np, dx, dw, db, R, H * d, E_in, pl.linear,
+                        reinterpret_cast<float*>(base + nphi * pl.dy + pl.feature), fs, st);
 }
 
 // ---- profiling ----------------------------------------------------------------------

@@ -96,6 +96,14 @@ bool plain_matrices(const Tensor& w, const OptTensor& sigma, double tau) {
 }
 
 // ---- feature map ------------------------------------------------------------------------
+void check_feature_grad(const Tensor& x, const Tensor& x0, const Tensor& w, const Tensor& g) {
+    check_feature_args(x, w);
+    check_half("grad_phi", g, 4);
+    TORCH_CHECK_VALUE(x.sizes() == x0.sizes() && g.size(0) == x0.size(0) && g.size(1) == x0.size(1) && g.size(2) == x0.size(2) &&
+                          g.size(3) == 2 * w.size(1), "grad_phi ", g.sizes(), " does not fit x ", x0.sizes(), " and ", w.size(1),
+                      " features");
+}
+
 // dx of one or two tensors through the same w, or the packed gradient [dx0 | dx1 | third] in `packed`; returns dW'
 // in fp16, undefined where w takes no gradient
 Tensor feature_grads(const Tensor& x0, const Tensor* x1, const Tensor& w, const Tensor& g0, const Tensor* g1,
@@ -108,14 +116,8 @@ Tensor feature_grads(const Tensor& x0, const Tensor* x1, const Tensor& w, const 
     }
     const int64_t R = x0.size(0) * x0.size(1);
     const int H = (int)x0.size(2), d = (int)x0.size(3), D = (int)w.size(1);
-    auto check = [&](const Tensor& x, const Tensor& g) {
-        check_feature_args(x, w);
-        check_half("grad_phi", g, 4);
-        TORCH_CHECK_VALUE(x.sizes() == x0.sizes() && g.size(0) == x0.size(0) && g.size(1) == x0.size(1) && g.size(2) == H &&
-                              g.size(3) == 2 * D, "grad_phi ", g.sizes(), " does not fit x ", x0.sizes(), " and ", D, " features");
-    };
-    check(x0, g0);
-    if (x1) check(*x1, *g1);
+    check_feature_grad(x0, x0, w, g0);
+    if (x1) check_feature_grad(*x1, x0, w, *g1);
     if (third) TORCH_CHECK_VALUE(third->numel() == x0.numel() && third->is_contiguous(), "third must hold the rows of x");
     dx0 = packed ? torch::empty({R, 3 * (int64_t)H * d}, x0.options()) : torch::empty_like(x0);
     if (x1 && !packed) *dx1 = torch::empty_like(*x1);
@@ -242,6 +244,41 @@ bool linear_grads(const std::vector<const void*>& dys, int64_t ld, const Tensor*
     return true;
 }
 
+// Those gradients and the feature map's where the library takes all of it: the first nphi layers went through the feature
+// map (outputs y), g their gradients, else those of the layers' outputs.  dwf as feature_grads.
+bool project_grads(const variable_list& g, const Tensor* y, int64_t nphi, const Tensor& wf, const Tensor* w, int64_t n, const Tensor& x,
+                   const std::vector<bool>& bias, double scale, bool need_wf, Tensor& dx, std::vector<Tensor>& dw,
+                   std::vector<OptTensor>& db, Tensor& dwf) {
+    const int64_t e_out = w[0].size(0), e_in = w[0].size(1), rows = x.size(0) * x.size(1);
+    const int H = (int)y[0].size(2), d = (int)y[0].size(3), D = (int)wf.size(1);
+    const size_t nbytes = rfa_project_grads_workspace_bytes(rows, H, D, d, (int)e_in, (int)n, (int)nphi);
+    if (nbytes == 0 || !aligned16(x) || !x.is_contiguous()) return false;
+    std::array<Tensor, 3> gc;
+    for (int64_t p = 0; p < n; ++p) {
+        gc[p] = g[p].contiguous();
+        if (!aligned16(gc[p])) return false;
+    }
+    for (int64_t p = 0; p < nphi; ++p) check_feature_grad(y[p], y[0], wf, gc[p]);
+    std::array<const void*, 3> wp{}, gp{}, yp{};
+    std::array<void*, 3> dwp{}, dbp{};
+    for (int64_t p = 0; p < n; ++p) {
+        wp[p] = ptr(w[p]);
+        gp[p] = ptr(gc[p]);
+        if (p < nphi) yp[p] = ptr(y[p]);
+        dw.push_back(torch::empty({e_out, e_in}, x.options()));
+        db.push_back(bias[p] ? OptTensor(torch::empty({e_out}, x.options())) : c10::nullopt);
+        dwp[p] = ptr(dw[p]);
+        dbp[p] = ptr(db[p]);
+    }
+    dx = torch::empty(x.sizes(), x.options());
+    if (need_wf) dwf = torch::empty({H, D, d}, x.options());
+    Launch l(x);
+    Tensor ws = workspace(nbytes, x);
+    check_rc(rfa_project_grads(ptr(x), yp.data(), ptr(wf), gp.data(), wp.data(), (int)n, (int)nphi, ptr(dx), dwp.data(), dbp.data(),
+                               need_wf ? ptr(dwf) : nullptr, rows, H, D, d, (int)e_in, (float)scale, ptr(ws), nbytes, l.stream));
+    return true;
+}
+
 struct ProjectNode : public torch::autograd::Function<ProjectNode> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& wf, double scale, int64_t heads,
                                  int64_t phi, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
@@ -293,7 +330,16 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
         std::vector<bool> bias;
         for (int64_t p = 0; p < n; ++p) bias.push_back((bias_bits >> p) & 1);
         Tensor dwf;
-        if (n == 3 && phi == 3 && need_x) {
+        const bool own_x = need_x && own_input_grad(rows, w, n);
+        std::vector<Tensor> dw;
+        std::vector<OptTensor> db;
+        if (own_x && (phi == 1 || phi == 3) &&
+            project_grads(g, y, phi == 3 ? 2 : 1, wf, w, n, x, bias, scale, need_wf, out[0], dw, db, dwf)) {
+            for (int64_t p = 0; p < n; ++p) {
+                out[5 + 2 * p] = dw[p];
+                out[6 + 2 * p] = opt(db[p]);
+            }
+        } else if (n == 3 && phi == 3 && need_x) {
             // [dy_q | dy_k | dv] side by side, written by the feature-map backward launch itself: one
             // GEMM for dx and one contraction for the three weight gradients
             const int64_t e_out = w[0].size(0);
@@ -302,18 +348,7 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
             dwf = feature_grads(y[0], &y[1], wf, g0, &g1, &g2, packed, nullptr, true, scale, need_wf);
             const char* base = static_cast<const char*>(packed.data_ptr());
             const std::vector<const void*> dyp{base, base + 2 * e_out, base + 4 * e_out};
-            const bool own = own_input_grad(rows, w, 3);
-            std::vector<Tensor> dw;
-            std::vector<OptTensor> db;
-            if (own && linear_grads(dyp, 3 * e_out, w, x, x2, bias, out[0], dw, db)) {
-                for (int64_t p = 0; p < n; ++p) {
-                    out[5 + 2 * p] = dw[p];
-                    out[6 + 2 * p] = opt(db[p]);
-                }
-                out[1] = dwf;
-                return out;
-            }
-            out[0] = own ? input_grad(dyp, 3 * e_out, w, x) : at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
+            out[0] = own_x ? input_grad(dyp, 3 * e_out, w, x) : at::mm(packed, at::cat({w[0], w[1], w[2]}, 0)).view(x.sizes());
             auto [dws, dbs] = param_grads(x2, {packed}, {bias_bits != 0});
             for (int64_t p = 0; p < n; ++p) {
                 out[5 + 2 * p] = dws[0].narrow(0, p * e_out, e_out);
@@ -335,22 +370,20 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
                 }
                 dys[p] = dys[p].reshape({rows, -1});
             }
-            bool own = need_x && own_input_grad(rows, w, n);
+            bool own = own_x;
             for (const Tensor& dy : dys) own = own && aligned16(dy);
-            std::vector<Tensor> dws;
-            std::vector<OptTensor> dbs;
             std::vector<const void*> dyp;
             for (Tensor& dy : dys) dyp.push_back(ptr(dy));
-            if (!own || !linear_grads(dyp, w[0].size(0), w, x, x2, bias, out[0], dws, dbs)) {
+            if (!own || !linear_grads(dyp, w[0].size(0), w, x, x2, bias, out[0], dw, db)) {
                 if (own) out[0] = input_grad(dyp, w[0].size(0), w, x);
                 for (int64_t p = 0; p < n && need_x && !own; ++p) {
                     out[0] = out[0].defined() ? out[0].addmm_(dys[p], w[p]) : at::mm(dys[p], w[p]);
                 }
-                std::tie(dws, dbs) = param_grads(x2, dys, bias);
+                std::tie(dw, db) = param_grads(x2, dys, bias);
             }
             for (int64_t p = 0; p < n; ++p) {
-                out[5 + 2 * p] = dws[p];
-                out[6 + 2 * p] = opt(dbs[p]);
+                out[5 + 2 * p] = dw[p];
+                out[6 + 2 * p] = opt(db[p]);
             }
             if (out[0].defined()) out[0] = out[0].view(x.sizes());
         }

@@ -404,13 +404,11 @@ __global__ __launch_bounds__(kFeatureBwdThreads) void k_feature_map_bwd(
 // conversion launch behind it (2.1 to 4.7 us, and 5 of host time).  One workgroup of 4 waves per 256 consecutive elements
 // (64 lanes x 16 bytes); wave p sums the shares b = p, p+4, ... with all its loads in
 // flight at once, then the 4 waves are added through LDS.  elems % 256 == 0.
-__global__ __launch_bounds__(kThreads) void k_feature_map_dw_reduce(const float* __restrict__ part,
-                                                                    float* __restrict__ dw,
-                                                                    half_t* __restrict__ dw16, int nblk,
-                                                                    int64_t elems) {
+__device__ __forceinline__ void feature_map_dw_sum(int block, const float* __restrict__ part, float* __restrict__ dw,
+                                                   half_t* __restrict__ dw16, int nblk, int64_t elems) {
     __shared__ f4 red[3][64];
     const int lane = threadIdx.x & 63, p = threadIdx.x >> 6;
-    const int64_t e = ((int64_t)blockIdx.x * 64 + lane) * 4;
+    const int64_t e = ((int64_t)block * 64 + lane) * 4;
     f4 acc = f4_zero();
     int b = p;
     for (; b + 28 < nblk; b += 32) {
@@ -430,6 +428,13 @@ __global__ __launch_bounds__(kThreads) void k_feature_map_dw_reduce(const float*
         if (dw16) *reinterpret_cast<h4*>(dw16 + e) = to_h4(acc);
         else *reinterpret_cast<f4*>(dw + e) = acc;
     }
+}
+
+__global__ __launch_bounds__(kThreads) void k_feature_map_dw_reduce(const float* __restrict__ part,
+                                                                    float* __restrict__ dw,
+                                                                    half_t* __restrict__ dw16, int nblk,
+                                                                    int64_t elems) {
+    feature_map_dw_sum(blockIdx.x, part, dw, dw16, nblk, elems);
 }
 
 // W' = (sigma * W if sigma) / tau, one element per thread, in the reference's own arithmetic

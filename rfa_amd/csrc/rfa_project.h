@@ -765,12 +765,27 @@ __global__ __launch_bounds__(kThreads * KG, 2) void k_linear_grads(
     }
 }
 
-// dW_p = sum of the partials (4 elements per thread), then db_p; grid = ceil(np * (Eo * Ei + Eo) / 4 / 256)
+// The feature map's dW' where its shares are summed beside those of the layers: `blocks` workgroups come first, one per
+// 256 elements (0: none).
+struct FeatureSum {
+    const float* part;
+    half_t* dw;
+    int blocks, shares;
+};
+
+// dW_p = sum of the partials (4 elements per thread), then db_p; grid = fs.blocks + ceil(np * (Eo * Ei + Eo) / 4 / 256).
+// What bounds it is one round trip to memory behind a launch, so the feature map's shares are summed beside the layers': the
+// reductions of a layer in training (8192 rows, three layers and one of 512, 64 features) 13.8 us in three launches, 10.4 in
+// two; those of an encoder-decoder layer 27.5 in five, 17.5 in three.
 __global__ __launch_bounds__(kThreads) void k_weight_grad_reduce(
     const float* __restrict__ part, const float* __restrict__ bpart, WeightGradArgs wa, int Eo, int Ei, int np,
-    int nsplit) {
+    int nsplit, FeatureSum fs) {
+    if ((int)blockIdx.x < fs.blocks) {
+        feature_map_dw_sum(blockIdx.x, fs.part, nullptr, fs.dw, fs.shares, (int64_t)fs.blocks * 256);
+        return;
+    }
     const int64_t per_w = (int64_t)Eo * Ei / 4, per_b = Eo / 4;
-    const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int64_t t = (int64_t)((int)blockIdx.x - fs.blocks) * kThreads + threadIdx.x;
     if (t < per_w * np) {
         const int p = (int)(t / per_w);
         const int64_t q = t % per_w;

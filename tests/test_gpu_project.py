@@ -705,3 +705,59 @@ def test_linear_grads(R, e_out, e_in, n):
     assert lib.rfa_linear_grads(*args, need - 1, stream) == -5              # the workspace is checked
     assert lib.rfa_linear_grads_workspace_bytes(R, e_out + 64, e_in, n) == 0
     assert lib.rfa_linear_grads_workspace_bytes(1 << 20, e_out, e_in, n) == 0
+
+
+@pytest.mark.parametrize("H,D,d,e_in,n,nphi", [(2, 64, 64, 128, 3, 2), (8, 64, 64, 512, 2, 1), (1, 128, 128, 256, 1, 1),
+                                               (4, 32, 64, 128, 2, 2), (2, 64, 128, 256, 3, 1)])
+@pytest.mark.parametrize("R", [1, 65, 300, 2049])
+def test_project_grads(R, H, D, d, e_in, n, nphi):
+    """Layers and the feature map behind the first of them, with one reduction for both: the bits of the calls of its parts."""
+    import ctypes
+    from rfa_amd import _lib
+    lib = _lib.load()
+    need = lib.rfa_project_grads_workspace_bytes(R, H, D, d, e_in, n, nphi)
+    e_out = H * d
+    assert need > 0
+    gen = torch.Generator("cuda").manual_seed(R + e_in)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").half()
+    new = lambda *shape: torch.full(shape, float("nan"), dtype=torch.float16, device="cuda")
+    x, wf = rand(R, e_in), rand(H, D, d)
+    y = [rand(R, e_out) for _ in range(nphi)]
+    grad = [rand(R, 2 * H * D) for _ in range(nphi)] + [rand(R, e_out) for _ in range(n - nphi)]
+    ws = [(rand(e_out, e_in) / e_out ** 0.5).half() for _ in range(n)]
+    work = torch.empty(need, dtype=torch.uint8, device="cuda")
+    array = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() if t is not None else None for t in ts])
+    stream = torch.cuda.current_stream().cuda_stream
+    print(f"project_grads R={R} H={H} D={D} d={d} E={e_in} layers={n} mapped={nphi}", flush=True)
+
+    def whole(with_wf, with_bias, nbytes=need):
+        dx, dw, dwf = new(R, e_in), [new(e_out, e_in) for _ in range(n)], new(H, D, d)
+        db = [new(e_out) if with_bias else None for _ in range(n)]
+        rc = lib.rfa_project_grads(x.data_ptr(), array(y), wf.data_ptr(), array(grad), array(ws), n, nphi, dx.data_ptr(), array(dw),
+                                   array(db), dwf.data_ptr() if with_wf else None, R, H, D, d, e_in, 0.3, work.data_ptr(), nbytes,
+                                   stream)
+        return rc, dx, dw, db, dwf
+
+    dy, dwf = [new(R, e_out) for _ in range(nphi)] + grad[nphi:], new(H, D, d)
+    fbytes = 2 * lib.rfa_feature_map_backward_workspace_bytes(R, H, D, d)
+    fwork = torch.empty(fbytes, dtype=torch.uint8, device="cuda")
+    two = nphi == 2
+    _lib.check(lib.rfa_feature_map_backward_half(
+        y[0].data_ptr(), y[1].data_ptr() if two else None, wf.data_ptr(), grad[0].data_ptr(), grad[1].data_ptr() if two else None,
+        None, dy[0].data_ptr(), dy[1].data_ptr() if two else None, None, dwf.data_ptr(), R, H, D, d, 0.3, fwork.data_ptr(), fbytes,
+        stream))
+    lbytes = lib.rfa_linear_grads_workspace_bytes(R, e_out, e_in, n)
+    lwork = torch.empty(lbytes, dtype=torch.uint8, device="cuda")
+    dx, dw, db = new(R, e_in), [new(e_out, e_in) for _ in range(n)], [new(e_out) for _ in range(n)]
+    _lib.check(lib.rfa_linear_grads(x.data_ptr(), array(dy), e_out, array(ws), n, dx.data_ptr(), array(dw), array(db), R, e_out, e_in,
+                                    lwork.data_ptr(), lbytes, stream))
+    for with_wf, with_bias in ((True, True), (False, True), (True, False)):
+        rc, gx, gw, gb, gwf = whole(with_wf, with_bias)
+        _lib.check(rc)
+        assert torch.equal(gx, dx) and all(torch.equal(a, b) for a, b in zip(gw, dw))
+        assert not with_bias or all(torch.equal(a, b) for a, b in zip(gb, db))
+        assert torch.equal(gwf, dwf) if with_wf else torch.isnan(gwf).all()
+    assert whole(True, True, need - 1)[0] == -5                             # the workspace is checked
+    assert lib.rfa_project_grads_workspace_bytes(R, H, D, 96, e_in, n, nphi) == 0
+    assert lib.rfa_project_grads_workspace_bytes(1 << 20, H, D, d, e_in, n, nphi) == 0
+    assert lib.rfa_project_grads_workspace_bytes(R, H, D, d, e_in, n, n + 1) == 0
