@@ -1964,9 +1964,11 @@ int rfa_build_random_matrices_backward(const void* w, const void* sigma, const v
         return fail(RFA_ERR_NULL_POINTER, "rfa_build_random_matrices_backward: dsigma asked for without sigma");
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto* gh = static_cast<const rfa::half_t*>(grad_out);
-    if (dsigma)
-        RFA_LAUNCH(BUILD_W, rfa::k_build_random_matrices_dsigma, dim3((unsigned)H), dim3(rfa::kThreads), 0, st,
-                   static_cast<const rfa::half_t*>(w), gh, static_cast<rfa::half_t*>(dsigma), tau, D, d);
+    if (dsigma) {
+        const int nb = std::max(1, std::min((d + 63) / 64, (1 << 20) / H));      // 2^31 threads at most
+        RFA_LAUNCH(BUILD_W, rfa::k_build_random_matrices_dsigma, dim3((unsigned)H * nb), dim3(64 * rfa::kDsigmaWaves), 0, st,
+                   static_cast<const rfa::half_t*>(w), gh, static_cast<rfa::half_t*>(dsigma), tau, D, d, nb);
+    }
     if (dw) {
         const int64_t total = (int64_t)H * D * d;
         RFA_LAUNCH(BUILD_W, rfa::k_build_random_matrices_dw, dim3((unsigned)((total + rfa::kThreads - 1) / rfa::kThreads)),

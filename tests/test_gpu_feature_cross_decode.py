@@ -277,6 +277,19 @@ def test_build_random_matrices_matches_the_aten_chain(H, D, d, tau, with_sigma):
         assert torch.equal(sf2.grad, sf.grad)
 
 
+@pytest.mark.parametrize("H,D,d", [(1, 1, 1), (2, 15, 63), (3, 17, 65), (2, 128, 128), (1, 129, 130), (2, 300, 64)])
+def test_build_random_matrices_sigma_gradient(H, D, d):
+    """Around the 16 rows and 64 columns that a workgroup of the sigma gradient takes at once, against the sum of the same
+    fp16 products in float64: D fp32 additions (2^-24 each, of the sum of magnitudes) and one rounding to fp16."""
+    from rfa_amd import rfa_hip
+    print(f"dsigma H={H} D={D} d={d}", flush=True)
+    w, g, sigma = _randn(H, D, d, seed=910).half(), _randn(H, D, d, seed=911).half(), _randn(H, 1, d, seed=912).half()
+    got, _ = rfa_hip.build_random_matrices_backward(w.cuda(), sigma.cuda(), g.cuda(), 0.7, True, False)
+    prod = ((g.float() / 0.7).half().float() * w.float()).half().double()
+    want, size = prod.sum(1, keepdim=True), prod.abs().sum(1, keepdim=True)
+    assert ((got.double().cpu().view_as(want) - want).abs() <= 2.0 ** -11 * want.abs() + D * 2.0 ** -24 * size + 2.0 ** -25).all()
+
+
 # ------------------------------------------------------------------------ cross
 def _cross_inputs(S, T, B, H, d, D, seed, lengths=None):
     W = O.make_w(d, D, H)
