@@ -2228,16 +2228,26 @@ int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int
     auto* wh = static_cast<const rfa::half_t*>(w);
     auto* bh = static_cast<const rfa::half_t*>(bias);
     auto* yh = static_cast<rfa::half_t*>(y);
-    const int rt = R <= 16 ? 1 : R <= 32 ? 2 : 4;
-    // two tiles of columns per workgroup (half the reads of x) once one tile each would overfill the chip
-    const int64_t row_blocks = (R + 16 * rt - 1) / (16 * rt);
-    const int ct = rt == 4 && row_blocks * (e_out / 16) > device_cus() ? 2 : 1;
-    const dim3 grid((unsigned)((e_out / 16 + ct - 1) / ct), (unsigned)row_blocks);
+    // The tile whose workgroups keep a CU busy shortest: rounds of workgroups times the rows of x and W that one reads;
+    // between equals the larger tile, whose operands are read by fewer.  Device us, 16 x 16 / 32 x 16 / 32 x 32 / 64 x 32 rows x
+    // columns (64 x 16 is nowhere the best): 64 rows 512 -> 512 2.8 / 3.3 / 3.8 / 5.0, 512 -> 1536 3.7 / 3.4 / 3.9 / 5.0,
+    // 1024 -> 1024 3.7 / 4.6 / 5.6 / 7.6, 1024 -> 3072 7.7 / 7.6 / 6.3 / 8.3; 512 rows 512 -> 512 5.6 / 4.7 / 3.9 / 5.1; 320 rows
+    // 1024 -> 1024 10.6 / 9.9 / 9.1 / 7.7; 32 rows 512 -> 6144 5.1 / 5.1 / 4.4 / 4.8.
+    static constexpr uint32_t kTiles[][2] = {{4, 2}, {2, 2}, {2, 1}, {1, 1}};
+    uint32_t rt = 0, ct = 0;
+    uint64_t least = 0;
+    const uint32_t cus = device_cus(), rows16 = ((uint32_t)R + 15) / 16, cols16 = e_out / 16;      // at most 2^16, 2^27
+    for (const auto& t : kTiles) {
+        const uint64_t wgs = (uint64_t)((rows16 + t[0] - 1) / t[0]) * ((cols16 + t[1] - 1) / t[1]);
+        const uint64_t cost = (wgs + cus - 1) / cus * (t[0] + t[1]);
+        if (rt == 0 || cost < least) { rt = t[0]; ct = t[1]; least = cost; }
+    }
+    const dim3 grid((cols16 + ct - 1) / ct, (rows16 + rt - 1) / rt);
 #define RFA_ROWS(RT, CT) \
     RFA_LAUNCH(LINEAR_ROWS, (rfa::k_linear_rows<RT, CT>), grid, dim3(rfa::kThreads), 0, st, xh, wh, bh, yh, (int)R, e_in, e_out)
     if (rt == 1) { RFA_ROWS(1, 1); }
-    else if (rt == 2) { RFA_ROWS(2, 1); }
-    else if (ct == 1) { RFA_ROWS(4, 1); }
+    else if (ct == 1) { RFA_ROWS(2, 1); }
+    else if (rt == 2) { RFA_ROWS(2, 2); }
     else { RFA_ROWS(4, 2); }
 #undef RFA_ROWS
     RFA_HIP_TRY(hipGetLastError());

@@ -479,8 +479,8 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
 
 // Without autograd the row kernel takes up to 512 rows while its workgroups (64 rows x 32 columns) are at most one to
 // a CU and the contraction is short (four waves share E_in), or a few rows of anything up to 192 M products.
-// Device us there, row kernel / library: 512 -> 512 64 rows 4.4 / 5.6, 512 rows 4.7 / 5.2; 1024 -> 3072 64 rows 7.1 / 8.3,
-// 128 rows 8.9 / 9.2; at worst 768 -> 2304 96 rows 7.9 / 6.3, 1024 -> 1024 320 rows 8.4 / 6.5; 2048 -> 2048 32 rows 7.7 /
+// Device us there, row kernel / library: 512 -> 512 64 rows 2.8 / 5.6, 512 rows 3.9 / 5.2; 1024 -> 3072 64 rows 6.3 / 8.3,
+// 128 rows 8.4 / 9.2; 768 -> 2304 96 rows 5.4 / 6.3; at worst 1024 -> 1024 320 rows 7.7 / 6.5; 2048 -> 2048 32 rows 7.7 /
 // 8.4.  Past it two rounds of workgroups: 1024 -> 1024 768 rows 14.0 / 8.7; rows of x that every column tile reads again,
 // from other XCDs' caches where they were just written (a layer's forward over 1024 rows of 512: 26.9 with the output
 // projection by it, 25.0 by the projection kernel); a long contraction: 2048 -> 2048 64 rows 11.2 / 8.9.

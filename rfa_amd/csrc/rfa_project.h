@@ -337,15 +337,16 @@ __global__ __launch_bounds__(kThreads * KG, 2) void k_project_phi(
 // ---------------------------------------------------------------------------
 // y[r][o] = x[r] . W[o] + b[o] for few rows: the projections of a decoding step.
 //
-// What bounds it is the trips to memory and the launch around them: a workgroup of four waves owns 16 columns (16 rows of
-// W) of up to 64 rows of x, the waves share the contraction, each with four 32-deep steps in flight together (the
+// What bounds it is the trips to memory and the launch around them: a workgroup of four waves owns 16 or 32 columns (rows of
+// W) of 16 to 64 rows of x, the waves share the contraction, each with four 32-deep steps in flight together (the
 // loads of a batch before its first product, no branch between them), operands straight from memory in the
 // lanes' own order; the four partial sums meet in LDS.  A lane's 16 bytes lie a whole row from its neighbour's, so
-// a load asks for 16 lines, and x is read again for every 16 columns: from 64 rows on these reads bound the kernel,
-// and 32 columns per workgroup halve them where that still leaves a workgroup per CU.
-// Measured, device us with the loads of a batch one behind the other / now / the library's product (which costs 19 us
-// of host time, this 4): 4 rows 512 -> 1536 2.9 / 2.8 / 3.9, 1024 -> 3072 4.2 / 3.8 / 5.7; 64 rows 512 -> 512 4.6 /
-// 4.4 / 5.6, 768 -> 768 6.8 / 6.1 / 5.7, 1024 -> 3072 7.7 / 7.1 / 8.3; 320 rows 1024 -> 1024 9.1 / 8.4 / 6.5.
+// a load asks for 16 lines: what a CU asks for decides, so the tile is the smallest that one round of workgroups allows.
+// Every tile adds in the same order: y of a row is the same whatever rows it comes with.
+// Measured, device us with 64 x 16 from 33 rows on and 64 x 32 past a workgroup per CU / now / the library's product (which
+// costs 19 us of host time, this 4): 4 rows 512 -> 1536 2.6 / 2.6 / 3.9, 1024 -> 3072 3.6 / 3.6 / 5.7; 64 rows 512 -> 512 4.2 /
+// 2.8 / 5.6, 768 -> 768 5.9 / 3.5 / 5.7, 1024 -> 1024 6.4 / 3.7, 1024 -> 3072 6.9 / 6.3 / 8.3; 160 rows 512 -> 512 4.3 / 3.3; 320 rows
+// 1024 -> 1024 7.7 / 7.7 / 6.5.  Eight waves with two steps each: 64 rows 1024 -> 3072 6.1, 768 -> 768 4.0, else the same.
 // grid = (ceil(Eo / (16 CT)), ceil(R / (16 RT)));  E % 32 == 0, Eo % 16 == 0
 // ---------------------------------------------------------------------------
 template <int RT, int CT>

@@ -586,6 +586,27 @@ def test_linear_rows_where_the_choice_changes(R, e_in, e_out):
     assert ((y.double() - want).abs() <= 2.0 ** -10 * want.abs() + 2e-5).all()
 
 
+@pytest.mark.parametrize("e_in,e_out", [(512, 512), (512, 1536), (1024, 1024), (1024, 3072), (160, 48)])
+def test_linear_rows_are_the_same_in_every_tile(e_in, e_out):
+    """The tile goes by rounds of workgroups; every tile adds a row's products in one order, so a row has the same bits
+    whatever rows it comes with: one at a time (16 x 16) against counts that take each tile, with rows past the last one."""
+    from rfa_amd import projection, rfa_hip
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    gen = torch.Generator("cuda").manual_seed(e_out)
+    x = torch.randn(256, e_in, generator=gen, device="cuda").half()
+    w = (torch.randn(e_out, e_in, generator=gen, device="cuda") / e_in ** 0.5).half()
+    b = torch.randn(e_out, generator=gen, device="cuda").half()
+    print(f"linear_rows in every tile {e_in}->{e_out}", flush=True)
+    with torch.no_grad():
+        one = [projection.linear_rows(x[r:r + 1], w, b) for r in (0, 17, 40)]
+        for R in (41, 64, 79, 128, 160, 256):
+            y = projection.linear_rows(x[:R], w, b)
+            if -(-R // 64) * -(-e_out // 32) > torch.cuda.get_device_properties(0).multi_processor_count:
+                continue                                     # another kernel's
+            assert all(torch.equal(y[r:r + 1], o) for r, o in zip((0, 17, 40), one)), R
+
+
 @pytest.mark.parametrize("e_in", [(1 << 22) + 128, (1 << 25) + 128])
 def test_output_projection_wider_than_the_kernels_address(e_in):
     """Widths that the input-gradient launch (2^22) and the projection launch (2^25) refuse go to the library."""
