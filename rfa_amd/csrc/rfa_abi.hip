@@ -330,14 +330,14 @@ double estimate_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cu
 // without totals beat four launches however few CUs they cover (T 256, 16 sequences) 38.3 / 20.9; (512, 8) 41.3 / 27.6;
 // single chunks as segments (1024, 4) 49.2 / 41.2; fewer, longer segments (4096, 24) 141 / 108.
 ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
-    const ScanPlan base = cover_plan(T, N, K, d);
-    if (T <= 0 || N <= 0 || tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0) return base;
+    if (T <= 0 || N <= 0 || tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0) return cover_plan(T, N, K, d);
     // called several times for one operation: the last answer of this thread, by all that goes into it
     struct Memo { int64_t T, N; int K, d, cus; unsigned knobs; ScanPlan plan; };
-    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, base};
+    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, {}};
     const int cus = device_cus();
     const unsigned knobs = tune::changes.load(std::memory_order_acquire);
     if (memo.T == T && memo.N == N && memo.K == K && memo.d == d && memo.cus == cus && memo.knobs == knobs) return memo.plan;
+    const ScanPlan base = cover_plan(T, N, K, d);
     const int64_t nchunks = (T + rfa::kChunk - 1) / rfa::kChunk;
     ScanPlan best = base;
     const double start = estimate_us(base, T, N, K, d, cus);
