@@ -59,6 +59,14 @@ void check_saved(const char* name, const Tensor& t, const Tensor& like) {
     TORCH_CHECK_TYPE(t.scalar_type() == torch::kFloat16, name, " must be float16 (got ", t.scalar_type(), ")");
 }
 
+// and the shapes, where launches take them together: layers w [e_out, E] over x [.., E] whose outputs have `rows` rows
+void check_saved_layers(const Tensor& x, const Tensor* w, int64_t n, int64_t rows, int64_t e_out) {
+    const int64_t e_in = x.dim() > 0 ? x.size(-1) : 0;
+    bool ok = x.dim() > 0 && x.numel() == rows * e_in;
+    for (int64_t p = 0; p < n; ++p) ok = ok && w[p].dim() == 2 && w[p].size(0) == e_out && w[p].size(1) == e_in;
+    TORCH_CHECK_VALUE(ok, "saved x ", x.sizes(), " and weight ", w[0].sizes(), " do not fit the gradient of ", rows, " rows of ", e_out);
+}
+
 Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : c10::nullopt; }
 
@@ -324,7 +332,15 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
         for (int64_t p = 0; p < n; ++p) check_saved("weight", w[p], g[0]);
         for (int64_t p = 0, i = 0; p < n; ++p)
             if ((phi >> p) & 1) check_saved("y", y[i++], g[0]);
-        const int64_t rows = x.size(0) * x.size(1);
+        const int64_t rows = g[0].size(0) * g[0].size(1), e_out = w[0].size(0);
+        TORCH_CHECK_VALUE(x.dim() == 3 && x.size(0) == g[0].size(0) && x.size(1) == g[0].size(1), "saved x ", x.sizes(),
+                          " does not fit the gradient ", g[0].sizes());
+        check_saved_layers(x, w, n, rows, e_out);
+        for (int64_t p = 0, i = 0; p < n; ++p) {
+            const Tensor& like = (phi >> p) & 1 ? y[i++] : g[p];
+            TORCH_CHECK_VALUE(like.dim() == 4 && like.size(0) == x.size(0) && like.size(1) == x.size(1) && like.size(2) == g[0].size(2) &&
+                                  like.size(2) * like.size(3) == e_out, "saved output ", like.sizes(), " does not fit ", rows, " rows of ", e_out);
+        }
         const Tensor x2 = x.reshape({rows, x.size(2)});
         variable_list out(11);                    // x, wf, scale, heads, phi, w0, b0, w1, b1, w2, b2
         std::vector<bool> bias;
@@ -342,7 +358,6 @@ struct ProjectNode : public torch::autograd::Function<ProjectNode> {
         } else if (n == 3 && phi == 3 && need_x) {
             // [dy_q | dy_k | dv] side by side, written by the feature-map backward launch itself: one
             // GEMM for dx and one contraction for the three weight gradients
-            const int64_t e_out = w[0].size(0);
             Tensor packed;
             const Tensor g0 = g[0].contiguous(), g1 = g[1].contiguous(), g2 = g[2].contiguous();
             dwf = feature_grads(y[0], &y[1], wf, g0, &g1, &g2, packed, nullptr, true, scale, need_wf);
@@ -462,6 +477,7 @@ struct LinearNode : public torch::autograd::Function<LinearNode> {
         check_saved("x", x, g[0]);
         check_saved("weight", w, g[0]);
         const Tensor dy2 = g[0].reshape({-1, g[0].size(-1)}), x2 = x.reshape({-1, x.size(-1)});
+        check_saved_layers(x, &w, 1, dy2.size(0), dy2.size(1));
         Tensor dx;
         const std::vector<bool> bias{ctx->saved_data["bias"].toBool()};
         if (ctx->saved_data["need_x"].toBool()) {

@@ -646,6 +646,46 @@ def test_native_nodes_check_what_saved_tensor_hooks_return(path):
     assert refused["type"] == refused["device"] == saved
 
 
+@pytest.mark.parametrize("change", ["longer", "shorter", "narrower"])
+def test_layers_check_the_shapes_of_what_saved_tensor_hooks_return(change):
+    """An input or a weight of a layer comes back from a hook with another shape: the backward pass raises before it
+    launches anything over rows or columns that are not there."""
+    from rfa_amd import rfa_hip
+    from rfa_amd.causal_attention import CausalAttention
+    if rfa_hip.native is None:
+        pytest.skip("the torch binding is not active")
+    T, B, H, d, D = 70, 3, 2, 64, 32
+    E = H * d
+    new = {"longer": lambda t: torch.cat([t, t[:1]]), "shorter": lambda t: t[:-1].contiguous(),
+           "narrower": lambda t: t[..., :E // 2].contiguous()}[change]
+    layer = CausalAttention(embed_dim=E, num_heads=H, head_dim=d, proj_dim=D).cuda().half().train()
+    x = torch.randn(T, B, E, device="cuda").half().requires_grad_()
+    W = O.make_w(d, D, H).half().cuda()
+    seen, which, total = [0], [-1], 0
+
+    def pack(t):
+        if t.shape[-1:] != (E,) or t.dim() not in (2, 3):       # what the layers save, not the scan
+            return t
+        seen[0] += 1
+        return new(t) if seen[0] - 1 == which[0] else t
+
+    while True:
+        seen[0] = 0
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+            out = layer(x, W)
+        if which[0] < 0:
+            out.backward(torch.ones_like(out))
+            total = seen[0]
+            assert total >= 6        # two inputs and four weights
+        else:
+            print(f"{change} saved tensor {which[0]}", flush=True)
+            with pytest.raises((RuntimeError, ValueError)):
+                out.backward(torch.ones_like(out))
+        which[0] += 1
+        if which[0] == total:
+            break
+
+
 def test_native_nodes_leave_odd_calls_to_the_python_functions():
     """Dispatch modes and tracing see the Python functions, and functorch transforms and forward-mode
     tangents meet the errors that those raise."""
