@@ -254,8 +254,8 @@ __global__ __launch_bounds__(kFeatureBwdThreads) void k_feature_map_bwd(
     int grp = blockIdx.x * kFeatureBwdWaves + wv;
     // Two sets of row registers: the loads of the next group are issued into the set the
     // current group does not use, so no set is ever copied.  Rows past R read the last row (no
-    // branch around the loads); their du is forced to 0, which keeps them out of dW', and their
-    // dx is not stored.
+    // branch around the loads); their du is replaced by 0 (a factor of 0 would leave NaN where that row's gradient is
+    // infinite), which keeps them out of dW', and their dx is not stored.
     struct Rows { h8 x[DH / 32], gs[D / 32], gc[D / 32]; };
     auto issue_loads = [&](Rows& t, int g) {
         const int64_t row = (int64_t)min(g * 16 + i, R - 1) * H + h;
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kFeatureBwdThreads) void k_feature_map_bwd(
         const float inv = rcp_nr(nrm + 1e-3f);
         const float coef = nrm > 0.f ? inv * rcp_nr(nrm) : 0.f;
         const float inv_turns = inv * 0.15915494309189535f;
-        const float sinv = r < R ? scale * inv : 0.f;
+        const float sinv = scale * inv;
 
         h8 du[D / 32];
 #pragma unroll
@@ -303,6 +303,7 @@ __global__ __launch_bounds__(kFeatureBwdThreads) void k_feature_map_bwd(
                     sincos_turns(acc[q][e] * inv_turns, s_, c_);
                     du[p][4 * q + e] = (half_t)(sinv * (c_ * (float)t.gs[p][4 * q + e] - s_ * (float)t.gc[p][4 * q + e]));
                 }
+            if (r >= R) du[p] = h8_zero();
             if (want_dw) *reinterpret_cast<h8*>(Us + i * LDU + 32 * p + 8 * G) = du[p];
         }
         if (kShared && want_dw) __syncthreads();      // the rows of all waves are in place

@@ -241,6 +241,38 @@ def test_feature_map_backward_where_waves_share_rows(R, wgs, d, D, knobs):
     assert torch.equal(packed, torch.cat([t.view(R, E) for t in (dx0, dx1, third)], 1)) and torch.equal(pw, dw)
 
 
+@pytest.mark.parametrize("d,D", [(64, 32), (64, 64), (128, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("R", [1, 17, 127, 128, 129, 1040])
+def test_feature_map_backward_of_an_infinity_in_the_last_row(R, d, D):
+    """Rows past the last one count for nothing, also where the row that stands in for them holds an infinity in its
+    gradient: dW' of that feature is infinite with the sign that the product has, everything else as without it."""
+    from rfa_amd import rfa_hip
+    H = 2
+    x0, x1 = (_randn(R, 1, H, d, seed=70 + i).half() for i in range(2))
+    x0[x0 == 0] = 1
+    w = (_randn(H, D, d, seed=72) * 0.9).half()
+    g0, g1 = (_randn(R, 1, H, 2 * D, seed=73 + i).half() for i in range(2))
+    g0[-1, 0, 0, 3] = 0
+    g0[-1, 0, 1, D + 5] = 0
+    x0, x1, w, g0, g1 = (t.cuda() for t in (x0, x1, w, g0, g1))
+    print(f"phi bwd with an infinity R={R} d={d} D={D}", flush=True)
+    clean = rfa_hip.feature_map_backward(x0, w, g0, O.SCALE), rfa_hip.feature_map_backward_pair(x1, x0, w, g1, g0, O.SCALE)
+    g0[-1, 0, 0, 3], g0[-1, 0, 1, D + 5] = float("inf"), float("-inf")
+    odd = rfa_hip.feature_map_backward(x0, w, g0, O.SCALE), rfa_hip.feature_map_backward_pair(x1, x0, w, g1, g0, O.SCALE)
+    last = x0[-1, 0].double()
+    u = torch.einsum("hc,hjc->hj", last / (last.norm(dim=-1, keepdim=True) + 1e-3), w.double())
+    sign = {(0, 3): u[0, 3].cos().sign() * last[0].sign(), (1, 5): u[1, 5].sin().sign() * last[1].sign()}
+    for was, now in zip(clean, odd):
+        assert torch.equal(now[0][:-1], was[0][:-1])             # dx of the other rows; in the pair of the other tensor
+        if len(now) == 3:
+            assert torch.equal(now[0], was[0]) and torch.equal(now[1][:-1], was[1][:-1])
+        keep = torch.ones(H, D, dtype=torch.bool, device="cuda")
+        for at, want in sign.items():
+            keep[at] = False
+            assert torch.isinf(now[-1][at]).all() and torch.equal(now[-1][at].sign().double(), want), at
+        assert torch.equal(now[-1][keep], was[-1][keep])
+
+
 @pytest.mark.parametrize("H,D,d,tau,with_sigma", [(8, 64, 64, 1.0, True), (3, 32, 128, 0.7, True),
                                                    (2, 128, 64, 2.0, False), (1, 5, 24, 1.3, True)])
 def test_build_random_matrices_matches_the_aten_chain(H, D, d, tau, with_sigma):
