@@ -301,6 +301,9 @@ int rfa_linear_weight_grad(const void* x, const void* const* dy, void* const* dw
  * all p, one rounding.  E_out a multiple of 32, E_in of 128, E_in and ld at most 2^22. */
 int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R,
                           int E_out, int E_in, void* stream);
+/* The tile that call takes for these sizes on the current device: its rows, and the groups of waves that share its
+ * contraction (a group's 32 columns each divide E_out).  For tests and sweeps; launches nothing. */
+int rfa_linear_input_grad_tile(int64_t R, int E_out, int E_in, int np, int* rows, int* groups);
 
 /* Both of those gradients in one launch (and its reduction): arguments as above, dy_p [R, E_out] with rows ld halves
  * apart for both.  Where rfa_linear_grads_workspace_bytes answers 0 the two calls above are to be used: E_out or E_in no

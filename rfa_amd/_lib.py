@@ -69,6 +69,7 @@ SIGNATURES = {
     "rfa_linear_weight_grad_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
     "rfa_linear_weight_grad": (c_int, [c_void_p] * 4 + [c_int, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rfa_linear_input_grad": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),
+    "rfa_linear_input_grad_tile": (c_int, [c_int64, c_int, c_int, c_int, POINTER(c_int), POINTER(c_int)]),
     "rfa_linear_grads_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
     "rfa_linear_grads": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                  c_int, c_void_p, c_size_t, c_void_p]),

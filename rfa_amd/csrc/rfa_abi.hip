@@ -965,6 +965,8 @@ template <int BM, int KG>
 int launch_input_grad(const rfa::InputGradArgs& ga, rfa::half_t* dx, int R, int Eo, int Ei, int np, int64_t ld,
                       hipStream_t st) {
     using Cfg = rfa::InputGradCfg<BM, KG>;
+    if (Eo % (Cfg::BK * KG) != 0)      // a stage would reach past a layer's last column
+        return fail(RFA_ERR_UNSUPPORTED, "rfa_linear_input_grad: E_out=%d is no multiple of the %d columns of a stage", Eo, Cfg::BK * KG);
     auto kern = rfa::k_input_grad<BM, KG>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     const int64_t tiles = (int64_t)((R + BM - 1) / BM) * (Ei / Cfg::BN);
@@ -974,17 +976,21 @@ int launch_input_grad(const rfa::InputGradArgs& ga, rfa::half_t* dx, int R, int 
     return RFA_OK;
 }
 
-// As the projections, with four groups for 64 rows where the contraction is 768 or longer; a group's columns divide each
-// layer's E_out.  Measured, us for 64 rows by one group / two / four, 128 by one / two, 256:
+// As the projections, with four groups for 64 rows where the contraction is 768 or longer.  Groups of waves share a
+// stage of 32 columns each, so they are for widths that they divide; other widths take one group.
+// Measured, us for 64 rows by one group / two / four, 128 by one / two, 256:
 // 512 rows of 512 -> 512 7.8 / 6.8 / 7.0 / 10.2 / 8.9 / 14.8; 512 of 3 x 512 17.5 / 12.9 / 11.6 / 22.5 / 16.7 / 32.2; 2048 of
 // 3 x 1024 32.7 / 23.9 / 21.9 / 41.4 / 29.6 / 58.6; 4096 of 3 x 768 31.9 / 27.5 / 31.7 / 33.5 / 25.4 / 46.0; 8192 of 512 11.2 /
 // 11.7 / 14.7 / 11.8 / 10.6 / 16.4, of 3 x 512 25.1 / 23.0 / 25.6 / 25.1 / 19.9 / 34.3, of 3 x 1024 80 / 72 / 83 / 63 / 67 / 67.
 TileShape input_grad_shape(int64_t R, int Eo, int Ei, int np) {
     const int64_t cus = device_cus(), tiles_c = Ei / 128;
     const int64_t t64 = (R + 63) / 64 * tiles_c, t128 = (R + 127) / 128 * tiles_c, t256 = (R + 255) / 256 * tiles_c;
-    if (Eo % 64 != 0 && t128 < cus) return {64, 1};
-    if (t64 <= cus) return {64, Eo % 128 == 0 && np * Eo >= 768 ? 4 : 2};
-    if (t128 <= cus && Eo % 64 == 0) return {128, 2};
+    if (Eo % 64 == 0) {
+        if (t64 <= cus) return {64, Eo % 128 == 0 && np * Eo >= 768 ? 4 : 2};
+        if (t128 <= cus) return {128, 2};
+    } else if (t128 < cus) {
+        return {64, 1};
+    }
     if (t256 >= cus && 5 * ((t256 + cus - 1) / cus) <= 3 * ((t128 + cus - 1) / cus)) return {256, 1};
     return {128, 1};
 }
@@ -2260,8 +2266,7 @@ size_t rfa_linear_weight_grad_workspace_bytes(int64_t R, int E_out, int E_in, in
     return (size_t)pl.nsplit * np * ((size_t)E_out * E_in + E_out) * 4;
 }
 
-int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R, int E_out,
-                          int E_in, void* stream) {
+static int check_input_grad_dims(int64_t R, int E_out, int E_in, int64_t ld, int np) {
     if (R < 0 || E_out <= 0 || E_in <= 0 || R > (int64_t(1) << 30) || ld < E_out || ld > (1 << 22) || E_in > (1 << 22))
         return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: bad sizes rows=%lld E_out=%d E_in=%d ld=%lld", (long long)R, E_out,
                     E_in, (long long)ld);
@@ -2270,6 +2275,21 @@ int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* 
                     E_out, E_in, (long long)ld);
     if (np < 1 || np > rfa::kMaxProjections)
         return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_input_grad: %d projections (1..%d supported)", np, rfa::kMaxProjections);
+    return RFA_OK;
+}
+
+int rfa_linear_input_grad_tile(int64_t R, int E_out, int E_in, int np, int* rows, int* groups) {
+    if (int rc = check_input_grad_dims(R, E_out, E_in, E_out, np)) return rc;
+    if (!rows || !groups) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_input_grad_tile: NULL pointer");
+    const TileShape t = input_grad_shape(R, E_out, E_in, np);
+    *rows = t.rows;
+    *groups = t.groups;
+    return RFA_OK;
+}
+
+int rfa_linear_input_grad(const void* const* dy, int64_t ld, const void* const* w, int np, void* dx, int64_t R, int E_out,
+                          int E_in, void* stream) {
+    if (int rc = check_input_grad_dims(R, E_out, E_in, ld, np)) return rc;
     if (R == 0) return RFA_OK;
     if (!dy || !w || !dx) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_input_grad: NULL pointer");
     rfa::InputGradArgs ga{};

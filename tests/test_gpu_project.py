@@ -688,6 +688,12 @@ def test_linear_input_grad(R, e_out, e_in, n):
     assert ((dx.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -20 * size + 2.0 ** -24).all()
 
 
+@pytest.mark.parametrize("e_out", [32, 96, 128])
+def test_linear_input_grad_of_a_tile_per_compute_unit(e_out):
+    """As many columns as give every compute unit one tile, where widths that two groups of waves divide and others part."""
+    test_linear_input_grad(50, e_out, 128 * torch.cuda.get_device_properties(0).multi_processor_count, 2)
+
+
 @pytest.mark.parametrize("e_out,e_in,n", [(128, 128, 1), (128, 256, 3), (384, 128, 2), (512, 512, 3), (1024, 1024, 1)])
 @pytest.mark.parametrize("R", [1, 31, 33, 64, 65, 200, 1000, 2049, 9000])
 def test_linear_grads(R, e_out, e_in, n):

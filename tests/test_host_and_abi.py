@@ -189,6 +189,26 @@ def test_causal_plans(K, d):
     assert {s: ask(*s) for s in shapes} == first
 
 
+def test_input_gradient_tiles_divide_their_widths():
+    """Groups of waves take 32 columns each of every layer's width, whatever tile the sizes choose; around every line of the
+    rule, the number of compute units in tiles (E_in = 128 of them) among them."""
+    import ctypes
+    lib = _lib.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available() else 256
+    rows, groups = ctypes.c_int(), ctypes.c_int()
+    seen = set()
+    for tiles in (1, 4, 24, cus // 2 - 1, cus // 2, cus - 1, cus, cus + 1, 2 * cus):
+        for R in (1, 64, 65, 128, 129, 256, 500, 4096, 100000):
+            for e_out in (32, 64, 96, 128, 160, 192, 256, 512, 544, 1024, 2080):
+                for n in (1, 3):
+                    assert lib.rfa_linear_input_grad_tile(R, e_out, 128 * tiles, n, rows, groups) == 0
+                    tile = (rows.value, groups.value)
+                    seen.add(tile)
+                    assert e_out % (32 * tile[1]) == 0, (R, e_out, tiles, n, tile)
+    assert seen <= {(64, 1), (64, 2), (64, 4), (128, 1), (128, 2), (256, 1)} and len(seen) == 6
+    assert lib.rfa_linear_input_grad_tile(64, 48, 128, 1, rows, groups) == -3
+
+
 def test_masked_rfa_has_no_cpu_path():
     """masked_rfa runs on the quadratic-form HIP kernels only: CPU tensors raise."""
     from rfa_amd.causal_attention import masked_rfa
