@@ -2,10 +2,10 @@
 of the tensors changes.
 
 An entry remembers, for every source tensor, a weak reference to the tensor object and its version
-counter, storage address, dtype, shape and device.  It answers only for the very same objects in the
-very same state: an in-place update moves the version counter, ``p.data = ...`` moves the address,
-and a tensor that has died cannot be impersonated by a new one that the allocator put at its
-address (or that Python gave its id), because the weak reference is dead.
+counter, storage address, dtype, shape, strides and device.  It answers only for the very same objects in the
+very same state: an in-place update moves the version counter, ``p.data = ...`` moves the address (or, for a
+view of the same storage, the strides), and a tensor that has died cannot be impersonated by a new one
+that the allocator put at its address (or that Python gave its id), because the weak reference is dead.
 """
 from __future__ import annotations
 
@@ -16,7 +16,7 @@ from torch import Tensor
 
 
 def _state(t: Optional[Tensor]):
-    return None if t is None else (t._version, t.data_ptr(), t.dtype, t.shape, t.device)
+    return None if t is None else (t._version, t.data_ptr(), t.dtype, t.shape, t.stride(), t.device)
 
 
 class _Entry:

@@ -556,7 +556,7 @@ class Sources {
         c10::weak_intrusive_ptr<at::TensorImpl> impl;
         uint32_t version;
         const void* data;
-        std::vector<int64_t> sizes;
+        std::vector<int64_t> sizes, strides;      // p.data = p.data.t() changes nothing but the strides
         at::ScalarType type;
         at::Device device;
     };
@@ -577,8 +577,8 @@ public:
             const OptTensor& t = *tensors[i];
             if (k.has_value() != t.has_value()) return false;
             if (k.has_value() && !(k->impl._unsafe_get_target() == t->unsafeGetTensorImpl() && k->version == t->_version() &&
-                                   k->data == t->data_ptr() && k->sizes == t->sizes() && k->type == t->scalar_type() &&
-                                   k->device == t->device()))
+                                   k->data == t->data_ptr() && k->sizes == t->sizes() && k->strides == t->strides() &&
+                                   k->type == t->scalar_type() && k->device == t->device()))
                 return false;
         }
         return true;
@@ -589,7 +589,8 @@ public:
             if (!t->has_value()) sources_.emplace_back(c10::nullopt);
             else
                 sources_.emplace_back(Source{c10::weak_intrusive_ptr<at::TensorImpl>((*t)->getIntrusivePtr()), (uint32_t)(*t)->_version(),
-                                             (*t)->data_ptr(), (*t)->sizes().vec(), (*t)->scalar_type(), (*t)->device()});
+                                             (*t)->data_ptr(), (*t)->sizes().vec(), (*t)->strides().vec(),
+                                             (*t)->scalar_type(), (*t)->device()});
         }
         extra_ = extra;
     }

@@ -205,13 +205,13 @@ def test_causal_module_decode_from_one_stacked_projection():
 
 
 @pytest.mark.parametrize("change", ["none", "replaced", "data", "in_place", "no_bias", "mixed_bias", "matrices", "tau", "sigma", "hook",
-                                    "steps", "strided"])
+                                    "steps", "strided", "transposed", "matrices_transposed"])
 def test_decode_step_sees_every_change(change):
     """A decoding step after one that filled the caches gives what a module without caches gives, whatever changed
     in between; the layers it is compared with run under autograd (nothing cached, three projections: a rounding of
     fp16 apart)."""
     import copy
-    from rfa_amd import CausalAttention
+    from rfa_amd import CausalAttention, rfa_hip
     torch.manual_seed(11)
     B, H, d, D = 3, 2, 64, 64
     E = H * d
@@ -221,13 +221,26 @@ def test_decode_step_sees_every_change(change):
         first = {}
         m(x[:2], W, saved_state=first)
         m(x[2:3], W, saved_state=dict(first))                       # fills the caches
-    seen, now = [], x[3:4]
+    seen, now, answered = [], x[3:4], []
+    if rfa_hip.native is not None:                                   # and the native step is the one that answers below
+        step = m._inference_cache["step"]
+
+        class Spy:
+            def rows(self, *args):
+                rows = step.rows(*args)
+                answered.append(rows is not None)
+                return rows
+        m._inference_cache["step"] = Spy()
     with torch.no_grad():
         if change == "replaced":
             m.k_proj = copy.deepcopy(m.k_proj)
             m.k_proj.weight.mul_(0.5)
         elif change == "data":
             m.v_proj.weight.data = m.v_proj.weight.data * 0.5
+        elif change == "transposed":             # same object, version, address and shape
+            m.q_proj.weight.data = m.q_proj.weight.data.t()
+        elif change == "matrices_transposed":
+            W.data = W.data.transpose(1, 2)
         elif change == "in_place":
             m.q_proj.bias.add_(0.5)
         elif change in ("no_bias", "mixed_bias"):
@@ -247,6 +260,7 @@ def test_decode_step_sees_every_change(change):
             now = torch.randn(1, E, B).cuda().half().transpose(1, 2)
         got_state, ref_state = dict(first), dict(first)
         got = m(now, W, saved_state=got_state)
+    assert answered == ([] if rfa_hip.native is None else [change != "mixed_bias"])
     m.requires_grad_(True)
     with torch.enable_grad():
         want = m(now, W, saved_state=ref_state).detach()

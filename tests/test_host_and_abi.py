@@ -322,6 +322,10 @@ def test_derived_values_answer_only_for_the_same_live_tensors_in_the_same_state(
     assert derived(slot, "k", (a, b, None), 2, make_from(a, b)) == 8.0 and len(made) == 4
     c = b.clone()                                                                                 # equal state, another object
     assert derived(slot, "k", (a, c, None), 2, make_from(a, c)) == 8.0 and len(made) == 5
+    sq, rows = torch.arange(4.0).view(2, 2), {}
+    assert torch.equal(derived(rows, "t", (sq,), None, lambda: sq.reshape(-1).clone()), torch.tensor([0.0, 1, 2, 3]))
+    sq.data = sq.data.t()                                        # version, address and shape as before, other strides
+    assert torch.equal(derived(rows, "t", (sq,), None, lambda: sq.reshape(-1).clone()), torch.tensor([0.0, 2, 1, 3]))
     assert derived(slot, "k", (a, None, None), 2, make_from(a)) == 0.0 and len(made) == 6       # None where a tensor was
     # a dead source: the entry must not answer for a newcomer in the same state, even at the same address
     t = torch.full((1024,), 3.0)
