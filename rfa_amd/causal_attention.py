@@ -208,11 +208,12 @@ class CausalAttention(nn.Module):
     # ---- inference-time caches ------------------------------------------------------------------
     # Decoding calls forward once per token with the same parameters: what depends on the parameters
     # alone is then kept between calls (only while autograd is off) for as long as every tensor it
-    # was made from is the same object in the same state (version counter, address, dtype, shape),
+    # was made from is the same object in the same state (version counter, address, dtype, shape, strides),
     # so an optimizer step, load_state_dict, a replaced parameter or another random_matrices tensor
-    # makes it anew.
+    # makes it anew.  Each stream has values of its own, at most four; a captured call forms its own as well.
     def _cached(self, name: str, sources, extra, make):
-        return derived(self.__dict__.setdefault("_inference_cache", {}), name, sources, extra, make)
+        cache = self.__dict__.setdefault("_inference_cache", {})
+        return derived(cache.setdefault("derived", {}), name, sources, extra, make, limit=8)
 
     def __getstate__(self):
         # copies and pickles of the module start without the cache (it holds weak references)

@@ -15,7 +15,10 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContextLight.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPException.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+
+#include <algorithm>
 
 namespace {
 
@@ -599,10 +602,31 @@ public:
 // The scaled matrices W' and the stacked q, k, v layer of one CausalAttention, and with them the first half of a decoding
 // step: rows [T, B, 3, H, d] of all three projections, W' and the tensors that the step writes its state to (none where it
 // stays in place).  In Python this half costs 16 us of a step whose kernels take 11 (four sequences of 8 heads).
+// What a stream made is for its own kernels alone: another one has nothing to wait on, and memory given back is used
+// again by the stream that it came from.  A captured step forms both anew: kept tensors would die under the graph
+// with the next change of a parameter, and the graph's own hold nothing before its first replay.
 class DecodeCache {
-    Sources matrix_sources_, layer_sources_;
-    Tensor w_, weight_;
-    OptTensor bias_;
+    struct Kept {
+        hipStream_t stream = nullptr;
+        Sources matrix_sources, layer_sources;
+        Tensor w, weight;
+        OptTensor bias;
+    };
+    static constexpr size_t kStreams = 4;
+    std::vector<Kept> kept_;       // the stream used last comes first
+
+    Kept& kept(hipStream_t stream) {
+        size_t i = 0;
+        while (i < kept_.size() && kept_[i].stream != stream) ++i;
+        if (i == kept_.size()) {
+            if (i == kStreams) kept_.pop_back();
+            kept_.emplace_back();
+            kept_.back().stream = stream;
+            i = kept_.size() - 1;
+        }
+        std::rotate(kept_.begin(), kept_.begin() + i, kept_.begin() + i + 1);
+        return kept_.front();
+    }
 
 public:
     using Rows = std::tuple<Tensor, Tensor, OptTensor, OptTensor>;
@@ -621,19 +645,24 @@ public:
         const OptTensor m(matrices);
         const Sources::List ms{&m, &sigma}, ls{&wq, &bq, &wk, &bk, &wv, &bv};
         if (heads < 1 || E % heads != 0 || !Sources::can_remember(ms) || !Sources::can_remember(ls)) return c10::nullopt;
-        if (!matrix_sources_.same(ms, tau)) {
-            w_ = build_random_matrices(matrices.contiguous(), sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt, tau);
-            matrix_sources_.remember(ms, tau);
+        const hipStream_t stream = c10::hip::getCurrentHIPStream(x.get_device()).stream();
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        C10_HIP_CHECK(hipStreamIsCapturing(stream, &capture));
+        Kept captured;
+        Kept& c = capture == hipStreamCaptureStatusNone ? kept(stream) : captured;
+        if (!c.matrix_sources.same(ms, tau)) {
+            c.w = build_random_matrices(matrices.contiguous(), sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt, tau);
+            c.matrix_sources.remember(ms, tau);
         }
-        if (!layer_sources_.same(ls, 0)) {
-            weight_ = at::cat({*wq, *wk, *wv}, 0);
-            bias_ = bq.has_value() ? OptTensor(at::cat({*bq, *bk, *bv}, 0)) : c10::nullopt;
-            layer_sources_.remember(ls, 0);
+        if (!c.layer_sources.same(ls, 0)) {
+            c.weight = at::cat({*wq, *wk, *wv}, 0);
+            c.bias = bq.has_value() ? OptTensor(at::cat({*bq, *bk, *bv}, 0)) : c10::nullopt;
+            c.layer_sources.remember(ls, 0);
         }
-        const OptTensor own = node_linear_rows(x, weight_, bias_);
-        const Tensor y = own.has_value() ? *own : at::linear(x, weight_, bias_);
+        const OptTensor own = node_linear_rows(x, c.weight, c.bias);
+        const Tensor y = own.has_value() ? *own : at::linear(x, c.weight, c.bias);
         auto fresh = [&](const Tensor& t) { return in_place ? c10::nullopt : OptTensor(torch::empty_like(t)); };
-        return Rows{y.view({x.size(0), x.size(1), 3, heads, E / heads}), w_, fresh(s), fresh(z)};
+        return Rows{y.view({x.size(0), x.size(1), 3, heads, E / heads}), c.w, fresh(s), fresh(z)};
     }
 };
 

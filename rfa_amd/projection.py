@@ -35,10 +35,7 @@ def _stacked_weights(weights: Sequence[Tensor]) -> Tensor:
     three weights are the same tensor objects in the same state (an optimizer step moves their
     version counters); under capture it is always formed, so that a replayed graph reads the
     weights of the day."""
-    make = lambda: torch.cat(list(weights), 0)
-    if torch.cuda.is_current_stream_capturing():
-        return make()
-    return derived(_STACKED, tuple(id(w) for w in weights), tuple(weights), None, make, limit=8)
+    return derived(_STACKED, tuple(id(w) for w in weights), tuple(weights), None, lambda: torch.cat(list(weights), 0), limit=8)
 
 
 def _packed_backward_ok(ctx, grads, weights) -> bool:

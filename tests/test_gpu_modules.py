@@ -204,6 +204,89 @@ def test_causal_module_decode_from_one_stacked_projection():
         rfa_hip.incremental_qkv = real
 
 
+def _decode_module(seed):
+    """A CausalAttention that advances its state in place, its matrices, tokens and a state after two of them."""
+    from rfa_amd import CausalAttention
+    torch.manual_seed(seed)
+    m = CausalAttention(embed_dim=128, num_heads=2, head_dim=64, proj_dim=64).cuda().half().eval()
+    W, x = O.make_w(64, 64, 2).cuda().half(), torch.randn(8, 3, 128).cuda().half()
+    first = {}
+    with torch.no_grad():
+        m(x[:2], W, saved_state=first)
+    m.decode_inplace = True
+    m.__dict__.pop("_inference_cache", None)
+    return m, W, x, first
+
+
+@pytest.fixture(params=["ext", "ctypes"])
+def decode_binding(request):
+    from rfa_amd import rfa_hip
+    if request.param == "ext" and not rfa_hip.ext_available():
+        pytest.skip("the torch binding has not been built")
+    before = rfa_hip.binding()
+    rfa_hip.use_binding(request.param)
+    yield request.param
+    rfa_hip.use_binding(before)
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_decode_step_reads_the_parameters_of_the_day(warm, decode_binding):
+    """A decoding step in a graph, captured before (nothing kept yet) or after eager steps: eager steps before the first
+    replay, changes of every parameter between replays and eager steps that make the kept values anew leave each replay
+    with the eager step's bits."""
+    m, W, x, first = _decode_module(21)
+    other, oW, ox, ofirst = _decode_module(22)
+    copy_of = lambda: {k: t.clone() for k, t in first.items()}
+    eager = lambda t: m(x[t:t + 1], W, saved_state=copy_of())
+    with torch.no_grad():
+        other(ox[2:3], oW, saved_state={k: t.clone() for k, t in ofirst.items()})        # loads the kernels, fills its own cache
+        if warm:
+            eager(2)
+        state, token, graph = copy_of(), x[2:3].clone(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        print(f"decode capture {decode_binding} warm={warm}", flush=True)
+        with torch.cuda.graph(graph):
+            out = m(token, W, saved_state=state)
+        assert state["prev_s"] is not first["prev_s"]
+        want = eager(2)                                            # before any replay
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        for t, change in enumerate([m.q_proj.weight, m.k_proj.bias, m.v_proj.weight, m.out_proj.weight, m.sigma, W], 2):
+            change.mul_(0.75)
+            want = eager(t)                                        # what was kept is replaced and given back
+            junk = [torch.full((384, 128), float("nan"), device="cuda").half() for _ in range(8)]
+            del junk
+            token.copy_(x[t:t + 1])
+            for key in first:
+                state[key].copy_(first[key])
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), t
+
+
+def test_decode_steps_on_several_streams(decode_binding):
+    """Each stream decodes with values that it made itself, also when there are more streams than values are kept for, and
+    when a parameter changes in between."""
+    m, W, x, first = _decode_module(23)
+    copy_of = lambda: {k: t.clone() for k, t in first.items()}
+    streams = [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(5)]
+    with torch.no_grad():
+        for round_ in range(3):
+            got = []
+            for s in streams + streams[::-1]:
+                s.wait_stream(torch.cuda.default_stream())
+                with torch.cuda.stream(s):
+                    got.append(m(x[2:3], W, saved_state=copy_of()))
+            torch.cuda.synchronize()
+            assert all(torch.equal(g, got[0]) for g in got)
+            m.q_proj.weight.mul_(0.5)
+            assert round_ == 0 or not torch.equal(got[0], last)
+            last = got[0]
+    if decode_binding == "ctypes":
+        assert len(m._inference_cache["derived"]) <= 8
+
+
 @pytest.mark.parametrize("change", ["none", "replaced", "data", "in_place", "no_bias", "mixed_bias", "matrices", "tau", "sigma", "hook",
                                     "steps", "strided", "transposed", "matrices_transposed"])
 def test_decode_step_sees_every_change(change):
