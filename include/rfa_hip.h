@@ -258,6 +258,10 @@ int rfa_feature_map_backward_half(const void* x0, const void* x1, const void* w,
  *   fp32 sums, E_in a multiple of 32 and E_out of 16.  Right for any R, meant for R up to a few hundred. */
 int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int64_t R, int e_in, int e_out,
                     void* stream);
+/* Up to three of them over the same rows, side by side: w, bias np pointers each (bias or its entries may be NULL), y fp16
+ * [R, np * E_out] with layer p in columns p E_out ...  The bits of rfa_linear_rows with the weights stacked. */
+int rfa_linear_rows_layers(const void* x, const void* const* w, const void* const* bias, int np, void* y, int64_t R, int e_in,
+                           int e_out, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Linear projections to heads with the feature map in the epilogue.

@@ -24,11 +24,12 @@ from . import rfa_hip
 
 
 def _stream(sources: Sequence[Optional[Tensor]]) -> Optional[int]:
-    """Handle of the stream that work on these tensors is issued to (0: the default one, or no device tensor), None
-    while it is captured."""
+    """Handle of the stream that work on these tensors is issued to (0: the default one, which cannot be captured, or no
+    device tensor), None while it is captured."""
     for t in sources:
         if t is not None and t.is_cuda:
-            return None if torch.cuda.is_current_stream_capturing() else rfa_hip._stream_ptr(t.device)
+            stream = rfa_hip._stream_ptr(t.device)
+            return None if stream and torch.cuda.is_current_stream_capturing() else stream
     return 0
 
 

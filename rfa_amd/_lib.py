@@ -66,6 +66,7 @@ SIGNATURES = {
     "rfa_feature_map_backward_half": (c_int, [c_void_p] * 10 + [c_int64, c_int, c_int, c_int, c_float, c_void_p, c_size_t, c_void_p]),
     "rfa_project_feature_map": (c_int, [c_void_p] * 5 + [c_int, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_float, c_void_p]),
     "rfa_linear_rows": (c_int, [c_void_p] * 4 + [c_int64, c_int, c_int, c_void_p]),
+    "rfa_linear_rows_layers": (c_int, [c_void_p] * 3 + [c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "rfa_linear_weight_grad_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
     "rfa_linear_weight_grad": (c_int, [c_void_p] * 4 + [c_int, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rfa_linear_input_grad": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),

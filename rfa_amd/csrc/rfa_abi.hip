@@ -2221,18 +2221,30 @@ int rfa_project_feature_map(const void* x, const void* const* weights, const voi
 }
 
 int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int64_t R, int e_in, int e_out, void* stream) {
+    return rfa_linear_rows_layers(x, &w, &bias, 1, y, R, e_in, e_out, stream);
+}
+
+int rfa_linear_rows_layers(const void* x, const void* const* w, const void* const* bias, int np, void* y, int64_t R, int e_in,
+                           int e_out, void* stream) {
+    const char* fn = "rfa_linear_rows";
     if (R < 0 || R > (1 << 20) || e_in <= 0 || e_out <= 0)
-        return fail(RFA_ERR_BAD_SHAPE, "rfa_linear_rows: bad sizes R=%lld E_in=%d E_out=%d", (long long)R, e_in, e_out);
+        return fail(RFA_ERR_BAD_SHAPE, "%s: bad sizes R=%lld E_in=%d E_out=%d", fn, (long long)R, e_in, e_out);
+    if (np < 1 || np > rfa::kMaxProjections || (np > 1 && e_out > (1 << 28)))
+        return fail(RFA_ERR_BAD_SHAPE, "%s: %d layers of %d (1..%d supported)", fn, np, e_out, rfa::kMaxProjections);
     if (e_in % 32 != 0 || e_out % 16 != 0)
-        return fail(RFA_ERR_UNSUPPORTED, "rfa_linear_rows: E_in must be a multiple of 32 and E_out of 16 (got %d, %d)", e_in, e_out);
+        return fail(RFA_ERR_UNSUPPORTED, "%s: E_in must be a multiple of 32 and E_out of 16 (got %d, %d)", fn, e_in, e_out);
     if (R == 0) return RFA_OK;
-    if (!x || !w || !y) return fail(RFA_ERR_NULL_POINTER, "rfa_linear_rows: NULL tensor pointer");
-    if (!aligned16(x) || !aligned16(w) || !aligned16(y))
-        return fail(RFA_ERR_ALIGNMENT, "rfa_linear_rows: tensors must be 16-byte aligned");
+    if (!x || !w || !y) return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor pointer", fn);
+    rfa::RowLayers layers{};
+    for (int p = 0; p < np; ++p) {
+        if (!w[p]) return fail(RFA_ERR_NULL_POINTER, "%s: NULL tensor pointer", fn);
+        if (!aligned16(w[p])) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
+        layers.w[p] = static_cast<const rfa::half_t*>(w[p]);
+        layers.bias[p] = bias ? static_cast<const rfa::half_t*>(bias[p]) : nullptr;
+    }
+    if (!aligned16(x) || !aligned16(y)) return fail(RFA_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", fn);
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto* xh = static_cast<const rfa::half_t*>(x);
-    auto* wh = static_cast<const rfa::half_t*>(w);
-    auto* bh = static_cast<const rfa::half_t*>(bias);
     auto* yh = static_cast<rfa::half_t*>(y);
     // The tile whose workgroups keep a CU busy shortest: rounds of workgroups times the rows of x and W that one reads;
     // between equals the larger tile, whose operands are read by fewer.  Device us, 16 x 16 / 32 x 16 / 32 x 32 / 64 x 32 rows x
@@ -2242,7 +2254,7 @@ int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int
     static constexpr uint32_t kTiles[][2] = {{4, 2}, {2, 2}, {2, 1}, {1, 1}};
     uint32_t rt = 0, ct = 0;
     uint64_t least = 0;
-    const uint32_t cus = device_cus(), rows16 = ((uint32_t)R + 15) / 16, cols16 = e_out / 16;      // at most 2^16, 2^27
+    const uint32_t cus = device_cus(), rows16 = ((uint32_t)R + 15) / 16, cols16 = e_out / 16 * np;      // at most 2^16, 2^27
     for (const auto& t : kTiles) {
         const uint64_t wgs = (uint64_t)((rows16 + t[0] - 1) / t[0]) * ((cols16 + t[1] - 1) / t[1]);
         const uint64_t cost = (wgs + cus - 1) / cus * (t[0] + t[1]);
@@ -2250,7 +2262,8 @@ int rfa_linear_rows(const void* x, const void* w, const void* bias, void* y, int
     }
     const dim3 grid((cols16 + ct - 1) / ct, (rows16 + rt - 1) / rt);
 #define RFA_ROWS(RT, CT) \
-    RFA_LAUNCH(LINEAR_ROWS, (rfa::k_linear_rows<RT, CT>), grid, dim3(rfa::kThreads), 0, st, xh, wh, bh, yh, (int)R, e_in, e_out)
+    if (np == 1) { RFA_LAUNCH(LINEAR_ROWS, (rfa::k_linear_rows<RT, CT, false>), grid, dim3(rfa::kThreads), 0, st, xh, layers, yh, (int)R, e_in, e_out, np); } \
+    else RFA_LAUNCH(LINEAR_ROWS, (rfa::k_linear_rows<RT, CT, true>), grid, dim3(rfa::kThreads), 0, st, xh, layers, yh, (int)R, e_in, e_out, np)
     if (rt == 1) { RFA_ROWS(1, 1); }
     else if (ct == 1) { RFA_ROWS(2, 1); }
     else if (rt == 2) { RFA_ROWS(2, 2); }

@@ -528,6 +528,28 @@ OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     return LinearNode::apply(x, w, b);
 }
 
+// x W^T + b of n layers [e_out, e_in] side by side by the row kernel, where few_rows wants it and the tensors are as it takes them
+OptTensor row_products(const Tensor& x, const Tensor* w, const OptTensor* b, int64_t n) {
+    const int64_t e_out = w[0].size(0), e_in = w[0].size(1), R = e_in ? x.numel() / e_in : 0;
+    if (R < 1 || e_out == 0 || e_in % 32 != 0 || e_out % 16 != 0 || x.size(-1) != e_in || !x.is_contiguous() || !aligned16(x) ||
+        !few_rows(R, e_in, n * e_out, at::cuda::getDeviceProperties(x.get_device())->multiProcessorCount))
+        return c10::nullopt;
+    std::array<const void*, 3> wp{}, bp{};
+    for (int64_t p = 0; p < n; ++p) {
+        if (w[p].size(0) != e_out || w[p].size(1) != e_in || !w[p].is_contiguous() || !aligned16(w[p]) || w[p].device() != x.device())
+            return c10::nullopt;
+        if (b[p].has_value() && (b[p]->size(0) != e_out || !b[p]->is_contiguous() || b[p]->device() != x.device())) return c10::nullopt;
+        wp[p] = ptr(w[p]);
+        bp[p] = ptr(b[p]);
+    }
+    auto shape = x.sizes().vec();
+    shape.back() = n * e_out;
+    Tensor y = torch::empty(shape, x.options());
+    Launch l(x);
+    check_rc(rfa_linear_rows_layers(ptr(x), wp.data(), bp.data(), (int)n, ptr(y), R, (int)e_in, (int)e_out, l.stream));
+    return y;
+}
+
 // y = x W^T + b without autograd: few rows by the row kernel, more by the projection kernel, the largest products
 // by the library (and all whenever autocast would choose the type).
 OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b) {
@@ -539,16 +561,7 @@ OptTensor node_linear_rows(const Tensor& x, const Tensor& w, const OptTensor& b)
     if (!few_rows(R, e_in, e_out, at::cuda::getDeviceProperties(x.get_device())->multiProcessorCount))
         return e_in <= kWidestOwnProjection && R * e_in * e_out <= (int64_t)1 << 31 && own_linear(x, w, b)
                    ? OptTensor(projection(x, w, b)) : c10::nullopt;
-    if (e_in % 32 != 0 || e_out % 16 != 0 || e_out == 0 ||
-        !x.is_contiguous() || !w.is_contiguous() || !aligned16(x) || !aligned16(w) || w.device() != x.device())
-        return c10::nullopt;
-    if (b.has_value() && (b->size(0) != e_out || !b->is_contiguous() || b->device() != x.device())) return c10::nullopt;
-    auto shape = x.sizes().vec();
-    shape.back() = e_out;
-    Tensor y = torch::empty(shape, x.options());
-    Launch l(x);
-    check_rc(rfa_linear_rows(ptr(x), ptr(w), ptr(b), ptr(y), R, (int)e_in, (int)e_out, l.stream));
-    return y;
+    return row_products(x, &w, &b, 1);
 }
 
 // ---- what decoding keeps between calls --------------------------------------------------------
@@ -603,8 +616,10 @@ public:
 // step: rows [T, B, 3, H, d] of all three projections, W' and the tensors that the step writes its state to (none where it
 // stays in place).  In Python this half costs 16 us of a step whose kernels take 11 (four sequences of 8 heads).
 // What a stream made is for its own kernels alone: another one has nothing to wait on, and memory given back is used
-// again by the stream that it came from.  A captured step forms both anew: kept tensors would die under the graph
-// with the next change of a parameter, and the graph's own hold nothing before its first replay.
+// again by the stream that it came from.  A captured step forms what it needs anew: kept tensors would die under the graph
+// with the next change of a parameter, and the graph's own hold nothing before its first replay.  Few rows then take the
+// layers where they are: 4 sequences of 8 heads of 64 11.7 us a replay, 64 of 16 25.9 (with stacks of weights and biases 16.6
+// and 33.4; with kept ones 9.7 and 23.2).  The kept stack stays where it can: one launch over it is 0.1 to 0.5 shorter.
 class DecodeCache {
     struct Kept {
         hipStream_t stream = nullptr;
@@ -646,23 +661,32 @@ public:
         const Sources::List ms{&m, &sigma}, ls{&wq, &bq, &wk, &bk, &wv, &bv};
         if (heads < 1 || E % heads != 0 || !Sources::can_remember(ms) || !Sources::can_remember(ls)) return c10::nullopt;
         const hipStream_t stream = c10::hip::getCurrentHIPStream(x.get_device()).stream();
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        C10_HIP_CHECK(hipStreamIsCapturing(stream, &capture));
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (stream) C10_HIP_CHECK(hipStreamIsCapturing(stream, &status));      // the default stream cannot be
+        const bool capturing = status != hipStreamCaptureStatusNone;
         Kept captured;
-        Kept& c = capture == hipStreamCaptureStatusNone ? kept(stream) : captured;
+        Kept& c = capturing ? captured : kept(stream);
         if (!c.matrix_sources.same(ms, tau)) {
             c.w = build_random_matrices(matrices.contiguous(), sigma.has_value() ? OptTensor(sigma->contiguous()) : c10::nullopt, tau);
             c.matrix_sources.remember(ms, tau);
         }
-        if (!c.layer_sources.same(ls, 0)) {
-            c.weight = at::cat({*wq, *wk, *wv}, 0);
-            c.bias = bq.has_value() ? OptTensor(at::cat({*bq, *bk, *bv}, 0)) : c10::nullopt;
-            c.layer_sources.remember(ls, 0);
+        OptTensor y;
+        if (capturing) {      // few rows: the layers where they are, the bits of their stack
+            const std::array<Tensor, 3> w{*wq, *wk, *wv};
+            const std::array<OptTensor, 3> b{bq, bk, bv};
+            y = row_products(x, w.data(), b.data(), 3);
         }
-        const OptTensor own = node_linear_rows(x, c.weight, c.bias);
-        const Tensor y = own.has_value() ? *own : at::linear(x, c.weight, c.bias);
+        if (!y.has_value()) {
+            if (!c.layer_sources.same(ls, 0)) {
+                c.weight = at::cat({*wq, *wk, *wv}, 0);
+                c.bias = bq.has_value() ? OptTensor(at::cat({*bq, *bk, *bv}, 0)) : c10::nullopt;
+                c.layer_sources.remember(ls, 0);
+            }
+            y = node_linear_rows(x, c.weight, c.bias);
+            if (!y.has_value()) y = at::linear(x, c.weight, c.bias);
+        }
         auto fresh = [&](const Tensor& t) { return in_place ? c10::nullopt : OptTensor(torch::empty_like(t)); };
-        return Rows{y.view({x.size(0), x.size(1), 3, heads, E / heads}), c.w, fresh(s), fresh(z)};
+        return Rows{y->view({x.size(0), x.size(1), 3, heads, E / heads}), c.w, fresh(s), fresh(z)};
     }
 };
 

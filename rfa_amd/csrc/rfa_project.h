@@ -347,12 +347,18 @@ __global__ __launch_bounds__(kThreads * KG, 2) void k_project_phi(
 // costs 19 us of host time, this 4): 4 rows 512 -> 1536 2.6 / 2.6 / 3.9, 1024 -> 3072 3.6 / 3.6 / 5.7; 64 rows 512 -> 512 4.2 /
 // 2.8 / 5.6, 768 -> 768 5.9 / 3.5 / 5.7, 1024 -> 1024 6.4 / 3.7, 1024 -> 3072 6.9 / 6.3 / 8.3; 160 rows 512 -> 512 4.3 / 3.3; 320 rows
 // 1024 -> 1024 7.7 / 7.7 / 6.5.  Eight waves with two steps each: 64 rows 1024 -> 3072 6.1, 768 -> 768 4.0, else the same.
-// grid = (ceil(Eo / (16 CT)), ceil(R / (16 RT)));  E % 32 == 0, Eo % 16 == 0
+// Up to three layers over the same rows side by side, y [R][np Eo]: their weights stay where they are, as a stack of them
+// would have to be formed again whenever one changes, and at every replay of a captured step.
+// grid = (ceil(np Eo / (16 CT)), ceil(R / (16 RT)));  E % 32 == 0, Eo % 16 == 0
 // ---------------------------------------------------------------------------
-template <int RT, int CT>
-__global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restrict__ x, const half_t* __restrict__ w,
-                                                          const half_t* __restrict__ bias, half_t* __restrict__ y, int R,
-                                                          int E, int Eo) {
+struct RowLayers {
+    const half_t* w[kMaxProjections];
+    const half_t* bias[kMaxProjections];      // NULL: none
+};
+
+template <int RT, int CT, bool SEVERAL>
+__global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restrict__ x, RowLayers layers, half_t* __restrict__ y,
+                                                          int R, int E, int Eo, int np) {
     __shared__ f4 red[4][RT * CT][64];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // the wave's bounds are scalar: no lane masks
@@ -360,10 +366,16 @@ __global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restri
     const int c0 = 16 * CT * blockIdx.x, r0 = 16 * RT * blockIdx.y;
     const int nk = E / 32, per_wave = (nk + 3) / 4;
     const int k_begin = min(wv * per_wave, nk), k_end = min(k_begin + per_wave, nk);
+    const int cols = SEVERAL ? np * Eo : Eo;
+    // 16 columns lie within one layer (past the last one: its last 16 again)
+    auto layer = [&](int c16) { return !SEVERAL || c16 < Eo ? 0 : (c16 - Eo < Eo ? 1 : 2); };
     const half_t* wp[CT];
     const half_t* xp[RT];
 #pragma unroll
-    for (int c = 0; c < CT; ++c) wp[c] = w + (int64_t)min(c0 + 16 * c + i, Eo - 1) * E + 8 * G;
+    for (int c = 0; c < CT; ++c) {
+        const int c16 = min(c0 + 16 * c, cols - 16), p = layer(c16);
+        wp[c] = (SEVERAL ? pick3(layers.w, p) : layers.w[0]) + (int64_t)(c16 - p * Eo + i) * E + 8 * G;
+    }
 #pragma unroll
     for (int a = 0; a < RT; ++a) xp[a] = x + (int64_t)min(r0 + 16 * a + i, R - 1) * E + 8 * G;
     f4 acc[RT][CT];      // y^T tiles: lane (i, G) holds columns 4G .. of row i
@@ -410,11 +422,13 @@ __global__ __launch_bounds__(kThreads) void k_linear_rows(const half_t* __restri
     for (int t = wv; t < RT * CT; t += 4) {
         const int r = r0 + 16 * (t / CT) + i, col = c0 + 16 * (t % CT) + 4 * G;
         const f4 s = (red[0][t][lane] + red[1][t][lane]) + (red[2][t][lane] + red[3][t][lane]);
-        if (r < R && col < Eo) {
+        if (r < R && col < cols) {
+            const int p = layer(c0 + 16 * (t % CT));
+            const half_t* const bias = SEVERAL ? pick3(layers.bias, p) : layers.bias[0];
             h4 o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (half_t)(s[e] + (bias ? (float)bias[col + e] : 0.f));
-            *reinterpret_cast<h4*>(y + (int64_t)r * Eo + col) = o;
+            for (int e = 0; e < 4; ++e) o[e] = (half_t)(s[e] + (bias ? (float)bias[col - p * Eo + e] : 0.f));
+            *reinterpret_cast<h4*>(y + (int64_t)r * cols + col) = o;
         }
     }
 }

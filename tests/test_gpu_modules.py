@@ -204,12 +204,12 @@ def test_causal_module_decode_from_one_stacked_projection():
         rfa_hip.incremental_qkv = real
 
 
-def _decode_module(seed):
+def _decode_module(seed, B=3):
     """A CausalAttention that advances its state in place, its matrices, tokens and a state after two of them."""
     from rfa_amd import CausalAttention
     torch.manual_seed(seed)
     m = CausalAttention(embed_dim=128, num_heads=2, head_dim=64, proj_dim=64).cuda().half().eval()
-    W, x = O.make_w(64, 64, 2).cuda().half(), torch.randn(8, 3, 128).cuda().half()
+    W, x = O.make_w(64, 64, 2).cuda().half(), torch.randn(8, B, 128).cuda().half()
     first = {}
     with torch.no_grad():
         m(x[:2], W, saved_state=first)
@@ -229,13 +229,14 @@ def decode_binding(request):
     rfa_hip.use_binding(before)
 
 
+@pytest.mark.parametrize("B", [3, 600])          # the layers where they are, a stack of them
 @pytest.mark.parametrize("warm", [False, True])
-def test_captured_decode_step_reads_the_parameters_of_the_day(warm, decode_binding):
+def test_captured_decode_step_reads_the_parameters_of_the_day(warm, B, decode_binding):
     """A decoding step in a graph, captured before (nothing kept yet) or after eager steps: eager steps before the first
     replay, changes of every parameter between replays and eager steps that make the kept values anew leave each replay
     with the eager step's bits."""
-    m, W, x, first = _decode_module(21)
-    other, oW, ox, ofirst = _decode_module(22)
+    m, W, x, first = _decode_module(21, B)
+    other, oW, ox, ofirst = _decode_module(22, B)
     copy_of = lambda: {k: t.clone() for k, t in first.items()}
     eager = lambda t: m(x[t:t + 1], W, saved_state=copy_of())
     with torch.no_grad():
@@ -244,7 +245,7 @@ def test_captured_decode_step_reads_the_parameters_of_the_day(warm, decode_bindi
             eager(2)
         state, token, graph = copy_of(), x[2:3].clone(), torch.cuda.CUDAGraph()
         torch.cuda.synchronize()
-        print(f"decode capture {decode_binding} warm={warm}", flush=True)
+        print(f"decode capture {decode_binding} B={B} warm={warm}", flush=True)
         with torch.cuda.graph(graph):
             out = m(token, W, saved_state=state)
         assert state["prev_s"] is not first["prev_s"]
@@ -265,10 +266,11 @@ def test_captured_decode_step_reads_the_parameters_of_the_day(warm, decode_bindi
             assert torch.equal(out, want), t
 
 
-def test_decode_steps_on_several_streams(decode_binding):
+@pytest.mark.parametrize("B", [3, 600])
+def test_decode_steps_on_several_streams(B, decode_binding):
     """Each stream decodes with values that it made itself, also when there are more streams than values are kept for, and
     when a parameter changes in between."""
-    m, W, x, first = _decode_module(23)
+    m, W, x, first = _decode_module(23, B)
     copy_of = lambda: {k: t.clone() for k, t in first.items()}
     streams = [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(5)]
     with torch.no_grad():

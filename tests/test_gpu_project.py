@@ -607,6 +607,33 @@ def test_linear_rows_are_the_same_in_every_tile(e_in, e_out):
             assert all(torch.equal(y[r:r + 1], o) for r, o in zip((0, 17, 40), one)), R
 
 
+@pytest.mark.parametrize("e_in,e_out", [(32, 16), (160, 48), (512, 512), (1024, 1024), (512, 2064)])
+@pytest.mark.parametrize("R", [1, 17, 64, 160])
+def test_linear_rows_of_several_layers(R, e_in, e_out):
+    """Layers side by side from where they are: the bits of one call over their stack, at widths where a tile of 32 columns
+    spans two layers, with and without a bias."""
+    import ctypes
+    from rfa_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator("cuda").manual_seed(R + e_out)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").half()
+    x, ws, bs = rand(R, e_in), [rand(e_out, e_in) for _ in range(3)], [rand(e_out) for _ in range(3)]
+    stream = torch.cuda.current_stream().cuda_stream
+    array = lambda ts: (ctypes.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+    print(f"linear_rows_layers R={R} {e_in}->{e_out}", flush=True)
+    for n in (1, 2, 3):
+        for biases in (bs[:n], [None] * n, [bs[0]] + [None] * (n - 1)):
+            got, want = (torch.full((R, n * e_out), float("nan"), device="cuda").half() for _ in range(2))
+            stack = torch.cat(ws[:n], 0)
+            bias = torch.cat([torch.zeros_like(bs[0]) if b is None else b for b in biases], 0)
+            _lib.check(lib.rfa_linear_rows_layers(x.data_ptr(), array(ws[:n]), array(biases), n, got.data_ptr(), R, e_in, e_out, stream))
+            _lib.check(lib.rfa_linear_rows(x.data_ptr(), stack.data_ptr(), bias.data_ptr(), want.data_ptr(), R, e_in, n * e_out, stream))
+            assert torch.equal(got, want), (n, len(biases))
+    _lib.check(lib.rfa_linear_rows_layers(x.data_ptr(), array(ws), None, 3, got.data_ptr(), R, e_in, e_out, stream))
+    assert lib.rfa_linear_rows_layers(x.data_ptr(), array(ws), None, 4, got.data_ptr(), R, e_in, e_out, stream) == -2
+    assert lib.rfa_linear_rows_layers(x.data_ptr(), array([ws[0], None]), None, 2, got.data_ptr(), R, e_in, e_out, stream) == -1
+
+
 @pytest.mark.parametrize("e_in", [(1 << 22) + 128, (1 << 25) + 128])
 def test_output_projection_wider_than_the_kernels_address(e_in):
     """Widths that the input-gradient launch (2^22) and the projection launch (2^25) refuse go to the library."""
