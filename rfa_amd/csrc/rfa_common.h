@@ -399,9 +399,10 @@ __global__ __launch_bounds__(kThreads) void k_mask_rows(const half_t* src, half_
     }
 }
 
-// 1 / x for x >= 1 (denominators): the hardware approximation and one Newton step, 3 vector
-// instructions where the correctly rounded quotient takes about ten; the result differs from
-// it by at most one unit in the last place, far below the fp16 rounding of whatever it scales.
+// 1 / x for normal x > 0 whose reciprocal is normal (denominators of at least 1; norms of fp16 rows, 6e-8 to 8e5): the
+// hardware approximation and one Newton step, 3 vector instructions where the correctly rounded quotient takes about
+// ten; the result differs from it by at most one unit in the last place, far below the fp16 rounding of whatever it
+// scales.  (x infinite: NaN, not 0.)
 __device__ __forceinline__ float rcp_nr(float x) {
     const float y = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
