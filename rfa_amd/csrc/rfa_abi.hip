@@ -291,53 +291,54 @@ ScanCost scan_cost(int K, int d) {
 
 ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool have_saved, int* s_ratio);
 
+double scan_rounds(double wgs, int K, int d, int cus) {
+    const double full = std::max(1.0, std::ceil(wgs / cus));
+    return K == 64 && d == 64 ? 1.5 * std::floor(full / 2) + std::fmod(full, 2.0) : full;
+}
+
+// of a forward alone; rebuilt: by workgroups that rebuild their states from the rows before them, where the cut allows it
+double forward_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cus, bool rebuilt) {
+    const ScanCost c = scan_cost(K, d);
+    const double nch = (double)((T + rfa::kChunk - 1) / rfa::kChunk), gap = 1.5;
+    double us, moved = (double)T * N * (K + d) * 4;
+    rfa::SegBounds b;
+    const double u = rebuilt ? recompute_bounds(T, p.nseg, &b) : 0;
+    if (p.nseg == 1) {
+        us = scan_rounds((double)N, K, d, cus) * (c.scan + c.scan_chunk * nch);
+    } else if (u > 0) {
+        us = scan_rounds((double)N * p.nseg, K, d, cus) * (c.scan + c.scan_chunk * u);
+    } else {
+        const double cps = p.seg_len / rfa::kChunk;
+        us = gap + scan_rounds((double)N * (p.nseg - 1), K, d, cus) * (c.totals + c.totals_chunk * cps) + (p.prefixed ? 5 : 0) +
+             scan_rounds((double)N * p.nseg, K, d, cus) * (c.scan + c.scan_chunk * cps + c.slot * (p.prefixed ? 1 : p.nseg - 1));
+        moved *= 1.5;
+    }
+    return std::max(us, moved / 3.5e6);
+}
+
 double estimate_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cus) {
     const ScanCost c = scan_cost(K, d);
     const double nch = (double)((T + rfa::kChunk - 1) / rfa::kChunk), rows = (double)T * N, gap = 1.5;
-    auto rounds = [&](double wgs) {
-        const double full = std::max(1.0, std::ceil(wgs / cus));
-        return K == 64 && d == 64 ? 1.5 * std::floor(full / 2) + std::fmod(full, 2.0) : full;
-    };
-    double fwd, moved = rows * (K + d) * 4;
-    rfa::SegBounds b;
-    const double u = p.layout == LAYOUT_FINAL ? recompute_bounds(T, p.nseg, &b) : 0;
-    if (p.nseg == 1) {
-        fwd = rounds((double)N) * (c.scan + c.scan_chunk * nch);
-    } else if (u > 0) {
-        fwd = rounds((double)N * p.nseg) * (c.scan + c.scan_chunk * u);
-    } else {
-        const double cps = p.seg_len / rfa::kChunk;
-        fwd = gap + rounds((double)N * (p.nseg - 1)) * (c.totals + c.totals_chunk * cps) + (p.prefixed ? 5 : 0) +
-              rounds((double)N * p.nseg) * (c.scan + c.scan_chunk * cps + c.slot * (p.prefixed ? 1 : p.nseg - 1));
-        moved *= 1.5;
-    }
-    fwd = std::max(fwd, moved / 3.5e6);
+    const double fwd = forward_us(p, T, N, K, d, cus, p.layout == LAYOUT_FINAL);
     if (p.layout == LAYOUT_FINAL)
-        return fwd + std::max(rounds((double)N * (K + d) / rfa::kSliceWidth) * (c.slices + c.slices_chunk * nch), rows * (8 * K + 10 * d) / 2.5e6);
+        return fwd + std::max(scan_rounds((double)N * (K + d) / rfa::kSliceWidth, K, d, cus) * (c.slices + c.slices_chunk * nch),
+                              rows * (8 * K + 10 * d) / 2.5e6);
     int ratio;
     const ScanPlan pb = backward_plan(p, K, d, true, &ratio);
     const int split = K >= 256 && d >= 128 ? 2 : 1;      // workgroups of a sweep to a segment
     const double slots = pb.nseg > 1 ? (p.prefixed ? 1 : pb.nseg - 1) : 0;
-    return fwd + std::max(gap + (pb.prefixed ? 9 : 0) + rounds((double)N * pb.nseg * split) *
+    return fwd + std::max(gap + (pb.prefixed ? 9 : 0) + scan_rounds((double)N * pb.nseg * split, K, d, cus) *
                                     (c.sweeps + c.sweeps_chunk * (pb.seg_len / rfa::kChunk) + c.sweeps_slot * slots),
                           rows * 12 * (K + d) / 3.5e6);
 }
 
-// Layout and segments of a forward (with or without a saved buffer: the same bits) and of the backward that follows it:
+// Layout and segments of a forward that saves and of the backward that follows it:
 // cover_plan (always that with the "nseg" or "sliced" knob), unless another is estimated more than 8 % shorter.  What that finds, us forward + backward at
 // K = 128, d = 64, before / after: segments that spill into a second round of workgroups (T 1024, 72 sequences, 4 segments
 // -> 3) 67.1 / 55.1, raw (777, 72) 58.5 / 45.8; short sequences, where the sliced backward's one launch and the forward
 // without totals beat four launches however few CUs they cover (T 256, 16 sequences) 38.3 / 20.9; (512, 8) 41.3 / 27.6;
 // single chunks as segments (1024, 4) 49.2 / 41.2; fewer, longer segments (4096, 24) 141 / 108.
-ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
-    if (T <= 0 || N <= 0 || tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0) return cover_plan(T, N, K, d);
-    // called several times for one operation: the last answer of this thread, by all that goes into it
-    struct Memo { int64_t T, N; int K, d, cus; unsigned knobs; ScanPlan plan; };
-    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, {}};
-    const int cus = device_cus();
-    const unsigned knobs = tune::changes.load(std::memory_order_acquire);
-    if (memo.T == T && memo.N == N && memo.K == K && memo.d == d && memo.cus == cus && memo.knobs == knobs) return memo.plan;
-    const ScanPlan base = cover_plan(T, N, K, d);
+ScanPlan find_pair_plan(int64_t T, int64_t N, int K, int d, int cus, const ScanPlan& base) {
     const int64_t nchunks = (T + rfa::kChunk - 1) / rfa::kChunk;
     ScanPlan best = base;
     const double start = estimate_us(base, T, N, K, d, cus);
@@ -356,8 +357,54 @@ ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
             if (us < least) { least = us; best = p; }
         }
     }
-    memo = Memo{T, N, K, d, cus, knobs, least * 1.08 < start ? best : base};
-    return memo.plan;
+    return least * 1.08 < start ? best : base;
+}
+
+// Segments of a forward that no backward follows: cover_plan's or the pair's, whose choice weighs both directions, whichever is
+// estimated shorter for the forward alone; more segments than cover_plan's that rebuild their states only if 8 % shorter.
+// Scanned totals count with their bytes, written, scanned and read, here (a state of 32768 floats at twice the rate).
+// us at the pair's / cover_plan's, taken for cover_plan's: K 256, d 128 (T 777, 40 sequences) 53.2 / 45.4, (777, 128) 75.9 / 64.9;
+// K 64, d 128 (512, 320) 40.6 / 35.4, (777, 16) 18.8 / 13.4; K 128, d 128 (777, 16) 26.0 / 23.3; K 256, d 64 (512, 16) 26.8 / 25.3.
+// Taken for the pair's: K 128, d 128 (777, 40) 18.9 / 26.8; K 256, d 128 (777, 16) 35.0 / 40.2; K 64, d 64 (4096, 40) 30.6 /
+// 38.9; K 128, d 64 (192, 16) 6.7 / 9.4.
+ScanPlan forward_plan(const ScanPlan& pair, const ScanPlan& base, int64_t T, int64_t N, int K, int d, int cus, bool rebuilt) {
+    if (pair.nseg == base.nseg) return pair;
+    auto cost = [&](const ScanPlan& p) {
+        const double bytes = p.prefixed ? (double)N * p.nseg * K * d * 4 : 0;
+        return forward_us(p, T, N, K, d, cus, rebuilt) + bytes / (K * d >= 32768 ? 2e6 : 1e6);
+    };
+    return cost(pair) * (pair.nseg > base.nseg && !pair.prefixed ? 1.08 : 1) <= cost(base) ? pair : base;
+}
+
+bool rebuilds_states(int64_t N, int K, int d) {
+    return K <= 128 && (int64_t)rfa::kChunk * N * (K > d ? K : d) * 2 < ((int64_t)1 << 32);      // as launch_forward asks
+}
+
+struct ScanPlans {
+    ScanPlan pair;         // a forward that saves, and the backward that follows it
+    ScanPlan forward;      // a forward alone
+};
+
+// Asked for several times in one operation: the last answer of this thread, by all that goes into it.
+ScanPlans scan_plans(int64_t T, int64_t N, int K, int d) {
+    struct Memo { int64_t T, N; int K, d, cus; unsigned knobs; ScanPlans plans; };
+    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, {}};
+    const int cus = device_cus();
+    const unsigned knobs = tune::changes.load(std::memory_order_acquire);
+    if (memo.T == T && memo.N == N && memo.K == K && memo.d == d && memo.cus == cus && memo.knobs == knobs) return memo.plans;
+    const ScanPlan base = cover_plan(T, N, K, d);
+    const bool fixed = tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0;
+    const ScanPlan pair = fixed ? base : find_pair_plan(T, N, K, d, cus, base);
+    memo = Memo{T, N, K, d, cus, knobs, {pair, forward_plan(pair, base, T, N, K, d, cus, rebuilds_states(N, K, d))}};
+    return memo.plans;
+}
+
+ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
+    return T <= 0 || N <= 0 ? cover_plan(T, N, K, d) : scan_plans(T, N, K, d).pair;
+}
+
+ScanPlan make_forward_plan(int64_t T, int64_t N, int K, int d) {
+    return T <= 0 || N <= 0 ? cover_plan(T, N, K, d) : scan_plans(T, N, K, d).forward;
 }
 
 // ---- description of a saved-state buffer ---------------------------------------------
@@ -1317,7 +1364,7 @@ int rfa_selftest_mfma_rate(int waves_per_simd, int iters, float* sink, double* f
 
 size_t rfa_causal_forward_workspace_bytes(int64_t T, int64_t N, int K, int d) {
     if (T <= 0 || N <= 0 || !rfa_shape_supported(K, d)) return 0;
-    // of the forward that takes it and of the one on static memory
+    // of the forward that saves, of the one that does not (one of these two plans) and of the one on static memory
     return std::max(layout_workspace(T, N, K, d, make_plan(T, N, K, d), false).total,
                     layout_workspace(T, N, K, d, cover_plan(T, N, K, d), false).total);
 }
@@ -1430,10 +1477,12 @@ int rfa_causal_forward(const void* q, const void* k, const void* v, void* out, i
 
 size_t rfa_static_scratch_bytes(void) { return kStaticScratchBytes; }
 
-// the plan (and the bits) of rfa_causal_forward where its totals fit the static array
+// As make_forward_plan for a forward that always adds up totals, where they fit the static array: the plan, and the bits, of
+// an rfa_causal_forward that adds them up too ("recompute" 0).
 static ScanPlan noalloc_plan(int64_t T, int64_t N, int K, int d) {
-    const ScanPlan p = make_plan(T, N, K, d);
-    return layout_workspace(T, N, K, d, p, false).total <= kStaticScratchBytes ? p : cover_plan(T, N, K, d);
+    const ScanPlan base = cover_plan(T, N, K, d);
+    const ScanPlan p = forward_plan(make_plan(T, N, K, d), base, T, N, K, d, device_cus(), false);
+    return layout_workspace(T, N, K, d, p, false).total <= kStaticScratchBytes ? p : base;
 }
 
 int rfa_causal_forward_noalloc(const void* q, const void* k, const void* v, void* out, int64_t T, int64_t N,
@@ -1517,7 +1566,7 @@ static int causal_forward_impl(const void* q, const void* k, const void* v, void
                                bool allow_recompute) {
     if (int rc = check_causal_dims(T, N, K, d)) return rc;
     if (T == 0 || N == 0) return RFA_OK;
-    const ScanPlan p = allow_recompute ? make_plan(T, N, K, d) : noalloc_plan(T, N, K, d);
+    const ScanPlan p = !allow_recompute ? noalloc_plan(T, N, K, d) : want_saved ? make_plan(T, N, K, d) : make_forward_plan(T, N, K, d);
     int* savedHdr = nullptr;
     float* savedS = nullptr;
     float* savedZ = nullptr;

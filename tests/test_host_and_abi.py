@@ -189,6 +189,30 @@ def test_causal_plans(K, d):
     assert {s: ask(*s) for s in shapes} == first
 
 
+def _forward_state_bytes(lib, T, N, K, d):
+    """Bytes of segment states that rfa_causal_forward asks for, from its refusal of a NULL workspace; no launch is reached."""
+    import ctypes
+    import re
+    buf = ctypes.create_string_buffer(64)
+    ptr = (ctypes.addressof(buf) + 15) // 16 * 16
+    assert lib.rfa_causal_forward(ptr, ptr, ptr, ptr, T, N, K, d, None, 0, None) == -5
+    return int(re.search(r"workspace of (\d+) bytes", lib.rfa_last_error().decode()).group(1))
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="pointers that no kernel may see")
+@pytest.mark.parametrize("T,N,K,d,nseg", [(777, 40, 256, 128, 5), (777, 16, 64, 128, 5), (777, 16, 128, 128, 5), (512, 16, 256, 64, 4),
+                                          (777, 72, 128, 64, 3), (256, 2, 64, 64, 4), (1024, 40, 128, 128, 4)])
+def test_forward_alone_is_not_cut_for_a_backward(T, N, K, d, nseg):
+    """A forward that no backward follows: the cut that covers the chip where the pair's is longer for it (the first four), the
+    pair's otherwise.  (256 compute units.)"""
+    lib = _lib.load()
+    align = lambda n: (n + 255) // 256 * 256
+    want = align(4 * N * nseg * K * d) + align(4 * N * nseg * K)
+    assert _forward_state_bytes(lib, T, N, K, d) == want
+    lib.rfa_causal_num_segments(100, 3, K, d)                   # another shape between
+    assert _forward_state_bytes(lib, T, N, K, d) == want <= lib.rfa_causal_forward_workspace_bytes(T, N, K, d)
+
+
 def test_input_gradient_tiles_divide_their_widths():
     """Groups of waves take 32 columns each of every layer's width, whatever tile the sizes choose; around every line of the
     rule, the number of compute units in tiles (E_in = 128 of them) among them."""
