@@ -216,8 +216,8 @@ void cut_segments(ScanPlan* p, int64_t T, int64_t want, int K, int d) {
 }
 
 // Enough (sequence, segment) workgroups to cover the compute units, at least two chunks per segment, at most 16 segments:
-// what the pair without a saved buffer and the forward on static memory run with (their buffers are sized by it), and
-// where the choice of make_plan starts.
+// what the backward without a saved buffer runs with, what a forward on static memory falls back to (their buffers are
+// sized by it), and where the choices below start.
 ScanPlan cover_plan(int64_t T, int64_t N, int K, int d) {
     ScanPlan p{1, rfa::kChunk, 0, LAYOUT_SEGMENTS};
     if (T <= 0 || N <= 0) return p;
@@ -385,18 +385,24 @@ struct ScanPlans {
     ScanPlan forward;      // a forward alone
 };
 
-// Asked for several times in one operation: the last answer of this thread, by all that goes into it.
-ScanPlans scan_plans(int64_t T, int64_t N, int K, int d) {
+// Asked for several times in one operation, and by a model's layers in turn: the last answers of this thread, by all that
+// goes into them.  Host us: a found answer 0.15, a new one 1.1 (cover_plan alone 0.35).
+const ScanPlans& scan_plans(int64_t T, int64_t N, int K, int d) {
     struct Memo { int64_t T, N; int K, d, cus; unsigned knobs; ScanPlans plans; };
-    static thread_local Memo memo{-1, -1, 0, 0, 0, 0, {}};
+    constexpr int kMemos = 8;
+    static thread_local Memo memos[kMemos];      // zeros: no shape
+    static thread_local int next = 0;
     const int cus = device_cus();
     const unsigned knobs = tune::changes.load(std::memory_order_acquire);
-    if (memo.T == T && memo.N == N && memo.K == K && memo.d == d && memo.cus == cus && memo.knobs == knobs) return memo.plans;
+    for (const Memo& m : memos)
+        if (m.T == T && m.N == N && m.K == K && m.d == d && m.cus == cus && m.knobs == knobs) return m.plans;
+    Memo& m = memos[next];
+    next = (next + 1) % kMemos;
     const ScanPlan base = cover_plan(T, N, K, d);
     const bool fixed = tune::get(tune::NSEG) >= 1 || tune::get(tune::SLICED) >= 0;
     const ScanPlan pair = fixed ? base : find_pair_plan(T, N, K, d, cus, base);
-    memo = Memo{T, N, K, d, cus, knobs, {pair, forward_plan(pair, base, T, N, K, d, cus, rebuilds_states(N, K, d))}};
-    return memo.plans;
+    m = Memo{T, N, K, d, cus, knobs, {pair, forward_plan(pair, base, T, N, K, d, cus, rebuilds_states(N, K, d))}};
+    return m.plans;
 }
 
 ScanPlan make_plan(int64_t T, int64_t N, int K, int d) {
