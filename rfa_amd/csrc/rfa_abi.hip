@@ -1106,21 +1106,10 @@ int launch_weight_grad_reduce(const float* part, const float* bpart, const rfa::
 }
 
 // ---- feature map launchers ---------------------------------------------------------
-int feature_bwd_blocks(int64_t R, int H, int ntens = 1) {
-    const int64_t nrb = (R + 63) / 64;
-    int64_t target = 512;               // about two workgroups per CU; few partial sums to reduce
-    if (tune::get(tune::FEATURE_WG) >= 1) target = tune::get(tune::FEATURE_WG);
-    int64_t nblk = (target + (int64_t)H * ntens - 1) / ((int64_t)H * ntens);
-    if (nblk > nrb) nblk = nrb;
-    if (nblk < 1) nblk = 1;
-    return (int)nblk;
-}
-
 // Workgroups along x for the streaming feature-map kernels: eight waves each, a wave per group of
 // 16 rows, one workgroup per CU in all (their registers leave room for one; a second round of
 // workgroups would pay the staging of W' and, in the backward, the sum over the waves again);
-// more rows make the waves walk further.  Never more than feature_bwd_blocks, which sizes the
-// workspace of the backward's partial sums.
+// more rows make the waves walk further.
 int feature_stream_blocks(int64_t R, int H, int ntens, int waves = rfa::kFeatureWaves) {
     const int64_t ngrp = (R + 15) / 16, full = (ngrp + waves - 1) / waves;
     int64_t target = std::min(device_cus(), 512);
@@ -1129,6 +1118,14 @@ int feature_stream_blocks(int64_t R, int H, int ntens, int waves = rfa::kFeature
     if (nblk > full) nblk = full;
     if (nblk < 1) nblk = 1;
     return (int)nblk;
+}
+
+bool feature_shape_supported(int D, int d) { return (D == 32 || D == 64 || D == 128) && (d == 64 || d == 128); }
+
+// Bytes of the backward's partial sums: a dW' of a head from every workgroup.
+size_t feature_share_bytes(int64_t R, int H, int D, int d, int ntens) {
+    if (R <= 0 || H <= 0 || !feature_shape_supported(D, d)) return 0;
+    return (size_t)ntens * feature_stream_blocks(R, H, ntens, rfa::kFeatureBwdWaves) * H * D * d * 4;
 }
 
 template <int D, int DH>
@@ -1157,7 +1154,7 @@ int launch_feature_bwd(const rfa::half_t* x, const rfa::half_t* w, const rfa::ha
     const int ntens = x1 ? 2 : 1;       // two tensors through the same w: one launch, one reduction
     if (dx_rs == 0) dx_rs = (int64_t)H * DH;
     using Cfg = rfa::FeatureBwdCfg<D, DH>;
-    const int nblk = feature_stream_blocks(R, H, ntens, rfa::kFeatureBwdWaves);      // never more than feature_bwd_blocks, which sized the workspace
+    const int nblk = feature_stream_blocks(R, H, ntens, rfa::kFeatureBwdWaves);      // feature_share_bytes sized the workspace by it
     auto kern = rfa::k_feature_map_bwd<D, DH>;
     if (int rc = set_lds(kern, Cfg::kLds)) return rc;
     RFA_LAUNCH(FEATURE_BWD, kern, dim3(nblk, H, ntens), dim3(rfa::kFeatureBwdThreads), Cfg::kLds, st,
@@ -1184,8 +1181,6 @@ __global__ void k_zero_f32(float* p, int64_t n) {
 void zero_f32(float* p, int64_t n, hipStream_t st) {
     if (n > 0) RFA_LAUNCH(ZERO_FILL, k_zero_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n);
 }
-
-bool feature_shape_supported(int D, int d) { return (D == 32 || D == 64 || D == 128) && (d == 64 || d == 128); }
 
 int check_causal_dims(int64_t T, int64_t N, int K, int d) {
     if (T < 0 || N < 0 || K <= 0 || d <= 0)
@@ -2097,8 +2092,7 @@ int rfa_feature_map_forward_pair(const void* x0, const void* x1, const void* w, 
 }
 
 size_t rfa_feature_map_backward_workspace_bytes(int64_t R, int H, int D, int d) {
-    if (R <= 0 || H <= 0 || !feature_shape_supported(D, d)) return 0;
-    return (size_t)feature_bwd_blocks(R, H) * H * D * d * 4;
+    return feature_share_bytes(R, H, D, d, 1);
 }
 
 int rfa_feature_map_backward(const void* x, const void* w, const void* grad_phi, void* dx, float* dw, int64_t R,
@@ -2129,7 +2123,7 @@ int rfa_feature_map_backward(const void* x, const void* w, const void* grad_phi,
 }
 
 size_t rfa_feature_map_backward_pair_workspace_bytes(int64_t R, int H, int D, int d) {
-    return 2 * rfa_feature_map_backward_workspace_bytes(R, H, D, d);
+    return feature_share_bytes(R, H, D, d, 2);
 }
 
 int rfa_feature_map_backward_pair(const void* x0, const void* x1, const void* w, const void* grad_phi0,
@@ -2499,7 +2493,7 @@ static bool make_project_grads_plan(int64_t R, int H, int D, int d, int Ei, int 
         return false;
     const auto round = [](size_t n) { return (n + 255) / 256 * 256; };
     p->dy = round((size_t)R * H * d * 2);
-    p->feature = round((size_t)nphi * rfa_feature_map_backward_workspace_bytes(R, H, D, d));
+    p->feature = round(feature_share_bytes(R, H, D, d, nphi));
     p->bytes = nphi * p->dy + p->feature + linear_grads_bytes(p->linear, np, H * d, Ei);
     return true;
 }

@@ -213,6 +213,24 @@ def test_forward_alone_is_not_cut_for_a_backward(T, N, K, d, nseg):
     assert _forward_state_bytes(lib, T, N, K, d) == want <= lib.rfa_causal_forward_workspace_bytes(T, N, K, d)
 
 
+@pytest.mark.parametrize("R,H,D,d", [(8192, 8, 128, 128), (8192, 8, 64, 64), (1, 3, 32, 64), (130, 5, 128, 64), (100000, 40, 64, 128),
+                                     (4096, 600, 32, 128)])
+def test_feature_map_workspaces_hold_what_the_launch_writes(R, H, D, d):
+    """A dW' of a head from each of its workgroups, about one to a compute unit over both tensors of a pair together."""
+    lib = _lib.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available() else 256
+    for n, got in ((1, lib.rfa_feature_map_backward_workspace_bytes(R, H, D, d)),
+                   (2, lib.rfa_feature_map_backward_pair_workspace_bytes(R, H, D, d))):
+        blocks = max(1, min(-(-cus // (H * n)), -(-R // 128)))
+        assert got == 4 * n * blocks * H * D * d
+    e_in, layers = 1024, lib.rfa_linear_grads_workspace_bytes(R, H * d, 1024, 3)
+    if layers:
+        whole = lib.rfa_project_grads_workspace_bytes(R, H, D, d, e_in, 3, 2)
+        assert 0 <= whole - layers - got - 2 * 2 * R * H * d < 3 * 256
+    with _lib.tuning(feature_wg=H):
+        assert lib.rfa_feature_map_backward_workspace_bytes(R, H, D, d) == 4 * H * D * d
+
+
 def test_input_gradient_tiles_divide_their_widths():
     """Groups of waves take 32 columns each of every layer's width, whatever tile the sizes choose; around every line of the
     rule, the number of compute units in tiles (E_in = 128 of them) among them."""
