@@ -239,12 +239,11 @@ ScanPlan cover_plan(int64_t T, int64_t N, int K, int d) {
 // prefix plus scan then take every workgroup about equally long.  Pays while a sequence has few
 // segments (the last one streams nearly the whole sequence): up to 4 ("recompute" knob: 0 never,
 // 1 whenever the kernel exists).  Returns u, or 0 if no such cut exists.
-double recompute_bounds(int64_t T, int nseg, rfa::SegBounds* b) {
-    const int knob = tune::get(tune::RECOMPUTE);
-    if (knob == 0 || nseg < 2 || nseg > rfa::kMaxSegments || (knob < 0 && nseg > 4)) return 0;
+constexpr double kPrefixCost = 0.12;
+constexpr int kMostRebuilt = 4;
+
+double rebuilt_bounds(int64_t T, int nseg, double cost, rfa::SegBounds* b) {
     const int nch = (int)((T + rfa::kChunk - 1) / rfa::kChunk);
-    const int cost_knob = tune::get(tune::PREFIX_COST);
-    const double cost = (cost_knob >= 0 ? cost_knob : 12) / 100.0;
     double u = (double)nch / nseg;
     if (cost > 0 && cost < 1 && nch > 64) {
         // uncut, the segments add up to u (1 - (1 - cost)^nseg) / cost: no smaller u covers the sequence (segments of
@@ -268,6 +267,12 @@ double recompute_bounds(int64_t T, int nseg, rfa::SegBounds* b) {
     return 0;
 }
 
+double recompute_bounds(int64_t T, int nseg, rfa::SegBounds* b) {
+    const int knob = tune::get(tune::RECOMPUTE), cost = tune::get(tune::PREFIX_COST);
+    if (knob == 0 || nseg < 2 || nseg > rfa::kMaxSegments || (knob < 0 && nseg > kMostRebuilt)) return 0;
+    return rebuilt_bounds(T, nseg, cost >= 0 ? cost / 100.0 : kPrefixCost, b);
+}
+
 // What a forward + backward of the saving pair takes with a given plan, us: every launch is a number of rounds of workgroups,
 // one to a CU (two of K = d = 64), each a start plus its chunks of 64 steps, and none is faster than its bytes at
 // 3.5 TB/s (2.5 in the sliced backward).  A workgroup of segment totals costs `totals` + `totals_chunk` a chunk, one of
@@ -289,20 +294,21 @@ ScanCost scan_cost(int K, int d) {
                     : ScanCost{2.9, 5.4, 4.0, 1.5, 8.0, 0, 0, 6.0, 9.1, 15.0};
 }
 
-ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool have_saved, int* s_ratio);
+ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool longer, int* s_ratio);
 
 double scan_rounds(double wgs, int K, int d, int cus) {
     const double full = std::max(1.0, std::ceil(wgs / cus));
     return K == 64 && d == 64 ? 1.5 * std::floor(full / 2) + std::fmod(full, 2.0) : full;
 }
 
-// of a forward alone; rebuilt: by workgroups that rebuild their states from the rows before them, where the cut allows it
+// of a forward alone; rebuilt: by workgroups that rebuild their states from the rows before them, where the cut allows it (at
+// the default cost: "recompute" and "prefix_cost" move the launch, never the plan that a saved buffer is laid out by)
 double forward_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cus, bool rebuilt) {
     const ScanCost c = scan_cost(K, d);
     const double nch = (double)((T + rfa::kChunk - 1) / rfa::kChunk), gap = 1.5;
     double us, moved = (double)T * N * (K + d) * 4;
     rfa::SegBounds b;
-    const double u = rebuilt ? recompute_bounds(T, p.nseg, &b) : 0;
+    const double u = rebuilt && p.nseg > 1 && p.nseg <= kMostRebuilt ? rebuilt_bounds(T, p.nseg, kPrefixCost, &b) : 0;
     if (p.nseg == 1) {
         us = scan_rounds((double)N, K, d, cus) * (c.scan + c.scan_chunk * nch);
     } else if (u > 0) {
@@ -324,7 +330,7 @@ double estimate_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cu
         return fwd + std::max(scan_rounds((double)N * (K + d) / rfa::kSliceWidth, K, d, cus) * (c.slices + c.slices_chunk * nch),
                               rows * (8 * K + 10 * d) / 2.5e6);
     int ratio;
-    const ScanPlan pb = backward_plan(p, K, d, true, &ratio);
+    const ScanPlan pb = backward_plan(p, K, d, true, &ratio);      // as by default: "nseg_same" moves the backward alone
     const int split = K >= 256 && d >= 128 ? 2 : 1;      // workgroups of a sweep to a segment
     const double slots = pb.nseg > 1 ? (p.prefixed ? 1 : pb.nseg - 1) : 0;
     return fwd + std::max(gap + (pb.prefixed ? 9 : 0) + scan_rounds((double)N * pb.nseg * split, K, d, cus) *
@@ -377,7 +383,7 @@ ScanPlan forward_plan(const ScanPlan& pair, const ScanPlan& base, int64_t T, int
 }
 
 bool rebuilds_states(int64_t N, int K, int d) {
-    return K <= 128 && (int64_t)rfa::kChunk * N * (K > d ? K : d) * 2 < ((int64_t)1 << 32);      // as launch_forward asks
+    return tune::get(tune::RECOMPUTE) != 0 && K <= 128 && (int64_t)rfa::kChunk * N * (K > d ? K : d) * 2 < ((int64_t)1 << 32);      // as launch_forward asks
 }
 
 struct ScanPlans {
@@ -605,12 +611,12 @@ int launch_prefill_phi(const rfa::half_t* q, const rfa::half_t* k, const rfa::ha
 
 // The cut into segments the backward sweeps use for a forward plan pf.  Where both sweeps run as two
 // workgroups per (sequence, segment) and the totals are scanned, the backward takes segments twice
-// as long: half as many workgroups already cover the compute units, in one round instead of two.
-ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool have_saved, int* s_ratio) {
+// as long: half as many workgroups already cover the compute units, in one round instead of two.  (longer: it may, the
+// totals are saved and the "nseg_same" knob does not forbid it.)
+ScanPlan backward_plan(const ScanPlan& pf, int K, int d, bool longer, int* s_ratio) {
     ScanPlan p = pf;
     *s_ratio = 1;
-    if (K >= 256 && d >= 128 && have_saved && pf.prefixed && pf.nseg >= 4 && pf.nseg % 2 == 0 &&
-        tune::get(tune::NSEG_SAME) <= 0) {
+    if (K >= 256 && d >= 128 && longer && pf.prefixed && pf.nseg >= 4 && pf.nseg % 2 == 0) {
         p.nseg = pf.nseg / 2;
         p.seg_len = 2 * pf.seg_len;
         p.prefixed = use_scanned_totals(p.nseg, K, d) ? 1 : 0;      // of dR, dr
@@ -627,7 +633,7 @@ int launch_backward(const rfa::half_t* q, const rfa::half_t* k, const rfa::half_
                     hipStream_t st) {
     // pf is the forward's cut into segments (that of the saved totals)
     int s_ratio = 1;
-    const ScanPlan p = backward_plan(pf, KD, DH, savedS != nullptr, &s_ratio);
+    const ScanPlan p = backward_plan(pf, KD, DH, savedS && tune::get(tune::NSEG_SAME) <= 0, &s_ratio);
     const int prefixed_s = pf.prefixed;
     const int prefixed = p.prefixed;   // of dR, dr
     const rfa::PlanWords pw = plan_words(T, N, KD, DH, pf);

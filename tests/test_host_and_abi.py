@@ -189,6 +189,19 @@ def test_causal_plans(K, d):
     assert {s: ask(*s) for s in shapes} == first
 
 
+def test_saved_layout_does_not_follow_the_knobs_of_one_direction():
+    """"recompute" and "prefix_cost" move a forward's launch, "nseg_same" a backward's: buffers saved under one setting are laid
+    out as those of another expect them (a copy of a buffer is read by the current plan)."""
+    lib = _lib.load()
+    shapes = [(T, N, K, d) for T in (128, 256, 512, 777, 1024, 4096) for N in (2, 8, 16, 24, 40, 72, 300)
+              for K, d in ((64, 64), (128, 64), (64, 128), (128, 128), (256, 128))]
+    ask = lambda: [(lib.rfa_causal_num_segments(*s), lib.rfa_causal_saved_state_bytes(*s)) for s in shapes]
+    first = ask()
+    for knobs in ({"recompute": 0}, {"recompute": 1}, {"prefix_cost": 0}, {"prefix_cost": 60}, {"nseg_same": 1}):
+        with _lib.tuning(**knobs):
+            assert ask() == first, knobs
+
+
 def _forward_state_bytes(lib, T, N, K, d):
     """Bytes of segment states that rfa_causal_forward asks for, from its refusal of a NULL workspace; no launch is reached."""
     import ctypes
