@@ -82,8 +82,8 @@ int rfa_causal_forward(const void* q, const void* k, const void* v, void* out, i
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): no counterpart in the
  * reference.  Same kernels and results as rfa_causal_forward; the segment totals live in a static
  * device array of rfa_static_scratch_bytes() = 16 MiB that every GPU the library runs on holds
- * until the process ends.  The call allocates and frees nothing.  Shapes whose
- * rfa_causal_forward_workspace_bytes exceed the array return RFA_ERR_WORKSPACE.  All calls on one
+ * until the process ends.  The call allocates and frees nothing.  Shapes whose totals, in as many
+ * segments as cover the chip, exceed the array return RFA_ERR_WORKSPACE.  All calls on one
  * GPU share that GPU's array: calls that overlap in time on one GPU (two streams, two threads)
  * race; calls on one stream, one after the other, are fine (nothing in the array has to start
  * at zero: every total the scan reads is written earlier in the same call).  The first call on a

@@ -1496,7 +1496,8 @@ int rfa_causal_forward_noalloc(const void* q, const void* k, const void* v, void
                                int K, int d, void* stream) {
     if (int rc = check_causal_dims(T, N, K, d)) return rc;
     if (T == 0 || N == 0) return RFA_OK;
-    const size_t need = layout_workspace(T, N, K, d, noalloc_plan(T, N, K, d), false).total;
+    // by cover_plan, whatever the cut of this call: which shapes the array is for does not follow an estimate
+    const size_t need = layout_workspace(T, N, K, d, cover_plan(T, N, K, d), false).total;
     if (need > kStaticScratchBytes)
         return fail(RFA_ERR_WORKSPACE,
                     "rfa_causal_forward_noalloc: this shape needs %zu bytes of segment totals, the static scratch "

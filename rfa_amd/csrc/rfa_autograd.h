@@ -528,11 +528,10 @@ OptTensor node_linear(const Tensor& x, const Tensor& w, const OptTensor& b) {
     return LinearNode::apply(x, w, b);
 }
 
-// x W^T + b of n layers [e_out, e_in] side by side by the row kernel, where few_rows wants it and the tensors are as it takes them
+// x W^T + b of n layers [e_out, e_in] side by side by the row kernel (for few_rows), where the tensors are as it takes them
 OptTensor row_products(const Tensor& x, const Tensor* w, const OptTensor* b, int64_t n) {
     const int64_t e_out = w[0].size(0), e_in = w[0].size(1), R = e_in ? x.numel() / e_in : 0;
-    if (R < 1 || e_out == 0 || e_in % 32 != 0 || e_out % 16 != 0 || x.size(-1) != e_in || !x.is_contiguous() || !aligned16(x) ||
-        !few_rows(R, e_in, n * e_out, at::cuda::getDeviceProperties(x.get_device())->multiProcessorCount))
+    if (R < 1 || e_out == 0 || e_in % 32 != 0 || e_out % 16 != 0 || x.size(-1) != e_in || !x.is_contiguous() || !aligned16(x))
         return c10::nullopt;
     std::array<const void*, 3> wp{}, bp{};
     for (int64_t p = 0; p < n; ++p) {
@@ -674,7 +673,8 @@ public:
         if (capturing) {      // few rows: the layers where they are, the bits of their stack
             const std::array<Tensor, 3> w{*wq, *wk, *wv};
             const std::array<OptTensor, 3> b{bq, bk, bv};
-            y = row_products(x, w.data(), b.data(), 3);
+            if (few_rows(x.size(0) * x.size(1), E, 3 * E, at::cuda::getDeviceProperties(x.get_device())->multiProcessorCount))
+                y = row_products(x, w.data(), b.data(), 3);
         }
         if (!y.has_value()) {
             if (!c.layer_sources.same(ls, 0)) {

@@ -213,6 +213,17 @@ def _forward_state_bytes(lib, T, N, K, d):
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="pointers that no kernel may see")
+@pytest.mark.parametrize("T,N,K,d", [(256, 131, 128, 128), (777, 40, 256, 128), (4096, 72, 128, 128), (8192, 254, 256, 128)])
+def test_forward_on_static_memory_refuses_by_the_cut_that_covers_the_chip(T, N, K, d):
+    """Totals of those segments past the static array are refused, also where another cut's would fit.  (256 compute units.)"""
+    import ctypes
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(64)
+    ptr = (ctypes.addressof(buf) + 15) // 16 * 16
+    assert lib.rfa_causal_forward_noalloc(ptr, ptr, ptr, ptr, T, N, K, d, None) == -5
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="pointers that no kernel may see")
 @pytest.mark.parametrize("T,N,K,d,nseg", [(777, 40, 256, 128, 5), (777, 16, 64, 128, 5), (777, 16, 128, 128, 5), (512, 16, 256, 64, 4),
                                           (777, 72, 128, 64, 3), (256, 2, 64, 64, 4), (1024, 40, 128, 128, 4)])
 def test_forward_alone_is_not_cut_for_a_backward(T, N, K, d, nseg):
