@@ -141,8 +141,9 @@ int rfa_causal_backward_saved(const void* q, const void* k, const void* v, const
  * case its kernels compare the header in the buffer with the plan they run, on the device: on a
  * mismatch dq, dk, dv are filled with NaN rather than computed from totals laid out
  * for another plan.  rfa_causal_backward_saved_workspace_bytes is the workspace that call needs
- * for a given saved buffer (= rfa_causal_backward_workspace_bytes unless the knobs changed since
- * the forward).  rfa_causal_saved_describe copies the 16 header ints to host memory and waits
+ * for a given saved buffer: that of the buffer's own plan, 0 where it holds the final state.  (At most
+ * rfa_causal_backward_workspace_bytes, which covers every plan of a backward, unless the knobs changed since
+ * the forward.)  rfa_causal_saved_describe copies the 16 header ints to host memory and waits
  * for the stream (a debugging aid).  No counterpart in the reference. */
 size_t rfa_causal_backward_saved_workspace_bytes(const void* saved, int64_t T, int64_t N, int K, int d);
 /* Rows [T, B] of `width` halves (a multiple of 8) with the padded ones zero: a copy of src to dst, or with
@@ -152,8 +153,8 @@ int rfa_mask_rows(const void* src, void* dst, const uint8_t* pad, int64_t stride
                   int64_t B, int64_t width, void* stream);
 int rfa_causal_saved_describe(const void* saved, int32_t* words16, void* stream);
 
-/* Number of time segments the causal kernels cut a sequence into for the given
- * shape on the current device (>= 1). */
+/* Number of time segments that a saving forward, and the backward behind it, cut a sequence into for the given
+ * shape on the current device (>= 1); a forward that no backward follows may take another number. */
 int rfa_causal_num_segments(int64_t T, int64_t N, int K, int d);
 
 /* Launch-heuristic overrides for sweeps and tests (process-wide; -1 restores the heuristic):
@@ -165,19 +166,18 @@ int rfa_causal_num_segments(int64_t T, int64_t N, int K, int d);
  *             with two groups of waves that share the tile's contraction (0 has two as well)
  *             (the name is older than the meaning: it chose between two kernels, of which one is left)
  *   "sliced"  1/0: rfa_causal_forward_save writes the final-state layout, whose backward is one
- *             launch that walks whole sequences by state slices (K <= 128; taken by itself at
- *             d = 64 when the slices cover 45 % of the compute units, at d = 128 only with K = 128
- *             and 90 %) / the
- *             segment-totals layout of the two-sweep backward
+ *             launch that walks whole sequences by state slices (K <= 128) / the segment-totals layout
+ *             of the two-sweep backward.  Unset: whichever, with the number of segments, is estimated
+ *             shorter for both directions; set, as "nseg", it also keeps the number of segments that covers the chip
  *   "recompute"  1/0: the forward with K <= 128 runs as one launch without segment totals (every
  *             workgroup rebuilds the state at its segment's first step from the k, v rows before
  *             it; segments of unequal length) whenever no backward wants the totals / never.
  *             Unset: for up to 4 segments.  Its output has the bits of the one-segment scan.
  *   "prefix_cost"  cost of a rebuilt 64-step block in percent of a scanned one (default 12): moves
  *             the cut of that forward into segments
- *   "feature_wg"  workgroups the feature-map kernels aim for (default: one per compute unit for the
- *             eight-wave streaming kernels, 512 for the row-block backward of the wide shapes; in
- *             the backward each leaves one partial dW' for the reduction)
+ *   "feature_wg"  workgroups the feature-map kernels aim for (default: one per compute unit over all
+ *             heads and tensors of a launch; in the backward each leaves one partial dW' for the reduction)
+ * "recompute", "prefix_cost" and "nseg_same" move one direction's launch and leave the layout of saved buffers alone.
  * Initial values come from the environment variables RFA_HIP_<NAME>, read once per process and
  * never on the launch path.  No counterpart in the reference. */
 int rfa_tuning_set(const char* name, int value);

@@ -339,8 +339,8 @@ double estimate_us(const ScanPlan& p, int64_t T, int64_t N, int K, int d, int cu
 }
 
 // Layout and segments of a forward that saves and of the backward that follows it:
-// cover_plan (always that with the "nseg" or "sliced" knob), unless another is estimated more than 8 % shorter.  What that finds, us forward + backward at
-// K = 128, d = 64, before / after: segments that spill into a second round of workgroups (T 1024, 72 sequences, 4 segments
+// cover_plan (always that with the "nseg" or "sliced" knob), unless another is estimated more than 8 % shorter.  What that finds, device us forward + backward
+// at K = 128, d = 64, before / after: segments that spill into a second round of workgroups (T 1024, 72 sequences, 4 segments
 // -> 3) 67.1 / 55.1, raw (777, 72) 58.5 / 45.8; short sequences, where the sliced backward's one launch and the forward
 // without totals beat four launches however few CUs they cover (T 256, 16 sequences) 38.3 / 20.9; (512, 8) 41.3 / 27.6;
 // single chunks as segments (1024, 4) 49.2 / 41.2; fewer, longer segments (4096, 24) 141 / 108.
@@ -1036,7 +1036,8 @@ int launch_input_grad(const rfa::InputGradArgs& ga, rfa::half_t* dx, int R, int 
 }
 
 // As the projections, with four groups for 64 rows where the contraction is 768 or longer.  Groups of waves share a
-// stage of 32 columns each, so they are for widths that they divide; other widths take one group.
+// stage of 32 columns each, so they are for widths that they divide; other widths take one group.  (The package's layers come
+// here past make_linear_grads_plan's sizes, mostly to 128 and 256 rows by one group, and with unaligned tensors at any.)
 // Measured, us for 64 rows by one group / two / four, 128 by one / two, 256:
 // 512 rows of 512 -> 512 7.8 / 6.8 / 7.0 / 10.2 / 8.9 / 14.8; 512 of 3 x 512 17.5 / 12.9 / 11.6 / 22.5 / 16.7 / 32.2; 2048 of
 // 3 x 1024 32.7 / 23.9 / 21.9 / 41.4 / 29.6 / 58.6; 4096 of 3 x 768 31.9 / 27.5 / 31.7 / 33.5 / 25.4 / 46.0; 8192 of 512 11.2 /

@@ -10,7 +10,7 @@
 // What bounds a layer without this is the host.  The Python functions over the same kernels (input gradients by the
 // library there) / these nodes, us: a layer of 8 heads of 64, 8192 tokens, forward + backward, 212 of kernels, 487 / 237;
 // 128 tokens of 4 heads, the scan alone, 125 / 75; an encoder-decoder layer, 16384 + 8192 rows, 611 / 324; a decoding step of
-// 64 sequences 71 / 28.
+// 64 sequences 71 / 23.
 #pragma once
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContextLight.h>
